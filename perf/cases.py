@@ -245,11 +245,11 @@ class Restore:
                 self.group.wait_layer(layer)
         return self.words
 
-    def __del__(self):
+    def __del__(self, close_fd=os.close):  # bound here: the module may go first
         if hasattr(self, "group"):
             self.group.close()
         for fd in getattr(self, "fds", ()):
-            os.close(fd)
+            close_fd(fd)
 
 
 _lanes = None
