@@ -134,6 +134,39 @@ hipError_t quiet_event_wait(hipEvent_t event, int device, int64_t expected_ns) {
   }
 }
 
+hipError_t quiet_word_wait(const uint64_t *word, uint64_t at_least, hipEvent_t behind, int device) {
+  auto there = [&] { return __atomic_load_n(word, __ATOMIC_ACQUIRE) >= at_least; };
+  const int setting = policy_peek(device).quiet_wait_us;
+  const int limit_us = setting < 0 ? -setting : setting;
+  Waiting here;
+  // who may keep a core busy looks all the time, as with the runtime's own waits
+  const bool spin = setting == 0 || (setting > 0 && here.others < kRuntimeWaits);
+  const auto close_until = std::chrono::steady_clock::now() + std::chrono::microseconds(30);
+  int nap_us = 20;
+  for (unsigned looks = 1;; ++looks) {
+    if (there())
+      return hipSuccess;
+    bool ask = looks % 4096 == 0;
+    if (!spin && looks % 16 == 0 && std::chrono::steady_clock::now() >= close_until) {
+      std::this_thread::sleep_for(std::chrono::microseconds(nap_us));
+      nap_us = std::min(nap_us * 2, std::max(1, limit_us));
+      ask = true;
+    } else {
+      __builtin_ia32_pause();
+    }
+    if (!ask)
+      continue;
+    const hipError_t q = hipEventQuery(behind); // the kernel may have ended in an error
+    if (q == hipErrorNotReady) {
+      (void)hipGetLastError();
+    } else if (q != hipSuccess) {
+      return q;
+    } else {
+      return there() ? hipSuccess : hipErrorUnknown;
+    }
+  }
+}
+
 hipError_t quiet_stream_wait(hipStream_t stream, int device) {
   constexpr int kMaxDevices = 64;
   const int setting = device < 0 || device >= kMaxDevices ? 0 : policy_peek(device).quiet_wait_us;
@@ -762,6 +795,27 @@ int kernel_plan_launch(const KernelPlan &p, int layer_offset, int num_layers,
   if (!p.no_alloc) // the bookkeeping creates events on first use
     link_direction_mark(p.device, p.h2d, stream,
                         (int64_t)p.num_blocks * num_layers * p.kv_dim * p.chunk_size);
+  return FKV_OK;
+}
+
+bool layers_launch_fits(const KernelPlan &p) {
+  // What fkv_copy_layers_kernel is built for: 16-byte vectors, chunks of a slice at least
+  // (shorter ones need the packed form), every base address in one LDS table, single
+  // wavefronts, and a counter to claim from.
+  return layers_device && p.h2d && p.host_visible && p.vec == 16 &&
+         p.chunk_size >= (int64_t)64 * kCopyUnroll * 16 && p.num_layers * p.kv_dim <= kCopyMaxLK &&
+         p.threads == 64 && p.claims && !p.no_alloc && !p.recorded;
+}
+
+int kernel_plan_launch_layers(const KernelPlan &p, int layers_per_batch, LayersLaunch t,
+                              hipStream_t stream) {
+  const int64_t bytes = (int64_t)p.num_blocks * p.num_layers * p.kv_dim * p.chunk_size;
+  t.a = plan_job(p, 0, p.num_layers);
+  t.pairs_per_batch = layers_per_batch * p.kv_dim;
+  t.batches = (p.num_layers + layers_per_batch - 1) / layers_per_batch;
+  const int workgroups = shape_for_now(p, bytes, stream, &t.a);
+  FKV_TRY(layers_device->launch(t, workgroups, stream));
+  link_direction_mark(p.device, p.h2d, stream, bytes);
   return FKV_OK;
 }
 

@@ -36,6 +36,9 @@ void pooled_stream_release(int device, bool non_blocking, hipStream_t stream);
 // thread behind what the stream holds and waits for that.
 hipError_t quiet_event_wait(hipEvent_t event, int device, int64_t expected_ns = 0);
 hipError_t quiet_stream_wait(hipStream_t stream, int device);
+// The same for a word in pinned host memory that a kernel raises to `at_least` before
+// `behind`, recorded behind the kernel, is reached.
+hipError_t quiet_word_wait(const uint64_t *word, uint64_t at_least, hipEvent_t behind, int device);
 // For the catch-all handler of an entry point: turns the exception in flight into a status
 // and an error text.  No C++ exception crosses the C ABI.
 int caught(const char *where) noexcept;
@@ -198,6 +201,34 @@ struct CopyJobs {
 };
 int launch_copy_jobs(const CopyKernelArgs *jobs, int njobs, int num_workgroups,
                      int threads_per_workgroup, hipStream_t stream);
+// ---- a layerwise restore in one launch -------------------------------------
+// Layers [0, a.lk / kv_dim) of a plan in batches of `pairs_per_batch` (layer, kv) pairs (the
+// last one may be shorter), copied in order by one kernel that announces each batch as it
+// lands; see fkv_copy_layers_kernel.
+struct LayersLaunch {
+  CopyKernelArgs a;
+  int32_t pairs_per_batch;
+  int32_t batches;
+  int32_t ranges;          // claims per batch, set by the launch
+  uint32_t *arrived;       // device, [batches]: ranges that have landed; zero between launches
+  uint64_t *landed;        // device, [batches]: `epoch` once the batch has landed
+  uint64_t *landed_host;   // the same in pinned host memory
+  uint64_t *tick_host;     // pinned, [batches]: when it landed, in ticks of the 100 MHz clock
+  uint64_t epoch;          // larger than that of any earlier launch
+};
+// What of it runs on the device.  A table instead of two functions because the library's host
+// code also runs without its kernels (over the emulated runtime of the sanitizer tests, where
+// the table stays empty and restores are launched batch by batch).
+struct LayersDevice {
+  int (*launch)(LayersLaunch t, int num_workgroups, hipStream_t stream);
+  // Makes `stream` wait until *landed (device `device`; `landed_host` is the same word in
+  // pinned memory) has reached `epoch`.  `overdue` (pinned) becomes 1 when that took longer
+  // than half a minute and the wait ended all the same.  `behind` lies behind the launch: a
+  // stream that is being captured is handed to it, and refused as ever.
+  int (*wait)(const uint64_t *landed, const uint64_t *landed_host, uint64_t epoch, uint64_t *overdue,
+              int device, hipEvent_t behind, hipStream_t stream);
+};
+extern const LayersDevice *layers_device;
 // Ranges of work that safety-net workgroups (see the kernel) have copied on the
 // current device since the process started; reads a device counter.
 uint64_t safety_net_ranges_of_current_device();
@@ -307,6 +338,11 @@ int kernel_plan_build(const fkv_transfer_desc &d, hipStream_t stream, KernelPlan
 // Enqueues the copy of layers [layer_offset, layer_offset + num_layers) of the plan.
 int kernel_plan_launch(const KernelPlan &p, int layer_offset, int num_layers,
                        hipStream_t stream);
+// All layers of the plan in one launch, `layers_per_batch` at a time; `t` brings the words
+// that announce the batches.  Only for plans layers_launch_fits accepts.
+bool layers_launch_fits(const KernelPlan &p);
+int kernel_plan_launch_layers(const KernelPlan &p, int layers_per_batch, LayersLaunch t,
+                              hipStream_t stream);
 // The same for layer ranges of several plans of one direction in one launch (the
 // members of one original layer of a multi-group restore); falls back to one launch
 // per plan where the plans cannot share one.
@@ -378,12 +414,13 @@ struct StagedPlan {
 // `batch_layers`) goes through the copy engines on the current device and, if so,
 // sizes the ring and uploads the tables on `scatter_stream`.  FKV_OK with
 // out->usable == false: use the kernel path.
+// `one_launch`: on the kernel path the restore would be a single launch;
 // `host_visible`: the device can read the host pool (else only the gathered route is open);
 // `kernel_allowed`: the caller lets batches go by kernel (the first batch of a gathered restore).
 int staged_plan_build(const fkv_transfer_desc &d, int batch_layers, StagedRing &ring,
                       GatherRing &pinned, hipStream_t scatter_stream, StagedPlan *out,
                       bool host_visible = true, bool kernel_allowed = true,
-                      bool several_gpus = false);
+                      bool several_gpus = false, bool one_launch = false);
 // The choice alone (no device): kRouteKernel, kRouteRuns (fills `segs` and `total_rows`)
 // or kRouteGathered.
 // `free_commands`: up to so many copy commands a batch are taken whatever the batch's size.

@@ -722,6 +722,224 @@ int launch_copy_jobs(const CopyKernelArgs *jobs, int njobs, int num_workgroups,
   }
 }
 
+#if defined(__HIP__) // not in the CPU model of the device: one workgroup at a time, no fences
+namespace {
+// A layerwise restore in one launch: every batch of layers, in order, announced as it lands.
+//
+// A launch a batch is bound by what lies around the launches: 8 us between two of them on a
+// stream, a ramp and a tail each, and 20 us of host time for a launch, its event and the
+// consumer's wait, next to 5 us (256 KiB) to 18 us (1 MiB) of link time.  Here the wavefronts
+// claim ranges of 64 KiB that run through all batches, so the link never drains between two
+// of them, and a batch costs the host nothing.
+//
+// A batch has landed when all its ranges are counted.  A range is counted behind a release
+// fence, which also waits for its stores; that, the answer of the counter and the next claim
+// are looked at when the first vectors of the following range have arrived, a round trip over
+// the link later, when they have long come back.  (Counted right behind its stores, with the
+// claim read through LDS, a range cost the wavefront 3 us more: 0.95 against 0.88 ms for 32
+// layers of 1 MiB with 16 wavefronts.)  Write-through stores instead of the fence measured
+// slower: 0.75 against 0.71 ms with 24 wavefronts.  Whoever counts the last range of a batch
+// writes its epoch to a word in device memory, which streams wait for, and one in pinned
+// memory, which the host looks at.
+//
+// Whole restores, the forward stream waiting for every layer (us, a launch a batch -> this):
+// 8 x 256 KiB to eventfds 164 -> 76, 32 x 1 MiB 774 -> 667, 61 x 7 MiB 9086 (rows gathered by
+// host threads) -> 7844, which is 55 GB/s.  Next to a fused attention of 76 us a layer:
+// 32 x 1 MiB 2956 -> 2822, 61 x 7 MiB 10383 -> 8122.
+__global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) {
+  using V = VecType<16>::type;
+  __shared__ uint64_t s_base_src[kCopyMaxLK], s_base_dst[kCopyMaxLK];
+  __shared__ int64_t s_off_src[kCopyIdTile], s_off_dst[kCopyIdTile];
+  __shared__ uint32_t s_claim;
+  const CopyKernelArgs &a = t.a;
+  Shares shares(a);
+  if (!shares.enter(&s_claim))
+    return;
+  const int lane = threadIdx.x;
+  constexpr int64_t kSliceBytes = (int64_t)kWave * kCopyUnroll * 16;
+  const uint32_t slices = (uint32_t)a.slices_per_chunk;
+  uint32_t tile = 0; // first of the block positions whose offsets are in LDS
+  auto load_tile = [&](uint32_t at) {
+    __syncthreads();
+    const uint32_t n = min((uint32_t)kCopyIdTile, (uint32_t)a.num_blocks - at);
+    for (uint32_t i = lane; i < n; i += kWave) {
+      s_off_src[i] = a.ids_src[at + i] * a.stride_src;
+      s_off_dst[i] = a.ids_dst[at + i] * a.stride_dst;
+    }
+    __syncthreads();
+    tile = at;
+  };
+  for (int i = lane; i < a.lk; i += kWave) {
+    s_base_src[i] = a.base_src[i];
+    s_base_dst[i] = a.base_dst[i];
+  }
+  load_tile(0);
+
+  // The batch whose range this wavefront has copied but not counted yet, and the one whose
+  // count is under way (-1: none).
+  int copied = -1, counted = -1;
+  uint32_t before = 0; // lane 0: ranges of `counted` that had landed before
+  auto announce = [&] { // whoever counted the last range of a batch
+    if (lane == 0 && counted >= 0 && before + 1 == (uint32_t)t.ranges) {
+      t.arrived[counted] = 0;
+      t.tick_host[counted] = (uint64_t)wall_clock64();
+      __hip_atomic_store(t.landed + counted, t.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(t.landed_host + counted, t.epoch, __ATOMIC_RELEASE,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    counted = -1;
+  };
+  auto count = [&] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); // the stores of the range, out of this XCD's L2
+    if (lane == 0)
+      before = __hip_atomic_fetch_add(t.arrived + copied, 1u, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
+    counted = copied;
+    copied = -1;
+  };
+  auto drain = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
+  // The claim after the current one; a safety-net workgroup claims none ahead of time.
+  auto claim_ahead = [&]() -> uint32_t {
+    const uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane((int)shares.next_claim);
+    if (lane == 0 && c < a.num_claims)
+      shares.next_claim = shares.claim_one();
+    return c;
+  };
+  auto claim_now = [&]() -> uint32_t {
+    uint32_t c, all;
+    return shares.next(&s_claim, &c, &all) ? c : a.num_claims;
+  };
+  uint32_t part = shares.safety_net ? claim_now() : claim_ahead();
+  while (part < a.num_claims) {
+    uint32_t ahead = a.num_claims;
+    const uint32_t batch = part / (uint32_t)t.ranges, range = part - batch * (uint32_t)t.ranges;
+    const uint32_t pair0 = batch * (uint32_t)t.pairs_per_batch;
+    const uint32_t pairs = min((uint32_t)t.pairs_per_batch, (uint32_t)a.lk - pair0);
+    const uint32_t spp = pairs * slices;
+    const uint64_t units = (uint64_t)a.num_blocks * spp;
+    const uint64_t s0 = units * range / (uint32_t)t.ranges;
+    const uint64_t s1 = units * (range + 1) / (uint32_t)t.ranges;
+    for (uint64_t s = s0; s < s1; ++s) {
+      const uint32_t p = (uint32_t)(s / spp);
+      const uint32_t r = (uint32_t)(s - (uint64_t)p * spp);
+      const uint32_t i = r / slices, sl = r - i * slices;
+      if (p - tile >= (uint32_t)kCopyIdTile) // behind the tile, or before it (wraps)
+        load_tile(p / kCopyIdTile * kCopyIdTile);
+      const int64_t off = (int64_t)sl * kSliceBytes;
+      const int64_t left = a.chunk_bytes - off;
+      const int nvec = (int)((left < kSliceBytes ? left : kSliceBytes) / 16);
+      const V *src = reinterpret_cast<const V *>(s_base_src[pair0 + i] +
+                                                 (uint64_t)s_off_src[p - tile] + off);
+      V *dst = reinterpret_cast<V *>(s_base_dst[pair0 + i] + (uint64_t)s_off_dst[p - tile] + off);
+      V v[kCopyUnroll];
+#pragma unroll
+      for (int u = 0; u < kCopyUnroll; ++u)
+        v[u] = __builtin_nontemporal_load(src + min(u * kWave + lane, nvec - 1));
+      // The vectors come from the other end of the link, so by the time they are here every
+      // store of the range before has completed, and the answers of the two counters have come:
+      // nothing is waited for that is not there.
+      if (s == s0 || counted >= 0)
+        drain();
+      announce();
+      if (s == s0) {
+        if (copied >= 0)
+          count();
+        if (!shares.safety_net)
+          ahead = claim_ahead();
+      }
+#pragma unroll
+      for (int u = 0; u < kCopyUnroll; ++u)
+        if (u * kWave + lane < nvec)
+          __builtin_nontemporal_store(v[u], dst + u * kWave + lane);
+    }
+    copied = (int)batch;
+    part = shares.safety_net ? claim_now() : ahead;
+  }
+  drain();
+  announce();
+  if (copied >= 0)
+    count();
+  announce();
+}
+
+__global__ void fkv_wait_landed_kernel(const uint64_t *landed, uint64_t epoch, uint64_t *overdue,
+                                       long long ticks) {
+  if (threadIdx.x != 0)
+    return;
+  const long long t0 = wall_clock64();
+  // relaxed: what the stream runs next starts with an acquire of its own
+  while (__hip_atomic_load(landed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) < epoch) {
+    if (wall_clock64() - t0 > ticks) {
+      __hip_atomic_store(overdue, (uint64_t)1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+      return;
+    }
+    __builtin_amdgcn_s_sleep(8);
+  }
+}
+
+int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
+  int64_t total = 0;
+  int grid_pct = 100;
+  FKV_TRY(prepare_job(t.a, &total, &grid_pct));
+  if (total == 0 || t.a.packed || t.a.vec != 16 || !t.a.claim || t.batches < 1)
+    return fail(FKV_ERR_RUNTIME, "copy kernel: a restore of this shape has no single launch");
+  int64_t grid = 1;
+  int threads = kWave;
+  // Half as many workgroups again as for a plain copy: the fence behind every range takes a
+  // wavefront out for a few microseconds (32 layers of 1 MiB: 16 wavefronts 881 us, 24 713, 32
+  // 677; next to a fused attention 2858 / 2822 / 2854).
+  shape_launch(t.a, total, (int64_t)t.a.num_blocks * t.a.lk * t.a.chunk_bytes, grid_pct * 3 / 2,
+               num_workgroups, kWave, &grid, &threads);
+  // Ranges of 64 KiB, or smaller ones where a batch would not go round the workgroups; none
+  // is empty, also in the last batch, which may be shorter than the others.
+  const int64_t per_pair = (int64_t)t.a.num_blocks * t.a.slices_per_chunk;
+  const int64_t last_pairs = t.a.lk - (int64_t)(t.batches - 1) * t.pairs_per_batch;
+  const int64_t ranges = std::min(per_pair * last_pairs,
+                                  std::max(grid, per_pair * t.pairs_per_batch / 8));
+  if (last_pairs < 1 || ranges * t.batches > (int64_t)INT32_MAX)
+    return fail(FKV_ERR_RUNTIME, "copy kernel: %d batches of %d of %d (layer, kv) pairs", t.batches,
+                t.pairs_per_batch, t.a.lk);
+  t.ranges = (int32_t)ranges;
+  t.a.num_claims = (uint32_t)(ranges * t.batches);
+  hipLaunchKernelGGL(fkv_copy_layers_kernel, dim3((unsigned)grid), dim3(kWave), 0, stream, t);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess)
+    return fail(FKV_ERR_RUNTIME, "copy kernel launch failed: %s", hipGetErrorString(e));
+  return FKV_OK;
+}
+
+int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t epoch,
+                uint64_t *overdue, int device, hipEvent_t behind, hipStream_t stream) {
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
+    (void)hipGetLastError();
+    capture = hipStreamCaptureStatusActive; // let the event decide
+  }
+  if (capture != hipStreamCaptureStatusNone) {
+    FKV_HIP_TRY(hipStreamWaitEvent(stream, behind, 0));
+    return FKV_OK;
+  }
+  if (__atomic_load_n(landed_host, __ATOMIC_ACQUIRE) >= epoch)
+    return FKV_OK; // it is there: whatever the stream gets next finds it
+  // a consumer on another GPU looks at the word in host memory
+  int of_stream = -1;
+  if (stream)
+    FKV_HIP_TRY(hipStreamGetDevice(stream, &of_stream));
+  DeviceGuard guard(of_stream);
+  if (!guard.ok())
+    return fail(FKV_ERR_RUNTIME, "cannot select the device of the consumer's stream");
+  constexpr long long kHalfMinute = 30ll * 100000000;
+  hipLaunchKernelGGL(fkv_wait_landed_kernel, dim3(1), dim3(kWave), 0, stream,
+                     guard.device() == device ? landed : landed_host, epoch, overdue, kHalfMinute);
+  FKV_HIP_TRY(hipGetLastError());
+  return FKV_OK;
+}
+
+const LayersDevice kLayersDevice{launch_layers, wait_landed};
+[[maybe_unused]] const bool layers_device_set = (layers_device = &kLayersDevice, true);
+} // namespace
+#endif
+
 } // namespace fkv
 
 // ---- what HBM delivers to a streaming kernel ---------------------------------

@@ -41,6 +41,7 @@
 #include <sys/eventfd.h>
 #include <unistd.h>
 
+#include <algorithm>
 #include <exception>
 #include <atomic>
 #include <condition_variable>
@@ -50,7 +51,70 @@
 #include <mutex>
 #include <thread>
 
+namespace fkv {
+const LayersDevice *layers_device = nullptr; // set where the kernels are part of the library
+}
+
 namespace {
+
+// The words by which a restore in one launch tells how far it is (see LayersLaunch): device
+// memory and pinned host memory of one group and GPU.  Taken from a pool per device and given
+// back when the group ends; never freed, because a consumer's stream may still hold a wait on
+// them when the group is gone (it finds its epoch reached: a later user's is larger).
+struct LandedWords {
+  uint64_t *dev = nullptr;  // [kCopyMaxLK] landed, then uint32_t [kCopyMaxLK] arrived
+  uint64_t *host = nullptr; // [kCopyMaxLK] landed, [kCopyMaxLK] ticks, overdue
+  uint32_t *arrived() const { return reinterpret_cast<uint32_t *>(dev + fkv::kCopyMaxLK); }
+  uint64_t *ticks() const { return host + fkv::kCopyMaxLK; }
+  uint64_t *overdue() const { return host + 2 * fkv::kCopyMaxLK; }
+};
+struct LandedPool {
+  std::mutex mu;
+  std::map<int, std::vector<LandedWords>> idle;
+};
+LandedPool &landed_pool() {
+  static LandedPool *p = new LandedPool(); // lives until the process ends
+  return *p;
+}
+// `device` is current.
+bool landed_words_acquire(int device, LandedWords *out) {
+  LandedPool &p = landed_pool();
+  {
+    std::lock_guard<std::mutex> lk(p.mu);
+    std::vector<LandedWords> &v = p.idle[device];
+    if (!v.empty()) {
+      *out = v.back();
+      v.pop_back();
+      return true;
+    }
+  }
+  constexpr size_t kDev = (size_t)fkv::kCopyMaxLK * 12, kHost = ((size_t)fkv::kCopyMaxLK * 2 + 1) * 8;
+  static const std::vector<uint8_t> zeros(kDev, 0);
+  void *d = nullptr, *h = nullptr;
+  if (hipHostMalloc(&h, kHost, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess ||
+      hipMalloc(&d, kDev) != hipSuccess ||
+      hipMemcpy(d, zeros.data(), kDev, hipMemcpyHostToDevice) != hipSuccess) {
+    (void)hipGetLastError();
+    if (d)
+      (void)hipFree(d);
+    if (h)
+      (void)hipHostFree(h);
+    return false;
+  }
+  std::memset(h, 0, kHost);
+  out->dev = static_cast<uint64_t *>(d);
+  out->host = static_cast<uint64_t *>(h);
+  return true;
+}
+void landed_words_release(int device, const LandedWords &w) {
+  if (!w.dev)
+    return;
+  LandedPool &p = landed_pool();
+  std::lock_guard<std::mutex> lk(p.mu);
+  p.idle[device].push_back(w);
+}
+// Numbers of the launches: each is larger than any before it in this process.
+std::atomic<uint64_t> g_layers_epoch{0};
 
 bool is(const char *a, const char *b) { return std::strcmp(a, b) == 0; }
 
@@ -207,6 +271,14 @@ struct fkv_layerwise {
     double trace_bytes = 0;
   };
   std::vector<std::unique_ptr<Batch>> batches;
+  // The whole restore is one launch that announces its batches itself: of the batch events
+  // only the last one exists, and `landed` says how far the launch is.
+  bool one_launch = false;
+  uint64_t epoch = 0;
+  std::vector<LandedWords> landed; // per GPU, taken on first use
+  bool has_landed(int b, int g) const {
+    return __atomic_load_n(landed[g].host + b, __ATOMIC_ACQUIRE) >= epoch;
+  }
   std::vector<int> layer_batch; // layer -> index into batches, -1: nothing in flight
   hipEvent_t started = nullptr; // on streams[0], before the first batch
   int counter_id = 0;
@@ -249,17 +321,26 @@ struct fkv_layerwise {
   }
 
   int poll_batches() {
+    unsigned looks = 0;
     return fkv::poll_batches_in_order(
         batches.size(), num_gpus, (int)hipSuccess, (int)hipErrorNotReady,
-        [this](size_t b, int g) {
+        [this, &looks](size_t b, int g) {
           // an event that has not been recorded yet reads as complete
           const int state = gate.peek((int)b);
           if (state <= 0)
             return (int)(state < 0 ? hipErrorLaunchFailure : hipErrorNotReady);
+          if (one_launch) {
+            if (has_landed((int)b, g))
+              return (int)hipSuccess;
+            if (++looks % 1024 != 0) // now and then: has the launch ended in an error?
+              return (int)hipErrorNotReady;
+          }
           (void)hipSetDevice(device_ids[g]);
-          const hipError_t e = hipEventQuery(batches[b]->done[g]);
+          const hipError_t e = hipEventQuery(one_launch ? batches.back()->done[g] : batches[b]->done[g]);
           if (e != hipSuccess)
             (void)hipGetLastError();
+          else if (one_launch && !has_landed((int)b, g))
+            return (int)hipErrorUnknown;
           return (int)e;
         },
         [this](size_t b) { notify(*batches[b]); }, poller_stop);
@@ -305,10 +386,29 @@ struct fkv_layerwise {
                        "%s: the previous layerwise restore failed while it was launched: %s", where,
                        feed_error.c_str());
     }
+    for (const LandedWords &w : landed)
+      if (w.host && __atomic_exchange_n(w.overdue(), (uint64_t)0, __ATOMIC_ACQ_REL))
+        return fkv::fail(FKV_ERR_RUNTIME, "%s: a consumer of the previous layerwise restore waited half "
+                         "a minute for its layer and went on without it", where);
     if (e == 0)
       return FKV_OK;
     return fkv::fail(FKV_ERR_RUNTIME, "%s: the previous layerwise restore failed on the device: %s",
                      where, hipGetErrorString((hipError_t)e));
+  }
+
+  // When batch `b` had landed on the first GPU, in ms after the restore began.
+  hipError_t batch_ms(int b, float *ms) const {
+    const hipError_t e =
+        hipEventElapsedTime(ms, started, (one_launch ? batches.back() : batches[b])->done[0]);
+    if (e != hipSuccess || !one_launch)
+      return e;
+    // The last one to land is what the event saw; the others by the device's own clock, each
+    // no earlier than the ones before it, which are announced first.
+    const uint64_t *t = landed[0].ticks();
+    const uint64_t end = *std::max_element(t, t + batches.size());
+    const uint64_t then = *std::max_element(t, t + b + 1);
+    *ms = std::max(0.0f, *ms - (float)((double)(end - then) / 1e5));
+    return e;
   }
 
   // Ends the notification machinery of the previous transfer and frees its
@@ -373,6 +473,7 @@ int finish_create(std::unique_ptr<fkv_layerwise> &g, const int64_t *gpu_device_i
   g->dma_turn.assign(g->num_gpus, 0u);
   g->alt_streams.assign(g->num_gpus, nullptr);
   g->alt_join.assign(g->num_gpus, nullptr);
+  g->landed.assign(g->num_gpus, LandedWords{});
   for (int i = 0; i < g->num_gpus; ++i) {
     hipError_t e = hipSetDevice(g->device_ids[i]);
     if (e == hipSuccess)
@@ -431,6 +532,57 @@ fkv_transfer_desc describe(const fkv_layerwise *g, const Lane &lane, int gpu, in
   return d;
 }
 
+// Fewer batches than this and the call is bound by the host's launches, not by the gaps
+// between them on the device (8 batches of 256 KiB: 0.15 ms either way).
+constexpr int kAltMinBatches = 12;
+// Batches up to this size alternate where nobody chose a size (kernel_alt_stream_kb = -1).
+constexpr int kAltDefaultKb = 4096;
+
+// Whether the kernel path of the restore that is being set up is one launch on GPU `i`: a
+// single lane (the jobs of several groups and of a sidecar share the launches of the batches),
+// more than one batch, a plan of a shape the kernel takes.  It is the faster way wherever it
+// can be had (batches of 112 / 464 KiB / 1 MiB / 7 MiB, 40 / 40 / 32 / 61 layers, the forward
+// stream waiting for each: 0.62 -> 0.20, 0.64 -> 0.47, 0.79 -> 0.71, 8.6 -> 7.8 ms).
+bool fits_one_launch(const fkv_layerwise *g, const std::vector<Lane> &lanes, int i) {
+  using namespace fkv;
+  if (!layers_device || g->multi_group || g->batches.size() < 2 || !lanes[0].used)
+    return false;
+  for (size_t k = 1; k < lanes.size(); ++k)
+    if (lanes[k].used)
+      return false;
+  const fkv_launch_policy pol = policy_of(g->device_ids[i]);
+  // tests of a restore that ends part-way, and callers who asked for batches on two streams
+  if (pol.test_fail_restore_batch > 0 ||
+      (pol.kernel_alt_stream_kb > 0 && (int)g->batches.size() >= kAltMinBatches))
+    return false;
+  return layers_launch_fits(lanes[0].plans[i]);
+}
+
+// All batches of the restore in one launch per GPU.
+int launch_layers_at_once(fkv_layerwise *g, std::vector<Lane> &lanes) {
+  using namespace fkv;
+  Lane &lane = lanes[0];
+  const int num_batches = (int)g->batches.size();
+  for (int i = 0; i < g->num_gpus; ++i) {
+    (void)hipSetDevice(g->device_ids[i]);
+    const KernelPlan &plan = lane.plans[i];
+    LayersLaunch t{};
+    t.arrived = g->landed[i].arrived();
+    t.landed = g->landed[i].dev;
+    t.landed_host = g->landed[i].host;
+    t.tick_host = g->landed[i].ticks();
+    t.epoch = g->epoch;
+    FKV_TRY(kernel_plan_launch_layers(plan, g->batches[0]->layers, t, g->streams[i]));
+    FKV_HIP_TRY(hipEventRecord(g->batches.back()->done[i], g->streams[i]));
+    stats().calls.fetch_add((uint64_t)num_batches, std::memory_order_relaxed);
+    stats().bytes_h2d.fetch_add((uint64_t)plan.num_blocks * plan.num_layers * plan.kv_dim *
+                                    (uint64_t)plan.chunk_size,
+                                std::memory_order_relaxed);
+  }
+  g->gate.publish(num_batches);
+  return FKV_OK;
+}
+
 // Enqueues every batch of the restore that is being set up, in order, records the batch
 // events and hands the plan memory back; `rc` is the status of the set-up so far (a
 // failed set-up enqueues nothing).  Runs on the calling thread, or on the group's
@@ -445,15 +597,13 @@ int launch_batches(fkv_layerwise *g, std::vector<Lane> &lanes, const EngineChoic
   const bool direct = choice.use_ce_transfer == 0;
   const int num_batches = (int)g->batches.size();
   const int give_up_at = policy_of(g->device_ids[0]).test_fail_restore_batch; // tests only
-  // Fewer batches than this and the call is bound by the host's launches, not by the gaps
-  // between them on the device (8 batches of 256 KiB: 0.15 ms either way).
-  constexpr int kAltMinBatches = 12;
   std::vector<char> two_dma_streams(g->num_gpus);
   std::vector<int64_t> alt_max_bytes(g->num_gpus, 0); // batches by kernel up to this size alternate
   for (int i = 0; i < g->num_gpus; ++i) {
     const fkv_launch_policy pol = policy_of(g->device_ids[i]);
     two_dma_streams[i] = pol.staged_dma_streams >= 2;
-    if (!direct || pol.kernel_alt_stream_kb <= 0 || num_batches < kAltMinBatches || rc != FKV_OK)
+    const int alt_kb = pol.kernel_alt_stream_kb < 0 ? kAltDefaultKb : pol.kernel_alt_stream_kb;
+    if (!direct || g->one_launch || alt_kb <= 0 || num_batches < kAltMinBatches || rc != FKV_OK)
       continue;
     (void)hipSetDevice(g->device_ids[i]);
     if (!g->alt_streams[i] &&
@@ -468,11 +618,13 @@ int launch_batches(fkv_layerwise *g, std::vector<Lane> &lanes, const EngineChoic
       g->alt_join[i] = nullptr;
       continue;
     }
-    alt_max_bytes[i] = (int64_t)pol.kernel_alt_stream_kb * 1024;
+    alt_max_bytes[i] = (int64_t)alt_kb * 1024;
   }
   std::vector<char> alt_used(g->num_gpus, 0);
   try { // an exception ends the launches like an error: the plans below are given back either way
-    for (int b = 0; b < num_batches && rc == FKV_OK; ++b) {
+    if (rc == FKV_OK && g->one_launch)
+      rc = launch_layers_at_once(g, lanes);
+    for (int b = 0; b < num_batches && rc == FKV_OK && !g->one_launch; ++b) {
       if (give_up_at > 0 && b == give_up_at - 1) {
         rc = fail(FKV_ERR_RUNTIME, "layerwise restore made to give up before batch %d (test_fail_restore_batch)", b);
         break;
@@ -922,12 +1074,6 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
     }
   }
   const int num_batches = (int)g->batches.size();
-  for (auto &b : g->batches)
-    for (int i = 0; i < g->num_gpus; ++i) {
-      FKV_HIP_TRY(hipSetDevice(g->device_ids[i]));
-      // a restore writes device memory only: no system-scope fence (see kBookkeepingEvent)
-      FKV_HIP_TRY(hipEventCreateWithFlags(&b->done[i], kTimingEventNoFence));
-    }
   FKV_HIP_TRY(hipSetDevice(g->device_ids[0]));
   FKV_HIP_TRY(hipEventCreateWithFlags(&g->started, kTimingEventNoFence));
   FKV_HIP_TRY(hipEventRecord(g->started, g->streams[0]));
@@ -968,7 +1114,8 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
         rc = staged_plan_build(d, g->multi_group ? 1 : c.layer_granularity,
                                g->rings[{lane_index, i}], g->pinned_rings[{lane_index, i}],
                                g->streams[i], &lane.staged[i], lane.plans[i].host_visible,
-                               /*kernel_allowed=*/direct, /*several_gpus=*/g->num_gpus > 1);
+                               /*kernel_allowed=*/direct, /*several_gpus=*/g->num_gpus > 1,
+                               /*one_launch=*/direct && fits_one_launch(g, lanes, i));
         if (rc == FKV_OK && lane.staged[i].usable && !g->dma_streams[i]) {
           hipError_t e = pooled_stream_acquire(g->device_ids[i], true, &g->dma_streams[i]);
           if (e != hipSuccess) {
@@ -996,6 +1143,30 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
   } catch (...) {
     rc = caught("plans of a layerwise restore");
   }
+  // The batch events; with everything in one launch only the last batch has one, and the words
+  // it is announced by.
+  g->one_launch = rc == FKV_OK && direct;
+  for (int i = 0; i < g->num_gpus && g->one_launch; ++i)
+    g->one_launch = fits_one_launch(g, lanes, i) && !lanes[0].staged[i].usable;
+  if (g->one_launch) {
+    g->epoch = g_layers_epoch.fetch_add(1, std::memory_order_relaxed) + 1;
+    for (int i = 0; i < g->num_gpus && g->one_launch; ++i) {
+      (void)hipSetDevice(g->device_ids[i]);
+      if (!g->landed[i].dev)
+        g->one_launch = landed_words_acquire(g->device_ids[i], &g->landed[i]);
+    }
+  }
+  for (int b = g->one_launch ? num_batches - 1 : 0; b < num_batches && rc == FKV_OK; ++b)
+    for (int i = 0; i < g->num_gpus && rc == FKV_OK; ++i) {
+      hipError_t e = hipSetDevice(g->device_ids[i]);
+      // a restore writes device memory only: no system-scope fence (see kBookkeepingEvent)
+      if (e == hipSuccess)
+        e = hipEventCreateWithFlags(&g->batches[b]->done[i], kTimingEventNoFence);
+      if (e != hipSuccess) {
+        (void)hipGetLastError();
+        rc = fail(FKV_ERR_RUNTIME, "event of a layerwise restore: %s", hipGetErrorString(e));
+      }
+    }
   // Staging memory that several restores in a row had no use for goes back (a group
   // with many lanes would otherwise hold buffers for every route it ever took).
   constexpr int kRingIdleCalls = 8;
@@ -1091,7 +1262,11 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
         return launch_failure();
       for (int i = 0; i < g->num_gpus; ++i) {
         (void)hipSetDevice(g->device_ids[i]);
-        hipError_t e = quiet_event_wait(g->batches[b]->done[i], g->device_ids[i], 0);
+        hipError_t e =
+            g->one_launch
+                ? quiet_word_wait(g->landed[i].host + b, g->epoch, g->batches.back()->done[i],
+                                  g->device_ids[i])
+                : quiet_event_wait(g->batches[b]->done[i], g->device_ids[i], 0);
         if (e != hipSuccess) {
           (void)hipGetLastError();
           (void)hipSetDevice(restore.device());
@@ -1102,7 +1277,10 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
       g->notify(*g->batches[b]);
     }
     g->join_feeder();
-    for (int i = 0; i < g->num_gpus; ++i) { // csrc/layerwise.cpp:1249-1256, 1634-1642
+    // Every batch of a single launch has been seen to land: nothing is left to wait for, unless
+    // the times of its event are asked for.
+    for (int i = 0; i < g->num_gpus && (!g->one_launch || c.enable_trace);
+         ++i) { // csrc/layerwise.cpp:1249-1256, 1634-1642
       (void)hipSetDevice(g->device_ids[i]);
       hipError_t e = quiet_stream_wait(g->streams[i], g->device_ids[i]);
       if (e != hipSuccess) {
@@ -1119,7 +1297,7 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
       float prev = 0;
       for (int b = 0; b < num_batches; ++b) {
         float ms = 0;
-        if (hipEventElapsedTime(&ms, g->started, g->batches[b]->done[0]) != hipSuccess) {
+        if (g->batch_ms(b, &ms) != hipSuccess) {
           (void)hipGetLastError();
           continue;
         }
@@ -1199,6 +1377,11 @@ int fkv_layerwise_wait_layer(fkv_layerwise *g, int32_t gpu_index, int32_t layer,
   if (!g->gate.wait(b))
     return fail(FKV_ERR_RUNTIME, "layer %d will not land: the restore failed while it was launched",
                 layer);
+  if (g->one_launch)
+    return layers_device->wait(g->landed[gpu_index].dev + b, g->landed[gpu_index].host + b, g->epoch,
+                               g->landed[gpu_index].overdue(), g->device_ids[gpu_index],
+                               g->batches.back()->done[gpu_index],
+                               static_cast<hipStream_t>(consumer_stream));
   FKV_HIP_TRY(hipStreamWaitEvent(static_cast<hipStream_t>(consumer_stream),
                                  g->batches[b]->done[gpu_index], 0));
   return FKV_OK;
@@ -1351,7 +1534,7 @@ int fkv_layerwise_batch_times_ms(fkv_layerwise *g, float *out_ms, int32_t capaci
     return fail(FKV_ERR_RUNTIME, "fkv_layerwise_batch_times_ms: the restore was not launched completely");
   DeviceGuard restore(g->device_ids[0]);
   for (int b = 0; b < (int)g->batches.size() && b < capacity; ++b)
-    FKV_HIP_TRY(hipEventElapsedTime(&out_ms[b], g->started, g->batches[b]->done[0]));
+    FKV_HIP_TRY(g->batch_ms(b, &out_ms[b]));
   return FKV_OK;
 } catch (...) {
   return fkv::caught(__func__);
@@ -1386,6 +1569,8 @@ void fkv_layerwise_destroy(fkv_layerwise *g) {
         (void)hipEventDestroy(g->alt_join[i]);
     }
     fkv::pooled_stream_release(g->device_ids[i], true, g->streams[i]);
+    if (i < (int)g->landed.size())
+      landed_words_release(g->device_ids[i], g->landed[i]);
   }
   (void)hipSetDevice(restore.device());
   (void)hipGetLastError();

@@ -170,7 +170,7 @@ void sanitize(fkv_launch_policy &p, const fkv_launch_policy &derived) {
   p.staged_scatter_threads = clampi(p.staged_scatter_threads, 64, kCopyBlockThreads);
   p.test_fail_restore_batch = clampi(p.test_fail_restore_batch, 0, 1 << 20);
   p.staged_dma_streams = clampi(p.staged_dma_streams, 1, 2);
-  p.kernel_alt_stream_kb = clampi(p.kernel_alt_stream_kb, 0, 1 << 20);
+  p.kernel_alt_stream_kb = clampi(p.kernel_alt_stream_kb, -1, 1 << 20);
   p.quiet_wait_us = clampi(p.quiet_wait_us, -10000, 10000);
 }
 
@@ -240,7 +240,7 @@ fkv_launch_policy defaults_for(uint32_t present) {
   p.model_seeded = 0;
   p.staged_scatter_threads = 256;
   p.staged_dma_streams = 2;
-  p.kernel_alt_stream_kb = 4096;
+  p.kernel_alt_stream_kb = -1;
   p.quiet_wait_us = 100;
   for (const EnvField &f : kEnv) {
     const char *v = std::getenv(f.name);

@@ -265,7 +265,8 @@ int64_t staged_row_of(const std::vector<StagedPlan::Seg> &segs, int64_t id) {
 
 int staged_plan_build(const fkv_transfer_desc &d, int batch_layers, StagedRing &ring,
                       GatherRing &pinned, hipStream_t scatter_stream, StagedPlan *out,
-                      bool host_visible, bool kernel_allowed, bool several_gpus) {
+                      bool host_visible, bool kernel_allowed, bool several_gpus,
+                      bool one_launch) {
   *out = StagedPlan{};
   int device = 0;
   FKV_HIP_TRY(hipGetDevice(&device));
@@ -306,6 +307,19 @@ int staged_plan_build(const fkv_transfer_desc &d, int batch_layers, StagedRing &
   }
   out->route = staged_route(d.cpu_block_ids, d.num_blocks, batch_row_bytes, pieces, pol, &out->segs,
                             &total_rows, free_commands);
+  // Where the alternative is one launch for the whole restore, gathered rows are left for
+  // batches long enough to hide what they cost the link: 15-25 us between two copies.
+  // Measured (72 KiB rows, 30 layers, gathered against one launch): 96 rows a layer 4.65 /
+  // 3.90 ms, 192 rows 8.3 / 7.8, 288 rows 12.1 / 11.5, 384 rows 15.9 / 15.3; next to a fused
+  // attention of 76 us a layer (61 layers, 96 rows) 10.4 / 8.1 ms.  Longer batches leave the
+  // compute units to the forward pass, as before.
+  constexpr double kGatherHandOverUs = 24;
+  if (out->route == kRouteGathered && pol.staged_gather == 1 && one_launch && host_visible &&
+      kernel_allowed) {
+    const double link_us = (double)total_rows * (double)batch_row_bytes / std::max(1, pol.model_link_mbps);
+    if (kGatherHandOverUs > link_us * pol.staged_overhead_pct / 100.0)
+      out->route = kRouteKernel;
+  }
   if (out->route == kRouteKernel)
     return FKV_OK;
   const bool gathered = out->route == kRouteGathered;

@@ -1,0 +1,111 @@
+"""A layerwise restore that goes out as one launch announcing its batches itself: bytes against
+the oracle, the layers a gated consumer sees, the eventfds, batch times, at the sizes where the
+cut into batches, ranges and slices can go wrong."""
+import os
+
+import numpy as np
+import pytest
+import torch
+
+from kvsetup import KVSetup, SGLANG, TRTLLM, VLLM
+
+pytestmark = pytest.mark.gpu
+
+# engine, layers, kv, chunk, blocks, layers per batch
+SHAPES = [
+    (VLLM, 2, 1, 8192, 1, 1),           # a slice a batch: fewer than workgroups
+    (VLLM, 5, 2, 8208, 7, 2),           # a vector behind the slice, a short last batch
+    (VLLM, 9, 1, 18432, 33, 1),         # 8 + 8 + 2 KiB
+    (SGLANG, 4, 2, 73728, 3, 3),
+    (TRTLLM, 3, 2, 16384, 129, 1),
+    (VLLM, 3, 1, 8192, 1025, 2),        # more blocks than an id tile, above the home-XCD size
+    (VLLM, 600, 1, 8192, 2, 7),         # many batches
+]
+POLICIES = dict(default={}, confined=dict(arbiter=2), safety_net=dict(arbiter=3),
+                everywhere=dict(arbiter=0))
+
+
+def restore(grp, s, gids, cids, gran, notify):
+    e = torch.empty(0, dtype=torch.int64)
+    grp.layerwise_transfer(
+        e, e, 0, 0, 0, 0, 0, torch.as_tensor(gids), torch.as_tensor(cids), s.cpu_kv_stride,
+        s.cpu_layer_stride, s.cpu_block_stride, s.chunk, s.cpu_kv_stride, s.cpu_layer_stride,
+        s.cpu_block_stride, 4, False, s.num_layers, gran, s.kv_dim, 1, counter_id=0,
+        kv_shared_across_ranks_mode="sharded", notify_mode=notify)
+
+
+@pytest.mark.parametrize("policy", list(POLICIES))
+@pytest.mark.parametrize("backend,layers,kv,chunk,n,gran", SHAPES)
+def test_restore_in_one_launch(gpu_device, backend, layers, kv, chunk, n, gran, policy):
+    from flexkv_amd.c_ext import LayerwiseTransferGroup, get_stats, launch_policy, reset_stats
+    from flexkv_amd.transfer.eventfd_channel import make_eventfd
+    pool = n + 5
+    s = KVSetup(backend, layers, kv, pool, pool, chunk, "BLOCKFIRST", seed=chunk + n)
+    dev = s.to_device(gpu_device)
+    fds = [make_eventfd() for _ in range(layers)]
+    i64 = lambda v: torch.tensor([v], dtype=torch.int64)  # noqa: E731
+    grp = LayerwiseTransferGroup(
+        num_gpus=1, gpu_blocks=[dev.gpu], cpu_blocks=dev.host, ssd_files={}, num_layers=layers,
+        gpu_kv_strides_tensor=i64(s.gpu_kv_stride), gpu_block_strides_tensor=i64(s.gpu_block_stride),
+        gpu_layer_strides_tensor=i64(s.gpu_layer_stride), gpu_chunk_sizes_tensor=i64(s.chunk),
+        iouring_entries=0, iouring_flags=0,
+        layer_eventfds_tensor=torch.tensor(fds, dtype=torch.int32), tp_size=1, is_blockfirst=True)
+    rng = np.random.default_rng(n)
+    consumer = torch.cuda.Stream()
+    for rep, notify in enumerate(("polling", "hostfunc", "polling")):
+        fresh = rng.integers(0, 256, s.host_bytes, dtype=np.uint8)
+        s.host_ref[:] = fresh
+        dev.host.copy_(torch.from_numpy(fresh))
+        gids = rng.permutation(pool)[:n].astype(np.int64)
+        cids = rng.permutation(pool)[:n].astype(np.int64)
+        per_layer = backend == VLLM and layers <= 16
+        seen = []
+        with launch_policy(staged_restore=0, staged_gather=0, **POLICIES[policy]):
+            reset_stats()
+            torch.cuda.synchronize()
+            restore(grp, s, gids, cids, gran, notify)
+            with torch.cuda.stream(consumer):
+                for l in range(layers):
+                    grp.wait_layer(l, consumer)
+                    if per_layer:
+                        seen.append(dev.gpu[l].clone())
+            grp.synchronize()
+            consumer.synchronize()
+            assert get_stats()["kernel_launches"] == 1
+        s.oracle_transfer(gids, cids, True)
+        dev.assert_matches_reference(f"restore {rep}")
+        for l, t in enumerate(seen):  # what the consumer saw of layer l is all of it
+            assert torch.equal(t, dev.gpu[l]), (rep, l)
+        for l, fd in enumerate(fds):
+            os.set_blocking(fd, False)
+            assert int.from_bytes(os.read(fd, 8), "little") == 1, (rep, l)
+        times = grp.batch_times_ms()
+        assert len(times) == -(-layers // gran) and times[0] >= 0
+        assert all(b >= a for a, b in zip(times, times[1:]))
+    grp.close()
+
+
+def test_shapes_that_go_batch_by_batch(gpu_device):
+    """Packed chunks and odd vector widths keep a launch a batch."""
+    from flexkv_amd.c_ext import get_stats, launch_policy, reset_stats
+    from flexkv_amd.c_ext import LayerwiseTransferGroup
+    i64 = lambda v: torch.tensor([v], dtype=torch.int64)  # noqa: E731
+    for chunk in (2304, 8200):
+        s = KVSetup(VLLM, 3, 1, 9, 9, chunk, "BLOCKFIRST", seed=chunk)
+        dev = s.to_device(gpu_device)
+        grp = LayerwiseTransferGroup(
+            num_gpus=1, gpu_blocks=[dev.gpu], cpu_blocks=dev.host, ssd_files={}, num_layers=3,
+            gpu_kv_strides_tensor=i64(s.gpu_kv_stride),
+            gpu_block_strides_tensor=i64(s.gpu_block_stride),
+            gpu_layer_strides_tensor=i64(s.gpu_layer_stride),
+            gpu_chunk_sizes_tensor=i64(s.chunk), iouring_entries=0, iouring_flags=0,
+            layer_eventfds_tensor=torch.empty(0, dtype=torch.int32), tp_size=1, is_blockfirst=True)
+        ids = np.arange(9, dtype=np.int64)[::-1].copy()
+        with launch_policy(staged_restore=0, staged_gather=0):
+            reset_stats()
+            restore(grp, s, ids, ids, 1, "hostfunc")
+            assert get_stats()["kernel_launches"] == 3
+        grp.synchronize()
+        s.oracle_transfer(ids, ids, True)
+        dev.assert_matches_reference(f"chunk {chunk}")
+        grp.close()
