@@ -164,8 +164,9 @@ struct CopyKernelArgs {
   int32_t slices_per_chunk;
   int32_t vec;      // 16, 8, 4, 2 or 1: widest access all addresses allow
   int32_t nt_store; // 1: nontemporal stores (destination in HBM), 0: plain (pinned host)
-  int32_t unroll;   // vector accesses in flight per lane: kCopyUnroll (also for 0), or
-                    // kCopyUnrollDeep where launch_copy_kernel finds the launch fit for it
+  int32_t unroll;   // 0: the host link bounds the launch; kCopyUnroll or kCopyUnrollDeep: HBM
+                    // does, and so many vectors per lane, if launch_copy_kernel finds it fit
+  int32_t per_slice; // set by launch_copy_kernel: HBM bounds it, see fkv_copy_slices_kernel
   int32_t packed;   // set by launch_copy_kernel: chunks shorter than a slice, see the kernel
   int32_t lane_runs; // stores into pinned host memory: a lane moves adjacent vectors (see copy_slice)
   int32_t packed_grid_pct; // workgroups to launch in packed mode, percent of the request (0 = 100)

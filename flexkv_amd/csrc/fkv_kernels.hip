@@ -58,6 +58,9 @@ namespace fkv {
 namespace {
 
 constexpr int kWave = 64;
+constexpr int kSliceWgThreads = 256; // workgroup of fkv_copy_slices_kernel
+constexpr size_t kSliceLdsBytes = 53 * 1024; // three workgroups fit the 160 KiB of a CU
+constexpr int64_t kSliceFewWgBytes = 64ll << 20;
 
 template <int VEC> struct VecType;
 template <> struct VecType<16> { typedef unsigned int type __attribute__((ext_vector_type(4))); };
@@ -300,7 +303,7 @@ __device__ __forceinline__ void copy_share(const CopyKernelArgs &a, uint64_t num
     const uint64_t t0 = s0 > tile_s0 ? s0 : tile_s0;
     const uint64_t tile_s1 = tile_s0 + (uint64_t)n * spp;
     const uint64_t t1 = s1 < tile_s1 ? s1 : tile_s1;
-    if (UNR == kCopyUnroll && a.packed) { // never with deep unroll: its chunks are whole slices
+    if (a.packed) {
       using V = typename VecType<VEC>::type;
       const uint32_t lim = (uint32_t)(t1 - tile_s0); // < kCopyIdTile * spp, checked on host
       const uint32_t ulk = (uint32_t)a.lk;
@@ -386,6 +389,53 @@ __global__ __launch_bounds__(kCopyBlockThreads) void fkv_copy_chunks_kernel(
   }
 }
 
+// A value that is the same for a whole wavefront, where the compiler cannot see it.
+__device__ __forceinline__ uint32_t wave_uniform(uint32_t v) {
+#if defined(__HIP__)
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+#else // the CPU model of the device: every work-item has its own
+  return v;
+#endif
+}
+
+// Launches that HBM bounds (both ends in device memory): a wavefront looks its slice up in the
+// tables, moves it and is done; nothing is staged, and no workgroup waits for itself.
+//
+// Three workgroups a CU where there are enough slices to fill the chip (kSliceLdsBytes of LDS
+// that nobody uses keep the others out).  More wavefronts in flight make the reads and writes
+// of HBM get in each other's way: 512 MiB of 32 KiB chunks into a dense buffer take 196 us with
+// eight workgroups a CU, 190 with four in 48 KiB, 181 with three, 181 with two, which is
+// 5.9 TB/s with the upload of the plan (the yardstick copy: 5.8).  A launch of 64 MiB gains
+// 3 %, one of 32 MiB nothing, and the scatter of a staged restore, 36 MiB next to the engine's
+// own kernels, should not ask for LDS that it does not need: the limit starts at 64 MiB.
+//
+// The form with the tables in LDS and 16 vectors a lane, which this one replaces for chunks of
+// 8 KiB and more, took (us, before -> this): 512 MiB out of 32 KiB chunks 195 -> 181, back
+// into them 205 -> 197, one tensor for all layers 187 -> 180; 288 MiB of 18 KiB chunks
+// 116 -> 105; 16 MiB 20 -> 14.  16 vectors a lane instead of 8 (hbm_unroll): 512 MiB 195.
+template <int UNR>
+__global__ __launch_bounds__(kSliceWgThreads) void fkv_copy_slices_kernel(CopyKernelArgs a) {
+  constexpr int64_t kSliceBytes = (int64_t)kWave * UNR * 16;
+  const uint32_t slices = (uint32_t)a.slices_per_chunk, spp = (uint32_t)a.lk * slices;
+  const uint64_t total = (uint64_t)a.num_blocks * spp;
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint32_t waves = blockDim.x / kWave;
+  const uint64_t step = (uint64_t)gridDim.x * waves;
+  for (uint64_t s = (uint64_t)blockIdx.x * waves + wave_uniform(threadIdx.x / kWave); s < total;
+       s += step) {
+    const uint32_t p = total <= 0xffffffffull ? (uint32_t)s / spp : (uint32_t)(s / spp);
+    const uint32_t r = (uint32_t)(s - (uint64_t)p * spp);
+    const uint32_t i = r / slices;
+    const int64_t off = (int64_t)(r - i * slices) * kSliceBytes;
+    const int64_t left = a.chunk_bytes - off;
+    const uint8_t *src = reinterpret_cast<const uint8_t *>(
+        a.base_src[i] + (uint64_t)((a.ids_src ? a.ids_src[p] : (int64_t)p) * a.stride_src) + off);
+    uint8_t *dst = reinterpret_cast<uint8_t *>(
+        a.base_dst[i] + (uint64_t)((a.ids_dst ? a.ids_dst[p] : (int64_t)p) * a.stride_dst) + off);
+    copy_slice<16, true, UNR, false>(src, dst, left < kSliceBytes ? left : kSliceBytes, lane);
+  }
+}
+
 // Several jobs in one launch (the members of one original layer of a multi-group
 // restore, which differ in chunk size and strides): the jobs lie one behind the
 // other on a line, each as long as its weight (its bytes), and a share of the launch
@@ -418,9 +468,12 @@ __global__ __launch_bounds__(kCopyBlockThreads) void fkv_copy_jobs_kernel(CopyJo
 template <int VEC>
 int launch_vec(const CopyKernelArgs &a, int grid, int threads, size_t lds_bytes,
                hipStream_t stream) {
-  if (a.nt_store && VEC == 16 && a.unroll == kCopyUnrollDeep)
-    hipLaunchKernelGGL((fkv_copy_chunks_kernel<16, true, kCopyUnrollDeep>), dim3(grid),
-                       dim3(threads), lds_bytes, stream, a);
+  if (VEC == 16 && a.per_slice && a.unroll == kCopyUnrollDeep)
+    hipLaunchKernelGGL(fkv_copy_slices_kernel<kCopyUnrollDeep>, dim3(grid), dim3(threads),
+                       lds_bytes, stream, a);
+  else if (VEC == 16 && a.per_slice)
+    hipLaunchKernelGGL(fkv_copy_slices_kernel<kCopyUnroll>, dim3(grid), dim3(threads), lds_bytes,
+                       stream, a);
   else if (a.nt_store)
     hipLaunchKernelGGL((fkv_copy_chunks_kernel<VEC, true, kCopyUnroll>), dim3(grid), dim3(threads),
                        lds_bytes, stream, a);
@@ -533,10 +586,12 @@ int prepare_job(CopyKernelArgs &a, int64_t *total, int *grid_pct) {
   if (a.chunk_bytes % a.vec)
     return fail(FKV_ERR_RUNTIME, "copy kernel: chunk %lld not a multiple of vector width %d",
                 (long long)a.chunk_bytes, a.vec);
-  // Deep unroll (16 vectors in flight per lane) is for launches that HBM bounds: both
-  // ends in device memory, 16-byte vectors, chunks of whole deep slices.  Measured on
-  // contiguous 4 GiB copies: 5.2 TB/s with 8 vectors per lane, 5.8 TB/s with 16.
-  if (!(a.unroll == kCopyUnrollDeep && a.vec == 16 && a.nt_store &&
+  // Launches that HBM bounds (their callers ask for an unroll) go by the slice where the
+  // chunks are at least as long as one; 16 vectors per lane for chunks of whole slices of that
+  // size, if asked for.
+  a.per_slice = a.unroll != 0 && a.vec == 16 && a.nt_store && !a.claim &&
+                a.chunk_bytes >= (int64_t)kWave * kCopyUnroll * 16;
+  if (!(a.per_slice && a.unroll == kCopyUnrollDeep &&
         a.chunk_bytes % ((int64_t)kWave * kCopyUnrollDeep * 16) == 0))
     a.unroll = kCopyUnroll;
   const int64_t slice_bytes = (int64_t)kWave * a.unroll * a.vec;
@@ -659,9 +714,18 @@ int launch_copy_kernel(CopyKernelArgs a, int num_workgroups, int threads_per_wor
     return FKV_OK;
   int64_t grid = 1;
   int threads = kWave;
+  if (a.per_slice && threads_per_workgroup > kSliceWgThreads) {
+    // the same number of wavefronts in smaller workgroups, which find room on a CU sooner
+    num_workgroups = (int)std::min<int64_t>(
+        (int64_t)num_workgroups * threads_per_workgroup / kSliceWgThreads, INT32_MAX);
+    threads_per_workgroup = kSliceWgThreads;
+  }
   shape_launch(a, total, (int64_t)a.num_blocks * a.lk * a.chunk_bytes, grid_pct,
                num_workgroups, threads_per_workgroup, &grid, &threads);
-  const size_t lds_bytes = (size_t)(2 * a.lk + 2 * kCopyIdTile) * sizeof(uint64_t);
+  const size_t lds_bytes =
+      !a.per_slice ? (size_t)(2 * a.lk + 2 * kCopyIdTile) * sizeof(uint64_t)
+      : (int64_t)a.num_blocks * a.lk * a.chunk_bytes >= kSliceFewWgBytes ? kSliceLdsBytes
+                                                                         : 0;
   switch (a.vec) {
   case 16: return launch_vec<16>(a, (int)grid, threads, lds_bytes, stream);
   case 8:  return launch_vec<8>(a, (int)grid, threads, lds_bytes, stream);
@@ -681,7 +745,7 @@ int launch_copy_jobs(const CopyKernelArgs *jobs, int njobs, int num_workgroups,
   int grid_pct = 100; // the largest any job asks for
   for (int j = 0; j < njobs; ++j) {
     CopyKernelArgs a = jobs[j];
-    a.unroll = kCopyUnroll;
+    a.unroll = 0;
     a.lane_runs = jobs[0].lane_runs; // the launch's choice, made for the first job
     if (a.vec != jobs[0].vec || a.nt_store != jobs[0].nt_store)
       return fail(FKV_ERR_RUNTIME, "copy kernel: jobs of one launch differ in vector width or store kind");

@@ -205,7 +205,7 @@ fkv_launch_policy defaults_for(uint32_t present) {
   p.staged_max_mb = 512;
   p.hbm_workgroups = 8192;
   p.hbm_wg_threads = 1024;
-  p.hbm_unroll = kCopyUnrollDeep;
+  p.hbm_unroll = kCopyUnroll;
   p.ce_staging_mb = 1024;
   p.ce_two_streams = 1;
   p.ce_rect_min_kb = 32768; // 32 MiB and more: the same rate either way (3 GiB in copies of 32 MiB:

@@ -722,7 +722,8 @@ typedef struct fkv_launch_policy {
    * the scatter of a staged restore */
   int32_t hbm_workgroups;
   int32_t hbm_wg_threads;
-  int32_t hbm_unroll;         /* 16-byte vectors in flight per lane in these launches: 8 or 16 */
+  int32_t hbm_unroll;         /* 16-byte vectors in flight per lane in these launches: 8 (default)
+                                 or 16 */
   int32_t ce_staging_mb;      /* FKV_CE_STAGING_MB: device staging of the copy-engine strategies */
   int32_t ce_two_streams;     /* 0: every copy of a copy-engine strategy on the caller's stream;
                                  2: runs of eight and more independent copies alternate between it
