@@ -42,8 +42,11 @@ struct StagingKernelArgs {
 
 typedef unsigned int vec16 __attribute__((ext_vector_type(4)));
 
-// Copies `bytes` from src to dst with one wavefront; VEC16: both are 16-byte aligned.
-template <bool VEC16, bool NTS>
+// Copies `bytes` from src to dst with one wavefront; VEC16: both are 16-byte aligned.  RUNS: a
+// lane moves adjacent vectors, 128 bytes, so that its stores complete a line of host memory
+// (see copy_slice in fkv_kernels.hip); its loads walk through one line, without the streaming
+// hint that might let the line go in between.
+template <bool VEC16, bool NTS, bool RUNS>
 __device__ __forceinline__ void wave_copy(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst,
                                           int64_t bytes, int lane) {
   int64_t done = 0;
@@ -52,18 +55,20 @@ __device__ __forceinline__ void wave_copy(const uint8_t *__restrict__ src, uint8
     vec16 *d = reinterpret_cast<vec16 *>(dst);
     const int64_t nvec = bytes / 16;
     constexpr int U = kCopyUnroll;
+    constexpr int kLane = RUNS ? U : 1, kAccess = RUNS ? 1 : 64;
     for (int64_t v0 = 0; v0 < nvec; v0 += 64 * U) {
       // all loads of a slice before the first store; lanes beyond the end re-read the
       // last vector rather than branch around the load
       vec16 r[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int64_t v = v0 + u * 64 + lane;
-        r[u] = __builtin_nontemporal_load(s + (v < nvec ? v : nvec - 1));
+        const int64_t v = v0 + u * kAccess + lane * kLane;
+        const vec16 *from = s + (v < nvec ? v : nvec - 1);
+        r[u] = RUNS ? *from : __builtin_nontemporal_load(from);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int64_t v = v0 + u * 64 + lane;
+        const int64_t v = v0 + u * kAccess + lane * kLane;
         if (v < nvec) {
           if (NTS)
             __builtin_nontemporal_store(r[u], d + v);
@@ -78,7 +83,7 @@ __device__ __forceinline__ void wave_copy(const uint8_t *__restrict__ src, uint8
     dst[j] = src[j];
 }
 
-template <bool WRITE_CPU, bool VEC16>
+template <bool WRITE_CPU, bool VEC16, bool RUNS = false>
 __global__ __launch_bounds__(kCopyBlockThreads) void fkv_staging_transfer_kernel(StagingKernelArgs a) {
   const int lane = threadIdx.x & 63;
   const int64_t wave = (int64_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
@@ -129,7 +134,7 @@ __global__ __launch_bounds__(kCopyBlockThreads) void fkv_staging_transfer_kernel
       }
       if (lane == 0)
         *cur_entry = (uint32_t)sz;
-      wave_copy<VEC16, false>(payload, cur_slot, sz, lane);
+      wave_copy<VEC16, false, RUNS>(payload, cur_slot, sz, lane);
     } else {
       if (sz > a.staging_stride) { // a stale or corrupt entry must not overrun the staging slot
         if (lane == 0) {
@@ -141,7 +146,7 @@ __global__ __launch_bounds__(kCopyBlockThreads) void fkv_staging_transfer_kernel
       }
       if (lane == 0)
         a.comp_sizes[i] = (uint64_t)sz;
-      wave_copy<VEC16, true>(cur_slot, payload, sz, lane);
+      wave_copy<VEC16, true, false>(cur_slot, payload, sz, lane);
     }
   }
 }
@@ -238,12 +243,30 @@ int fkv_staging_transfer(const fkv_staging_transfer_desc *dp, void *stream_v) tr
   // payloads, whose last slice is short: twice the workgroups of the fixed-size
   // kernel make up for it (16-29 KiB payloads: 45 GB/s with 16 wavefronts, 55.0 with
   // 24, 55.7 with 32).
-  int grid = cta * (write_cpu ? pol.d2h_wg_per_cta : 2 * pol.h2d_wg_per_cta);
+  // Writing, the short last slices leave a third of the bytes in flight out, and as many
+  // workgroups more make up for it (us, 48 / 64 / 96 wavefronts: 2048 payloads of 16-29 KiB
+  // 887 / 877 / 866, of 4-7 KiB in 8 KiB slots, with adjacent vectors 259 / 249; more would
+  // cost the kernels next to them more than they bring).
+  int grid = cta * (write_cpu ? (pol.d2h_wg_per_cta * 4 + 2) / 3 : 2 * pol.h2d_wg_per_cta);
   const int threads = write_cpu ? pol.d2h_wg_threads : pol.h2d_wg_threads;
   grid = std::max(1, std::min(grid, (d.bsz + threads / 64 - 1) / (threads / 64)));
-#define FKV_LAUNCH_STAGING(W, V)                                                              \
-  hipLaunchKernelGGL((fkv_staging_transfer_kernel<W, V>), dim3(grid), dim3(threads), 0, stream, a)
-  if (write_cpu && vec16)
+#define FKV_LAUNCH_STAGING(...)                                                               \
+  hipLaunchKernelGGL((fkv_staging_transfer_kernel<__VA_ARGS__>), dim3(grid), dim3(threads), 0,  \
+                     stream, a)
+  // Adjacent vectors per lane on the same terms as the fixed-size kernel: not next to a
+  // transfer from the host, where the plain order moves 2 % more in sum.  And only for calls
+  // that fill the link for a while: the loads of a slice take longer in this order, which a
+  // short call waits for.  With 64 wavefronts (us, plain / adjacent): 96 payloads of 16-29 KiB
+  // 51 / 53, 256 124 / 128, 384 181 / 182-191, 768 351 / 336, 2048 877 / 857; 512 of 4-7 KiB
+  // 69 / 72.  With 48: 2048 of 9-16 KiB in 18 KiB slots 527 / 502.
+  constexpr int kRunsMinPayloads = 16; // per wavefront
+  const bool runs = d.bsz / kRunsMinPayloads >= grid * (threads / 64) &&
+                    (pol.d2h_lane_runs == 2 ||
+                     (pol.d2h_lane_runs == 1 &&
+                      !(pol.arbiter != 0 && link_direction_busy(device, /*h2d=*/true, stream))));
+  if (write_cpu && vec16 && runs)
+    FKV_LAUNCH_STAGING(true, true, true);
+  else if (write_cpu && vec16)
     FKV_LAUNCH_STAGING(true, true);
   else if (write_cpu)
     FKV_LAUNCH_STAGING(true, false);

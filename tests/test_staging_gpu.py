@@ -90,6 +90,20 @@ def test_write_then_read_matches_the_oracle(gpu_device, layout, cap, stride, siz
     c.check("after the reads")
 
 
+@pytest.mark.parametrize("lane_runs", [0, 1])
+@pytest.mark.parametrize("size_range", [(1, 140), (120, 136), (8000, 8208), (0, 9000)])
+def test_many_payloads_in_either_order_of_vectors(gpu_device, lane_runs, size_range):
+    """Enough payloads for the order in which a lane moves adjacent vectors: around one lane's
+    128 bytes, a whole slice and a byte more."""
+    from flexkv_amd.c_ext import launch_policy
+    rng = np.random.default_rng(size_range[1])
+    L, NB = 4, 300
+    c = Case(gpu_device, rng, L, 1, NB, NB, 9008, 9008, "BLOCKFIRST", size_range, L * NB)
+    with launch_policy(d2h_lane_runs=2 * lane_runs):
+        c.run(0, 0, L * NB, True)
+    c.check("after the writes")
+
+
 def test_unaligned_addresses_take_the_byte_path(gpu_device):
     """A staging stride and a host slot that are no multiples of 16."""
     rng = np.random.default_rng(4)
