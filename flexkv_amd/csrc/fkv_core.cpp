@@ -658,7 +658,7 @@ void kernel_plan_point(KernelPlan *out, const uint8_t *dv, uint64_t *claims) {
 }
 
 int kernel_plan_build(const fkv_transfer_desc &d, hipStream_t stream, KernelPlan *out,
-                      bool host_optional) {
+                      bool host_optional, bool one_launch) {
   int device = 0;
   FKV_HIP_TRY(hipGetDevice(&device));
   const size_t plan_bytes = kernel_plan_bytes(d);
@@ -672,16 +672,25 @@ int kernel_plan_build(const fkv_transfer_desc &d, hipStream_t stream, KernelPlan
   }
   const fkv_launch_policy pol = policy_of(device);
   // Kernels read the plan from a device copy, which a small kernel uploads first,
-  // or where it is, in the pinned slot.  Next to a transfer in the other direction
-  // every command on a stream costs idle time, and the upload is one: two threads
-  // that put and get 25 MB (100 MB) requests move 88.8 (95.4) instead of 87.0 (94.1)
-  // GB/s without it.  A lone transfer is no faster for it and a multi-group restore
-  // 1.5 % slower, so the plan is read in place only while the other direction is
-  // busy.  plan_mirror of the launch policy = 1 / 0: always / never upload.
+  // or where it is, in the pinned slot.  In place it costs the kernel a round trip over the
+  // link, uploaded a command on the stream, so a plan that one launch reads once (`one_launch`)
+  // stays where it is, as long as a workgroup's part of it is one round trip: the ids of its
+  // blocks one a lane, and two tables of two entries a lane (a block of 2 MiB 67.7 -> 65.1 us
+  // from the host, 71.8 -> 68.6 to it; 10 MiB 220 -> 217, three layer groups 825 -> 818; 1024
+  // blocks of 2304 bytes 72.6 -> 70.1; with 160 (layer, kv) pairs 37.5 -> 37.7, with 256
+  // 73.0 -> 73.9).  A restore that reads its plan a launch a batch is 1.5 % slower
+  // in place; but next to a transfer in the other direction every command on a stream costs
+  // idle time, and nothing is uploaded then: two threads that put and get 25 MB (100 MB)
+  // requests move 88.8 (95.4) instead of 87.0 (94.1) GB/s.  plan_mirror of the launch
+  // policy = 1 / 0: always / never upload.
+  constexpr int kInPlacePairs = 128, kInPlaceBlocksPerWorkgroup = 64;
+  const bool one_round_trip = one_launch && d.num_layers * d.kv_dim <= kInPlacePairs &&
+                              d.num_blocks <= kInPlaceBlocksPerWorkgroup * out->workgroups;
   const bool mirror_plan =
       pol.plan_mirror >= 0
           ? pol.plan_mirror != 0
-          : !(pol.arbiter == 1 && link_direction_busy(device, !out->h2d, stream));
+          : !(one_round_trip ||
+              (pol.arbiter == 1 && link_direction_busy(device, !out->h2d, stream)));
   uint8_t *dv = nullptr;
   rc = plan_publish(slot, plan_bytes, mirror_plan, stream, &dv);
   if (rc != FKV_OK) {
@@ -861,7 +870,7 @@ void kernel_plan_release(KernelPlan *p, hipStream_t stream) {
 int run_kernel_path(const fkv_transfer_desc &d, hipStream_t stream) {
   set_last_path(FKV_PATH_KERNEL);
   KernelPlan plan;
-  FKV_TRY(kernel_plan_build(d, stream, &plan));
+  FKV_TRY(kernel_plan_build(d, stream, &plan, /*host_optional=*/false, /*one_launch=*/true));
   KernelPlanHold hold{&plan, stream};
   return kernel_plan_launch(plan, 0, d.num_layers, stream);
 }
@@ -1143,7 +1152,8 @@ int run_kernel_path_multi(const fkv_transfer_desc *descs, int count, hipStream_t
   } give_back{plans, stream};
   int rc = FKV_OK, built = 0;
   for (; built < count && rc == FKV_OK; ++built)
-    rc = fkv::kernel_plan_build(descs[built], stream, &plans[built]);
+    rc = fkv::kernel_plan_build(descs[built], stream, &plans[built], /*host_optional=*/false,
+                                /*one_launch=*/true);
   if (rc != FKV_OK)
     --built; // the one that failed holds nothing
   for (int k = 0; k < built && rc == FKV_OK; k += fkv::kCopyMaxJobs) {

@@ -334,8 +334,9 @@ int kernel_plan_fill(const fkv_transfer_desc &d, uint8_t *h, bool may_probe_devi
 void kernel_plan_point(KernelPlan *out, const uint8_t *dv, uint64_t *claims);
 // Builds and uploads (on `stream`) the plan for all layers of `d`.  With `host_optional` a
 // host pool the device cannot read is no error: the plan then has host_visible == false.
+// `one_launch`: the plan is read by one launch and not again.
 int kernel_plan_build(const fkv_transfer_desc &d, hipStream_t stream, KernelPlan *out,
-                      bool host_optional = false);
+                      bool host_optional = false, bool one_launch = false);
 // Enqueues the copy of layers [layer_offset, layer_offset + num_layers) of the plan.
 int kernel_plan_launch(const KernelPlan &p, int layer_offset, int num_layers,
                        hipStream_t stream);

@@ -272,6 +272,26 @@ __device__ __forceinline__ void copy_share(const CopyKernelArgs &a, uint64_t num
   const int wave = tid / kWave;
   const int nwaves = blockDim.x / kWave;
 
+  uint64_t s0 = total * num0 / den;
+  uint64_t s1 = total * num1 / den;
+  if (a.packed) { // from pieces to vectors
+    s0 *= kPiece;
+    s1 = s1 * kPiece < total_units ? s1 * kPiece : total_units;
+  }
+  const bool any = s0 < s1;
+
+  const uint32_t pos_lo = (uint32_t)(s0 / spp);
+  const uint32_t pos_hi = any ? (uint32_t)((s1 - 1) / spp) : pos_lo;
+  // This work-item's ids of the first tile are asked for before the tables: where the plan is
+  // read in place, out of pinned host memory, that is one round trip over the link instead
+  // of two.
+  int64_t id_src = (int64_t)pos_lo + tid, id_dst = id_src;
+  if (any && (uint32_t)tid < min((uint32_t)kCopyIdTile, pos_hi - pos_lo + 1)) {
+    if (a.ids_src)
+      id_src = a.ids_src[pos_lo + tid];
+    if (a.ids_dst)
+      id_dst = a.ids_dst[pos_lo + tid];
+  }
   if (load_tables) {
     __syncthreads(); // nobody still reads the tables of the job before
     for (int i = tid; i < a.lk; i += blockDim.x) {
@@ -279,24 +299,19 @@ __device__ __forceinline__ void copy_share(const CopyKernelArgs &a, uint64_t num
       s_base_dst[i] = a.base_dst[i];
     }
   }
-  uint64_t s0 = total * num0 / den;
-  uint64_t s1 = total * num1 / den;
-  if (s0 >= s1)
+  if (!any)
     return;
-  if (a.packed) { // from pieces to vectors
-    s0 *= kPiece;
-    s1 = s1 * kPiece < total_units ? s1 * kPiece : total_units;
-  }
-
-  const uint32_t pos_lo = (uint32_t)(s0 / spp);
-  const uint32_t pos_hi = (uint32_t)((s1 - 1) / spp);
   for (uint32_t tile = pos_lo; tile <= pos_hi; tile += kCopyIdTile) {
     const uint32_t n = min((uint32_t)kCopyIdTile, pos_hi - tile + 1);
     __syncthreads(); // previous tile fully consumed; base tables visible
     for (uint32_t i = tid; i < n; i += blockDim.x) {
       const int64_t p = (int64_t)tile + i;
-      s_off_src[i] = (a.ids_src ? a.ids_src[p] : p) * a.stride_src;
-      s_off_dst[i] = (a.ids_dst ? a.ids_dst[p] : p) * a.stride_dst;
+      if (tile != pos_lo || i != (uint32_t)tid) {
+        id_src = a.ids_src ? a.ids_src[p] : p;
+        id_dst = a.ids_dst ? a.ids_dst[p] : p;
+      }
+      s_off_src[i] = id_src * a.stride_src;
+      s_off_dst[i] = id_dst * a.stride_dst;
     }
     __syncthreads();
     const uint64_t tile_s0 = (uint64_t)tile * spp;
