@@ -1011,9 +1011,11 @@ int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t ep
   if (__atomic_load_n(landed_host, __ATOMIC_ACQUIRE) >= epoch)
     return FKV_OK; // it is there: whatever the stream gets next finds it
   // a consumer on another GPU looks at the word in host memory
-  int of_stream = -1;
-  if (stream)
-    FKV_HIP_TRY(hipStreamGetDevice(stream, &of_stream));
+  int of_stream = -1; // the null stream: that of the current device
+  if (stream && hipStreamGetDevice(stream, &of_stream) != hipSuccess) {
+    (void)hipGetLastError();
+    of_stream = -1;
+  }
   DeviceGuard guard(of_stream);
   if (!guard.ok())
     return fail(FKV_ERR_RUNTIME, "cannot select the device of the consumer's stream");

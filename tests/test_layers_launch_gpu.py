@@ -83,6 +83,8 @@ def test_restore_in_one_launch(gpu_device, backend, layers, kv, chunk, n, gran, 
         assert len(times) == -(-layers // gran) and times[0] >= 0
         assert all(b >= a for a, b in zip(times, times[1:]))
     grp.close()
+    for fd in fds:
+        os.close(fd)
 
 
 def test_shapes_that_go_batch_by_batch(gpu_device):
