@@ -822,8 +822,8 @@ namespace {
 // memory, which the host looks at.
 //
 // Whole restores, the forward stream waiting for every layer (us, a launch a batch -> this):
-// 8 x 256 KiB to eventfds 164 -> 76, 32 x 1 MiB 774 -> 667, 61 x 7 MiB 9086 (rows gathered by
-// host threads) -> 7844, which is 55 GB/s.  Next to a fused attention of 76 us a layer:
+// 8 x 256 KiB to eventfds 160 -> 75, 32 x 1 MiB 753 -> 645, 61 x 7 MiB 9080 (rows gathered by
+// host threads) -> 7708, which is 56 GB/s.  Next to a fused attention of 76 us a layer:
 // 32 x 1 MiB 2956 -> 2822, 61 x 7 MiB 10383 -> 8122.
 __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) {
   using V = VecType<16>::type;
