@@ -218,8 +218,8 @@ struct LayersLaunch {
   uint64_t epoch;          // larger than that of any earlier launch
 };
 // What of it runs on the device.  A table instead of two functions because the library's host
-// code also runs without its kernels (over the emulated runtime of the sanitizer tests, where
-// the table stays empty and restores are launched batch by batch).
+// code also runs without its kernels (over the emulated runtime of the sanitizer tests, which
+// brings a table of its own; without one restores are launched batch by batch).
 struct LayersDevice {
   int (*launch)(LayersLaunch t, int num_workgroups, hipStream_t stream);
   // Makes `stream` wait until *landed (device `device`; `landed_host` is the same word in

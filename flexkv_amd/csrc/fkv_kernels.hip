@@ -413,6 +413,24 @@ __device__ __forceinline__ uint32_t wave_uniform(uint32_t v) {
 #endif
 }
 
+// The first lane's value in all lanes, where a workgroup is a single wavefront.
+__device__ __forceinline__ uint32_t from_first_lane(uint32_t v) {
+#if defined(__HIP__)
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+#else
+  return cpu_device_model::from_first_work_item(v);
+#endif
+}
+
+// Waits for every load and store of such a wavefront.
+__device__ __forceinline__ void drain_wave() {
+#if defined(__HIP__)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#else
+  __syncthreads(); // every work-item has got as far
+#endif
+}
+
 // Launches that HBM bounds (both ends in device memory): a wavefront looks its slice up in the
 // tables, moves it and is done; nothing is staged, and no workgroup waits for itself.
 //
@@ -801,7 +819,6 @@ int launch_copy_jobs(const CopyKernelArgs *jobs, int njobs, int num_workgroups,
   }
 }
 
-#if defined(__HIP__) // not in the CPU model of the device: one workgroup at a time, no fences
 namespace {
 // A layerwise restore in one launch: every batch of layers, in order, announced as it lands.
 //
@@ -876,10 +893,9 @@ __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) 
     counted = copied;
     copied = -1;
   };
-  auto drain = [] { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); };
   // The claim after the current one; a safety-net workgroup claims none ahead of time.
   auto claim_ahead = [&]() -> uint32_t {
-    const uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane((int)shares.next_claim);
+    const uint32_t c = from_first_lane(shares.next_claim);
     if (lane == 0 && c < a.num_claims)
       shares.next_claim = shares.claim_one();
     return c;
@@ -918,7 +934,7 @@ __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) 
       // store of the range before has completed, and the answers of the two counters have come:
       // nothing is waited for that is not there.
       if (s == s0 || counted >= 0)
-        drain();
+        drain_wave();
       announce();
       if (s == s0) {
         if (copied >= 0)
@@ -934,7 +950,7 @@ __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) 
     copied = (int)batch;
     part = shares.safety_net ? claim_now() : ahead;
   }
-  drain();
+  drain_wave();
   announce();
   if (copied >= 0)
     count();
@@ -942,9 +958,7 @@ __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) 
 }
 
 __global__ void fkv_wait_landed_kernel(const uint64_t *landed, uint64_t epoch, uint64_t *overdue,
-                                       long long ticks) {
-  if (threadIdx.x != 0)
-    return;
+                                       long long ticks) { // one work-item
   const long long t0 = wall_clock64();
   // relaxed: what the stream runs next starts with an acquire of its own
   while (__hip_atomic_load(landed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) < epoch) {
@@ -1020,8 +1034,9 @@ int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t ep
   if (!guard.ok())
     return fail(FKV_ERR_RUNTIME, "cannot select the device of the consumer's stream");
   constexpr long long kHalfMinute = 30ll * 100000000;
-  hipLaunchKernelGGL(fkv_wait_landed_kernel, dim3(1), dim3(kWave), 0, stream,
-                     guard.device() == device ? landed : landed_host, epoch, overdue, kHalfMinute);
+  const uint64_t *word = guard.device() == device ? landed : landed_host;
+  hipLaunchKernelGGL(fkv_wait_landed_kernel, dim3(1), dim3(1), 0, stream, word, epoch, overdue,
+                     kHalfMinute);
   FKV_HIP_TRY(hipGetLastError());
   return FKV_OK;
 }
@@ -1029,7 +1044,6 @@ int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t ep
 const LayersDevice kLayersDevice{launch_layers, wait_landed};
 [[maybe_unused]] const bool layers_device_set = (layers_device = &kLayersDevice, true);
 } // namespace
-#endif
 
 } // namespace fkv
 

@@ -8,14 +8,18 @@
 // the host runs as it does in the product.  Test infrastructure (emulated_hip_runtime.cpp
 // holds the implementation); nothing here is fast.
 //
-// What the model does not have: wavefronts (no cross-lane operations; the kernels here use
-// none), more than one workgroup in flight (a workgroup never waits for another one in
+// A launch of a single work-item runs on the stream's own thread, next to whatever workgroup
+// is running: that is the kernel that makes a stream wait for a word another kernel writes.
+//
+// What the model does not have: wavefronts (of the cross-lane operations only the first
+// lane's value, in workgroups that are one wavefront), more than one workgroup in flight (a workgroup never waits for another one in
 // these kernels: the safety net of a confined launch only looks at a counter for a bounded
 // time), memory that is not coherent.
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cstddef>
 #include <cstdint>
@@ -32,6 +36,17 @@ extern thread_local Index thread_index, block_index;
 extern thread_local Extent block_extent, grid_extent;
 
 void sync_threads();
+// The value work-item 0 brings, for every work-item of the workgroup; all of them call it.
+uint32_t from_first_work_item(uint32_t v);
+// Fences between work-items, pairwise by time: an acquire is ordered behind every release
+// before it.  One word instead of a fence instruction, which ThreadSanitizer does not follow.
+inline std::atomic<int> fence_word{0};
+inline void fence(int order) {
+  if (order == __ATOMIC_RELEASE || order == __ATOMIC_ACQ_REL)
+    fence_word.fetch_add(1, std::memory_order_release);
+  if (order == __ATOMIC_ACQUIRE || order == __ATOMIC_ACQ_REL)
+    (void)fence_word.load(std::memory_order_acquire);
+}
 // The launch's dynamically sized LDS, one array per workgroup, zeroed never (as on the device).
 void *dynamic_lds();
 // XCDs take the workgroups of a launch in turn; which one takes workgroup 0 changes
@@ -68,7 +83,13 @@ void launch(hipStream_t stream, dim3 grid, dim3 block, size_t lds_bytes, std::fu
 #ifndef __HIP_MEMORY_SCOPE_AGENT
 #define __HIP_MEMORY_SCOPE_AGENT 4
 #endif
+#ifndef __HIP_MEMORY_SCOPE_SYSTEM
+#define __HIP_MEMORY_SCOPE_SYSTEM 5
+#endif
 #define __hip_atomic_load(pointer, order, scope) __atomic_load_n(pointer, order)
+#define __hip_atomic_store(pointer, value, order, scope) __atomic_store_n(pointer, value, order)
+#define __hip_atomic_fetch_add(pointer, value, order, scope) __atomic_fetch_add(pointer, value, order)
+#define __builtin_amdgcn_fence(order, scope) cpu_device_model::fence(order)
 #undef hipLaunchKernelGGL
 #define hipLaunchKernelGGL(kernel, grid, block, lds_bytes, stream, ...)                             \
   cpu_device_model::launch(stream, grid, block, lds_bytes, [=] { (kernel)(__VA_ARGS__); })

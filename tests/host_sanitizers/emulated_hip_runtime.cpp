@@ -48,6 +48,7 @@ struct ihipStream_t {
   std::deque<std::function<void()>> queue;
   bool busy = false, quit = false;
   int hardware_queue = 0; // streams are dealt over four, the null stream sits on the first
+  int device = 0;         // the one that was current when it was made
   std::thread worker;
   ihipStream_t() : worker([this] { run(); }) {}
   ~ihipStream_t() {
@@ -259,6 +260,7 @@ hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned int) {
   *s = made.get();
   static std::atomic<int> dealt{0};
   made->hardware_queue = ++dealt % 4;
+  made->device = t_device;
   std::lock_guard<std::mutex> lk(rt().mu);
   if (rt().streams.empty())
     rt().streams.push_back(std::make_shared<ihipStream_t>());
@@ -287,6 +289,10 @@ hipError_t hipStreamDestroy(hipStream_t s) {
 }
 hipError_t hipStreamSynchronize(hipStream_t s) {
   of(s)->drain();
+  return hipSuccess;
+}
+hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t *device) {
+  *device = s ? s->device : t_device;
   return hipSuccess;
 }
 hipError_t hipStreamQuery(hipStream_t s) { return of(s)->is_idle() ? hipSuccess : hipErrorNotReady; }
@@ -584,6 +590,15 @@ std::atomic<unsigned> g_launch_number{0};
 } // namespace
 
 void sync_threads() { crew().barrier(); }
+uint32_t from_first_work_item(uint32_t v) {
+  static uint32_t slot;
+  if (thread_index.x == 0)
+    slot = v;
+  sync_threads();
+  const uint32_t first = slot;
+  sync_threads(); // everyone has read it before the next one is written
+  return first;
+}
 void *dynamic_lds() { return crew().lds.data(); }
 unsigned xcc_id() { return crew().xcc; }
 void nap() { std::this_thread::yield(); }
@@ -602,6 +617,15 @@ void launch(hipStream_t stream, dim3 grid, dim3 block, size_t lds_bytes, std::fu
   if (refused(kThrow)) // as if the library had run out of host memory at this point
     throw std::bad_alloc();
   const unsigned number = g_launch_number.fetch_add(1);
+  if (threads == 1 && grid.x == 1 && grid.y == 1 && grid.z == 1) {
+    of(stream)->push([=] {
+      thread_index = block_index = Index{};
+      block_extent = grid_extent = Extent{};
+      work_item();
+      fence(__ATOMIC_ACQUIRE); // as the next command of a stream begins on the device
+    });
+    return;
+  }
   of(stream)->push([=] {
     std::lock_guard<std::mutex> device(g_device);
     Crew &c = crew();
@@ -694,6 +718,43 @@ int launch_copy_jobs(const CopyKernelArgs *jobs, int njobs, int num_workgroups,
   });
   return FKV_OK;
 }
+
+// What fkv_copy_layers_kernel does: every batch of layers in order, announced as it lands.
+int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
+  if (t.a.lk < 1 || t.a.lk > kCopyMaxLK || t.a.num_blocks < 1 || t.batches < 1 || num_workgroups < 1 ||
+      t.pairs_per_batch < 1 || (t.a.lk + t.pairs_per_batch - 1) / t.pairs_per_batch != t.batches)
+    return fail(FKV_ERR_RUNTIME, "emulated restore kernel: bad launch");
+  if (refused(kLaunch))
+    return fail(FKV_ERR_RUNTIME, "emulated restore kernel: launch refused");
+  if (refused(kThrow))
+    throw std::bad_alloc();
+  stats().kernel_launches.fetch_add(1, std::memory_order_relaxed);
+  of(stream)->push([t] {
+    for (int b = 0; b < t.batches; ++b) {
+      CopyKernelArgs a = t.a;
+      a.base_src += (size_t)b * t.pairs_per_batch;
+      a.base_dst += (size_t)b * t.pairs_per_batch;
+      a.lk = std::min(t.pairs_per_batch, t.a.lk - b * t.pairs_per_batch);
+      copy_rows(a);
+      t.tick_host[b] = (uint64_t)(std::chrono::steady_clock::now().time_since_epoch().count() / 10);
+      __atomic_store_n(t.landed + b, t.epoch, __ATOMIC_RELEASE);
+      __atomic_store_n(t.landed_host + b, t.epoch, __ATOMIC_RELEASE);
+    }
+  });
+  return FKV_OK;
+}
+int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t epoch, uint64_t *, int,
+                hipEvent_t, hipStream_t stream) {
+  if (__atomic_load_n(landed_host, __ATOMIC_ACQUIRE) >= epoch)
+    return FKV_OK;
+  of(stream)->push([=] {
+    while (__atomic_load_n(landed, __ATOMIC_ACQUIRE) < epoch)
+      std::this_thread::yield();
+  });
+  return FKV_OK;
+}
+const LayersDevice kLayersDevice{launch_layers, wait_landed};
+[[maybe_unused]] const bool layers_device_set = (layers_device = &kLayersDevice, true);
 
 uint64_t safety_net_ranges_of_current_device() { return 0; }
 

@@ -1,0 +1,265 @@
+// Layerwise restores that go out as one launch announcing its batches itself, over the
+// emulated HIP runtime, for sanitizer builds: the words a launch announces its batches by and
+// their reuse by later groups, consumers that wait for a word, both notify modes with
+// eventfds, one and two GPUs, several groups at once, runtime calls refused part-way.  The
+// launch is the stand-in of the emulated runtime, or the kernel itself on the CPU device model.
+// Every byte is compared with a plain model.
+#include <hip/hip_runtime_api.h>
+#include <sys/eventfd.h>
+#include <unistd.h>
+
+#include <algorithm>
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <numeric>
+#include <random>
+#include <thread>
+#include <vector>
+
+#include "fkv_transfer.h"
+
+extern "C" {
+long fkv_emulated_fail(int category, long after, long count); // emulated_hip_runtime.cpp
+unsigned long long fkv_emulated_workgroups_run();
+}
+
+#define REQUIRE(cond, ...)                                                                          \
+  do {                                                                                              \
+    if (!(cond)) {                                                                                  \
+      fprintf(stderr, "FAILED %s:%d: %s\n  ", __FILE__, __LINE__, #cond);                           \
+      fprintf(stderr, __VA_ARGS__);                                                                 \
+      fprintf(stderr, "\n  last error: %s\n", fkv_last_error());                                    \
+      exit(1);                                                                                      \
+    }                                                                                               \
+  } while (0)
+
+namespace {
+
+using Rng = std::mt19937_64;
+int pick(Rng &rng, int lo, int hi) { return lo + (int)(rng() % (uint64_t)(hi - lo + 1)); }
+
+void set_policy(int alt_kb = -1, int gather = 0) {
+  for (int device = 0; device < 2; ++device) {
+    fkv_launch_policy p{};
+    REQUIRE(fkv_launch_policy_reset(device) == FKV_OK && fkv_launch_policy_get(device, &p) == FKV_OK,
+            "policy");
+    p.model_seed = 0;
+    p.staged_restore = 0;
+    p.staged_gather = gather;
+    p.kernel_alt_stream_kb = alt_kb;
+    REQUIRE(fkv_launch_policy_set(device, &p) == FKV_OK, "policy");
+  }
+}
+
+uint64_t launches() {
+  fkv_stats s{};
+  fkv_get_stats(&s);
+  return s.kernel_launches;
+}
+
+// Engine tensors per GPU and layer, [kv, pool, chunk], a block-first host pool, a group.
+struct Group {
+  int ranks, layers, kv, pool;
+  int64_t chunk;
+  std::vector<uint8_t *> dev; // [rank * layers + layer]
+  std::vector<std::vector<uint8_t>> model;
+  uint8_t *host = nullptr;
+  std::vector<int32_t> fds;
+  fkv_layerwise *g = nullptr;
+  std::vector<int64_t> gids, cids;
+
+  size_t layer_bytes() const { return (size_t)(kv * pool * chunk); }
+  int64_t block() const { return layers * kv * chunk; }
+
+  Group(Rng &rng, int ranks_, int layers_, int kv_, int pool_, int64_t chunk_)
+      : ranks(ranks_), layers(layers_), kv(kv_), pool(pool_), chunk(chunk_) {
+    std::vector<uint64_t> ptrs;
+    for (int i = 0; i < ranks * layers; ++i) {
+      uint8_t *d = nullptr;
+      REQUIRE(hipMalloc((void **)&d, layer_bytes()) == hipSuccess, "engine tensor");
+      memset(d, i, layer_bytes());
+      dev.push_back(d);
+      model.emplace_back(layer_bytes(), (uint8_t)i);
+      ptrs.push_back((uint64_t)(uintptr_t)d);
+      fds.push_back(eventfd(0, EFD_NONBLOCK));
+    }
+    REQUIRE(hipHostMalloc((void **)&host, (size_t)(pool * block()), 0) == hipSuccess, "host pool");
+    std::vector<int64_t> kvs(ranks, pool * chunk), bs(ranks, chunk), ls(ranks, (int64_t)layer_bytes()),
+        cs(ranks, chunk), devs;
+    for (int r = 0; r < ranks; ++r)
+      devs.push_back(r);
+    fkv_layerwise_params p{};
+    p.num_gpus = ranks;
+    p.num_tensors_per_gpu = layers;
+    p.gpu_block_ptrs_flat = ptrs.data();
+    p.cpu_blocks_ptr = host;
+    p.num_layers = layers;
+    p.tp_size = ranks;
+    p.gpu_kv_strides = kvs.data();
+    p.gpu_block_strides = bs.data();
+    p.gpu_layer_strides = ls.data();
+    p.gpu_chunk_sizes = cs.data();
+    p.gpu_device_ids = devs.data();
+    p.layer_eventfds = fds.data();
+    p.num_layer_eventfds = (int32_t)fds.size();
+    fkv_ce_config_default(&p.ce);
+    p.ce.is_blockfirst = 1;
+    REQUIRE(fkv_layerwise_create(&p, &g) == FKV_OK, "create");
+    refill(rng);
+  }
+  void refill(Rng &rng) { // new bytes in the host pool
+    for (int64_t i = 0; i < pool * block(); i += 8) {
+      const uint64_t v = rng();
+      memcpy(host + i, &v, 8);
+    }
+  }
+  int restore(Rng &rng, int n, int gran, int notify) {
+    gids.resize(pool);
+    cids.resize(pool);
+    std::iota(gids.begin(), gids.end(), 0);
+    std::iota(cids.begin(), cids.end(), 0);
+    std::shuffle(gids.begin(), gids.end(), rng);
+    std::shuffle(cids.begin(), cids.end(), rng);
+    gids.resize(n);
+    cids.resize(n);
+    return fkv_layerwise_transfer(g, gids.data(), cids.data(), n, block(), chunk, kv * chunk, block(),
+                                  4, 0, layers, gran, kv, 1, 0, "sharded", notify, 0);
+  }
+  void model_restore() {
+    for (int r = 0; r < ranks; ++r)
+      for (int l = 0; l < layers; ++l)
+        for (int k = 0; k < kv; ++k)
+          for (size_t q = 0; q < gids.size(); ++q)
+            memcpy(model[r * layers + l].data() + (k * pool + gids[q]) * chunk,
+                   host + cids[q] * block() + (l * kv + k) * chunk, (size_t)chunk);
+  }
+  void check(const char *when) {
+    model_restore();
+    for (size_t i = 0; i < dev.size(); ++i)
+      REQUIRE(memcmp(dev[i], model[i].data(), layer_bytes()) == 0, "%s: tensor %zu differs", when, i);
+  }
+  int units(size_t i) {
+    uint64_t v = 0;
+    return read(fds[i], &v, 8) == 8 ? (int)v : 0;
+  }
+  void destroy() {
+    fkv_layerwise_destroy(g);
+    for (int fd : fds)
+      close(fd);
+    for (uint8_t *d : dev)
+      REQUIRE(hipFree(d) == hipSuccess, "free");
+    REQUIRE(hipHostFree(host) == hipSuccess, "free");
+  }
+};
+
+int64_t some_chunk(Rng &rng) {
+  return std::vector<int64_t>{8192, 8208, 18432, 8192 + 16 * pick(rng, 1, 700)}[pick(rng, 0, 3)];
+}
+
+// Restores one after the other on one group, a consumer that waits for each layer.
+void seeded_case(uint64_t seed) {
+  Rng rng(seed);
+  const int pool = pick(rng, 2, 7);
+  Group g(rng, pick(rng, 1, 2), pick(rng, 2, 9), pick(rng, 1, 2), pool, some_chunk(rng));
+  hipStream_t consumer = nullptr;
+  REQUIRE(hipSetDevice(0) == hipSuccess &&
+              hipStreamCreateWithFlags(&consumer, hipStreamNonBlocking) == hipSuccess, "stream");
+  std::vector<std::vector<uint8_t>> seen(g.layers, std::vector<uint8_t>(g.layer_bytes()));
+  for (int rep = 0; rep < 4; ++rep) {
+    g.refill(rng);
+    const int gran = pick(rng, 1, g.layers), batches = (g.layers + gran - 1) / gran;
+    const int notify = rep & 1 ? FKV_NOTIFY_POLLING : FKV_NOTIFY_HOSTFUNC;
+    const uint64_t before = launches();
+    REQUIRE(g.restore(rng, pick(rng, 1, pool), gran, notify) == FKV_OK, "seed %llu", (unsigned long long)seed);
+    if (batches > 1)
+      REQUIRE(launches() - before == (uint64_t)g.ranks, "seed %llu: not one launch a GPU",
+              (unsigned long long)seed);
+    for (int l = 0; l < g.layers; ++l) {
+      REQUIRE(fkv_layerwise_wait_layer(g.g, 0, l, consumer) == FKV_OK, "wait_layer");
+      REQUIRE(hipMemcpyAsync(seen[l].data(), g.dev[l], g.layer_bytes(), hipMemcpyDeviceToHost, consumer) ==
+                  hipSuccess, "consumer copy");
+    }
+    REQUIRE(hipStreamSynchronize(consumer) == hipSuccess, "consumer");
+    REQUIRE(fkv_layerwise_synchronize(g.g) == FKV_OK, "synchronize");
+    g.check("restore");
+    for (int l = 0; l < g.layers; ++l)
+      REQUIRE(seen[l] == g.model[l], "seed %llu: the consumer saw other bytes of layer %d",
+              (unsigned long long)seed, l);
+    for (size_t i = 0; i < g.fds.size(); ++i)
+      REQUIRE(g.units(i) == 1, "seed %llu: eventfd %zu", (unsigned long long)seed, i);
+    std::vector<float> ms(batches);
+    int32_t count = 0;
+    REQUIRE(fkv_layerwise_batch_times_ms(g.g, ms.data(), batches, &count) == FKV_OK && count == batches,
+            "batch times");
+    REQUIRE(std::is_sorted(ms.begin(), ms.end()), "batch times out of order");
+  }
+  REQUIRE(hipStreamDestroy(consumer) == hipSuccess, "stream");
+  g.destroy();
+}
+
+// Groups that restore at the same time, each from a thread of its own.
+void several_at_once(uint64_t seed) {
+  std::vector<std::thread> threads;
+  for (int t = 0; t < 3; ++t)
+    threads.emplace_back([seed, t] {
+      Rng rng(seed * 8 + t);
+      for (int k = 0; k < 2; ++k) { // the second group takes words that another one gave back
+        Group g(rng, 1, pick(rng, 2, 6), 1, 4, 8192);
+        for (int rep = 0; rep < 3; ++rep) {
+          g.refill(rng);
+          REQUIRE(g.restore(rng, pick(rng, 1, 4), 1, rep & 1) == FKV_OK, "restore");
+          REQUIRE(fkv_layerwise_synchronize(g.g) == FKV_OK, "synchronize");
+          g.check("several at once");
+        }
+        g.destroy();
+      }
+    });
+  for (auto &t : threads)
+    t.join();
+}
+
+// The runtime refuses something part-way: the restore fails or makes up for it, and the next
+// one is whole.
+void refused_case(uint64_t seed) {
+  Rng rng(seed);
+  Group g(rng, pick(rng, 1, 2), pick(rng, 2, 5), 1, 4, 8192);
+  for (int rep = 0; rep < 4; ++rep) {
+    const bool inject = rep % 2 == 0;
+    g.refill(rng);
+    if (inject)
+      fkv_emulated_fail(pick(rng, 0, 7), pick(rng, 0, 5), pick(rng, 1, 3));
+    const int rc = g.restore(rng, pick(rng, 1, 4), 1, pick(rng, 0, 1));
+    const int src = fkv_layerwise_synchronize(g.g);
+    for (int c = 0; c < 8; ++c)
+      fkv_emulated_fail(c, 0, 0);
+    const bool whole = rc == FKV_OK && src == FKV_OK;
+    REQUIRE(whole || inject, "seed %llu rep %d: a clean restore failed", (unsigned long long)seed, rep);
+    if (whole)
+      g.check("refused calls");
+    for (size_t i = 0; i < g.fds.size(); ++i) {
+      const int units = g.units(i);
+      REQUIRE(whole ? units == 1 : units <= 1, "seed %llu: eventfd %zu has %d", (unsigned long long)seed, i, units);
+    }
+    for (size_t i = 0; i < g.dev.size(); ++i)
+      memcpy(g.model[i].data(), g.dev[i], g.layer_bytes());
+  }
+  g.destroy();
+}
+
+} // namespace
+
+int main(int argc, char **argv) {
+  const int cases = argc > 1 ? atoi(argv[1]) : 20;
+  set_policy();
+  for (int i = 0; i < cases; ++i)
+    seeded_case(21000 + i);
+  for (int i = 0; i < (cases + 3) / 4; ++i)
+    several_at_once(22000 + i);
+  for (int i = 0; i < cases; ++i)
+    refused_case(23000 + i);
+  printf("ok: %d groups of single-launch restores, kernels from their sources: %s\n", cases,
+         fkv_emulated_workgroups_run() ? "yes" : "no");
+  return 0;
+}
