@@ -223,11 +223,11 @@ struct LayersLaunch {
 struct LayersDevice {
   int (*launch)(LayersLaunch t, int num_workgroups, hipStream_t stream);
   // Makes `stream` wait until *landed (device `device`; `landed_host` is the same word in
-  // pinned memory) has reached `epoch`.  `overdue` (pinned) becomes 1 when that took longer
-  // than half a minute and the wait ended all the same.  `behind` lies behind the launch: a
-  // stream that is being captured is handed to it, and refused as ever.
-  int (*wait)(const uint64_t *landed, const uint64_t *landed_host, uint64_t epoch, uint64_t *overdue,
-              int device, hipEvent_t behind, hipStream_t stream);
+  // pinned memory) has reached `epoch`, however long that takes, or until the host has raised
+  // `given_up` (pinned) that far: the launch ended in an error, the batch never lands.  `behind`
+  // lies behind the launch: a stream that is being captured is handed to it, and refused as ever.
+  int (*wait)(const uint64_t *landed, const uint64_t *landed_host, uint64_t epoch,
+              const uint64_t *given_up, int device, hipEvent_t behind, hipStream_t stream);
 };
 extern const LayersDevice *layers_device;
 // Ranges of work that safety-net workgroups (see the kernel) have copied on the

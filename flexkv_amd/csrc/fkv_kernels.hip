@@ -957,15 +957,20 @@ __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) 
   announce();
 }
 
-__global__ void fkv_wait_landed_kernel(const uint64_t *landed, uint64_t epoch, uint64_t *overdue,
-                                       long long ticks) { // one work-item
-  const long long t0 = wall_clock64();
+// Holds its stream until a batch has landed, as an event behind the batch would: for as long as
+// that takes.  The launch it waits for was submitted before it, but may lie behind other work of
+// its hardware queue for any length of time (a collective that waits for another rank), so no
+// clock ends the wait; the host does, should it find that the launch ended in an error.  One
+// work-item.
+__global__ void fkv_wait_landed_kernel(const uint64_t *landed, uint64_t epoch,
+                                       const uint64_t *given_up) {
   // relaxed: what the stream runs next starts with an acquire of its own
-  while (__hip_atomic_load(landed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) < epoch) {
-    if (wall_clock64() - t0 > ticks) {
-      __hip_atomic_store(overdue, (uint64_t)1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  for (uint32_t looks = 1;
+       __hip_atomic_load(landed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) < epoch; ++looks) {
+    // that word lies at the other end of the link: every 0.1 ms or so
+    if (looks % 64 == 0 &&
+        __hip_atomic_load(given_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) >= epoch)
       return;
-    }
     __builtin_amdgcn_s_sleep(8);
   }
 }
@@ -1012,7 +1017,7 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
 }
 
 int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t epoch,
-                uint64_t *overdue, int device, hipEvent_t behind, hipStream_t stream) {
+                const uint64_t *given_up, int device, hipEvent_t behind, hipStream_t stream) {
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
     (void)hipGetLastError();
@@ -1033,10 +1038,8 @@ int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t ep
   DeviceGuard guard(of_stream);
   if (!guard.ok())
     return fail(FKV_ERR_RUNTIME, "cannot select the device of the consumer's stream");
-  constexpr long long kHalfMinute = 30ll * 100000000;
   const uint64_t *word = guard.device() == device ? landed : landed_host;
-  hipLaunchKernelGGL(fkv_wait_landed_kernel, dim3(1), dim3(1), 0, stream, word, epoch, overdue,
-                     kHalfMinute);
+  hipLaunchKernelGGL(fkv_wait_landed_kernel, dim3(1), dim3(1), 0, stream, word, epoch, given_up);
   FKV_HIP_TRY(hipGetLastError());
   return FKV_OK;
 }

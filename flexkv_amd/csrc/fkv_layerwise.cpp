@@ -63,10 +63,11 @@ namespace {
 // them when the group is gone (it finds its epoch reached: a later user's is larger).
 struct LandedWords {
   uint64_t *dev = nullptr;  // [kCopyMaxLK] landed, then uint32_t [kCopyMaxLK] arrived
-  uint64_t *host = nullptr; // [kCopyMaxLK] landed, [kCopyMaxLK] ticks, overdue
+  uint64_t *host = nullptr; // [kCopyMaxLK] landed, [kCopyMaxLK] ticks, given up
   uint32_t *arrived() const { return reinterpret_cast<uint32_t *>(dev + fkv::kCopyMaxLK); }
   uint64_t *ticks() const { return host + fkv::kCopyMaxLK; }
-  uint64_t *overdue() const { return host + 2 * fkv::kCopyMaxLK; }
+  // Epoch of the newest launch the host knows to have ended in an error: waits up to it end.
+  uint64_t *given_up() const { return host + 2 * fkv::kCopyMaxLK; }
 };
 struct LandedPool {
   std::mutex mu;
@@ -315,9 +316,23 @@ struct fkv_layerwise {
     if (status != (int)hipSuccess) {
       // A real device error: the layers behind it were not announced; the next call
       // on the group reports it.
-      int none = 0;
-      restore_error.compare_exchange_strong(none, status);
+      note_device_error(status);
     }
+  }
+
+  // An error of the restore on the device: the first one is kept for the next call, and
+  // streams that wait for words its launch will not write any more are let go.
+  void note_device_error(int e) {
+    int none = 0;
+    restore_error.compare_exchange_strong(none, e);
+    give_up_waits();
+  }
+  void give_up_waits() {
+    if (!one_launch)
+      return;
+    for (const LandedWords &w : landed)
+      if (w.host)
+        __atomic_store_n(w.given_up(), epoch, __ATOMIC_RELEASE);
   }
 
   int poll_batches() {
@@ -366,8 +381,7 @@ struct fkv_layerwise {
       hipError_t e = hipStreamSynchronize(streams[g]);
       if (e != hipSuccess) {
         (void)hipGetLastError();
-        int none = 0;
-        restore_error.compare_exchange_strong(none, (int)e);
+        note_device_error((int)e);
         poller_stop.store(true, std::memory_order_release);
       }
     }
@@ -386,10 +400,6 @@ struct fkv_layerwise {
                        "%s: the previous layerwise restore failed while it was launched: %s", where,
                        feed_error.c_str());
     }
-    for (const LandedWords &w : landed)
-      if (w.host && __atomic_exchange_n(w.overdue(), (uint64_t)0, __ATOMIC_ACQ_REL))
-        return fkv::fail(FKV_ERR_RUNTIME, "%s: a consumer of the previous layerwise restore waited half "
-                         "a minute for its layer and went on without it", where);
     if (e == 0)
       return FKV_OK;
     return fkv::fail(FKV_ERR_RUNTIME, "%s: the previous layerwise restore failed on the device: %s",
@@ -420,10 +430,8 @@ struct fkv_layerwise {
     for (int g = 0; g < num_gpus; ++g) {
       (void)hipSetDevice(device_ids[g]);
       hipError_t e = hipStreamSynchronize(streams[g]);
-      if (e != hipSuccess) {
-        int none = 0;
-        restore_error.compare_exchange_strong(none, (int)e);
-      }
+      if (e != hipSuccess)
+        note_device_error((int)e);
     }
     for (int g = 0; g < (int)dma_streams.size(); ++g)
       for (hipStream_t s : {dma_streams[g], dma_streams2[g]})
@@ -1269,6 +1277,7 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
                 : quiet_event_wait(g->batches[b]->done[i], g->device_ids[i], 0);
         if (e != hipSuccess) {
           (void)hipGetLastError();
+          g->give_up_waits();
           (void)hipSetDevice(restore.device());
           return fail(FKV_ERR_RUNTIME, "layerwise_transfer failed on GPU %d: %s", i,
                       hipGetErrorString(e));
@@ -1285,6 +1294,7 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
       hipError_t e = quiet_stream_wait(g->streams[i], g->device_ids[i]);
       if (e != hipSuccess) {
         (void)hipGetLastError();
+        g->give_up_waits();
         (void)hipSetDevice(restore.device());
         return fail(FKV_ERR_RUNTIME, "%s failed on GPU %d: %s",
                     g->multi_group ? "layerwise_transfer_multi_group" : "layerwise_transfer", i,
@@ -1379,7 +1389,7 @@ int fkv_layerwise_wait_layer(fkv_layerwise *g, int32_t gpu_index, int32_t layer,
                 layer);
   if (g->one_launch)
     return layers_device->wait(g->landed[gpu_index].dev + b, g->landed[gpu_index].host + b, g->epoch,
-                               g->landed[gpu_index].overdue(), g->device_ids[gpu_index],
+                               g->landed[gpu_index].given_up(), g->device_ids[gpu_index],
                                g->batches.back()->done[gpu_index],
                                static_cast<hipStream_t>(consumer_stream));
   FKV_HIP_TRY(hipStreamWaitEvent(static_cast<hipStream_t>(consumer_stream),
@@ -1514,7 +1524,12 @@ int fkv_layerwise_synchronize(fkv_layerwise *g) try {
   DeviceGuard restore(-1);
   for (int i = 0; i < g->num_gpus; ++i) {
     FKV_HIP_TRY(hipSetDevice(g->device_ids[i]));
-    FKV_HIP_TRY(quiet_stream_wait(g->streams[i], g->device_ids[i]));
+    const hipError_t e = quiet_stream_wait(g->streams[i], g->device_ids[i]);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      g->give_up_waits();
+      return fail(FKV_ERR_RUNTIME, "fkv_layerwise_synchronize: GPU %d: %s", i, hipGetErrorString(e));
+    }
   }
   (void)hipSetDevice(restore.device());
   return g->take_restore_error("fkv_layerwise_synchronize");

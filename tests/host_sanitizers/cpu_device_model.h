@@ -53,11 +53,12 @@ void *dynamic_lds();
 // from launch to launch.
 unsigned xcc_id();
 void nap();
+extern std::atomic<long> clock_speed;  // times the rate of the real clock (fkv_emulated_clock_speed)
 inline long long wall_clock_ticks() { // the device's constant 100 MHz clock
   return std::chrono::duration_cast<std::chrono::nanoseconds>(
              std::chrono::steady_clock::now().time_since_epoch())
              .count() /
-         10;
+         10 * clock_speed.load(std::memory_order_relaxed);
 }
 void launch(hipStream_t stream, dim3 grid, dim3 block, size_t lds_bytes, std::function<void()> work_item);
 } // namespace cpu_device_model

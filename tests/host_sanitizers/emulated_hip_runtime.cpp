@@ -121,7 +121,7 @@ hipError_t remember(hipError_t e) {
 // calls of it fail (fkv_emulated_fail below).  What a real runtime does when memory, streams
 // or events run out, or a launch is refused.
 enum Category { kDeviceAlloc, kPinnedAlloc, kStreamCreate, kEventCreate, kCopy, kLaunch, kEventRecord,
-                kThrow, kCategories };
+                kThrow, kStreamSync, kCategories };
 std::atomic<long> g_fail_after[kCategories];
 std::atomic<long> g_fail_count[kCategories];
 std::atomic<long> g_failed_calls{0};
@@ -136,6 +136,26 @@ bool refused(Category c) {
   g_failed_calls.fetch_add(1);
   return true;
 }
+
+// Kernels held back on request (fkv_emulated_hold_kernels): a device whose queue is busy with
+// somebody else's work.  A launch of one work-item is not held.
+struct Hold {
+  std::mutex mu;
+  std::condition_variable cv;
+  bool on = false;
+  void pass() {
+    std::unique_lock<std::mutex> lk(mu);
+    cv.wait(lk, [this] { return !on; });
+  }
+  void set(bool held) {
+    {
+      std::lock_guard<std::mutex> lk(mu);
+      on = held;
+    }
+    cv.notify_all();
+  }
+};
+Hold g_hold;
 
 struct Runtime {
   std::mutex mu;
@@ -288,6 +308,8 @@ hipError_t hipStreamDestroy(hipStream_t s) {
   return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t s) {
+  if (refused(kStreamSync)) // the stream ended in an error
+    return remember(hipErrorLaunchFailure);
   of(s)->drain();
   return hipSuccess;
 }
@@ -485,6 +507,7 @@ hipError_t hipIpcCloseMemHandle(void *) { return remember(hipErrorNotSupported);
 namespace cpu_device_model {
 thread_local Index thread_index, block_index;
 thread_local Extent block_extent, grid_extent;
+std::atomic<long> clock_speed{1};
 
 namespace {
 // The work-items of the workgroup that is running: a crew of host threads that lives as
@@ -627,6 +650,7 @@ void launch(hipStream_t stream, dim3 grid, dim3 block, size_t lds_bytes, std::fu
     return;
   }
   of(stream)->push([=] {
+    g_hold.pass();
     std::lock_guard<std::mutex> device(g_device);
     Crew &c = crew();
     // exactly as large as asked for: an access beyond it is one the device would not forgive either
@@ -730,6 +754,7 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
     throw std::bad_alloc();
   stats().kernel_launches.fetch_add(1, std::memory_order_relaxed);
   of(stream)->push([t] {
+    g_hold.pass();
     for (int b = 0; b < t.batches; ++b) {
       CopyKernelArgs a = t.a;
       a.base_src += (size_t)b * t.pairs_per_batch;
@@ -743,12 +768,13 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
   });
   return FKV_OK;
 }
-int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t epoch, uint64_t *, int,
-                hipEvent_t, hipStream_t stream) {
+int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t epoch,
+                const uint64_t *given_up, int, hipEvent_t, hipStream_t stream) {
   if (__atomic_load_n(landed_host, __ATOMIC_ACQUIRE) >= epoch)
     return FKV_OK;
   of(stream)->push([=] {
-    while (__atomic_load_n(landed, __ATOMIC_ACQUIRE) < epoch)
+    while (__atomic_load_n(landed, __ATOMIC_ACQUIRE) < epoch &&
+           __atomic_load_n(given_up, __ATOMIC_ACQUIRE) < epoch)
       std::this_thread::yield();
   });
   return FKV_OK;
@@ -794,7 +820,8 @@ extern "C" long fkv_emulated_host_waited_copies() { return g_host_waited_copies.
 
 // Test hook: the next `count` calls of `category` (0 device allocation, 1 pinned allocation,
 // 2 stream creation, 3 event creation, 4 copy, 5 kernel launch, 6 event record; 7: a kernel
-// launch throws std::bad_alloc, as an allocation of the library's own might) fail once `after`
+// launch throws std::bad_alloc, as an allocation of the library's own might; 8: a stream's
+// synchronization finds that the stream ended in an error) fail once `after`
 // more of them have succeeded; count 0 switches it off.  Returns the calls refused so far.
 extern "C" long fkv_emulated_fail(int category, long after, long count) {
   if (category >= 0 && category < kCategories) {
@@ -802,6 +829,17 @@ extern "C" long fkv_emulated_fail(int category, long after, long count) {
     g_fail_count[category].store(count);
   }
   return g_failed_calls.load();
+}
+
+// Test hooks: kernels that have not begun wait while `on`; the device's clock runs `factor`
+// times as fast as the real one (the CPU device model).
+extern "C" void fkv_emulated_hold_kernels(int on) { g_hold.set(on != 0); }
+extern "C" void fkv_emulated_clock_speed(long factor) {
+#ifdef FKV_KERNELS_FROM_SOURCE
+  cpu_device_model::clock_speed.store(factor);
+#else
+  (void)factor;
+#endif
 }
 
 // Entry points of the library that live beside its kernels: not part of what runs here.

@@ -9,6 +9,7 @@
 #include <unistd.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -23,6 +24,8 @@
 extern "C" {
 long fkv_emulated_fail(int category, long after, long count); // emulated_hip_runtime.cpp
 unsigned long long fkv_emulated_workgroups_run();
+void fkv_emulated_hold_kernels(int on);
+void fkv_emulated_clock_speed(long factor);
 }
 
 #define REQUIRE(cond, ...)                                                                          \
@@ -31,7 +34,7 @@ unsigned long long fkv_emulated_workgroups_run();
       fprintf(stderr, "FAILED %s:%d: %s\n  ", __FILE__, __LINE__, #cond);                           \
       fprintf(stderr, __VA_ARGS__);                                                                 \
       fprintf(stderr, "\n  last error: %s\n", fkv_last_error());                                    \
-      exit(1);                                                                                      \
+      _exit(1); /* kernels may be held: no destructor of the runtime could end */                   \
     }                                                                                               \
   } while (0)
 
@@ -199,6 +202,45 @@ void seeded_case(uint64_t seed) {
   g.destroy();
 }
 
+// A restore that is held up for minutes by other work on its queue: its consumer waits, and goes
+// on without the layer only when the host has found that the launch ended in an error.
+void held_up_case(uint64_t seed) {
+  Rng rng(seed);
+  Group g(rng, 1, 3, 1, 3, 8192);
+  hipStream_t consumer = nullptr;
+  REQUIRE(hipStreamCreateWithFlags(&consumer, hipStreamNonBlocking) == hipSuccess, "stream");
+  std::vector<uint8_t> seen(g.layer_bytes());
+  for (int rep = 0; rep < 3; ++rep) {
+    const bool fails = rep == 1;
+    g.refill(rng);
+    fkv_emulated_hold_kernels(1);
+    REQUIRE(g.restore(rng, 3, 1, FKV_NOTIFY_POLLING) == FKV_OK, "restore");
+    REQUIRE(fkv_layerwise_wait_layer(g.g, 0, 2, consumer) == FKV_OK, "wait_layer");
+    REQUIRE(hipMemcpyAsync(seen.data(), g.dev[2], g.layer_bytes(), hipMemcpyDeviceToHost, consumer) ==
+                hipSuccess, "consumer copy");
+    fkv_emulated_clock_speed(100000); // ten minutes of the device's clock in 6 ms
+    std::this_thread::sleep_for(std::chrono::milliseconds(50));
+    REQUIRE(hipStreamQuery(consumer) == hipErrorNotReady, "the consumer went on without its layer");
+    if (fails) {
+      fkv_emulated_fail(8, 0, 8);
+      REQUIRE(fkv_layerwise_synchronize(g.g) != FKV_OK, "the stream's error is reported");
+      fkv_emulated_fail(8, 0, 0);
+      REQUIRE(hipStreamSynchronize(consumer) == hipSuccess, "nobody waits for a launch that failed");
+    }
+    fkv_emulated_hold_kernels(0);
+    fkv_emulated_clock_speed(1);
+    // (what the poller saw of the error is reported by this call)
+    REQUIRE((fkv_layerwise_synchronize(g.g) == FKV_OK) == !fails, "synchronize");
+    REQUIRE(hipStreamSynchronize(consumer) == hipSuccess && hipDeviceSynchronize() == hipSuccess, "end");
+    g.check("held up");
+    REQUIRE(fails || seen == g.model[2], "the consumer saw other bytes");
+    for (size_t i = 0; i < g.fds.size(); ++i)
+      (void)g.units(i);
+  }
+  REQUIRE(hipStreamDestroy(consumer) == hipSuccess, "stream");
+  g.destroy();
+}
+
 // Groups that restore at the same time, each from a thread of its own.
 void several_at_once(uint64_t seed) {
   std::vector<std::thread> threads;
@@ -255,6 +297,7 @@ int main(int argc, char **argv) {
   set_policy();
   for (int i = 0; i < cases; ++i)
     seeded_case(21000 + i);
+  held_up_case(20500);
   for (int i = 0; i < (cases + 3) / 4; ++i)
     several_at_once(22000 + i);
   for (int i = 0; i < cases; ++i)
