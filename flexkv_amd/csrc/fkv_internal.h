@@ -211,8 +211,8 @@ struct LayersLaunch {
   int32_t pairs_per_batch;
   int32_t batches;
   int32_t ranges;          // claims per batch, set by the launch
-  uint32_t *arrived;       // device, [batches]: ranges that have landed; zero between launches
-  uint64_t *landed;        // device, [batches]: `epoch` once the batch has landed
+  uint32_t *arrived;       // device, [batches]: counts of Landing; zero between launches
+  uint64_t *landed;        // device, [batches]: `epoch` once the batch and all before it have landed
   uint64_t *landed_host;   // the same in pinned host memory
   uint64_t *tick_host;     // pinned, [batches]: when it landed, in ticks of the 100 MHz clock
   uint64_t epoch;          // larger than that of any earlier launch

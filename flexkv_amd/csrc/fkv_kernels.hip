@@ -48,6 +48,7 @@
 // by this kernel.  Stores into HBM are nontemporal too; stores into pinned host
 // memory are plain, which measured about 1 GB/s faster over the link.
 #include "fkv_internal.h"
+#include "fkv_landing.h"
 
 #include <algorithm>
 #include <chrono>
@@ -834,9 +835,10 @@ namespace {
 // the link later, when they have long come back.  (Counted right behind its stores, with the
 // claim read through LDS, a range cost the wavefront 3 us more: 0.95 against 0.88 ms for 32
 // layers of 1 MiB with 16 wavefronts.)  Write-through stores instead of the fence measured
-// slower: 0.75 against 0.71 ms with 24 wavefronts.  Whoever counts the last range of a batch
-// writes its epoch to a word in device memory, which streams wait for, and one in pinned
-// memory, which the host looks at.
+// slower: 0.75 against 0.71 ms with 24 wavefronts.  Whoever completes the count of a
+// batch (see Landing: its ranges, and the announcement of the batch before) writes its epoch to a
+// word in device memory, which streams wait for, and one in pinned memory, which the host looks
+// at.
 //
 // Whole restores, the forward stream waiting for every layer (us, a launch a batch -> this):
 // 8 x 256 KiB to eventfds 160 -> 75, 32 x 1 MiB 753 -> 645, 61 x 7 MiB 9080 (rows gathered by
@@ -871,28 +873,7 @@ __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) 
   }
   load_tile(0);
 
-  // The batch whose range this wavefront has copied but not counted yet, and the one whose
-  // count is under way (-1: none).
-  int copied = -1, counted = -1;
-  uint32_t before = 0; // lane 0: ranges of `counted` that had landed before
-  auto announce = [&] { // whoever counted the last range of a batch
-    if (lane == 0 && counted >= 0 && before + 1 == (uint32_t)t.ranges) {
-      t.arrived[counted] = 0;
-      t.tick_host[counted] = (uint64_t)wall_clock64();
-      __hip_atomic_store(t.landed + counted, t.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-      __hip_atomic_store(t.landed_host + counted, t.epoch, __ATOMIC_RELEASE,
-                         __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    counted = -1;
-  };
-  auto count = [&] {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent"); // the stores of the range, out of this XCD's L2
-    if (lane == 0)
-      before = __hip_atomic_fetch_add(t.arrived + copied, 1u, __ATOMIC_RELAXED,
-                                      __HIP_MEMORY_SCOPE_AGENT);
-    counted = copied;
-    copied = -1;
-  };
+  Landing landing(t, lane == 0);
   // The claim after the current one; a safety-net workgroup claims none ahead of time.
   auto claim_ahead = [&]() -> uint32_t {
     const uint32_t c = from_first_lane(shares.next_claim);
@@ -933,12 +914,12 @@ __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) 
       // The vectors come from the other end of the link, so by the time they are here every
       // store of the range before has completed, and the answers of the two counters have come:
       // nothing is waited for that is not there.
-      if (s == s0 || counted >= 0)
+      if (s == s0 || landing.counted >= 0)
         drain_wave();
-      announce();
+      landing.announce();
       if (s == s0) {
-        if (copied >= 0)
-          count();
+        if (landing.copied >= 0)
+          landing.count();
         if (!shares.safety_net)
           ahead = claim_ahead();
       }
@@ -947,14 +928,14 @@ __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) 
         if (u * kWave + lane < nvec)
           __builtin_nontemporal_store(v[u], dst + u * kWave + lane);
     }
-    copied = (int)batch;
+    landing.copied = (int)batch;
     part = shares.safety_net ? claim_now() : ahead;
   }
   drain_wave();
-  announce();
-  if (copied >= 0)
-    count();
-  announce();
+  landing.announce();
+  if (landing.copied >= 0)
+    landing.count();
+  landing.announce();
 }
 
 // Holds its stream until a batch has landed, as an event behind the batch would: for as long as

@@ -274,3 +274,17 @@ def test_single_launch_restores_under_sanitizers(tmp_path, sanitizer, kernels_fr
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-6000:]
     assert "ok: %d groups of single-launch restores" % cases in r.stdout
     assert ("sources: " + ("yes" if kernels_from_source else "no")) in r.stdout
+
+
+@pytest.mark.parametrize("sanitizer", SANITIZERS)
+def test_batches_are_announced_in_order(tmp_path, sanitizer):
+    """The counting and announcing of a single-launch restore (fkv_landing.h): wavefronts take
+    turns in seeded orders, some of them slow, and a batch is announced when it and all before it
+    have landed, not sooner."""
+    exe = build_over_emulated_runtime(tmp_path, "landing_driver.cpp", sanitizer,
+                                      kernels_from_source=True)
+    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:verify_asan_link_order=0",
+               TSAN_OPTIONS="halt_on_error=1", TMPDIR=str(tmp_path))
+    r = subprocess.run([exe, "300"], capture_output=True, text=True, env=env, timeout=300)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-6000:]
+    assert "ok: 300 landings by turns" in r.stdout

@@ -87,6 +87,44 @@ def test_restore_in_one_launch(gpu_device, backend, layers, kv, chunk, n, gran, 
         os.close(fd)
 
 
+@pytest.mark.parametrize("layers,blocks", [(24, 16), (61, 3), (40, 64)])
+def test_a_consumer_of_one_layer_has_all_before_it(gpu_device, layers, blocks):
+    """A stream that waits for one layer only, the last or one in the middle, sees every layer up
+    to it: batches of few ranges, many of them under way together."""
+    from flexkv_amd.c_ext import LayerwiseTransferGroup, get_stats, launch_policy, reset_stats
+    chunk, pool = 16384, blocks + 4
+    s = KVSetup(VLLM, layers, 1, pool, pool, chunk, "BLOCKFIRST", seed=layers)
+    dev = s.to_device(gpu_device)
+    i64 = lambda v: torch.tensor([v], dtype=torch.int64)  # noqa: E731
+    grp = LayerwiseTransferGroup(
+        num_gpus=1, gpu_blocks=[dev.gpu], cpu_blocks=dev.host, ssd_files={}, num_layers=layers,
+        gpu_kv_strides_tensor=i64(s.gpu_kv_stride), gpu_block_strides_tensor=i64(s.gpu_block_stride),
+        gpu_layer_strides_tensor=i64(s.gpu_layer_stride), gpu_chunk_sizes_tensor=i64(s.chunk),
+        iouring_entries=0, iouring_flags=0, layer_eventfds_tensor=torch.empty(0, dtype=torch.int32),
+        tp_size=1, is_blockfirst=True)
+    rng = np.random.default_rng(layers)
+    consumer = torch.cuda.Stream()
+    seen = [torch.empty_like(t) for t in dev.gpu]
+    for rep in range(6):
+        last = layers - 1 if rep % 2 == 0 else layers // 2
+        dev.host.copy_(torch.from_numpy(rng.integers(0, 256, s.host_bytes, dtype=np.uint8)))
+        ids = [rng.permutation(pool)[:blocks].astype(np.int64) for _ in range(2)]
+        with launch_policy(staged_restore=0, staged_gather=0):
+            reset_stats()
+            torch.cuda.synchronize()
+            restore(grp, s, *ids, 1, "polling")
+            with torch.cuda.stream(consumer):
+                grp.wait_layer(last, consumer)
+                for l in range(last + 1):
+                    seen[l].copy_(dev.gpu[l])
+            consumer.synchronize()
+            grp.synchronize()
+            assert get_stats()["kernel_launches"] == 1
+        for l in range(last + 1):
+            assert torch.equal(seen[l], dev.gpu[l]), (rep, l)
+    grp.close()
+
+
 def test_shapes_that_go_batch_by_batch(gpu_device):
     """Packed chunks and odd vector widths keep a launch a batch."""
     from flexkv_amd.c_ext import get_stats, launch_policy, reset_stats
