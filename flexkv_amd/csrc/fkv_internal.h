@@ -211,8 +211,8 @@ struct LayersLaunch {
   int32_t pairs_per_batch;
   int32_t batches;
   int32_t ranges;          // claims per batch, set by the launch
-  uint32_t *arrived;       // device, [batches]: counts of Landing; zero between launches
-  uint64_t *landed;        // device, [batches]: `epoch` once the batch and all before it have landed
+  uint32_t *arrived;       // device, [batches]: ranges that have landed; zero between launches
+  uint64_t *landed;        // device, [batches]: `epoch` once the batch has landed
   uint64_t *landed_host;   // the same in pinned host memory
   uint64_t *tick_host;     // pinned, [batches]: when it landed, in ticks of the 100 MHz clock
   uint64_t epoch;          // larger than that of any earlier launch
@@ -222,11 +222,12 @@ struct LayersLaunch {
 // brings a table of its own; without one restores are launched batch by batch).
 struct LayersDevice {
   int (*launch)(LayersLaunch t, int num_workgroups, hipStream_t stream);
-  // Makes `stream` wait until *landed (device `device`; `landed_host` is the same word in
-  // pinned memory) has reached `epoch`, however long that takes, or until the host has raised
-  // `given_up` (pinned) that far: the launch ended in an error, the batch never lands.  `behind`
-  // lies behind the launch: a stream that is being captured is handed to it, and refused as ever.
-  int (*wait)(const uint64_t *landed, const uint64_t *landed_host, uint64_t epoch,
+  // Makes `stream` wait until the first `count` words of `landed` (device `device`; `landed_host`
+  // are the same in pinned memory) have reached `epoch`, however long that takes, or until the
+  // host has raised `given_up` (pinned) that far: the launch ended in an error, the batches
+  // never land.  `behind` lies behind the launch: a stream that is being captured is handed to
+  // it, and refused as ever.
+  int (*wait)(const uint64_t *landed, const uint64_t *landed_host, int count, uint64_t epoch,
               const uint64_t *given_up, int device, hipEvent_t behind, hipStream_t stream);
 };
 extern const LayersDevice *layers_device;

@@ -432,6 +432,15 @@ __device__ __forceinline__ void drain_wave() {
 #endif
 }
 
+// A launch of one wavefront that waits for what another launch writes.
+#if defined(__HIP__)
+#define FKV_LAUNCH_BESIDE(kernel, stream, ...)                                                      \
+  hipLaunchKernelGGL(kernel, dim3(1), dim3(kWave), 0, stream, __VA_ARGS__)
+#else // the CPU model of the device runs one launch at a time, except for these
+#define FKV_LAUNCH_BESIDE(kernel, stream, ...)                                                      \
+  cpu_device_model::launch_beside(stream, kWave, [=] { (kernel)(__VA_ARGS__); })
+#endif
+
 // Launches that HBM bounds (both ends in device memory): a wavefront looks its slice up in the
 // tables, moves it and is done; nothing is staged, and no workgroup waits for itself.
 //
@@ -835,10 +844,9 @@ namespace {
 // the link later, when they have long come back.  (Counted right behind its stores, with the
 // claim read through LDS, a range cost the wavefront 3 us more: 0.95 against 0.88 ms for 32
 // layers of 1 MiB with 16 wavefronts.)  Write-through stores instead of the fence measured
-// slower: 0.75 against 0.71 ms with 24 wavefronts.  Whoever completes the count of a
-// batch (see Landing: its ranges, and the announcement of the batch before) writes its epoch to a
-// word in device memory, which streams wait for, and one in pinned memory, which the host looks
-// at.
+// slower: 0.75 against 0.71 ms with 24 wavefronts.  Whoever counts the last range of a batch
+// writes its epoch to a word in device memory, which streams wait for, and one in pinned
+// memory, which the host looks at (see Landing).
 //
 // Whole restores, the forward stream waiting for every layer (us, a launch a batch -> this):
 // 8 x 256 KiB to eventfds 160 -> 75, 32 x 1 MiB 753 -> 645, 61 x 7 MiB 9080 (rows gathered by
@@ -938,22 +946,24 @@ __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) 
   landing.announce();
 }
 
-// Holds its stream until a batch has landed, as an event behind the batch would: for as long as
-// that takes.  The launch it waits for was submitted before it, but may lie behind other work of
-// its hardware queue for any length of time (a collective that waits for another rank), so no
-// clock ends the wait; the host does, should it find that the launch ended in an error.  One
-// work-item.
-__global__ void fkv_wait_landed_kernel(const uint64_t *landed, uint64_t epoch,
-                                       const uint64_t *given_up) {
+// Holds its stream until batches have landed, as an event behind them would: for as long as that
+// takes.  The launch it waits for was submitted before it, but may lie behind other work of its
+// hardware queue for any length of time (a collective that waits for another rank), so no clock
+// ends the wait; the host does, should it find that the launch ended in an error.  One
+// wavefront, a word a lane: the words are written in any order.
+__global__ __launch_bounds__(kWave) void fkv_wait_landed_kernel(const uint64_t *landed, uint32_t count,
+                                                                uint64_t epoch,
+                                                                const uint64_t *given_up) {
+  uint32_t looks = 0;
   // relaxed: what the stream runs next starts with an acquire of its own
-  for (uint32_t looks = 1;
-       __hip_atomic_load(landed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) < epoch; ++looks) {
-    // that word lies at the other end of the link: every 0.1 ms or so
-    if (looks % 64 == 0 &&
-        __hip_atomic_load(given_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) >= epoch)
-      return;
-    __builtin_amdgcn_s_sleep(8);
-  }
+  for (uint32_t i = threadIdx.x; i < count; i += kWave)
+    while (__hip_atomic_load(landed + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) < epoch) {
+      // that word lies at the other end of the link: every 0.1 ms or so
+      if (++looks % 64 == 0 &&
+          __hip_atomic_load(given_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) >= epoch)
+        return;
+      __builtin_amdgcn_s_sleep(8);
+    }
 }
 
 int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
@@ -997,7 +1007,7 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
   return FKV_OK;
 }
 
-int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t epoch,
+int wait_landed(const uint64_t *landed, const uint64_t *landed_host, int count, uint64_t epoch,
                 const uint64_t *given_up, int device, hipEvent_t behind, hipStream_t stream) {
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {
@@ -1008,9 +1018,12 @@ int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t ep
     FKV_HIP_TRY(hipStreamWaitEvent(stream, behind, 0));
     return FKV_OK;
   }
-  if (__atomic_load_n(landed_host, __ATOMIC_ACQUIRE) >= epoch)
-    return FKV_OK; // it is there: whatever the stream gets next finds it
-  // a consumer on another GPU looks at the word in host memory
+  int first = 0; // not known to have landed yet
+  while (first < count && __atomic_load_n(landed_host + first, __ATOMIC_ACQUIRE) >= epoch)
+    ++first;
+  if (first == count)
+    return FKV_OK; // they are there: whatever the stream gets next finds them
+  // a consumer on another GPU looks at the words in host memory
   int of_stream = -1; // the null stream: that of the current device
   if (stream && hipStreamGetDevice(stream, &of_stream) != hipSuccess) {
     (void)hipGetLastError();
@@ -1019,8 +1032,8 @@ int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t ep
   DeviceGuard guard(of_stream);
   if (!guard.ok())
     return fail(FKV_ERR_RUNTIME, "cannot select the device of the consumer's stream");
-  const uint64_t *word = guard.device() == device ? landed : landed_host;
-  hipLaunchKernelGGL(fkv_wait_landed_kernel, dim3(1), dim3(1), 0, stream, word, epoch, given_up);
+  const uint64_t *words = (guard.device() == device ? landed : landed_host) + first;
+  FKV_LAUNCH_BESIDE(fkv_wait_landed_kernel, stream, words, (uint32_t)(count - first), epoch, given_up);
   FKV_HIP_TRY(hipGetLastError());
   return FKV_OK;
 }

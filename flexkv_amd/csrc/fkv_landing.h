@@ -8,16 +8,16 @@
 namespace fkv {
 
 // One wavefront's part.  Wavefronts run on from batch to batch and the last ranges of several
-// batches are under way together, but a batch is announced only behind the one before it: whoever
-// waits for a batch has all earlier ones too, as with a launch per batch on one stream.  That
-// the batch before has been announced counts like a range of its own; nobody waits for it, who
-// completes a count announces that batch and passes the word on to the next.
+// batches are under way together, so a batch may be announced before an earlier one: whoever
+// waits for a batch looks at the words of all up to it.  (Announced in order, by a count that
+// is passed on from batch to batch, eight batches of 256 KiB that land within 36 us took 81
+// instead of 71 us.)
 struct Landing {
   const LayersLaunch &t;
   const bool first_lane;
   int copied = -1;     // batch of the range this wavefront has copied but not counted yet (-1: none)
   int counted = -1;    // the one whose count is under way
-  uint32_t before = 0; // first lane: what had been counted of it before
+  uint32_t before = 0; // first lane: ranges of it that had landed before
 
   __device__ __forceinline__ Landing(const LayersLaunch &t, bool first_lane)
       : t(t), first_lane(first_lane) {}
@@ -32,20 +32,14 @@ struct Landing {
     copied = -1;
   }
 
-  // Whoever has completed a count.
+  // Whoever has counted the last range of a batch.
   __device__ __forceinline__ void announce() {
-    if (first_lane && counted >= 0) {
-      int b = counted;
-      uint32_t had = before;
-      while (had + 1 == (uint32_t)t.ranges + (b > 0 ? 1u : 0u)) {
-        t.arrived[b] = 0; // for the next launch
-        t.tick_host[b] = (uint64_t)wall_clock64();
-        __hip_atomic_store(t.landed + b, t.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-        __hip_atomic_store(t.landed_host + b, t.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-        if (++b == t.batches)
-          break;
-        had = __hip_atomic_fetch_add(t.arrived + b, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-      }
+    if (first_lane && counted >= 0 && before + 1 == (uint32_t)t.ranges) {
+      t.arrived[counted] = 0; // for the next launch
+      t.tick_host[counted] = (uint64_t)wall_clock64();
+      __hip_atomic_store(t.landed + counted, t.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+      __hip_atomic_store(t.landed_host + counted, t.epoch, __ATOMIC_RELEASE,
+                         __HIP_MEMORY_SCOPE_SYSTEM);
     }
     counted = -1;
   }

@@ -413,7 +413,7 @@ struct fkv_layerwise {
     if (e != hipSuccess || !one_launch)
       return e;
     // The last one to land is what the event saw; the others by the device's own clock, each
-    // no earlier than the ones before it, which are announced first.
+    // no earlier than the ones before it, as whoever waits for a batch waits for those too.
     const uint64_t *t = landed[0].ticks();
     const uint64_t end = *std::max_element(t, t + batches.size());
     const uint64_t then = *std::max_element(t, t + b + 1);
@@ -1387,8 +1387,8 @@ int fkv_layerwise_wait_layer(fkv_layerwise *g, int32_t gpu_index, int32_t layer,
   if (!g->gate.wait(b))
     return fail(FKV_ERR_RUNTIME, "layer %d will not land: the restore failed while it was launched",
                 layer);
-  if (g->one_launch)
-    return layers_device->wait(g->landed[gpu_index].dev + b, g->landed[gpu_index].host + b, g->epoch,
+  if (g->one_launch) // for every batch up to it, as an event on the stream would
+    return layers_device->wait(g->landed[gpu_index].dev, g->landed[gpu_index].host, b + 1, g->epoch,
                                g->landed[gpu_index].given_up(), g->device_ids[gpu_index],
                                g->batches.back()->done[gpu_index],
                                static_cast<hipStream_t>(consumer_stream));

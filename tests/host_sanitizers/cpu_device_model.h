@@ -8,8 +8,9 @@
 // the host runs as it does in the product.  Test infrastructure (emulated_hip_runtime.cpp
 // holds the implementation); nothing here is fast.
 //
-// A launch of a single work-item runs on the stream's own thread, next to whatever workgroup
-// is running: that is the kernel that makes a stream wait for a word another kernel writes.
+// launch_beside: a wavefront without barriers, run on the stream's own thread (work-item by
+// work-item) next to whatever workgroup is running, is the kernel that makes a stream wait for
+// words another kernel writes.
 //
 // What the model does not have: wavefronts (of the cross-lane operations only the first
 // lane's value, in workgroups that are one wavefront), more than one workgroup in flight (a workgroup never waits for another one in
@@ -60,6 +61,7 @@ inline long long wall_clock_ticks() { // the device's constant 100 MHz clock
              .count() /
          10 * clock_speed.load(std::memory_order_relaxed);
 }
+void launch_beside(hipStream_t stream, unsigned work_items, std::function<void()> work_item);
 void launch(hipStream_t stream, dim3 grid, dim3 block, size_t lds_bytes, std::function<void()> work_item);
 } // namespace cpu_device_model
 

@@ -626,6 +626,23 @@ void *dynamic_lds() { return crew().lds.data(); }
 unsigned xcc_id() { return crew().xcc; }
 void nap() { std::this_thread::yield(); }
 
+void launch_beside(hipStream_t stream, unsigned work_items, std::function<void()> work_item) {
+  if (refused(kLaunch)) {
+    remember(hipErrorLaunchFailure);
+    return;
+  }
+  of(stream)->push([=] {
+    block_index = Index{};
+    grid_extent = Extent{};
+    block_extent = Extent{work_items, 1, 1};
+    for (unsigned i = 0; i < work_items; ++i) {
+      thread_index = Index{i, 0, 0};
+      work_item();
+    }
+    fence(__ATOMIC_ACQUIRE); // as the next command of a stream begins on the device
+  });
+}
+
 void launch(hipStream_t stream, dim3 grid, dim3 block, size_t lds_bytes, std::function<void()> work_item) {
   const uint64_t threads = (uint64_t)block.x * block.y * block.z;
   if (threads == 0 || threads > 1024 || grid.x == 0 || grid.y == 0 || grid.z == 0 ||
@@ -640,15 +657,6 @@ void launch(hipStream_t stream, dim3 grid, dim3 block, size_t lds_bytes, std::fu
   if (refused(kThrow)) // as if the library had run out of host memory at this point
     throw std::bad_alloc();
   const unsigned number = g_launch_number.fetch_add(1);
-  if (threads == 1 && grid.x == 1 && grid.y == 1 && grid.z == 1) {
-    of(stream)->push([=] {
-      thread_index = block_index = Index{};
-      block_extent = grid_extent = Extent{};
-      work_item();
-      fence(__ATOMIC_ACQUIRE); // as the next command of a stream begins on the device
-    });
-    return;
-  }
   of(stream)->push([=] {
     g_hold.pass();
     std::lock_guard<std::mutex> device(g_device);
@@ -768,14 +776,18 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
   });
   return FKV_OK;
 }
-int wait_landed(const uint64_t *landed, const uint64_t *landed_host, uint64_t epoch,
+int wait_landed(const uint64_t *landed, const uint64_t *landed_host, int count, uint64_t epoch,
                 const uint64_t *given_up, int, hipEvent_t, hipStream_t stream) {
-  if (__atomic_load_n(landed_host, __ATOMIC_ACQUIRE) >= epoch)
+  int first = 0;
+  while (first < count && __atomic_load_n(landed_host + first, __ATOMIC_ACQUIRE) >= epoch)
+    ++first;
+  if (first == count)
     return FKV_OK;
   of(stream)->push([=] {
-    while (__atomic_load_n(landed, __ATOMIC_ACQUIRE) < epoch &&
-           __atomic_load_n(given_up, __ATOMIC_ACQUIRE) < epoch)
-      std::this_thread::yield();
+    for (int b = first; b < count; ++b)
+      while (__atomic_load_n(landed + b, __ATOMIC_ACQUIRE) < epoch &&
+             __atomic_load_n(given_up, __ATOMIC_ACQUIRE) < epoch)
+        std::this_thread::yield();
   });
   return FKV_OK;
 }

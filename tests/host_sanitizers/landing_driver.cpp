@@ -1,5 +1,5 @@
 // The counting and announcing of batches by the wavefronts of a single-launch restore
-// (fkv_landing.h), without the copies: wavefronts as state machines that take turns in a seeded
+// (fkv_landing.h) and the streams that wait for them, without the copies: wavefronts as state machines that take turns in a seeded
 // order, some of them slow, every word checked after every step.
 #include "cpu_device_model.h"
 
@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <random>
+#include <thread>
 #include <vector>
 
 #define REQUIRE(cond, ...)                                                                          \
@@ -92,22 +93,57 @@ void turns(uint64_t seed) {
       const int i = pick(rng, 0, waves - 1);
       if (pick(rng, 1, 100) <= speed[i])
         wave[i].step(w, &next, &counted);
-      bool whole = true; // every batch so far has all its ranges counted
-      for (int b = 0; b < w.t.batches; ++b) {
-        whole = whole && counted[b] == w.t.ranges;
-        REQUIRE(whole || (w.landed[b] < w.t.epoch && w.landed_host[b] < w.t.epoch),
-                "seed %llu: batch %d of %d announced before all up to it had landed",
+      for (int b = 0; b < w.t.batches; ++b)
+        REQUIRE(counted[b] == w.t.ranges || (w.landed[b] < w.t.epoch && w.landed_host[b] < w.t.epoch),
+                "seed %llu: batch %d of %d announced before it had landed",
                 (unsigned long long)seed, b, w.t.batches);
-      }
       busy = false;
       for (const Wavefront &v : wave)
         busy = busy || v.at != Wavefront::kDone;
     }
     for (int b = 0; b < w.t.batches; ++b)
-      REQUIRE(w.landed[b] == w.t.epoch && w.landed_host[b] == w.t.epoch && w.arrived[b] == 0 &&
-                  (b == 0 || w.ticks[b] >= w.ticks[b - 1]),
+      REQUIRE(w.landed[b] == w.t.epoch && w.landed_host[b] == w.t.epoch && w.arrived[b] == 0,
               "seed %llu: batch %d at the end", (unsigned long long)seed, b);
   }
+}
+
+// Words written in any order: a stream that waits for one batch goes on when every word up to
+// that one is there, at the device's words and at those the host sees.
+void any_order(uint64_t seed, hipStream_t stream) {
+  Rng rng(seed);
+  Words w(pick(rng, 1, 150), 1);
+  w.t.epoch = 5;
+  uint64_t given_up = 4;
+  hipEvent_t behind = nullptr;
+  REQUIRE(hipEventCreate(&behind) == hipSuccess, "event");
+  std::vector<int> order(w.t.batches);
+  for (int b = 0; b < w.t.batches; ++b)
+    order[b] = b;
+  std::shuffle(order.begin(), order.end(), rng);
+  const int only = pick(rng, 0, w.t.batches - 1), begun = pick(rng, 0, w.t.batches);
+  auto write = [&](int k) {
+    __atomic_store_n(&w.landed[order[k]], w.t.epoch, __ATOMIC_RELEASE);
+    __atomic_store_n(&w.landed_host[order[k]], w.t.epoch, __ATOMIC_RELEASE);
+  };
+  for (int k = 0; k < begun; ++k)
+    write(k);
+  REQUIRE(fkv::layers_device->wait(w.t.landed, w.t.landed_host, only + 1, w.t.epoch, &given_up, 0, behind,
+                                   stream) == FKV_OK, "wait");
+  for (int k = begun; k <= w.t.batches; ++k) {
+    bool there = true;
+    for (int b = 0; b <= only; ++b)
+      there = there && w.landed[b] == w.t.epoch;
+    if (there) {
+      REQUIRE(hipStreamSynchronize(stream) == hipSuccess, "stream");
+      break;
+    }
+    if (k % 16 == begun % 16)
+      std::this_thread::sleep_for(std::chrono::milliseconds(2));
+    REQUIRE(hipStreamQuery(stream) == hipErrorNotReady,
+            "seed %llu: the stream went on without a batch before %d", (unsigned long long)seed, only);
+    write(k);
+  }
+  REQUIRE(hipEventDestroy(behind) == hipSuccess, "event");
 }
 
 } // namespace
@@ -116,6 +152,11 @@ int main(int argc, char **argv) {
   const int cases = argc > 1 ? atoi(argv[1]) : 100;
   for (int i = 0; i < cases; ++i)
     turns(31000 + i);
+  hipStream_t stream = nullptr;
+  REQUIRE(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) == hipSuccess, "stream");
+  for (int i = 0; i < cases / 4; ++i)
+    any_order(33000 + i, stream);
+  REQUIRE(hipStreamDestroy(stream) == hipSuccess, "stream");
   printf("ok: %d landings by turns\n", cases);
   return 0;
 }

@@ -277,10 +277,11 @@ def test_single_launch_restores_under_sanitizers(tmp_path, sanitizer, kernels_fr
 
 
 @pytest.mark.parametrize("sanitizer", SANITIZERS)
-def test_batches_are_announced_in_order(tmp_path, sanitizer):
+def test_landing_of_batches_and_waits_for_them(tmp_path, sanitizer):
     """The counting and announcing of a single-launch restore (fkv_landing.h): wavefronts take
-    turns in seeded orders, some of them slow, and a batch is announced when it and all before it
-    have landed, not sooner."""
+    turns in seeded orders, some of them slow, and a batch is announced when it has landed, not
+    sooner; a stream that waits for a batch goes on when it and all before it are there, in
+    whatever order the words are written."""
     exe = build_over_emulated_runtime(tmp_path, "landing_driver.cpp", sanitizer,
                                       kernels_from_source=True)
     env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:verify_asan_link_order=0",
