@@ -32,10 +32,14 @@ struct Landing {
     copied = -1;
   }
 
-  // Whoever has counted the last range of a batch.
+  // Whoever has counted the last range of a batch.  The other wavefronts' counts lie behind a
+  // release of what they wrote; the acquire makes what they wrote part of what the words release.  (On this
+  // chip each of them has written its L2 back before it counted, and nothing would be missing.)
   __device__ __forceinline__ void announce() {
     if (first_lane && counted >= 0 && before + 1 == (uint32_t)t.ranges) {
-      t.arrived[counted] = 0; // for the next launch
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+      __hip_atomic_store(t.arrived + counted, 0u, __ATOMIC_RELAXED, // for the next launch
+                         __HIP_MEMORY_SCOPE_AGENT);
       t.tick_host[counted] = (uint64_t)wall_clock64();
       __hip_atomic_store(t.landed + counted, t.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
       __hip_atomic_store(t.landed_host + counted, t.epoch, __ATOMIC_RELEASE,

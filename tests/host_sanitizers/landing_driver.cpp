@@ -1,6 +1,6 @@
 // The counting and announcing of batches by the wavefronts of a single-launch restore
 // (fkv_landing.h) and the streams that wait for them, without the copies: wavefronts as state machines that take turns in a seeded
-// order, some of them slow, every word checked after every step.
+// order, some of them slow, every word checked after every step; and as host threads, for ThreadSanitizer.
 #include "cpu_device_model.h"
 
 #include "fkv_landing.h"
@@ -107,6 +107,47 @@ void turns(uint64_t seed) {
   }
 }
 
+// Wavefronts as host threads, copies as plain stores: whoever has seen the words of a batch and of
+// all before it reads every byte of them.
+void threads(uint64_t seed) {
+  Rng rng(seed);
+  Words w(pick(rng, 1, 10), pick(rng, 1, 6));
+  w.t.epoch = 7;
+  std::vector<int> bytes(w.parts(), 0); // what the copies write: plain memory
+  std::atomic<int> next{0}, ready{0};
+  std::vector<std::thread> all;
+  for (int i = 0; i < 6; ++i)
+    all.emplace_back([&] {
+      fkv::Landing landing(w.t, true);
+      ready.fetch_add(1, std::memory_order_relaxed);
+      while (ready.load(std::memory_order_relaxed) < 6) // all of them get some of the work
+        std::this_thread::yield();
+      for (int part; (part = next.fetch_add(1, std::memory_order_relaxed)) < w.parts();) {
+        landing.announce();
+        if (landing.copied >= 0)
+          landing.count();
+        bytes[part] = part + 1;
+        landing.announce();
+        landing.copied = w.batch_of(part);
+        std::this_thread::yield();
+      }
+      landing.announce();
+      if (landing.copied >= 0)
+        landing.count();
+      landing.announce();
+    });
+  for (int reader = 0; reader < 2; ++reader)
+    all.emplace_back([&, only = pick(rng, 0, w.t.batches - 1), host = reader == 1] {
+      for (int b = 0; b <= only; ++b)
+        while (__atomic_load_n((host ? w.t.landed_host : w.t.landed) + b, __ATOMIC_ACQUIRE) < w.t.epoch)
+          std::this_thread::yield();
+      for (int part = 0; part < (only + 1) * w.t.ranges; ++part)
+        REQUIRE(bytes[part] == part + 1, "seed %llu: batch %d, part %d", (unsigned long long)seed, only, part);
+    });
+  for (auto &t : all)
+    t.join();
+}
+
 // Words written in any order: a stream that waits for one batch goes on when every word up to
 // that one is there, at the device's words and at those the host sees.
 void any_order(uint64_t seed, hipStream_t stream) {
@@ -152,11 +193,13 @@ int main(int argc, char **argv) {
   const int cases = argc > 1 ? atoi(argv[1]) : 100;
   for (int i = 0; i < cases; ++i)
     turns(31000 + i);
+  for (int i = 0; i < cases; ++i)
+    threads(32000 + i);
   hipStream_t stream = nullptr;
   REQUIRE(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) == hipSuccess, "stream");
   for (int i = 0; i < cases / 4; ++i)
     any_order(33000 + i, stream);
   REQUIRE(hipStreamDestroy(stream) == hipSuccess, "stream");
-  printf("ok: %d landings by turns\n", cases);
+  printf("ok: %d landings by turns and by threads\n", cases);
   return 0;
 }

@@ -280,7 +280,7 @@ def test_single_launch_restores_under_sanitizers(tmp_path, sanitizer, kernels_fr
 def test_landing_of_batches_and_waits_for_them(tmp_path, sanitizer):
     """The counting and announcing of a single-launch restore (fkv_landing.h): wavefronts take
     turns in seeded orders, some of them slow, and a batch is announced when it has landed, not
-    sooner; a stream that waits for a batch goes on when it and all before it are there, in
+    sooner, and its bytes are ordered before the announcement (as threads); a stream that waits for a batch goes on when it and all before it are there, in
     whatever order the words are written."""
     exe = build_over_emulated_runtime(tmp_path, "landing_driver.cpp", sanitizer,
                                       kernels_from_source=True)
@@ -288,4 +288,4 @@ def test_landing_of_batches_and_waits_for_them(tmp_path, sanitizer):
                TSAN_OPTIONS="halt_on_error=1", TMPDIR=str(tmp_path))
     r = subprocess.run([exe, "300"], capture_output=True, text=True, env=env, timeout=300)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-6000:]
-    assert "ok: 300 landings by turns" in r.stdout
+    assert "ok: 300 landings by turns and by threads" in r.stdout
