@@ -1286,10 +1286,7 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
       g->notify(*g->batches[b]);
     }
     g->join_feeder();
-    // Every batch of a single launch has been seen to land: nothing is left to wait for, unless
-    // the times of its event are asked for.
-    for (int i = 0; i < g->num_gpus && (!g->one_launch || c.enable_trace);
-         ++i) { // csrc/layerwise.cpp:1249-1256, 1634-1642
+    for (int i = 0; i < g->num_gpus; ++i) { // csrc/layerwise.cpp:1249-1256, 1634-1642
       (void)hipSetDevice(g->device_ids[i]);
       hipError_t e = quiet_stream_wait(g->streams[i], g->device_ids[i]);
       if (e != hipSuccess) {

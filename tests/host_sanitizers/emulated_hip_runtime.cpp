@@ -156,6 +156,12 @@ struct Hold {
   }
 };
 Hold g_hold;
+// How long a restore in one launch goes on after its last batch has landed (fkv_emulated_kernel_tail).
+std::atomic<long> g_tail_us{0};
+void kernel_tail() {
+  if (const long us = g_tail_us.load(std::memory_order_relaxed))
+    std::this_thread::sleep_for(std::chrono::microseconds(us));
+}
 
 struct Runtime {
   std::mutex mu;
@@ -671,6 +677,7 @@ void launch(hipStream_t stream, dim3 grid, dim3 block, size_t lds_bytes, std::fu
           c.xcc = (x + number * 3) % 8;
           c.run_workgroup(work_item, Index{x, y, z}, block_ext, grid_ext);
         }
+    kernel_tail();
   });
 }
 } // namespace cpu_device_model
@@ -773,6 +780,7 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
       __atomic_store_n(t.landed + b, t.epoch, __ATOMIC_RELEASE);
       __atomic_store_n(t.landed_host + b, t.epoch, __ATOMIC_RELEASE);
     }
+    kernel_tail();
   });
   return FKV_OK;
 }
@@ -843,8 +851,10 @@ extern "C" long fkv_emulated_fail(int category, long after, long count) {
   return g_failed_calls.load();
 }
 
-// Test hooks: kernels that have not begun wait while `on`; the device's clock runs `factor`
-// times as fast as the real one (the CPU device model).
+// Test hooks: kernels that have not begun wait while `on`; a kernel's work is done this long
+// before the kernel is; the device's clock runs `factor` times as fast as the real one (the CPU
+// device model).
+extern "C" void fkv_emulated_kernel_tail(long us) { g_tail_us.store(us); }
 extern "C" void fkv_emulated_hold_kernels(int on) { g_hold.set(on != 0); }
 extern "C" void fkv_emulated_clock_speed(long factor) {
 #ifdef FKV_KERNELS_FROM_SOURCE

@@ -26,6 +26,7 @@ long fkv_emulated_fail(int category, long after, long count); // emulated_hip_ru
 unsigned long long fkv_emulated_workgroups_run();
 void fkv_emulated_hold_kernels(int on);
 void fkv_emulated_clock_speed(long factor);
+void fkv_emulated_kernel_tail(long us);
 }
 
 #define REQUIRE(cond, ...)                                                                          \
@@ -241,6 +242,25 @@ void held_up_case(uint64_t seed) {
   g.destroy();
 }
 
+// A call that returns when everything has landed (HOSTFUNC) leaves nothing running: the times of
+// its batches are there, and whatever it used is free.
+void drained_case(uint64_t seed) {
+  Rng rng(seed);
+  Group g(rng, 2, 3, 1, 3, 8192);
+  fkv_emulated_kernel_tail(3000);
+  for (int rep = 0; rep < 3; ++rep) {
+    g.refill(rng);
+    REQUIRE(g.restore(rng, 2, 1, FKV_NOTIFY_HOSTFUNC) == FKV_OK, "restore");
+    float ms[3];
+    int32_t count = 0;
+    REQUIRE(fkv_layerwise_batch_times_ms(g.g, ms, 3, &count) == FKV_OK && count == 3,
+            "the call returned before its streams had drained");
+    g.check("drained");
+  }
+  fkv_emulated_kernel_tail(0);
+  g.destroy();
+}
+
 // Groups that restore at the same time, each from a thread of its own.
 void several_at_once(uint64_t seed) {
   std::vector<std::thread> threads;
@@ -298,6 +318,7 @@ int main(int argc, char **argv) {
   for (int i = 0; i < cases; ++i)
     seeded_case(21000 + i);
   held_up_case(20500);
+  drained_case(20600);
   for (int i = 0; i < (cases + 3) / 4; ++i)
     several_at_once(22000 + i);
   for (int i = 0; i < cases; ++i)
