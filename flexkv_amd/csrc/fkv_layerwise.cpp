@@ -239,11 +239,12 @@ struct fkv_layerwise {
   // either way).  Created with the first; nullptr = all copies on the first.
   std::vector<hipStream_t> dma_streams2;
   std::vector<unsigned> dma_turn;
-  // Restores by kernel in small batches: every other batch is launched on a second stream
-  // per GPU, which starts behind the first batch of the call (and so behind its plan
-  // uploads) and is joined back into `streams` before the plans are released, so that a batch starts while its predecessor's last requests are in
-  // flight and its event is being recorded (8 us between two launches on one stream,
-  // next to 18 us of link time for 1 MiB).  Created on first use.
+  // Restores by kernel in small batches that are not a single launch: every other batch is
+  // launched on a second stream per GPU, which starts behind the first batch of the call (and so
+  // behind its plan uploads) and is joined back into `streams` before the plans are released, so
+  // that a batch starts while its predecessor's last requests are in flight and its event is
+  // being recorded (8 us between two launches on one stream, next to 18 us of link time for
+  // 1 MiB).  Created on first use.
   std::vector<hipStream_t> alt_streams;
   std::vector<hipEvent_t> alt_join;
   std::map<std::pair<int, int>, fkv::StagedRing> rings;
@@ -559,9 +560,8 @@ bool fits_one_launch(const fkv_layerwise *g, const std::vector<Lane> &lanes, int
     if (lanes[k].used)
       return false;
   const fkv_launch_policy pol = policy_of(g->device_ids[i]);
-  // tests of a restore that ends part-way, and callers who asked for batches on two streams
-  if (pol.test_fail_restore_batch > 0 ||
-      (pol.kernel_alt_stream_kb > 0 && (int)g->batches.size() >= kAltMinBatches))
+  // tests of a restore that ends part-way, and callers who asked for batches on one stream or two
+  if (pol.test_fail_restore_batch > 0 || pol.kernel_alt_stream_kb >= 0)
     return false;
   return layers_launch_fits(lanes[0].plans[i]);
 }

@@ -797,9 +797,10 @@ typedef struct fkv_launch_policy {
                                  the last requests of its predecessor are in flight (two launches
                                  on one stream lie 8 us apart, next to 18 us of link time for
                                  1 MiB); events, notifications and wait_layer stay per batch and
-                                 in order.  0 = one stream; -1 (default): a restore of one layer
-                                 group goes out as a single launch that announces its batches
-                                 itself where its shape allows that, and as with 4096 otherwise */
+                                 in order.  0 = every batch on one stream.  -1 (default): a
+                                 restore of one layer group goes out as a single launch that
+                                 announces its batches itself where its shape allows that, and as
+                                 with 4096 otherwise */
   int32_t quiet_wait_us;        /* how a call waits for its transfer (sync = 1, the thread group, the
                                  layerwise restore in HOSTFUNC mode, fkv_layerwise_synchronize): the
                                  runtime's own waits keep a core busy for as long as they last (a

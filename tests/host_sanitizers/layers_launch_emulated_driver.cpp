@@ -261,6 +261,23 @@ void drained_case(uint64_t seed) {
   g.destroy();
 }
 
+// kernel_alt_stream_kb chosen by the caller: batch by batch, on one stream (0) or two.
+void by_policy(uint64_t seed) {
+  Rng rng(seed);
+  for (int layers : {3, 13}) // fewer and more batches than two streams are worth
+    for (int alt_kb : {-1, 0, 1, 4096}) {
+      Group g(rng, 1, layers, 1, 2, 8192);
+      set_policy(alt_kb);
+      const uint64_t before = launches();
+      REQUIRE(g.restore(rng, 2, 1, FKV_NOTIFY_HOSTFUNC) == FKV_OK, "restore");
+      REQUIRE(launches() - before == (uint64_t)(alt_kb < 0 ? 1 : layers),
+              "kernel_alt_stream_kb %d, %d batches: %d launches", alt_kb, layers, (int)(launches() - before));
+      g.check("by policy");
+      g.destroy();
+    }
+  set_policy();
+}
+
 // Groups that restore at the same time, each from a thread of its own.
 void several_at_once(uint64_t seed) {
   std::vector<std::thread> threads;
@@ -319,6 +336,7 @@ int main(int argc, char **argv) {
     seeded_case(21000 + i);
   held_up_case(20500);
   drained_case(20600);
+  by_policy(20700);
   for (int i = 0; i < (cases + 3) / 4; ++i)
     several_at_once(22000 + i);
   for (int i = 0; i < cases; ++i)

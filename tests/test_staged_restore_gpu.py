@@ -251,6 +251,7 @@ def test_small_batches_by_kernel_alternate_over_two_streams(gpu_device, notify):
             st = get_stats()
         # batches 2, 4, .. 16 of 17
         assert st["second_stream_batches"] == (8 if alt_kb else 0), st
+        assert st["kernel_launches"] == L, st
         s.oracle_transfer(gids, cids, True)
         dev.assert_matches_reference(f"restore {rep}, second stream {'on' if alt_kb else 'off'}")
         for l in range(L):
