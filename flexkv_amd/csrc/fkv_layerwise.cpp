@@ -77,8 +77,10 @@ LandedPool &landed_pool() {
   static LandedPool *p = new LandedPool(); // lives until the process ends
   return *p;
 }
-// `device` is current.
-bool landed_words_acquire(int device, LandedWords *out) {
+// `device` is current.  New words are cleared by a kernel on `stream`, and the call waits for it:
+// a stream of the group's own that holds no more than the upload of a plan.  (A hipMemcpy waits
+// for the null stream, on which an engine may have its forward pass.)
+bool landed_words_acquire(int device, hipStream_t stream, LandedWords *out) {
   LandedPool &p = landed_pool();
   {
     std::lock_guard<std::mutex> lk(p.mu);
@@ -90,11 +92,17 @@ bool landed_words_acquire(int device, LandedWords *out) {
     }
   }
   constexpr size_t kDev = (size_t)fkv::kCopyMaxLK * 12, kHost = ((size_t)fkv::kCopyMaxLK * 2 + 1) * 8;
-  static const std::vector<uint8_t> zeros(kDev, 0);
+  static_assert(kDev <= kHost, "the device words are cleared from the host's");
   void *d = nullptr, *h = nullptr;
-  if (hipHostMalloc(&h, kHost, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess ||
-      hipMalloc(&d, kDev) != hipSuccess ||
-      hipMemcpy(d, zeros.data(), kDev, hipMemcpyHostToDevice) != hipSuccess) {
+  bool ok = hipHostMalloc(&h, kHost, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess &&
+            hipMalloc(&d, kDev) == hipSuccess;
+  if (ok) {
+    std::memset(h, 0, kHost);
+    ok = fkv::launch_plan_upload(d, h, kDev, stream) == FKV_OK;
+    ok = hipStreamSynchronize(stream) == hipSuccess && ok;
+  }
+  if (!ok) {
+    fkv::clear_error();
     (void)hipGetLastError();
     if (d)
       (void)hipFree(d);
@@ -102,7 +110,6 @@ bool landed_words_acquire(int device, LandedWords *out) {
       (void)hipHostFree(h);
     return false;
   }
-  std::memset(h, 0, kHost);
   out->dev = static_cast<uint64_t *>(d);
   out->host = static_cast<uint64_t *>(h);
   return true;
@@ -1161,7 +1168,7 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
     for (int i = 0; i < g->num_gpus && g->one_launch; ++i) {
       (void)hipSetDevice(g->device_ids[i]);
       if (!g->landed[i].dev)
-        g->one_launch = landed_words_acquire(g->device_ids[i], &g->landed[i]);
+        g->one_launch = landed_words_acquire(g->device_ids[i], g->streams[i], &g->landed[i]);
     }
   }
   for (int b = g->one_launch ? num_batches - 1 : 0; b < num_batches && rc == FKV_OK; ++b)

@@ -27,6 +27,7 @@ unsigned long long fkv_emulated_workgroups_run();
 void fkv_emulated_hold_kernels(int on);
 void fkv_emulated_clock_speed(long factor);
 void fkv_emulated_kernel_tail(long us);
+long fkv_emulated_host_waited_copies();
 }
 
 #define REQUIRE(cond, ...)                                                                          \
@@ -160,6 +161,23 @@ struct Group {
 
 int64_t some_chunk(Rng &rng) {
   return std::vector<int64_t>{8192, 8208, 18432, 8192 + 16 * pick(rng, 1, 700)}[pick(rng, 0, 3)];
+}
+
+// The words of a process's first group are set up without a copy on the null stream, which
+// would wait for whatever the engine has queued there.
+void first_words(uint64_t seed) {
+  Rng rng(seed);
+  Group g(rng, 2, 3, 1, 2, 8192);
+  set_policy(0); // plan memory and its counters: a restore of the same group, batch by batch
+  REQUIRE(g.restore(rng, 2, 1, FKV_NOTIFY_HOSTFUNC) == FKV_OK, "restore");
+  g.check("batch by batch");
+  set_policy();
+  const long before = fkv_emulated_host_waited_copies();
+  REQUIRE(g.restore(rng, 2, 1, FKV_NOTIFY_HOSTFUNC) == FKV_OK, "restore");
+  REQUIRE(fkv_emulated_host_waited_copies() == before, "%ld copies that wait for the null stream",
+          fkv_emulated_host_waited_copies() - before);
+  g.check("first words");
+  g.destroy();
 }
 
 // Restores one after the other on one group, a consumer that waits for each layer.
@@ -332,6 +350,7 @@ void refused_case(uint64_t seed) {
 int main(int argc, char **argv) {
   const int cases = argc > 1 ? atoi(argv[1]) : 20;
   set_policy();
+  first_words(20400);
   for (int i = 0; i < cases; ++i)
     seeded_case(21000 + i);
   held_up_case(20500);
