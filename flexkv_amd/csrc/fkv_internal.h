@@ -210,12 +210,15 @@ struct LayersLaunch {
   CopyKernelArgs a;
   int32_t pairs_per_batch;
   int32_t batches;
-  int32_t ranges;          // claims per batch, set by the launch
+  int32_t ranges, last_ranges; // claims of a batch and of the last one, set by the launch
   uint32_t *arrived;       // device, [batches]: ranges that have landed; zero between launches
   uint64_t *landed;        // device, [batches]: `epoch` once the batch has landed
   uint64_t *landed_host;   // the same in pinned host memory
   uint64_t *tick_host;     // pinned, [batches]: when it landed, in ticks of the 100 MHz clock
   uint64_t epoch;          // larger than that of any earlier launch
+  __host__ __device__ uint32_t ranges_of(int batch) const {
+    return (uint32_t)(batch + 1 == batches ? last_ranges : ranges);
+  }
 };
 // What of it runs on the device.  A table instead of two functions because the library's host
 // code also runs without its kernels (over the emulated runtime of the sanitizer tests, which

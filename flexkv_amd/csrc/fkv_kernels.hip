@@ -897,12 +897,13 @@ __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) 
   while (part < a.num_claims) {
     uint32_t ahead = a.num_claims;
     const uint32_t batch = part / (uint32_t)t.ranges, range = part - batch * (uint32_t)t.ranges;
+    const uint32_t ranges = t.ranges_of((int)batch);
     const uint32_t pair0 = batch * (uint32_t)t.pairs_per_batch;
     const uint32_t pairs = min((uint32_t)t.pairs_per_batch, (uint32_t)a.lk - pair0);
     const uint32_t spp = pairs * slices;
     const uint64_t units = (uint64_t)a.num_blocks * spp;
-    const uint64_t s0 = units * range / (uint32_t)t.ranges;
-    const uint64_t s1 = units * (range + 1) / (uint32_t)t.ranges;
+    const uint64_t s0 = units * range / ranges;
+    const uint64_t s1 = units * (range + 1) / ranges;
     for (uint64_t s = s0; s < s1; ++s) {
       const uint32_t p = (uint32_t)(s / spp);
       const uint32_t r = (uint32_t)(s - (uint64_t)p * spp);
@@ -979,27 +980,20 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
   // 677; next to a fused attention 2858 / 2822 / 2854).
   shape_launch(t.a, total, (int64_t)t.a.num_blocks * t.a.lk * t.a.chunk_bytes, grid_pct * 3 / 2,
                num_workgroups, kWave, &grid, &threads);
-  // Ranges of 128 KiB, or smaller ones where the whole restore would not make two rounds of
-  // the workgroups that take part; none is empty, also in the last batch, which may be shorter
-  // than the others.  A batch need not go round the workgroups: they run on into the next one.
-  // (Ranges of 64 KiB, and as many a batch as there are workgroups: 32 layers of 1 MiB 703 us
-  // instead of 694, 61 of 7 MiB 7.90 ms instead of 7.78; of 256 KiB: 720 us and 7.71 ms.)
-  const int64_t per_pair = (int64_t)t.a.num_blocks * t.a.slices_per_chunk;
-  const int64_t last_pairs = t.a.lk - (int64_t)(t.batches - 1) * t.pairs_per_batch;
   const uint32_t present = t.a.xcd_present ? t.a.xcd_present : 0xffu;
   const int64_t working =
       t.a.xcd_mask ? grid * __builtin_popcount(t.a.xcd_mask & present) /
                          std::max(1, __builtin_popcount(present))
                    : grid;
-  const int64_t ranges = std::min(
-      per_pair * last_pairs,
-      std::max({(int64_t)1, (2 * working + t.batches - 1) / t.batches,
-                per_pair * t.pairs_per_batch / 16}));
-  if (last_pairs < 1 || ranges * t.batches > (int64_t)INT32_MAX)
+  const int64_t last_pairs = t.a.lk - (int64_t)(t.batches - 1) * t.pairs_per_batch;
+  const LayersCut cut = cut_layers(t.batches, t.pairs_per_batch, last_pairs,
+                                   (int64_t)t.a.num_blocks * t.a.slices_per_chunk, working);
+  if (last_pairs < 1 || cut.claims(t.batches) > (int64_t)INT32_MAX)
     return fail(FKV_ERR_RUNTIME, "copy kernel: %d batches of %d of %d (layer, kv) pairs", t.batches,
                 t.pairs_per_batch, t.a.lk);
-  t.ranges = (int32_t)ranges;
-  t.a.num_claims = (uint32_t)(ranges * t.batches);
+  t.ranges = (int32_t)cut.ranges;
+  t.last_ranges = (int32_t)cut.last_ranges;
+  t.a.num_claims = (uint32_t)cut.claims(t.batches);
   hipLaunchKernelGGL(fkv_copy_layers_kernel, dim3((unsigned)grid), dim3(kWave), 0, stream, t);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess)

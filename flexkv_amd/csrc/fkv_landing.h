@@ -5,7 +5,29 @@
 
 #include "fkv_internal.h"
 
+#include <algorithm>
+
 namespace fkv {
+
+// How a restore of `batches` batches of `pairs_per_batch` (layer, kv) pairs, the last one of
+// `last_pairs`, each of `per_pair` slices, is cut for `working` wavefronts.  Ranges of 16 slices
+// (128 KiB), or smaller ones where the whole restore would not make two rounds of the wavefronts;
+// the last batch, which may be shorter than the others, into ranges of about the same size.  None
+// is empty.  A batch need not go round the wavefronts: they run on into the next one.  (Ranges of
+// 64 KiB, and as many a batch as there are wavefronts: 32 layers of 1 MiB 703 us instead of 694,
+// 61 of 7 MiB 7.90 ms instead of 7.78; of 256 KiB: 720 us and 7.71 ms.)
+struct LayersCut {
+  int64_t ranges = 0, last_ranges = 0; // of a batch, of the last one (no more than that)
+  int64_t claims(int64_t batches) const { return ranges * (batches - 1) + last_ranges; }
+};
+inline LayersCut cut_layers(int64_t batches, int64_t pairs_per_batch, int64_t last_pairs,
+                            int64_t per_pair, int64_t working) {
+  const int64_t slices = per_pair * pairs_per_batch, one = 1;
+  LayersCut c;
+  c.ranges = std::min(slices, std::max({one, (2 * working + batches - 1) / batches, slices / 16}));
+  c.last_ranges = (c.ranges * last_pairs + pairs_per_batch - 1) / pairs_per_batch;
+  return c;
+}
 
 // One wavefront's part.  Wavefronts run on from batch to batch and the last ranges of several
 // batches are under way together, so a batch may be announced before an earlier one: whoever
@@ -36,7 +58,7 @@ struct Landing {
   // release of what they wrote; the acquire makes what they wrote part of what the words release.  (On this
   // chip each of them has written its L2 back before it counted, and nothing would be missing.)
   __device__ __forceinline__ void announce() {
-    if (first_lane && counted >= 0 && before + 1 == (uint32_t)t.ranges) {
+    if (first_lane && counted >= 0 && before + 1 == t.ranges_of(counted)) {
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
       __hip_atomic_store(t.arrived + counted, 0u, __ATOMIC_RELAXED, // for the next launch
                          __HIP_MEMORY_SCOPE_AGENT);

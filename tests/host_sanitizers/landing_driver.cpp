@@ -25,16 +25,33 @@ namespace {
 using Rng = std::mt19937_64;
 int pick(Rng &rng, int lo, int hi) { return lo + (int)(rng() % (uint64_t)(hi - lo + 1)); }
 
+// How a restore is cut: no empty range, whatever the last batch is; no range of more than 16 or so
+// slices, and enough of them for every wavefront, as far as there are slices.
+void cuts(uint64_t seed) {
+  Rng rng(seed);
+  const int64_t pairs = pick(rng, 1, 64), batches = pick(rng, 1, 40), last = pick(rng, 1, (int)pairs),
+                per_pair = std::vector<int>{1, 2, 7, 100, 5000}[pick(rng, 0, 4)], working = pick(rng, 1, 96);
+  const fkv::LayersCut c = fkv::cut_layers(batches, pairs, last, per_pair, working);
+  const int64_t slices = pairs * per_pair;
+  REQUIRE(c.ranges >= 1 && c.ranges <= slices && c.last_ranges >= 1 && c.last_ranges <= last * per_pair &&
+              c.last_ranges <= c.ranges, "seed %llu: an empty range", (unsigned long long)seed);
+  REQUIRE(c.ranges == slices || (c.ranges * 32 > slices && c.ranges * batches >= 2 * working),
+          "seed %llu: %lld ranges of %lld slices for %lld wavefronts", (unsigned long long)seed,
+          (long long)c.ranges, (long long)slices, (long long)working);
+  REQUIRE(c.last_ranges == last * per_pair || c.last_ranges * pairs >= c.ranges * last,
+          "seed %llu: longer ranges in the last batch", (unsigned long long)seed);
+}
+
 struct Words {
   std::vector<uint32_t> arrived;
   std::vector<uint64_t> landed, landed_host, ticks;
   fkv::LayersLaunch t{};
-  Words(int batches, int ranges) : arrived(batches), landed(batches), landed_host(batches), ticks(batches) {
-    t.batches = batches, t.ranges = ranges;
+  Words(int batches, int ranges, int last_ranges) : arrived(batches), landed(batches), landed_host(batches), ticks(batches) {
+    t.batches = batches, t.ranges = ranges, t.last_ranges = last_ranges;
     t.arrived = arrived.data(), t.landed = landed.data();
     t.landed_host = landed_host.data(), t.tick_host = ticks.data();
   }
-  int parts() const { return t.ranges * t.batches; }
+  int parts() const { return t.ranges * (t.batches - 1) + t.last_ranges; }
   int batch_of(int part) const { return part / t.ranges; }
 };
 
@@ -81,7 +98,8 @@ struct Wavefront {
 
 void turns(uint64_t seed) {
   Rng rng(seed);
-  Words w(pick(rng, 1, 12), pick(rng, 1, 5));
+  const int ranges = pick(rng, 1, 5);
+  Words w(pick(rng, 1, 12), ranges, pick(rng, 1, ranges));
   const int waves = pick(rng, 1, 9);
   for (w.t.epoch = 1; w.t.epoch <= 3; ++w.t.epoch) {
     std::vector<Wavefront> wave(waves, Wavefront(w));
@@ -94,7 +112,7 @@ void turns(uint64_t seed) {
       if (pick(rng, 1, 100) <= speed[i])
         wave[i].step(w, &next, &counted);
       for (int b = 0; b < w.t.batches; ++b)
-        REQUIRE(counted[b] == w.t.ranges || (w.landed[b] < w.t.epoch && w.landed_host[b] < w.t.epoch),
+        REQUIRE(counted[b] == (int)w.t.ranges_of(b) || (w.landed[b] < w.t.epoch && w.landed_host[b] < w.t.epoch),
                 "seed %llu: batch %d of %d announced before it had landed",
                 (unsigned long long)seed, b, w.t.batches);
       busy = false;
@@ -111,7 +129,8 @@ void turns(uint64_t seed) {
 // all before it reads every byte of them.
 void threads(uint64_t seed) {
   Rng rng(seed);
-  Words w(pick(rng, 1, 10), pick(rng, 1, 6));
+  const int ranges = pick(rng, 1, 6);
+  Words w(pick(rng, 1, 10), ranges, pick(rng, 1, ranges));
   w.t.epoch = 7;
   std::vector<int> bytes(w.parts(), 0); // what the copies write: plain memory
   std::atomic<int> next{0}, ready{0};
@@ -141,7 +160,7 @@ void threads(uint64_t seed) {
       for (int b = 0; b <= only; ++b)
         while (__atomic_load_n((host ? w.t.landed_host : w.t.landed) + b, __ATOMIC_ACQUIRE) < w.t.epoch)
           std::this_thread::yield();
-      for (int part = 0; part < (only + 1) * w.t.ranges; ++part)
+      for (int part = 0; part < w.parts() && w.batch_of(part) <= only; ++part)
         REQUIRE(bytes[part] == part + 1, "seed %llu: batch %d, part %d", (unsigned long long)seed, only, part);
     });
   for (auto &t : all)
@@ -152,7 +171,7 @@ void threads(uint64_t seed) {
 // that one is there, at the device's words and at those the host sees.
 void any_order(uint64_t seed, hipStream_t stream) {
   Rng rng(seed);
-  Words w(pick(rng, 1, 150), 1);
+  Words w(pick(rng, 1, 150), 1, 1);
   w.t.epoch = 5;
   uint64_t given_up = 4;
   hipEvent_t behind = nullptr;
@@ -191,6 +210,8 @@ void any_order(uint64_t seed, hipStream_t stream) {
 
 int main(int argc, char **argv) {
   const int cases = argc > 1 ? atoi(argv[1]) : 100;
+  for (int i = 0; i < 20 * cases; ++i)
+    cuts(30000 + i);
   for (int i = 0; i < cases; ++i)
     turns(31000 + i);
   for (int i = 0; i < cases; ++i)

@@ -278,7 +278,8 @@ def test_single_launch_restores_under_sanitizers(tmp_path, sanitizer, kernels_fr
 
 @pytest.mark.parametrize("sanitizer", SANITIZERS)
 def test_landing_of_batches_and_waits_for_them(tmp_path, sanitizer):
-    """The counting and announcing of a single-launch restore (fkv_landing.h): wavefronts take
+    """The cut into ranges, the counting and announcing of a single-launch restore
+    (fkv_landing.h): ranges of like size in all batches, none empty; wavefronts take
     turns in seeded orders, some of them slow, and a batch is announced when it has landed, not
     sooner, and its bytes are ordered before the announcement (as threads); a stream that waits for a batch goes on when it and all before it are there, in
     whatever order the words are written."""

@@ -20,6 +20,8 @@ SHAPES = [
     (TRTLLM, 3, 2, 16384, 129, 1),
     (VLLM, 3, 1, 8192, 1025, 2),        # more blocks than an id tile, above the home-XCD size
     (VLLM, 600, 1, 8192, 2, 7),         # many batches
+    (VLLM, 33, 1, 16384, 1, 32),        # a last batch of a single block and layer
+    (SGLANG, 11, 2, 18432, 9, 5),
 ]
 POLICIES = dict(default={}, confined=dict(arbiter=2), safety_net=dict(arbiter=3),
                 everywhere=dict(arbiter=0))
