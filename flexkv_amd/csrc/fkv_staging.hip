@@ -243,11 +243,7 @@ int fkv_staging_transfer(const fkv_staging_transfer_desc *dp, void *stream_v) tr
   // payloads, whose last slice is short: twice the workgroups of the fixed-size
   // kernel make up for it (16-29 KiB payloads: 45 GB/s with 16 wavefronts, 55.0 with
   // 24, 55.7 with 32).
-  // Writing, the short last slices leave a third of the bytes in flight out, and as many
-  // workgroups more make up for it (us, 48 / 64 / 96 wavefronts: 2048 payloads of 16-29 KiB
-  // 887 / 877 / 866, of 4-7 KiB in 8 KiB slots, with adjacent vectors 259 / 249; more would
-  // cost the kernels next to them more than they bring).
-  int grid = cta * (write_cpu ? (pol.d2h_wg_per_cta * 4 + 2) / 3 : 2 * pol.h2d_wg_per_cta);
+  int grid = cta * (write_cpu ? pol.d2h_wg_per_cta : 2 * pol.h2d_wg_per_cta);
   const int threads = write_cpu ? pol.d2h_wg_threads : pol.h2d_wg_threads;
   grid = std::max(1, std::min(grid, (d.bsz + threads / 64 - 1) / (threads / 64)));
 #define FKV_LAUNCH_STAGING(...)                                                               \
