@@ -252,14 +252,14 @@ int fkv_staging_transfer(const fkv_staging_transfer_desc *dp, void *stream_v) tr
   // Adjacent vectors per lane on the same terms as the fixed-size kernel: not next to a
   // transfer from the host, where the plain order moves 2 % more in sum.  And only for calls
   // that fill the link for a while: the loads of a slice take longer in this order, which a
-  // short call waits for.  With 64 wavefronts (us, plain / adjacent): 96 payloads of 16-29 KiB
-  // 51 / 53, 256 124 / 128, 384 181 / 182-191, 768 351 / 336, 2048 877 / 857; 512 of 4-7 KiB
-  // 69 / 72.  With 48: 2048 of 9-16 KiB in 18 KiB slots 527 / 502.
-  constexpr int kRunsMinPayloads = 16; // per wavefront
-  const bool runs = d.bsz / kRunsMinPayloads >= grid * (threads / 64) &&
-                    (pol.d2h_lane_runs == 2 ||
-                     (pol.d2h_lane_runs == 1 &&
-                      !(pol.arbiter != 0 && link_direction_busy(device, /*h2d=*/true, stream))));
+  // shorter call waits for.  The line lies at the same bytes for all sizes (us, plain / adjacent,
+  // by MiB of slots 50-90 % full): slots of 2 KiB 8: 219 / 241, 16: 415 / 403, 24: 603 / 553;
+  // 4 KiB 8: 173 / 188, 16: 320 / 308, 24: 455 / 425; 8 KiB 8: 153 / 163, 12: 216 / 222,
+  // 16: 283 / 274; 32 KiB 8: 143 / 150, 12: 201 / 201, 16: 260 / 254, 48: 687 / 679.
+  constexpr int64_t kRunsMinBytes = 16 << 20; // of slots
+  const bool runs = pol.d2h_lane_runs == 2 ||
+                    (pol.d2h_lane_runs == 1 && d.bsz * d.staging_stride >= kRunsMinBytes &&
+                     !(pol.arbiter != 0 && link_direction_busy(device, /*h2d=*/true, stream)));
   if (write_cpu && vec16 && runs)
     FKV_LAUNCH_STAGING(true, true, true);
   else if (write_cpu && vec16)
