@@ -731,9 +731,10 @@ CopyKernelArgs plan_job(const KernelPlan &p, int l0, int nl) {
 
 // Which XCDs, how many workgroups and how many ranges per workgroup a launch of
 // `bytes` gets now; `a` is the (first) job of the launch.  Decided when a launch is
-// made, not when its plan is built (a layerwise restore launches for tens of
-// milliseconds after its plan was built): while the other direction is busy
-// GPU->host keeps to its busy XCDs and host->GPU to its own; on an idle link large
+// made, not when its plan is built (a layerwise restore batch by batch launches for
+// tens of milliseconds after its plan was built; one in a single launch is decided once, which
+// costs it nothing: host->GPU has the same XCDs at home and while the other direction is
+// busy): while the other direction is busy GPU->host keeps to its busy XCDs and host->GPU to its own; on an idle link large
 // launches keep to their direction's home XCDs, so that a transfer of the other
 // direction that starts while they run finds its own XCDs free.  On the home XCDs
 // a launch gets no more workgroups than on all XCDs: what a copy costs the kernels
@@ -747,7 +748,9 @@ CopyKernelArgs plan_job(const KernelPlan &p, int l0, int nl) {
 // with one range each the slowest one holds up the launch: a restore next to
 // fused-attention calls moves 37 GB/s with one range per workgroup and 54 GB/s with
 // two.
-int shape_for_now(const KernelPlan &p, int64_t bytes, hipStream_t stream, CopyKernelArgs *a) {
+// `beside` (may be null): whether the launch is shaped to run next to the other direction.
+int shape_for_now(const KernelPlan &p, int64_t bytes, hipStream_t stream, CopyKernelArgs *a,
+                  bool *beside = nullptr) {
   const fkv_launch_policy pol = p.no_alloc ? policy_peek(p.device) : policy_of(p.device);
   int workgroups = p.workgroups;
   const uint32_t all = pol.xcd_present_mask;
@@ -773,6 +776,8 @@ int shape_for_now(const KernelPlan &p, int64_t bytes, hipStream_t stream, CopyKe
     workgroups = busy_workgroups;
     a->claims_per_wg = pol.busy_claims_per_wg;
     a->lane_runs = !p.h2d && pol.d2h_lane_runs == 2; // next to traffic the other way: see copy_slice
+    if (beside)
+      *beside = true;
   } else if (pol.arbiter == 1 && home_mask != all && pol.home_min_kb >= 0 &&
              bytes >= (int64_t)pol.home_min_kb * 1024) {
     a->xcd_mask = home_mask;
@@ -822,7 +827,16 @@ int kernel_plan_launch_layers(const KernelPlan &p, int layers_per_batch, LayersL
   t.a = plan_job(p, 0, p.num_layers);
   t.pairs_per_batch = layers_per_batch * p.kv_dim;
   t.batches = (p.num_layers + layers_per_batch - 1) / layers_per_batch;
-  const int workgroups = shape_for_now(p, bytes, stream, &t.a);
+  bool beside = false;
+  const int workgroups = shape_for_now(p, bytes, stream, &t.a, &beside);
+  // Half as many workgroups again as for a plain copy: the fence behind every range takes a
+  // wavefront out for a few microseconds.  (16 / 20 / 24 wavefronts: 32 layers of 1 MiB 874 / 765 /
+  // 732 us, 61 of 7 MiB 9.52 / 8.23 / 7.84 ms; next to the latter three 2048^3 GEMMs take 118 /
+  // 121 / 126 us, 80 alone, a fused attention 112 / 113 / 115, 82 alone.)  Next to a transfer the
+  // other way there are half as many again already, and more would slow that one down: a put of
+  // 512 MiB takes 10.97 instead of 12.56 ms with 24 instead of 36 wavefronts beside it, the restore
+  // 10.35 instead of 8.49, both together 11.16 instead of 12.71 ms.
+  t.grid_pct = beside ? 100 : 150;
   FKV_TRY(layers_device->launch(t, workgroups, stream));
   link_direction_mark(p.device, p.h2d, stream, bytes);
   return FKV_OK;

@@ -210,6 +210,7 @@ struct LayersLaunch {
   CopyKernelArgs a;
   int32_t pairs_per_batch;
   int32_t batches;
+  int32_t grid_pct;        // host side: workgroups to launch, percent of a plain copy's
   int32_t ranges, last_ranges; // claims of a batch and of the last one, set by the launch
   uint32_t *arrived;       // device, [batches]: ranges that have landed; zero between launches
   uint64_t *landed;        // device, [batches]: `epoch` once the batch has landed

@@ -975,11 +975,8 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
     return fail(FKV_ERR_RUNTIME, "copy kernel: a restore of this shape has no single launch");
   int64_t grid = 1;
   int threads = kWave;
-  // Half as many workgroups again as for a plain copy: the fence behind every range takes a
-  // wavefront out for a few microseconds (32 layers of 1 MiB: 16 wavefronts 881 us, 24 713, 32
-  // 677; next to a fused attention 2858 / 2822 / 2854).
-  shape_launch(t.a, total, (int64_t)t.a.num_blocks * t.a.lk * t.a.chunk_bytes, grid_pct * 3 / 2,
-               num_workgroups, kWave, &grid, &threads);
+  shape_launch(t.a, total, (int64_t)t.a.num_blocks * t.a.lk * t.a.chunk_bytes,
+               grid_pct * t.grid_pct / 100, num_workgroups, kWave, &grid, &threads);
   const uint32_t present = t.a.xcd_present ? t.a.xcd_present : 0xffu;
   const int64_t working =
       t.a.xcd_mask ? grid * __builtin_popcount(t.a.xcd_mask & present) /

@@ -296,6 +296,55 @@ void by_policy(uint64_t seed) {
   set_policy();
 }
 
+// Next to a transfer from the GPU a restore asks for no more workgroups than a launch per batch
+// does: the writer pays for them.  (Workgroups launched, confined ones of which half the XCDs'
+// stay; only where the kernel itself runs.)
+void next_to_a_put(uint64_t seed) {
+  Rng rng(seed);
+  Group g(rng, 1, 8, 1, 16, 8192);
+  std::vector<uint64_t> ptrs;
+  for (uint8_t *d : g.dev)
+    ptrs.push_back((uint64_t)(uintptr_t)d);
+  std::vector<int64_t> ids{0};
+  hipStream_t other = nullptr;
+  REQUIRE(hipStreamCreateWithFlags(&other, hipStreamNonBlocking) == hipSuccess, "stream");
+  fkv_launch_policy p{};
+  REQUIRE(fkv_launch_policy_get(0, &p) == FKV_OK, "policy");
+  p.busy_window_ms = 20000; // a put counts for as long as this program runs
+  REQUIRE(fkv_launch_policy_set(0, &p) == FKV_OK, "policy");
+  uint8_t *sink = nullptr;
+  REQUIRE(hipHostMalloc((void **)&sink, (size_t)g.block(), 0) == hipSuccess, "sink");
+  fkv_transfer_desc d{};
+  d.backend = FKV_BACKEND_VLLM;
+  d.num_layers_total = d.num_layers = d.num_gpu_tensor_ptrs = g.layers;
+  d.gpu_tensor_ptrs = ptrs.data();
+  d.device = 0;
+  d.gpu_kv_stride = d.gpu_layer_stride = (int64_t)g.layer_bytes();
+  d.gpu_block_stride = d.cpu_kv_stride = d.cpu_layer_stride = d.chunk_size = g.chunk;
+  d.cpu_ptr = sink;
+  d.cpu_block_stride = g.block();
+  d.kv_dim = d.num_blocks = d.sync = 1;
+  d.gpu_block_ids = d.cpu_block_ids = ids.data();
+  d.transfer_num_cta = 4;
+  fkv_ce_config_default(&d.ce);
+  REQUIRE(fkv_transfer_kv_blocks(&d, other) == FKV_OK, "put");
+  auto workgroups = [&](int alt_kb) {
+    p.kernel_alt_stream_kb = alt_kb;
+    REQUIRE(fkv_launch_policy_set(0, &p) == FKV_OK, "policy");
+    const unsigned long long before = fkv_emulated_workgroups_run();
+    const uint64_t launched = launches();
+    g.refill(rng);
+    REQUIRE(g.restore(rng, 16, 4, FKV_NOTIFY_HOSTFUNC) == FKV_OK, "restore");
+    g.check("next to a put");
+    return (fkv_emulated_workgroups_run() - before) / (launches() - launched);
+  };
+  const unsigned long long batches = workgroups(0), single = workgroups(-1);
+  REQUIRE(single <= batches, "%llu workgroups, %llu of a launch per batch", single, batches);
+  REQUIRE(hipHostFree(sink) == hipSuccess && hipStreamDestroy(other) == hipSuccess, "free");
+  set_policy();
+  g.destroy();
+}
+
 // Groups that restore at the same time, each from a thread of its own.
 void several_at_once(uint64_t seed) {
   std::vector<std::thread> threads;
@@ -356,6 +405,7 @@ int main(int argc, char **argv) {
   held_up_case(20500);
   drained_case(20600);
   by_policy(20700);
+  next_to_a_put(20800);
   for (int i = 0; i < (cases + 3) / 4; ++i)
     several_at_once(22000 + i);
   for (int i = 0; i < cases; ++i)
