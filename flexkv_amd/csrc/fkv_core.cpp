@@ -157,7 +157,7 @@ hipError_t quiet_word_wait(const uint64_t *word, uint64_t at_least, hipEvent_t b
     if (!ask)
       continue;
     const hipError_t q = hipEventQuery(behind); // the kernel may have ended in an error
-    if (q == hipErrorNotReady) {
+    if (q == hipErrorNotReady || capture_forbids(q)) {
       (void)hipGetLastError();
     } else if (q != hipSuccess) {
       return q;

@@ -39,6 +39,11 @@ hipError_t quiet_stream_wait(hipStream_t stream, int device);
 // The same for a word in pinned host memory that a kernel raises to `at_least` before
 // `behind`, recorded behind the kernel, is reached.
 hipError_t quiet_word_wait(const uint64_t *word, uint64_t at_least, hipEvent_t behind, int device);
+// The runtime gave no answer because some thread is capturing a stream: says nothing about the
+// work that was asked about.
+inline bool capture_forbids(hipError_t e) {
+  return e >= hipErrorStreamCaptureUnsupported && e <= hipErrorStreamCaptureWrongThread;
+}
 // For the catch-all handler of an entry point: turns the exception in flight into a status
 // and an error text.  No C++ exception crosses the C ABI.
 int caught(const char *where) noexcept;
@@ -229,8 +234,8 @@ struct LayersDevice {
   // Makes `stream` wait until the first `count` words of `landed` (device `device`; `landed_host`
   // are the same in pinned memory) have reached `epoch`, however long that takes, or until the
   // host has raised `given_up` (pinned) that far: the launch ended in an error, the batches
-  // never land.  `behind` lies behind the launch: a stream that is being captured is handed to
-  // it, and refused as ever.
+  // never land.  `behind` lies behind the launch: a stream that is being captured waits for
+  // that instead, which the runtime takes or refuses as it does any event from outside the capture.
   int (*wait)(const uint64_t *landed, const uint64_t *landed_host, int count, uint64_t epoch,
               const uint64_t *given_up, int device, hipEvent_t behind, hipStream_t stream);
 };

@@ -333,10 +333,10 @@ struct fkv_layerwise {
   void note_device_error(int e) {
     int none = 0;
     restore_error.compare_exchange_strong(none, e);
-    give_up_waits();
+    give_up_waits((hipError_t)e);
   }
-  void give_up_waits() {
-    if (!one_launch)
+  void give_up_waits(hipError_t e) {
+    if (!one_launch || fkv::capture_forbids(e))
       return;
     for (const LandedWords &w : landed)
       if (w.host)
@@ -364,7 +364,7 @@ struct fkv_layerwise {
             (void)hipGetLastError();
           else if (one_launch && !has_landed((int)b, g))
             return (int)hipErrorUnknown;
-          return (int)e;
+          return (int)(fkv::capture_forbids(e) ? hipErrorNotReady : e);
         },
         [this](size_t b) { notify(*batches[b]); }, poller_stop);
   }
@@ -389,6 +389,8 @@ struct fkv_layerwise {
       hipError_t e = hipStreamSynchronize(streams[g]);
       if (e != hipSuccess) {
         (void)hipGetLastError();
+        if (fkv::capture_forbids(e))
+          continue; // the poller ends with the last batch all the same
         note_device_error((int)e);
         poller_stop.store(true, std::memory_order_release);
       }
@@ -1284,7 +1286,7 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
                 : quiet_event_wait(g->batches[b]->done[i], g->device_ids[i], 0);
         if (e != hipSuccess) {
           (void)hipGetLastError();
-          g->give_up_waits();
+          g->give_up_waits(e);
           (void)hipSetDevice(restore.device());
           return fail(FKV_ERR_RUNTIME, "layerwise_transfer failed on GPU %d: %s", i,
                       hipGetErrorString(e));
@@ -1298,7 +1300,7 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
       hipError_t e = quiet_stream_wait(g->streams[i], g->device_ids[i]);
       if (e != hipSuccess) {
         (void)hipGetLastError();
-        g->give_up_waits();
+        g->give_up_waits(e);
         (void)hipSetDevice(restore.device());
         return fail(FKV_ERR_RUNTIME, "%s failed on GPU %d: %s",
                     g->multi_group ? "layerwise_transfer_multi_group" : "layerwise_transfer", i,
@@ -1531,7 +1533,7 @@ int fkv_layerwise_synchronize(fkv_layerwise *g) try {
     const hipError_t e = quiet_stream_wait(g->streams[i], g->device_ids[i]);
     if (e != hipSuccess) {
       (void)hipGetLastError();
-      g->give_up_waits();
+      g->give_up_waits(e);
       return fail(FKV_ERR_RUNTIME, "fkv_layerwise_synchronize: GPU %d: %s", i, hipGetErrorString(e));
     }
   }

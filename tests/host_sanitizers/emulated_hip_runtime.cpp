@@ -121,7 +121,7 @@ hipError_t remember(hipError_t e) {
 // calls of it fail (fkv_emulated_fail below).  What a real runtime does when memory, streams
 // or events run out, or a launch is refused.
 enum Category { kDeviceAlloc, kPinnedAlloc, kStreamCreate, kEventCreate, kCopy, kLaunch, kEventRecord,
-                kThrow, kStreamSync, kCategories };
+                kThrow, kStreamSync, kEventQuery, kCategories };
 std::atomic<long> g_fail_after[kCategories];
 std::atomic<long> g_fail_count[kCategories];
 std::atomic<long> g_failed_calls{0};
@@ -364,6 +364,8 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
 hipError_t hipEventQuery(hipEvent_t e) {
   if (!e)
     return remember(hipErrorInvalidHandle);
+  if (refused(kEventQuery)) // some thread is capturing a stream in global mode
+    return remember(hipErrorStreamCaptureUnsupported);
   std::lock_guard<std::mutex> lk(e->mu);
   return e->completed >= e->recorded ? hipSuccess : hipErrorNotReady;
 }
@@ -841,7 +843,8 @@ extern "C" long fkv_emulated_host_waited_copies() { return g_host_waited_copies.
 // Test hook: the next `count` calls of `category` (0 device allocation, 1 pinned allocation,
 // 2 stream creation, 3 event creation, 4 copy, 5 kernel launch, 6 event record; 7: a kernel
 // launch throws std::bad_alloc, as an allocation of the library's own might; 8: a stream's
-// synchronization finds that the stream ended in an error) fail once `after`
+// synchronization finds that the stream ended in an error; 9: an event is asked during a capture,
+// when the runtime does not answer) fail once `after`
 // more of them have succeeded; count 0 switches it off.  Returns the calls refused so far.
 extern "C" long fkv_emulated_fail(int category, long after, long count) {
   if (category >= 0 && category < kCategories) {

@@ -260,6 +260,43 @@ void held_up_case(uint64_t seed) {
   g.destroy();
 }
 
+// While some thread captures a stream the runtime does not answer whether an event has been
+// reached: that is no error of the restore, and nobody is let go for it.
+void no_answer_case(uint64_t seed) {
+  Rng rng(seed);
+  Group g(rng, 1, 3, 1, 3, 8192);
+  hipStream_t consumer = nullptr;
+  REQUIRE(hipStreamCreateWithFlags(&consumer, hipStreamNonBlocking) == hipSuccess, "stream");
+  std::vector<uint8_t> seen(g.layer_bytes());
+  for (int notify : {FKV_NOTIFY_POLLING, FKV_NOTIFY_HOSTFUNC}) {
+    g.refill(rng);
+    fkv_emulated_hold_kernels(1);
+    fkv_emulated_fail(9, 0, 1000000);
+    std::thread call([&] { REQUIRE(g.restore(rng, 3, 1, notify) == FKV_OK, "restore"); });
+    if (notify == FKV_NOTIFY_POLLING) {
+      call.join();
+      REQUIRE(fkv_layerwise_wait_layer(g.g, 0, 2, consumer) == FKV_OK, "wait_layer");
+      REQUIRE(hipMemcpyAsync(seen.data(), g.dev[2], g.layer_bytes(), hipMemcpyDeviceToHost, consumer) ==
+                  hipSuccess, "consumer copy");
+    }
+    std::this_thread::sleep_for(std::chrono::milliseconds(50));
+    if (notify == FKV_NOTIFY_POLLING)
+      REQUIRE(hipStreamQuery(consumer) == hipErrorNotReady, "the consumer went on without its layer");
+    fkv_emulated_hold_kernels(0);
+    if (notify == FKV_NOTIFY_HOSTFUNC)
+      call.join();
+    REQUIRE(fkv_layerwise_synchronize(g.g) == FKV_OK, "synchronize");
+    fkv_emulated_fail(9, 0, 0);
+    REQUIRE(hipStreamSynchronize(consumer) == hipSuccess, "consumer");
+    g.check("no answer");
+    REQUIRE(notify == FKV_NOTIFY_HOSTFUNC || seen == g.model[2], "the consumer saw other bytes");
+    for (size_t i = 0; i < g.fds.size(); ++i)
+      REQUIRE(g.units(i) == 1, "eventfd %zu", i);
+  }
+  REQUIRE(hipStreamDestroy(consumer) == hipSuccess, "stream");
+  g.destroy();
+}
+
 // A call that returns when everything has landed (HOSTFUNC) leaves nothing running: the times of
 // its batches are there, and whatever it used is free.
 void drained_case(uint64_t seed) {
@@ -403,6 +440,7 @@ int main(int argc, char **argv) {
   for (int i = 0; i < cases; ++i)
     seeded_case(21000 + i);
   held_up_case(20500);
+  no_answer_case(20550);
   drained_case(20600);
   by_policy(20700);
   next_to_a_put(20800);
