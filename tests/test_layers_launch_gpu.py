@@ -127,6 +127,102 @@ def test_a_consumer_of_one_layer_has_all_before_it(gpu_device, layers, blocks):
     grp.close()
 
 
+def vllm_group(s, dev, layers):
+    from flexkv_amd.c_ext import LayerwiseTransferGroup
+    i64 = lambda v: torch.tensor([v], dtype=torch.int64)  # noqa: E731
+    return LayerwiseTransferGroup(
+        num_gpus=1, gpu_blocks=[dev.gpu], cpu_blocks=dev.host, ssd_files={}, num_layers=layers,
+        gpu_kv_strides_tensor=i64(s.gpu_kv_stride), gpu_block_strides_tensor=i64(s.gpu_block_stride),
+        gpu_layer_strides_tensor=i64(s.gpu_layer_stride), gpu_chunk_sizes_tensor=i64(s.chunk),
+        iouring_entries=0, iouring_flags=0, layer_eventfds_tensor=torch.empty(0, dtype=torch.int32),
+        tp_size=1, is_blockfirst=True)
+
+
+def test_groups_restoring_at_once(gpu_device):
+    """Three groups, a thread and a consumer stream each, at the same time; then the words of the
+    groups go to new ones."""
+    import threading
+    from flexkv_amd.c_ext import launch_policy
+    layers, blocks = 12, 24
+    failures = []
+
+    def restores(seed):
+        try:
+            s = KVSetup(VLLM, layers, 1, 32, 32, 16384, "BLOCKFIRST", seed=seed)
+            dev = s.to_device(gpu_device)
+            consumer, rng = torch.cuda.Stream(), np.random.default_rng(seed)
+            for _ in range(2):
+                grp = vllm_group(s, dev, layers)
+                for rep in range(5):
+                    fresh = rng.integers(0, 256, s.host_bytes, dtype=np.uint8)
+                    s.host_ref[:] = fresh
+                    dev.host.copy_(torch.from_numpy(fresh))
+                    ids = [rng.permutation(32)[:blocks].astype(np.int64) for _ in range(2)]
+                    restore(grp, s, *ids, 1, "polling" if rep % 2 else "hostfunc")
+                    with torch.cuda.stream(consumer):
+                        grp.wait_layer(layers - 1, consumer)
+                        seen = [t.clone() for t in dev.gpu]
+                    consumer.synchronize()
+                    grp.synchronize()
+                    s.oracle_transfer(*ids, True)
+                    dev.assert_matches_reference(f"group {seed} restore {rep}")
+                    for l, t in enumerate(seen):
+                        assert torch.equal(t, dev.gpu[l]), (seed, rep, l)
+                grp.close()
+        except BaseException as e:  # noqa: B902 - handed to the test's thread
+            failures.append(e)
+
+    with launch_policy(staged_restore=0, staged_gather=0):
+        threads = [threading.Thread(target=restores, args=(60 + k,)) for k in range(3)]
+        [t.start() for t in threads]
+        [t.join() for t in threads]
+    if failures:
+        raise failures[0]
+
+
+def test_wait_layer_while_the_stream_is_captured(gpu_device):
+    """The wait of a captured stream is the runtime's business, as an event from outside the
+    capture is; the graph holds none of the words, and restores before and after are whole."""
+    from flexkv_amd.c_ext import launch_policy
+    layers, blocks = 9, 7
+    s = KVSetup(VLLM, layers, 1, 12, 12, 16384, "BLOCKFIRST", seed=77)
+    dev = s.to_device(gpu_device)
+    grp = vllm_group(s, dev, layers)
+    rng = np.random.default_rng(78)
+    stream, counter = torch.cuda.Stream(), torch.zeros(4, device=gpu_device)
+    with launch_policy(staged_restore=0, staged_gather=0):
+        for rep in range(3):
+            fresh = rng.integers(0, 256, s.host_bytes, dtype=np.uint8)
+            s.host_ref[:] = fresh
+            dev.host.copy_(torch.from_numpy(fresh))
+            ids = [rng.permutation(12)[:blocks].astype(np.int64) for _ in range(2)]
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.stream(stream):
+                restore(grp, s, *ids, 1, "polling")
+                graph.capture_begin(capture_error_mode="thread_local")
+                counter.add_(1)
+                try:
+                    grp.wait_layer(layers - 1, stream)
+                except RuntimeError:
+                    pass
+                graph.capture_end()
+                grp.wait_layer(layers - 1, stream)
+                seen = [t.clone() for t in dev.gpu]
+            grp.synchronize()
+            torch.cuda.synchronize()
+            s.oracle_transfer(*ids, True)
+            dev.assert_matches_reference(f"restore {rep}")
+            for l, t in enumerate(seen):
+                assert torch.equal(t, dev.gpu[l]), (rep, l)
+            before = float(counter[0])
+            for k in range(3):
+                graph.replay()
+                torch.cuda.synchronize()
+                assert float(counter[0]) == before + k + 1
+    grp.close()
+
+
 def test_shapes_that_go_batch_by_batch(gpu_device):
     """Packed chunks and odd vector widths keep a launch a batch."""
     from flexkv_amd.c_ext import get_stats, launch_policy, reset_stats
