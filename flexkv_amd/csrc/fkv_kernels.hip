@@ -842,16 +842,15 @@ namespace {
 // fence, which also waits for its stores; that, the answer of the counter and the next claim
 // are looked at when the first vectors of the following range have arrived, a round trip over
 // the link later, when they have long come back.  (Counted right behind its stores, with the
-// claim read through LDS, a range cost the wavefront 3 us more: 0.95 against 0.88 ms for 32
-// layers of 1 MiB with 16 wavefronts.)  Write-through stores instead of the fence measured
-// slower: 0.75 against 0.71 ms with 24 wavefronts.  Whoever counts the last range of a batch
+// claim read through LDS, a range cost the wavefront 3 us more: 8 % of 32 layers of 1 MiB with 16
+// wavefronts.)  Write-through stores instead of the fence were 5 % slower with 24 wavefronts.  Whoever counts the last range of a batch
 // writes its epoch to a word in device memory, which streams wait for, and one in pinned
 // memory, which the host looks at (see Landing).
 //
-// Whole restores, the forward stream waiting for every layer (us, a launch a batch -> this):
-// 8 x 256 KiB to eventfds 160 -> 75, 32 x 1 MiB 753 -> 645, 61 x 7 MiB 9080 (rows gathered by
-// host threads) -> 7708, which is 56 GB/s.  Next to a fused attention of 76 us a layer:
-// 32 x 1 MiB 2956 -> 2822, 61 x 7 MiB 10383 -> 8122.
+// Whole restores, the forward stream waiting for every layer (us, before -> this): 8 x 256 KiB
+// to eventfds 159 -> 78, 32 x 1 MiB 773 -> 647, 61 x 7 MiB 9190 (rows gathered by host threads)
+// -> 7709, which is 56 GB/s.  Next to a fused attention of 76 us a layer: 32 x 1 MiB 2845 -> 2798,
+// 61 x 7 MiB 9193 -> 7994; next to three 2048^3 GEMMs a layer: 2691 -> 2585, 9224 -> 8076.
 __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) {
   using V = VecType<16>::type;
   __shared__ uint64_t s_base_src[kCopyMaxLK], s_base_dst[kCopyMaxLK];

@@ -311,8 +311,11 @@ int staged_plan_build(const fkv_transfer_desc &d, int batch_layers, StagedRing &
   // batches long enough to hide what they cost the link: 15-25 us between two copies.
   // Measured (72 KiB rows, 30 layers, gathered against one launch): 96 rows a layer 4.65 /
   // 3.90 ms, 192 rows 8.3 / 7.8, 288 rows 12.1 / 11.5, 384 rows 15.9 / 15.3; next to a fused
-  // attention of 76 us a layer (61 layers, 96 rows) 10.4 / 8.1 ms.  Longer batches leave the
-  // compute units to the forward pass, as before.
+  // attention of 76 us a layer (61 layers, 96 rows) 9.2 / 8.0 ms, to three 2048^3 GEMMs a layer
+  // 9.2 / 8.1.  The price is paid by kernels that do not wait for the restore: while it lasts, three
+  // such GEMMs take 126 us instead of 85 (79 alone), the attention 115 instead of 85 (81), a
+  // streaming kernel 23.7 instead of 22.7 (20.2); staged_gather = 2 keeps to gathered rows.  Longer
+  // batches leave the compute units to the forward pass either way.
   constexpr double kGatherHandOverUs = 24;
   if (out->route == kRouteGathered && pol.staged_gather == 1 && one_launch && host_visible &&
       kernel_allowed) {

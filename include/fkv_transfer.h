@@ -417,9 +417,11 @@ int fkv_layerwise_transfer(fkv_layerwise *g, const int64_t *gpu_block_ids,
 
 /* Make `consumer_stream` (a hipStream_t on GPU `gpu_index` of the group) wait
  * until `layer` (an original layer id for a multi-group instance) of the most
- * recent transfer has landed.  This is the in-process counterpart of the
- * eventfd a consumer in another process blocks on
- * (flexkv/integration/sglang/comm.py:705-744); the reference has no such call. */
+ * recent transfer has landed, for as long as that takes.  The layers before it have landed too
+ * where the restore is a single launch or its batches keep to one stream
+ * (kernel_alt_stream_kb of the launch policy says which); an engine waits for each layer it
+ * uses.  This is the in-process counterpart of the eventfd a consumer in another process
+ * blocks on (flexkv/integration/sglang/comm.py:705-744); the reference has no such call. */
 int fkv_layerwise_wait_layer(fkv_layerwise *g, int32_t gpu_index, int32_t layer,
                              void *consumer_stream);
 /* Names the stream on which the engine computes next to this group's restores on GPU
