@@ -798,8 +798,8 @@ typedef struct fkv_launch_policy {
                                  second stream, so that it starts while
                                  the last requests of its predecessor are in flight (two launches
                                  on one stream lie 8 us apart, next to 18 us of link time for
-                                 1 MiB); events, notifications and wait_layer stay per batch and
-                                 in order.  0 = every batch on one stream.  -1 (default): a
+                                 1 MiB); events, notifications and wait_layer stay per batch, the
+                                 notifications in order.  0 = every batch on one stream.  -1 (default): a
                                  restore of one layer group goes out as a single launch that
                                  announces its batches itself where its shape allows that, and as
                                  with 4096 otherwise */
