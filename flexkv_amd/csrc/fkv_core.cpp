@@ -162,7 +162,10 @@ hipError_t quiet_word_wait(const uint64_t *word, uint64_t at_least, hipEvent_t b
     } else if (q != hipSuccess) {
       return q;
     } else {
-      return there() ? hipSuccess : hipErrorUnknown;
+      for (const auto until = std::chrono::steady_clock::now() + kLateWord; !there();)
+        if (std::chrono::steady_clock::now() >= until)
+          return hipErrorUnknown;
+      return hipSuccess;
     }
   }
 }

@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <chrono>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -38,6 +39,9 @@ hipError_t quiet_event_wait(hipEvent_t event, int device, int64_t expected_ns = 
 hipError_t quiet_stream_wait(hipStream_t stream, int device);
 // The same for a word in pinned host memory that a kernel raises to `at_least` before
 // `behind`, recorded behind the kernel, is reached.
+// The word may become visible a little after the event (recorded without a system-scope fence):
+// only a launch that has been over for kLateWord without it has ended in an error.
+constexpr std::chrono::milliseconds kLateWord{100};
 hipError_t quiet_word_wait(const uint64_t *word, uint64_t at_least, hipEvent_t behind, int device);
 // The runtime gave no answer because some thread is capturing a stream: says nothing about the
 // work that was asked about.

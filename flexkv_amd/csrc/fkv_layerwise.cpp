@@ -347,16 +347,19 @@ struct fkv_layerwise {
 
   int poll_batches() {
     unsigned looks = 0;
+    std::chrono::steady_clock::time_point over{}; // when a launch was first seen to be over
     return fkv::poll_batches_in_order(
         batches.size(), num_gpus, (int)hipSuccess, (int)hipErrorNotReady,
-        [this, &looks](size_t b, int g) {
+        [this, &looks, &over](size_t b, int g) {
           // an event that has not been recorded yet reads as complete
           const int state = gate.peek((int)b);
           if (state <= 0)
             return (int)(state < 0 ? hipErrorLaunchFailure : hipErrorNotReady);
           if (one_launch) {
-            if (has_landed((int)b, g))
+            if (has_landed((int)b, g)) {
+              over = {};
               return (int)hipSuccess;
+            }
             if (++looks % 1024 != 0) // now and then: has the launch ended in an error?
               return (int)hipErrorNotReady;
           }
@@ -364,8 +367,12 @@ struct fkv_layerwise {
           const hipError_t e = hipEventQuery(one_launch ? batches.back()->done[g] : batches[b]->done[g]);
           if (e != hipSuccess)
             (void)hipGetLastError();
-          else if (one_launch && !has_landed((int)b, g))
-            return (int)hipErrorUnknown;
+          else if (one_launch && !has_landed((int)b, g)) {
+            const auto now = std::chrono::steady_clock::now();
+            if (over == std::chrono::steady_clock::time_point{})
+              over = now;
+            return (int)(now - over < fkv::kLateWord ? hipErrorNotReady : hipErrorUnknown);
+          }
           return (int)(fkv::capture_forbids(e) ? hipErrorNotReady : e);
         },
         [this](size_t b) { notify(*batches[b]); }, poller_stop);

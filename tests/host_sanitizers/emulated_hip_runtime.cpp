@@ -158,6 +158,8 @@ struct Hold {
 Hold g_hold;
 // How long a restore in one launch goes on after its last batch has landed (fkv_emulated_kernel_tail).
 std::atomic<long> g_tail_us{0};
+// How long the words of a restore in one launch take to the host (fkv_emulated_late_words).
+std::atomic<long> g_late_us{0};
 void kernel_tail() {
   if (const long us = g_tail_us.load(std::memory_order_relaxed))
     std::this_thread::sleep_for(std::chrono::microseconds(us));
@@ -780,7 +782,14 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
       copy_rows(a);
       t.tick_host[b] = (uint64_t)(std::chrono::steady_clock::now().time_since_epoch().count() / 10);
       __atomic_store_n(t.landed + b, t.epoch, __ATOMIC_RELEASE);
-      __atomic_store_n(t.landed_host + b, t.epoch, __ATOMIC_RELEASE);
+      auto to_host = [t, b] { __atomic_store_n(t.landed_host + b, t.epoch, __ATOMIC_RELEASE); };
+      if (const long us = g_late_us.load(std::memory_order_relaxed))
+        std::thread([to_host, us] { // the words are never freed
+          std::this_thread::sleep_for(std::chrono::microseconds(us));
+          to_host();
+        }).detach();
+      else
+        to_host();
     }
     kernel_tail();
   });
@@ -858,6 +867,9 @@ extern "C" long fkv_emulated_fail(int category, long after, long count) {
 // before the kernel is; the device's clock runs `factor` times as fast as the real one (the CPU
 // device model).
 extern "C" void fkv_emulated_kernel_tail(long us) { g_tail_us.store(us); }
+// The stand-in for a restore in one launch: its words reach the host this long after they were
+// written, maybe behind the event that follows the launch.
+extern "C" void fkv_emulated_late_words(long us) { g_late_us.store(us); }
 extern "C" void fkv_emulated_hold_kernels(int on) { g_hold.set(on != 0); }
 extern "C" void fkv_emulated_clock_speed(long factor) {
 #ifdef FKV_KERNELS_FROM_SOURCE

@@ -28,6 +28,7 @@ void fkv_emulated_hold_kernels(int on);
 void fkv_emulated_clock_speed(long factor);
 void fkv_emulated_kernel_tail(long us);
 long fkv_emulated_host_waited_copies();
+void fkv_emulated_late_words(long us);
 }
 
 #define REQUIRE(cond, ...)                                                                          \
@@ -382,6 +383,23 @@ void next_to_a_put(uint64_t seed) {
   g.destroy();
 }
 
+// The words of a launch may reach the host a little after the event behind it is seen: no error.
+void late_words_case(uint64_t seed) {
+  Rng rng(seed);
+  Group g(rng, 1, 3, 1, 3, 8192);
+  fkv_emulated_late_words(1000);
+  for (int rep = 0; rep < 6; ++rep) {
+    g.refill(rng);
+    REQUIRE(g.restore(rng, 3, 1, rep & 1 ? FKV_NOTIFY_POLLING : FKV_NOTIFY_HOSTFUNC) == FKV_OK, "restore");
+    REQUIRE(fkv_layerwise_synchronize(g.g) == FKV_OK, "synchronize");
+    g.check("late words");
+    for (size_t i = 0; i < g.fds.size(); ++i)
+      REQUIRE(g.units(i) == 1, "rep %d: eventfd %zu", rep, i);
+  }
+  fkv_emulated_late_words(0);
+  g.destroy();
+}
+
 // Groups that restore at the same time, each from a thread of its own.
 void several_at_once(uint64_t seed) {
   std::vector<std::thread> threads;
@@ -441,6 +459,7 @@ int main(int argc, char **argv) {
     seeded_case(21000 + i);
   held_up_case(20500);
   no_answer_case(20550);
+  late_words_case(20580);
   drained_case(20600);
   by_policy(20700);
   next_to_a_put(20800);
