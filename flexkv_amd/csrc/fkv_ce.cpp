@@ -551,7 +551,10 @@ int device_staging_copy(const fkv_transfer_desc &d, int it0, int nit, int p0, in
     }
     std::memcpy(h + 2 * tab, d.gpu_block_ids + p0, ids);
     uint8_t *dv = nullptr;
-    int rc = plan_publish(slot, 2 * tab + ids, /*mirror=*/true, stream, &dv);
+    const int vec = common_vector_width(&acc, 1);
+    const bool carried = fits_arguments(lk, np, vec); // as in fkv_layout_transform
+    CopyReport report;
+    int rc = plan_publish(slot, 2 * tab + ids, /*mirror=*/!carried, stream, &dv);
     if (rc == FKV_OK) {
       CopyKernelArgs a{};
       const uint64_t *dg = reinterpret_cast<const uint64_t *>(dv);
@@ -566,10 +569,13 @@ int device_staging_copy(const fkv_transfer_desc &d, int it0, int nit, int p0, in
       a.chunk_bytes = d.chunk_size;
       a.num_blocks = np;
       a.lk = lk;
-      a.vec = common_vector_width(&acc, 1);
+      a.vec = vec;
       a.nt_store = 1;
       a.unroll = pol.hbm_unroll;
+      a.host_tables = carried;
+      a.report = &report;
       rc = launch_copy_kernel(a, kStagingWorkgroups, kStagingThreads, stream);
+      hold.drained = report.in_arguments;
     }
     if (rc != FKV_OK)
       return rc;

@@ -661,7 +661,7 @@ void kernel_plan_point(KernelPlan *out, const uint8_t *dv, uint64_t *claims) {
 }
 
 int kernel_plan_build(const fkv_transfer_desc &d, hipStream_t stream, KernelPlan *out,
-                      bool host_optional, bool one_launch) {
+                      bool host_optional) {
   int device = 0;
   FKV_HIP_TRY(hipGetDevice(&device));
   const size_t plan_bytes = kernel_plan_bytes(d);
@@ -673,35 +673,41 @@ int kernel_plan_build(const fkv_transfer_desc &d, hipStream_t stream, KernelPlan
     plan_release(slot, stream, true);
     return rc;
   }
-  const fkv_launch_policy pol = policy_of(device);
-  // Kernels read the plan from a device copy, which a small kernel uploads first,
-  // or where it is, in the pinned slot.  In place it costs the kernel a round trip over the
+  out->slot = slot;
+  kernel_plan_point(out, plan_host(slot), plan_counters(slot, d.num_layers)); // nullptr: launches are not confined
+  return FKV_OK;
+}
+
+int kernel_plan_publish(KernelPlan *p, hipStream_t stream, bool one_launch) {
+  const fkv_launch_policy pol = policy_of(p->device);
+  const int pairs = p->num_layers * p->kv_dim;
+  // A plan that one launch reads travels in its arguments if it fits (see tables_from_arguments
+  // in fkv_kernels.hip): a block of 2 MiB takes 59.6 instead of 63.8 us from the host, a restore of
+  // 8 layers of 256 KiB 75.0 instead of 78.6, three layer groups 815.8 instead of 816.9.
+  //
+  // Other plans are read from a device copy, which a small kernel uploads first,
+  // or where they are, in the pinned slot.  In place a plan costs the kernel a round trip over the
   // link, uploaded a command on the stream, so a plan that one launch reads once (`one_launch`)
   // stays where it is, as long as a workgroup's part of it is one round trip: the ids of its
-  // blocks one a lane, and two tables of two entries a lane (a block of 2 MiB 67.7 -> 65.1 us
-  // from the host, 71.8 -> 68.6 to it; 10 MiB 220 -> 217, three layer groups 825 -> 818; 1024
-  // blocks of 2304 bytes 72.6 -> 70.1; with 160 (layer, kv) pairs 37.5 -> 37.7, with 256
+  // blocks one a lane, and two tables of two entries a lane (1024
+  // blocks of 2304 bytes 72.6 -> 70.1 us; with 160 (layer, kv) pairs 37.5 -> 37.7, with 256
   // 73.0 -> 73.9).  A restore that reads its plan a launch a batch is 1.5 % slower
   // in place; but next to a transfer in the other direction every command on a stream costs
   // idle time, and nothing is uploaded then: two threads that put and get 25 MB (100 MB)
   // requests move 88.8 (95.4) instead of 87.0 (94.1) GB/s.  plan_mirror of the launch
   // policy = 1 / 0: always / never upload.
   constexpr int kInPlacePairs = 128, kInPlaceBlocksPerWorkgroup = 64;
-  const bool one_round_trip = one_launch && d.num_layers * d.kv_dim <= kInPlacePairs &&
-                              d.num_blocks <= kInPlaceBlocksPerWorkgroup * out->workgroups;
+  p->host_tables = one_launch && pol.plan_mirror < 0 && fits_arguments(pairs, 2 * (int64_t)p->num_blocks, p->vec);
+  const bool one_round_trip = one_launch && pairs <= kInPlacePairs &&
+                              p->num_blocks <= kInPlaceBlocksPerWorkgroup * p->workgroups;
   const bool mirror_plan =
       pol.plan_mirror >= 0
           ? pol.plan_mirror != 0
-          : !(one_round_trip ||
-              (pol.arbiter == 1 && link_direction_busy(device, !out->h2d, stream)));
+          : !(p->host_tables || one_round_trip ||
+              (pol.arbiter == 1 && link_direction_busy(p->device, !p->h2d, stream)));
   uint8_t *dv = nullptr;
-  rc = plan_publish(slot, plan_bytes, mirror_plan, stream, &dv);
-  if (rc != FKV_OK) {
-    plan_release(slot, stream, false);
-    return rc;
-  }
-  out->slot = slot;
-  kernel_plan_point(out, dv, plan_counters(slot, d.num_layers)); // nullptr: launches are not confined
+  FKV_TRY(plan_publish(p->slot, 2 * ((size_t)pairs + (size_t)p->num_blocks) * 8, mirror_plan, stream, &dv));
+  kernel_plan_point(p, dv, p->claims);
   return FKV_OK;
 }
 
@@ -729,6 +735,7 @@ CopyKernelArgs plan_job(const KernelPlan &p, int l0, int nl) {
   a.packed_grid_pct = 150; // replaced by the policy's when the launch is shaped
   a.xcd_mask = 0;
   a.claim = p.claims ? p.claims + l0 : nullptr; // a launch per first layer at most
+  a.host_tables = p.host_tables;
   return a;
 }
 
@@ -791,7 +798,7 @@ int shape_for_now(const KernelPlan &p, int64_t bytes, hipStream_t stream, CopyKe
 } // namespace
 
 int kernel_plan_launch(const KernelPlan &p, int layer_offset, int num_layers,
-                       hipStream_t stream) {
+                       hipStream_t stream, CopyReport *report) {
   if (!p.host_visible)
     return fail(FKV_ERR_INVALID_ARG, "kernel transfer: the host pool is not device-visible "
                 "(allocate it pinned or register it)");
@@ -805,6 +812,7 @@ int kernel_plan_launch(const KernelPlan &p, int layer_offset, int num_layers,
   for (int l0 = layer_offset; l0 < layer_offset + num_layers; l0 += layers_per_launch) {
     const int nl = std::min(layers_per_launch, layer_offset + num_layers - l0);
     CopyKernelArgs a = plan_job(p, l0, nl);
+    a.report = report; // tables that fit the arguments go out in one launch
     const int workgroups =
         shape_for_now(p, (int64_t)p.num_blocks * a.lk * p.chunk_size, stream, &a);
     FKV_TRY(launch_copy_kernel(a, workgroups, p.threads, stream));
@@ -846,7 +854,7 @@ int kernel_plan_launch_layers(const KernelPlan &p, int layers_per_batch, LayersL
 }
 
 int kernel_plans_launch(const KernelPlan *const *plans, const int *layer_offsets,
-                        const int *num_layers, int count, hipStream_t stream) {
+                        const int *num_layers, int count, hipStream_t stream, CopyReport *report) {
   // One launch for all of them when they can share one: same direction, device,
   // vector width and launch shape, each range within one LDS table.
   const bool fuse = policy_of(plans[0]->device).fuse_launches != 0;
@@ -862,8 +870,15 @@ int kernel_plans_launch(const KernelPlan *const *plans, const int *layer_offsets
                num_layers[i] * p.kv_dim <= kCopyMaxLK;
   }
   if (!together) {
-    for (int i = 0; i < count; ++i)
-      FKV_TRY(kernel_plan_launch(*plans[i], layer_offsets[i], num_layers[i], stream));
+    CopyReport all{/*in_arguments=*/true, /*claims=*/false};
+    for (int i = 0; i < count; ++i) {
+      CopyReport one;
+      FKV_TRY(kernel_plan_launch(*plans[i], layer_offsets[i], num_layers[i], stream, &one));
+      all.in_arguments = all.in_arguments && one.in_arguments;
+      all.claims = all.claims || one.claims;
+    }
+    if (report)
+      *report = all;
     return FKV_OK;
   }
   CopyKernelArgs jobs[kCopyMaxJobs];
@@ -872,6 +887,7 @@ int kernel_plans_launch(const KernelPlan *const *plans, const int *layer_offsets
     jobs[i] = plan_job(*plans[i], layer_offsets[i], num_layers[i]);
     bytes += (int64_t)plans[i]->num_blocks * jobs[i].lk * plans[i]->chunk_size;
   }
+  jobs[0].report = report;
   const int workgroups = shape_for_now(*plans[0], bytes, stream, &jobs[0]);
   FKV_TRY(launch_copy_jobs(jobs, count, workgroups, plans[0]->threads, stream));
   link_direction_mark(plans[0]->device, plans[0]->h2d, stream, bytes);
@@ -880,16 +896,20 @@ int kernel_plans_launch(const KernelPlan *const *plans, const int *layer_offsets
 
 void kernel_plan_release(KernelPlan *p, hipStream_t stream) {
   if (p->slot)
-    plan_release(p->slot, stream, false);
+    plan_release(p->slot, stream, p->unread);
   p->slot = nullptr;
 }
 
 int run_kernel_path(const fkv_transfer_desc &d, hipStream_t stream) {
   set_last_path(FKV_PATH_KERNEL);
   KernelPlan plan;
-  FKV_TRY(kernel_plan_build(d, stream, &plan, /*host_optional=*/false, /*one_launch=*/true));
+  FKV_TRY(kernel_plan_build(d, stream, &plan));
   KernelPlanHold hold{&plan, stream};
-  return kernel_plan_launch(plan, 0, d.num_layers, stream);
+  FKV_TRY(kernel_plan_publish(&plan, stream, /*one_launch=*/true));
+  CopyReport report;
+  FKV_TRY(kernel_plan_launch(plan, 0, d.num_layers, stream, &report));
+  plan.unread = report.in_arguments && !report.claims;
+  return FKV_OK;
 }
 
 int validate(const fkv_transfer_desc &d) {
@@ -1169,10 +1189,11 @@ int run_kernel_path_multi(const fkv_transfer_desc *descs, int count, hipStream_t
   } give_back{plans, stream};
   int rc = FKV_OK, built = 0;
   for (; built < count && rc == FKV_OK; ++built)
-    rc = fkv::kernel_plan_build(descs[built], stream, &plans[built], /*host_optional=*/false,
-                                /*one_launch=*/true);
+    rc = fkv::kernel_plan_build(descs[built], stream, &plans[built]);
   if (rc != FKV_OK)
     --built; // the one that failed holds nothing
+  for (int k = 0; k < built && rc == FKV_OK; ++k)
+    rc = fkv::kernel_plan_publish(&plans[k], stream, /*one_launch=*/true);
   for (int k = 0; k < built && rc == FKV_OK; k += fkv::kCopyMaxJobs) {
     const int n = std::min(fkv::kCopyMaxJobs, built - k);
     const fkv::KernelPlan *group[fkv::kCopyMaxJobs];
@@ -1182,7 +1203,10 @@ int run_kernel_path_multi(const fkv_transfer_desc *descs, int count, hipStream_t
       first[j] = 0;
       layers[j] = descs[k + j].num_layers;
     }
-    rc = fkv::kernel_plans_launch(group, first, layers, n, stream);
+    fkv::CopyReport report;
+    rc = fkv::kernel_plans_launch(group, first, layers, n, stream, &report);
+    for (int j = 0; j < n && rc == FKV_OK; ++j)
+      plans[k + j].unread = report.in_arguments && !report.claims;
   }
   return rc;
 }

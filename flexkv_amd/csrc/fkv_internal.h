@@ -192,7 +192,26 @@ struct CopyKernelArgs {
   uint32_t epoch; // set by launch_copy_kernel: a number no other launch in flight has
   int32_t claims_per_wg; // ranges per working workgroup: confined launches (0 = 1), and
                          // launches on all XCDs that have counters (0 = fixed shares)
+  int32_t host_tables;   // host side: the host reads the four arrays at these addresses too, and
+                         // the launch may carry them in its arguments (fits_arguments)
+  struct CopyReport *report; // host side: what became of the launch; may be null
 };
+// Filled in by a launch for its caller.
+struct CopyReport {
+  bool in_arguments = false; // the tables travelled in the arguments: nothing on the device reads
+                             // them where they were, whenever it runs
+  bool claims = false;       // workgroups of the launch look at its claim counter, until it ends
+};
+// Tables in the arguments of a launch: 4 KiB in all, of which up to kCopyMaxJobs jobs take 0.8.
+constexpr int kArgPlanWords = 400;
+struct ArgPlan {
+  uint64_t w[kArgPlanWords];
+};
+// Whether a launch over `pairs` (layer, kv) pairs and `ids` block ids (of both lists together),
+// every address a multiple of `vec`, can carry its tables.
+inline bool fits_arguments(int64_t pairs, int64_t ids, int vec) {
+  return vec == 16 && 2 * pairs + ids <= kArgPlanWords;
+}
 constexpr int kCopyBlockThreads = 1024;  // largest workgroup the kernel is built for
 constexpr int kCopyUnroll = 8;           // vector accesses in flight per lane
 constexpr int kCopyUnrollDeep = 16;      // the same for launches that HBM bounds
@@ -311,6 +330,9 @@ struct KernelPlan {
   bool recorded = false; // the launches are being recorded into a graph: shaped once for every
                          // replay, without a look at what the link is doing right now
   uint64_t *claims = nullptr; // a claim counter per layer of the plan, device memory
+  bool host_tables = false; // not uploaded: the addresses above are those of the pinned slot, and
+                            // the one launch of the plan carries the tables in its arguments
+  bool unread = false;      // ... and has been made: nothing on the device looks at the slot
 };
 void kernel_plan_release(KernelPlan *p, hipStream_t stream);
 // Give plan memory back when the scope ends, by whichever way it ends.
@@ -325,9 +347,10 @@ struct KernelPlanHold {
 struct PlanSlotHold {
   PlanSlot *slot;
   hipStream_t stream;
+  bool drained = false; // nothing on the device looks at the slot
   ~PlanSlotHold() {
     if (slot)
-      plan_release(slot, stream, false);
+      plan_release(slot, stream, drained);
   }
 };
 // Link-bound launches of the last while, per device and direction (see fkv_core.cpp).
@@ -346,14 +369,17 @@ size_t kernel_plan_bytes(const fkv_transfer_desc &d);
 int kernel_plan_fill(const fkv_transfer_desc &d, uint8_t *h, bool may_probe_device,
                      KernelPlan *out, bool host_optional = false);
 void kernel_plan_point(KernelPlan *out, const uint8_t *dv, uint64_t *claims);
-// Builds and uploads (on `stream`) the plan for all layers of `d`.  With `host_optional` a
+// Builds the plan for all layers of `d`.  With `host_optional` a
 // host pool the device cannot read is no error: the plan then has host_visible == false.
-// `one_launch`: the plan is read by one launch and not again.
 int kernel_plan_build(const fkv_transfer_desc &d, hipStream_t stream, KernelPlan *out,
-                      bool host_optional = false, bool one_launch = false);
+                      bool host_optional = false);
+// Makes its tables known to the launches that follow on `stream`: uploaded, read where they are,
+// or carried in the arguments.  `one_launch`: the plan is read by one launch and not again.
+int kernel_plan_publish(KernelPlan *p, hipStream_t stream, bool one_launch);
 // Enqueues the copy of layers [layer_offset, layer_offset + num_layers) of the plan.
+// `report` (may be null): see CopyReport, for all launches of the call together.
 int kernel_plan_launch(const KernelPlan &p, int layer_offset, int num_layers,
-                       hipStream_t stream);
+                       hipStream_t stream, CopyReport *report = nullptr);
 // All layers of the plan in one launch, `layers_per_batch` at a time; `t` brings the words
 // that announce the batches.  Only for plans layers_launch_fits accepts.
 bool layers_launch_fits(const KernelPlan &p);
@@ -363,7 +389,8 @@ int kernel_plan_launch_layers(const KernelPlan &p, int layers_per_batch, LayersL
 // members of one original layer of a multi-group restore); falls back to one launch
 // per plan where the plans cannot share one.
 int kernel_plans_launch(const KernelPlan *const *plans, const int *layer_offsets,
-                        const int *num_layers, int count, hipStream_t stream);
+                        const int *num_layers, int count, hipStream_t stream,
+                        CopyReport *report = nullptr);
 // The plan memory is recycled once everything enqueued on `stream` so far has run.
 void kernel_plan_release(KernelPlan *p, hipStream_t stream);
 int run_kernel_path(const fkv_transfer_desc &d, hipStream_t stream);

@@ -53,6 +53,7 @@
 #include <algorithm>
 #include <chrono>
 #include <cstdlib>
+#include <cstring>
 #include <vector>
 
 namespace fkv {
@@ -389,9 +390,28 @@ __device__ __forceinline__ void copy_share(const CopyKernelArgs &a, uint64_t num
   }
 }
 
-template <int VEC, bool NTS, int U, bool LR = false>
-__global__ __launch_bounds__(kCopyBlockThreads) void fkv_copy_chunks_kernel(
-    CopyKernelArgs a) {
+// Tables that travel in the arguments of a launch instead of lying in memory of their own.
+//
+// What bounds a small call is what happens before its first load: a plan in pinned host memory
+// costs every workgroup a round trip over the link (5000 cycles, 2.2 us), a plan in device memory
+// a kernel that brings it there (3 us and the 5 to 10 us between two commands of a stream).
+// Arguments are written to device memory by the host itself as part of the launch (a lane has
+// its words after 500 cycles) for 0.1 us of host time.  Calls, before -> this (us): transforms of a
+// few blocks 14.9 -> 9.8, one of 512 MiB (64 pairs, 256 blocks) 180.8 -> 177.0, payloads of 48 MiB
+// to the host 872 -> 865; transfers and restores at kernel_plan_publish.  In these launches the
+// four pointers of the arguments hold the number of the first word, plus one; 0: no such list.
+template <typename T> __device__ __forceinline__ const T *in_arguments(const T *word, const ArgPlan &plan) {
+  return word ? reinterpret_cast<const T *>(plan.w + (reinterpret_cast<uintptr_t>(word) - 1)) : nullptr;
+}
+__device__ __forceinline__ void tables_from_arguments(CopyKernelArgs &a, const ArgPlan &plan) {
+  a.base_src = in_arguments(a.base_src, plan);
+  a.base_dst = in_arguments(a.base_dst, plan);
+  a.ids_src = in_arguments(a.ids_src, plan);
+  a.ids_dst = in_arguments(a.ids_dst, plan);
+}
+
+template <int VEC, bool NTS, int U, bool LR>
+__device__ __forceinline__ void copy_chunks(const CopyKernelArgs &a) {
   extern __shared__ uint64_t lds[];
   __shared__ uint32_t s_claim;
   Shares shares(a);
@@ -403,6 +423,17 @@ __global__ __launch_bounds__(kCopyBlockThreads) void fkv_copy_chunks_kernel(
     copy_share<VEC, NTS, U, LR>(a, part, part + 1, parts, lds, load_tables);
     load_tables = false;
   }
+}
+template <int VEC, bool NTS, int U, bool LR = false>
+__global__ __launch_bounds__(kCopyBlockThreads) void fkv_copy_chunks_kernel(
+    CopyKernelArgs a) {
+  copy_chunks<VEC, NTS, U, LR>(a);
+}
+template <bool NTS, bool LR>
+__global__ __launch_bounds__(kCopyBlockThreads) void fkv_copy_chunks_args_kernel(CopyKernelArgs a,
+                                                                                 ArgPlan plan) {
+  tables_from_arguments(a, plan);
+  copy_chunks<16, NTS, kCopyUnroll, LR>(a);
 }
 
 // A value that is the same for a whole wavefront, where the compiler cannot see it.
@@ -456,8 +487,7 @@ __device__ __forceinline__ void drain_wave() {
 // 8 KiB and more, took (us, before -> this): 512 MiB out of 32 KiB chunks 195 -> 181, back
 // into them 205 -> 197, one tensor for all layers 187 -> 180; 288 MiB of 18 KiB chunks
 // 116 -> 105; 16 MiB 20 -> 14.  16 vectors a lane instead of 8 (hbm_unroll): 512 MiB 195.
-template <int UNR>
-__global__ __launch_bounds__(kSliceWgThreads) void fkv_copy_slices_kernel(CopyKernelArgs a) {
+template <int UNR> __device__ __forceinline__ void copy_slices(const CopyKernelArgs &a) {
   constexpr int64_t kSliceBytes = (int64_t)kWave * UNR * 16;
   const uint32_t slices = (uint32_t)a.slices_per_chunk, spp = (uint32_t)a.lk * slices;
   const uint64_t total = (uint64_t)a.num_blocks * spp;
@@ -478,13 +508,37 @@ __global__ __launch_bounds__(kSliceWgThreads) void fkv_copy_slices_kernel(CopyKe
     copy_slice<16, true, UNR, false>(src, dst, left < kSliceBytes ? left : kSliceBytes, lane);
   }
 }
+template <int UNR>
+__global__ __launch_bounds__(kSliceWgThreads) void fkv_copy_slices_kernel(CopyKernelArgs a) {
+  copy_slices<UNR>(a);
+}
+template <int UNR>
+__global__ __launch_bounds__(kSliceWgThreads) void fkv_copy_slices_args_kernel(CopyKernelArgs a,
+                                                                               ArgPlan plan) {
+  tables_from_arguments(a, plan);
+  copy_slices<UNR>(a);
+}
 
 // Several jobs in one launch (the members of one original layer of a multi-group
 // restore, which differ in chunk size and strides): the jobs lie one behind the
 // other on a line, each as long as its weight (its bytes), and a share of the launch
 // is a stretch of that line.  Counters, mask and grid are those of job 0.
-template <int VEC, bool NTS, int U, bool LR = false>
-__global__ __launch_bounds__(kCopyBlockThreads) void fkv_copy_jobs_kernel(CopyJobs t) {
+// The argument behind the first one of the running kernel, by its place in the argument memory:
+// where the pointers into it are chosen in a loop over the jobs, the compiler would first copy
+// all of it to scratch memory.
+template <typename First> __device__ __forceinline__ const ArgPlan &plan_behind(const ArgPlan &plan) {
+#if defined(__HIP__)
+  static_assert(sizeof(First) % alignof(ArgPlan) == 0, "no gap between the two arguments");
+  return *reinterpret_cast<const ArgPlan *>(
+      (const char *)__builtin_amdgcn_kernarg_segment_ptr() + sizeof(First));
+#else
+  return plan;
+#endif
+}
+
+// `plan`: nothing, or the tables of all jobs (see tables_from_arguments).
+template <int VEC, bool NTS, int U, bool LR, typename... Plan>
+__device__ __forceinline__ void copy_jobs(const CopyJobs &t, const Plan &...plan) {
   extern __shared__ uint64_t lds[];
   __shared__ uint32_t s_claim;
   Shares shares(t.job[0]);
@@ -501,17 +555,89 @@ __global__ __launch_bounds__(kCopyBlockThreads) void fkv_copy_jobs_kernel(CopyJo
       const uint64_t w = t.weight[j];
       const uint64_t lo = b0 > off ? (b0 - off < w ? b0 - off : w) : 0;
       const uint64_t hi = b1 > off ? (b1 - off < w ? b1 - off : w) : 0;
-      if (lo < hi)
-        copy_share<VEC, NTS, U, LR>(t.job[j], lo, hi, w, lds, true);
+      if (lo < hi) {
+        CopyKernelArgs a = t.job[j];
+        (tables_from_arguments(a, plan), ...);
+        copy_share<VEC, NTS, U, LR>(a, lo, hi, w, lds, true);
+      }
       off += w;
     }
   }
+}
+template <int VEC, bool NTS, int U, bool LR = false>
+__global__ __launch_bounds__(kCopyBlockThreads) void fkv_copy_jobs_kernel(CopyJobs t) {
+  copy_jobs<VEC, NTS, U, LR>(t);
+}
+template <bool NTS, bool LR>
+__global__ __launch_bounds__(kCopyBlockThreads) void fkv_copy_jobs_args_kernel(CopyJobs t, ArgPlan plan) {
+  copy_jobs<16, NTS, kCopyUnroll, LR>(t, plan_behind<CopyJobs>(plan));
+}
+
+// Puts the tables of a job into `plan`, behind the `*at` words that are taken, and the numbers of
+// their words into `a`; a list that lies there already (`jobs` before this one, of a call over
+// several layer groups that share their blocks) is not put there again.  False: no room, or the
+// host cannot read the tables.
+bool into_arguments(CopyKernelArgs &a, const CopyKernelArgs *jobs, int njobs, ArgPlan &plan, int *at) {
+  if (!a.host_tables || a.vec != 16)
+    return false;
+  auto put = [&](const void *from, int n) -> uintptr_t {
+    if (n > kArgPlanWords - *at)
+      return 0;
+    std::memcpy(plan.w + *at, from, (size_t)n * 8);
+    *at += n;
+    return (uintptr_t)(*at - n + 1);
+  };
+  auto table = [&](const uint64_t **words) {
+    *words = reinterpret_cast<const uint64_t *>(put(*words, a.lk));
+    return *words != nullptr;
+  };
+  auto list = [&](const int64_t **ids) {
+    if (!*ids)
+      return true;
+    for (int j = 0; j < njobs; ++j)
+      if (jobs[j].num_blocks == a.num_blocks)
+        for (const int64_t *there : {jobs[j].ids_src, jobs[j].ids_dst})
+          if (there && std::memcmp(plan.w + (reinterpret_cast<uintptr_t>(there) - 1), *ids,
+                                   (size_t)a.num_blocks * 8) == 0) {
+            *ids = there;
+            return true;
+          }
+    *ids = reinterpret_cast<const int64_t *>(put(*ids, a.num_blocks));
+    return *ids != nullptr;
+  };
+  return table(&a.base_src) && table(&a.base_dst) && list(&a.ids_src) && list(&a.ids_dst);
+}
+
+// A launch whose tables travel in its arguments; false: they do not fit.
+bool launch_with_plan(CopyKernelArgs a, int grid, int threads, size_t lds_bytes, hipStream_t stream) {
+  ArgPlan plan;
+  int words = 0;
+  if (!into_arguments(a, nullptr, 0, plan, &words))
+    return false;
+  if (a.report)
+    a.report->in_arguments = true;
+#define FKV_LAUNCH_WITH_PLAN(...)                                                             \
+  hipLaunchKernelGGL((__VA_ARGS__), dim3(grid), dim3(threads), lds_bytes, stream, a, plan)
+  if (a.per_slice && a.unroll == kCopyUnrollDeep)
+    FKV_LAUNCH_WITH_PLAN(fkv_copy_slices_args_kernel<kCopyUnrollDeep>);
+  else if (a.per_slice)
+    FKV_LAUNCH_WITH_PLAN(fkv_copy_slices_args_kernel<kCopyUnroll>);
+  else if (a.nt_store)
+    FKV_LAUNCH_WITH_PLAN(fkv_copy_chunks_args_kernel<true, false>);
+  else if (a.lane_runs)
+    FKV_LAUNCH_WITH_PLAN(fkv_copy_chunks_args_kernel<false, true>);
+  else
+    FKV_LAUNCH_WITH_PLAN(fkv_copy_chunks_args_kernel<false, false>);
+#undef FKV_LAUNCH_WITH_PLAN
+  return true;
 }
 
 template <int VEC>
 int launch_vec(const CopyKernelArgs &a, int grid, int threads, size_t lds_bytes,
                hipStream_t stream) {
-  if (VEC == 16 && a.per_slice && a.unroll == kCopyUnrollDeep)
+  if (VEC == 16 && launch_with_plan(a, grid, threads, lds_bytes, stream))
+    ;
+  else if (VEC == 16 && a.per_slice && a.unroll == kCopyUnrollDeep)
     hipLaunchKernelGGL(fkv_copy_slices_kernel<kCopyUnrollDeep>, dim3(grid), dim3(threads),
                        lds_bytes, stream, a);
   else if (VEC == 16 && a.per_slice)
@@ -722,6 +848,8 @@ void shape_launch(CopyKernelArgs &a, int64_t total, int64_t bytes, int grid_pct,
     if (a.num_claims <= (uint32_t)grid) // nothing to hand out: fixed shares
       a.num_claims = 0;
   }
+  if (a.report)
+    a.report->claims = a.report->claims || a.num_claims != 0;
   stats().kernel_launches.fetch_add(1, std::memory_order_relaxed);
   if (a.xcd_mask != 0)
     stats().confined_launches.fetch_add(1, std::memory_order_relaxed);
@@ -729,10 +857,36 @@ void shape_launch(CopyKernelArgs &a, int64_t total, int64_t bytes, int grid_pct,
   *threads_out = threads;
 }
 
+// Puts the tables of all jobs, lists that several of them share once, into the arguments of their
+// launch; false (and nothing changed) where they do not fit.
+bool jobs_into_arguments(CopyJobs &t, ArgPlan &plan) {
+  CopyKernelArgs packed[kCopyMaxJobs];
+  int words = 0;
+  for (int j = 0; j < t.njobs; ++j) {
+    packed[j] = t.job[j];
+    if (!into_arguments(packed[j], packed, j, plan, &words))
+      return false;
+  }
+  std::copy(packed, packed + t.njobs, t.job);
+  return true;
+}
+
 template <int VEC>
-int launch_jobs_vec(const CopyJobs &t, int grid, int threads, size_t lds_bytes,
-                    hipStream_t stream) {
-  if (t.job[0].nt_store)
+int launch_jobs_vec(CopyJobs &t, int grid, int threads, size_t lds_bytes, hipStream_t stream) {
+  ArgPlan plan;
+  if (VEC == 16 && jobs_into_arguments(t, plan)) {
+    if (t.job[0].report)
+      t.job[0].report->in_arguments = true;
+    if (t.job[0].nt_store)
+      hipLaunchKernelGGL((fkv_copy_jobs_args_kernel<true, false>), dim3(grid), dim3(threads), lds_bytes,
+                         stream, t, plan);
+    else if (t.job[0].lane_runs)
+      hipLaunchKernelGGL((fkv_copy_jobs_args_kernel<false, true>), dim3(grid), dim3(threads), lds_bytes,
+                         stream, t, plan);
+    else
+      hipLaunchKernelGGL((fkv_copy_jobs_args_kernel<false, false>), dim3(grid), dim3(threads), lds_bytes,
+                         stream, t, plan);
+  } else if (t.job[0].nt_store)
     hipLaunchKernelGGL((fkv_copy_jobs_kernel<VEC, true, kCopyUnroll>), dim3(grid), dim3(threads),
                        lds_bytes, stream, t);
   else if (VEC == 16 && t.job[0].lane_runs)
@@ -815,6 +969,7 @@ int launch_copy_jobs(const CopyKernelArgs *jobs, int njobs, int num_workgroups,
   t.job[0].xcd_present = jobs[0].xcd_present;
   t.job[0].safety_net_wait_us = jobs[0].safety_net_wait_us;
   t.job[0].packed_grid_pct = jobs[0].packed_grid_pct;
+  t.job[0].report = jobs[0].report;
   int64_t grid = 1;
   int threads = kWave;
   shape_launch(t.job[0], total, bytes, grid_pct, num_workgroups, threads_per_workgroup, &grid,
@@ -851,12 +1006,11 @@ namespace {
 // to eventfds 159 -> 78, 32 x 1 MiB 773 -> 647, 61 x 7 MiB 9190 (rows gathered by host threads)
 // -> 7709, which is 56 GB/s.  Next to a fused attention of 76 us a layer: 32 x 1 MiB 2845 -> 2798,
 // 61 x 7 MiB 9193 -> 7994; next to three 2048^3 GEMMs a layer: 2691 -> 2585, 9224 -> 8076.
-__global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) {
+__device__ __forceinline__ void copy_layers(const LayersLaunch &t, const CopyKernelArgs &a) {
   using V = VecType<16>::type;
   __shared__ uint64_t s_base_src[kCopyMaxLK], s_base_dst[kCopyMaxLK];
   __shared__ int64_t s_off_src[kCopyIdTile], s_off_dst[kCopyIdTile];
   __shared__ uint32_t s_claim;
-  const CopyKernelArgs &a = t.a;
   Shares shares(a);
   if (!shares.enter(&s_claim))
     return;
@@ -945,6 +1099,12 @@ __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) 
     landing.count();
   landing.announce();
 }
+__global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) { copy_layers(t, t.a); }
+__global__ __launch_bounds__(kWave) void fkv_copy_layers_args_kernel(LayersLaunch t, ArgPlan plan) {
+  CopyKernelArgs a = t.a;
+  tables_from_arguments(a, plan);
+  copy_layers(t, a);
+}
 
 // Holds its stream until batches have landed, as an event behind them would: for as long as that
 // takes.  The launch it waits for was submitted before it, but may lie behind other work of its
@@ -990,7 +1150,15 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
   t.ranges = (int32_t)cut.ranges;
   t.last_ranges = (int32_t)cut.last_ranges;
   t.a.num_claims = (uint32_t)cut.claims(t.batches);
-  hipLaunchKernelGGL(fkv_copy_layers_kernel, dim3((unsigned)grid), dim3(kWave), 0, stream, t);
+  LayersLaunch with_plan = t;
+  ArgPlan plan;
+  int words = 0;
+  if (into_arguments(with_plan.a, nullptr, 0, plan, &words)) {
+    hipLaunchKernelGGL(fkv_copy_layers_args_kernel, dim3((unsigned)grid), dim3(kWave), 0, stream,
+                       with_plan, plan);
+  } else {
+    hipLaunchKernelGGL(fkv_copy_layers_kernel, dim3((unsigned)grid), dim3(kWave), 0, stream, t);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess)
     return fail(FKV_ERR_RUNTIME, "copy kernel launch failed: %s", hipGetErrorString(e));

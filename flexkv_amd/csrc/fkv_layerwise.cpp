@@ -1183,6 +1183,12 @@ int fkv_layerwise_transfer_call(fkv_layerwise *g, const fkv_layerwise_call *call
         g->one_launch = landed_words_acquire(g->device_ids[i], g->streams[i], &g->landed[i]);
     }
   }
+  for (Lane &lane : lanes)
+    for (int i = 0; i < (int)lane.plans.size() && rc == FKV_OK; ++i)
+      if (lane.plans[i].slot) {
+        (void)hipSetDevice(g->device_ids[i]);
+        rc = kernel_plan_publish(&lane.plans[i], g->streams[i], /*one_launch=*/g->one_launch);
+      }
   for (int b = g->one_launch ? num_batches - 1 : 0; b < num_batches && rc == FKV_OK; ++b)
     for (int i = 0; i < g->num_gpus && rc == FKV_OK; ++i) {
       hipError_t e = hipSetDevice(g->device_ids[i]);

@@ -34,7 +34,7 @@ struct StagingKernelArgs {
   int64_t chunk_capacity;
   int32_t *overflow;          // device counter or nullptr
   int64_t cpu_kv_stride, cpu_layer_stride, cpu_block_stride;
-  const int64_t *cpu_ids;     // device-visible, [num_blocks]
+  const int64_t *cpu_ids;     // device-visible, [num_blocks]; nullptr: in the launch's arguments
   uint32_t *size_table;       // device-visible alias of the host size table
   int64_t table_block_stride, table_layer_stride; // in entries
   int32_t start_layer, kv_dim, num_blocks, batch_start, bsz;
@@ -84,7 +84,10 @@ __device__ __forceinline__ void wave_copy(const uint8_t *__restrict__ src, uint8
 }
 
 template <bool WRITE_CPU, bool VEC16, bool RUNS = false>
-__global__ __launch_bounds__(kCopyBlockThreads) void fkv_staging_transfer_kernel(StagingKernelArgs a) {
+__global__ __launch_bounds__(kCopyBlockThreads) void fkv_staging_transfer_kernel(StagingKernelArgs a,
+                                                                                 ArgPlan plan) {
+  const int64_t *const cpu_ids =
+      a.cpu_ids ? a.cpu_ids : reinterpret_cast<const int64_t *>(plan.w);
   const int lane = threadIdx.x & 63;
   const int64_t wave = (int64_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
   const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x / 64);
@@ -95,7 +98,7 @@ __global__ __launch_bounds__(kCopyBlockThreads) void fkv_staging_transfer_kernel
     const int64_t layer = g / per_layer;
     const int64_t kv = (g % per_layer) / a.num_blocks;
     const int64_t b = g % a.num_blocks;
-    const int64_t id = a.cpu_ids[b];
+    const int64_t id = cpu_ids[b];
     *slot = a.cpu + (layer + a.start_layer) * a.cpu_layer_stride + kv * a.cpu_kv_stride +
             id * a.cpu_block_stride;
     *entry = a.size_table + id * a.table_block_stride +
@@ -151,10 +154,15 @@ __global__ __launch_bounds__(kCopyBlockThreads) void fkv_staging_transfer_kernel
   }
 }
 
+// `base` == nullptr: the table of `planes` base addresses and the ids behind it lie in `plan`.
 __global__ void fkv_chunk_ptrs_kernel(void **__restrict__ out, const uint64_t *__restrict__ base,
                                       const int64_t *__restrict__ ids, int64_t block_stride,
                                       int32_t kv_dim, int32_t num_blocks, int32_t batch_start,
-                                      int32_t bsz) {
+                                      int32_t bsz, int32_t planes, ArgPlan plan) {
+  if (!base) {
+    base = plan.w;
+    ids = reinterpret_cast<const int64_t *>(plan.w + planes);
+  }
   const int64_t per_layer = (int64_t)kv_dim * num_blocks;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < bsz;
        i += (int64_t)gridDim.x * blockDim.x) {
@@ -205,14 +213,21 @@ int fkv_staging_transfer(const fkv_staging_transfer_desc *dp, void *stream_v) tr
                 "fkv_staging_transfer: the host cache and the size table must be device-visible "
                 "(pinned or registered)");
   }
+  // The ids travel with the launch where they fit (see tables_from_arguments in fkv_kernels.hip),
+  // else in plan memory.
   const size_t ids_bytes = (size_t)d.num_blocks * 8;
-  PlanSlot *slot = plan_acquire(device, ids_bytes);
-  if (!slot)
-    return FKV_ERR_RUNTIME;
-  PlanSlotHold hold{slot, stream};
-  std::memcpy(plan_host(slot), d.cpu_block_ids, ids_bytes);
+  PlanSlotHold hold{nullptr, stream};
   uint8_t *dv = nullptr;
-  FKV_TRY(plan_publish(slot, ids_bytes, /*mirror=*/true, stream, &dv));
+  ArgPlan plan;
+  if (d.num_blocks <= kArgPlanWords) {
+    std::memcpy(plan.w, d.cpu_block_ids, ids_bytes);
+  } else {
+    hold.slot = plan_acquire(device, ids_bytes);
+    if (!hold.slot)
+      return FKV_ERR_RUNTIME;
+    std::memcpy(plan_host(hold.slot), d.cpu_block_ids, ids_bytes);
+    FKV_TRY(plan_publish(hold.slot, ids_bytes, /*mirror=*/true, stream, &dv));
+  }
   StagingKernelArgs a{};
   a.staging = static_cast<uint8_t *>(d.staging);
   a.staging_stride = d.staging_stride;
@@ -248,7 +263,7 @@ int fkv_staging_transfer(const fkv_staging_transfer_desc *dp, void *stream_v) tr
   grid = std::max(1, std::min(grid, (d.bsz + threads / 64 - 1) / (threads / 64)));
 #define FKV_LAUNCH_STAGING(...)                                                               \
   hipLaunchKernelGGL((fkv_staging_transfer_kernel<__VA_ARGS__>), dim3(grid), dim3(threads), 0,  \
-                     stream, a)
+                     stream, a, plan)
   // Adjacent vectors per lane on the same terms as the fixed-size kernel: not next to a
   // transfer from the host, where the plain order moves 2 % more in sum.  And only for calls
   // that fill the link for a while: the loads of a slice take longer in this order, which a
@@ -322,29 +337,33 @@ int fkv_build_gpu_chunk_ptrs(const fkv_chunk_ptrs_desc *dp, void *stream_v) try 
   // base addresses of the (layer, kv) planes the batch touches, engine addressing resolved
   const int nplanes = (int)(last_layer + 1) * d.kv_dim;
   const size_t tab = (size_t)nplanes * 8, ids_bytes = (size_t)d.num_blocks * 8;
-  PlanSlot *slot = plan_acquire(device, tab + ids_bytes);
-  if (!slot)
-    return FKV_ERR_RUNTIME;
-  PlanSlotHold hold{slot, stream};
-  uint8_t *h = plan_host(slot);
-  uint64_t *base = reinterpret_cast<uint64_t *>(h);
+  const bool carried = (int64_t)nplanes + d.num_blocks <= kArgPlanWords; // as the ids above
+  ArgPlan plan;
+  PlanSlotHold hold{nullptr, stream};
+  uint64_t *h = plan.w;
+  if (!carried) {
+    hold.slot = plan_acquire(device, tab + ids_bytes);
+    if (!hold.slot)
+      return FKV_ERR_RUNTIME;
+    h = reinterpret_cast<uint64_t *>(plan_host(hold.slot));
+  }
   for (int64_t l = 0; l <= last_layer; ++l)
     for (int kv = 0; kv < d.kv_dim; ++kv)
-      base[l * d.kv_dim + kv] =
+      h[l * d.kv_dim + kv] =
           l < first_layer ? 0
                           : gpu_chunk_addr(d.backend, d.gpu_tensor_ptrs, d.num_layers_total,
                                            d.gpu_kv_stride, d.gpu_block_stride, d.gpu_layer_stride,
                                            d.start_layer_id + l, kv, 0);
-  std::memcpy(h + tab, d.gpu_block_ids, ids_bytes);
+  std::memcpy(h + nplanes, d.gpu_block_ids, ids_bytes);
   uint8_t *dv = nullptr;
-  int rc = plan_publish(slot, tab + ids_bytes, /*mirror=*/true, stream, &dv);
+  int rc = carried ? FKV_OK : plan_publish(hold.slot, tab + ids_bytes, /*mirror=*/true, stream, &dv);
   if (rc == FKV_OK) {
     const int threads = 256;
     const int grid = std::max(1, std::min((d.bsz + threads - 1) / threads, 1024));
     hipLaunchKernelGGL(fkv_chunk_ptrs_kernel, dim3(grid), dim3(threads), 0, stream, d.out_ptrs,
                        reinterpret_cast<const uint64_t *>(dv),
-                       reinterpret_cast<const int64_t *>(dv + tab), d.gpu_block_stride, d.kv_dim,
-                       d.num_blocks, d.batch_start, d.bsz);
+                       carried ? nullptr : reinterpret_cast<const int64_t *>(dv + tab), d.gpu_block_stride,
+                       d.kv_dim, d.num_blocks, d.batch_start, d.bsz, nplanes, plan);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess)
       rc = fail(FKV_ERR_RUNTIME, "chunk pointer launch failed: %s", hipGetErrorString(e));

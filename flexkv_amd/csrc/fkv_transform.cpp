@@ -77,7 +77,12 @@ extern "C" int fkv_layout_transform(const fkv_layout_transform_desc *dp, void *s
     }
     std::memcpy(h + 2 * tab, d.gpu_block_ids, ids);
     uint8_t *dv = nullptr;
-    int rc = plan_publish(slot, 2 * tab + ids, /*mirror=*/true, stream, &dv);
+    const int vec = common_vector_width(&acc, 1);
+    // Small tables travel with the launch (see tables_from_arguments in fkv_kernels.hip): nothing
+    // is uploaded, and nothing on the device looks at the slot.
+    const bool carried = fits_arguments(lk, d.num_blocks, vec);
+    CopyReport report;
+    int rc = plan_publish(slot, 2 * tab + ids, /*mirror=*/!carried, stream, &dv);
     if (rc == FKV_OK) {
       CopyKernelArgs a{};
       const uint64_t *dg = reinterpret_cast<const uint64_t *>(dv);
@@ -92,11 +97,14 @@ extern "C" int fkv_layout_transform(const fkv_layout_transform_desc *dp, void *s
       a.chunk_bytes = d.chunk_size;
       a.num_blocks = d.num_blocks;
       a.lk = lk;
-      a.vec = common_vector_width(&acc, 1);
+      a.vec = vec;
       a.nt_store = 1;
       a.unroll = pol.hbm_unroll;
       a.xcd_mask = 0;
+      a.host_tables = carried;
+      a.report = &report;
       rc = launch_copy_kernel(a, workgroups, threads, stream);
+      hold.drained = report.in_arguments;
     }
     if (rc != FKV_OK)
       return rc;
