@@ -466,17 +466,22 @@ int default_num_cta(bool is_h2d) {
   return is_h2d ? h2d : d2h;
 }
 
-// Launch shape of the link-bound kernel.  Measured on MI355X with 4 requested CTAs:
+// Launch shape of the link-bound kernel.  Measured on MI355X with 4 requested CTAs (512 MiB):
 // GB/s over the link (a plain pinned hipMemcpy reaches 57.0 GPU->host / 57.3
 // host->GPU) and the slowdown of a kernel running next to the copy (a 2048^3 bf16
 // GEMM / fused attention / a streaming elementwise kernel):
-//   host->GPU  16 x  64 lanes : 57.2 GB/s,  1.9x /  1.10x /  1.05x   <- default
-//              24 x  64       : 57.4 GB/s,  2.9x /  1.16x /  1.10x
-//              12 x 1024      : 57.1 GB/s, 16x   /  2.1x  / 11x (stalled until the copy ends)
-//   GPU->host  48 x  64 lanes : 56.4 GB/s, streaming neighbour 2.7x   <- default
-//              24 x  64       : 54.7 GB/s, streaming neighbour 1.9x
-//              12 x 1024      : 56.6 GB/s, streaming neighbour 4.2x
-// So every requested CTA becomes four (host->GPU) or twelve (GPU->host)
+//   host->GPU   8 x 64 lanes : 40.8 GB/s, 1.5x / 1.9x / 1.1x
+//              12 x 64       : 57.0 GB/s, 1.6x / 1.9x / 1.2x
+//              16 x 64       : 57.3 GB/s, 1.8x / 2.4x / 1.2x   <- default
+//              24 x 64       : 57.4 GB/s, 2.7x / 3.6x / 1.4x
+//   GPU->host  16 x 64 lanes : 55.2 GB/s, 3.0x / 3.2x / 1.4x
+//              24 x 64       : 56.5 GB/s, 4.8x / 3.8x / 2.7x
+//              32 x 64       : 56.8 GB/s, 6.9x / 3.9x / 6.3x   <- default
+//              48 x 64       : 56.8 GB/s, 9.7x / 4.0x / 7.6x
+// (A wavefront that waited for the stores of a slice before it asked for the next one needed
+// 16 and 48 for these rates: 12 moved 50.0 GB/s from the host, 24 55.2 to it.)  Workgroups of
+// 1024 lanes stall the neighbours of a copy until it ends.
+// So every requested CTA becomes four (host->GPU) or eight (GPU->host)
 // single-wavefront workgroups: {h2d,d2h}_wg_per_cta and {h2d,d2h}_wg_threads of the
 // launch policy.
 
@@ -763,6 +768,7 @@ int shape_for_now(const KernelPlan &p, int64_t bytes, hipStream_t stream, CopyKe
                   bool *beside = nullptr) {
   const fkv_launch_policy pol = p.no_alloc ? policy_peek(p.device) : policy_of(p.device);
   int workgroups = p.workgroups;
+  bool next_to_other = false;
   const uint32_t all = pol.xcd_present_mask;
   const uint32_t busy_mask = p.h2d ? pol.h2d_busy_mask : pol.d2h_busy_mask;
   const uint32_t home_mask = p.h2d ? pol.h2d_home_mask : pol.d2h_home_mask;
@@ -786,13 +792,20 @@ int shape_for_now(const KernelPlan &p, int64_t bytes, hipStream_t stream, CopyKe
     workgroups = busy_workgroups;
     a->claims_per_wg = pol.busy_claims_per_wg;
     a->lane_runs = !p.h2d && pol.d2h_lane_runs == 2; // next to traffic the other way: see copy_slice
-    if (beside)
-      *beside = true;
+    next_to_other = true;
   } else if (pol.arbiter == 1 && home_mask != all && pol.home_min_kb >= 0 &&
              bytes >= (int64_t)pol.home_min_kb * 1024) {
     a->xcd_mask = home_mask;
     a->claims_per_wg = pol.home_claims_per_wg;
   }
+  // A short copy to the host spends its time getting under way, which more wavefronts do sooner,
+  // and its neighbours are free again in no time: 48 instead of 32 take 61.8 instead of 63.2 us
+  // for 2 MiB, 216.0 instead of 218.6 for 10 MiB, and no less for 64 MiB.
+  constexpr int64_t kShortCopyBytes = 16 << 20;
+  if (!p.h2d && !next_to_other && bytes < kShortCopyBytes)
+    workgroups = workgroups * 3 / 2;
+  if (beside)
+    *beside = next_to_other;
   return workgroups;
 }
 } // namespace

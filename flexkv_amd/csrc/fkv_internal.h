@@ -154,6 +154,15 @@ inline uint8_t *cpu_chunk_ptr(const fkv_transfer_desc &d, int64_t layer, int64_t
          d.cpu_startoff_inside_chunks;
 }
 
+// Memory behind an address that a kernel has computed from numbers: global, which the compiler
+// cannot know.  Without this it emits flat accesses, which count with those of LDS: the first
+// store of a slice then waits for all its loads instead of for its own.
+#if defined(__HIP__)
+#define FKV_GLOBAL __attribute__((address_space(1)))
+#else // the CPU model of the device
+#define FKV_GLOBAL
+#endif
+
 // ---- the gather/scatter kernel -----------------------------------------
 // One launch copies `num_blocks * lk` chunks of `chunk_bytes`:
 //   for pos, i:  src = base_src[i] + ids_src[pos]*stride_src

@@ -82,16 +82,29 @@ __device__ __forceinline__ uint32_t xcd_of_this_wave() {
 // accesses of a lane walk through one 128-byte line: a streaming hint lets the line go
 // between two of them (measured: 5.6 % of the lines fetched from HBM a second time).
 template <typename V, bool NT> __device__ __forceinline__ V get(const V *p) {
+  const FKV_GLOBAL V *g = (const FKV_GLOBAL V *)p;
   if (NT)
-    return __builtin_nontemporal_load(p);
-  return *p;
+    return __builtin_nontemporal_load(g);
+  return *g;
 }
 
 template <typename V, bool NT> __device__ __forceinline__ void put(V v, V *p) {
+  FKV_GLOBAL V *g = (FKV_GLOBAL V *)p;
   if (NT)
-    __builtin_nontemporal_store(v, p);
+    __builtin_nontemporal_store(v, g);
   else
-    *p = v;
+    *g = v;
+}
+
+// Ends a stretch with predicated stores, of which the compiler must think that they left a load
+// unused.  It would otherwise wait for everything in flight, the stores of whole slices too,
+// wherever such a stretch joins the path of those: a wavefront then asked for its next slice only
+// when the last store of the current one had been acknowledged, which over the link takes as long
+// as a load.
+__device__ __forceinline__ void nothing_in_flight() {
+#if defined(__HIP__)
+  __builtin_amdgcn_s_waitcnt(0x0f70); // vmcnt(0)
+#endif
 }
 
 // Which vector of the slice access u of a lane moves.  Ordinarily an access of the
@@ -134,6 +147,7 @@ __device__ __forceinline__ void copy_slice(const uint8_t *__restrict__ src,
     for (int u = 0; u < UNR; ++u)
       if (first + u * kAccessStep < nvec)
         put<V, NTS>(r[u], d + first + u * kAccessStep);
+    nothing_in_flight();
   }
 }
 
@@ -367,10 +381,17 @@ __device__ __forceinline__ void copy_share(const CopyKernelArgs &a, uint64_t num
           d[u] = reinterpret_cast<V *>(s_base_dst[i] + (uint64_t)s_off_dst[p]) + w;
           r[u] = get<V, !LR>(src);
         }
+        if (v0 + kPiece <= lim) {
 #pragma unroll
-        for (int u = 0; u < UNR; ++u)
-          if (v0 + u * kStep + lane * kLaneStep < lim)
+          for (int u = 0; u < UNR; ++u)
             put<V, NTS>(r[u], d[u]);
+        } else {
+#pragma unroll
+          for (int u = 0; u < UNR; ++u)
+            if (v0 + u * kStep + lane * kLaneStep < lim)
+              put<V, NTS>(r[u], d[u]);
+          nothing_in_flight();
+        }
       }
       continue;
     }
@@ -1072,7 +1093,7 @@ __device__ __forceinline__ void copy_layers(const LayersLaunch &t, const CopyKer
       V v[kCopyUnroll];
 #pragma unroll
       for (int u = 0; u < kCopyUnroll; ++u)
-        v[u] = __builtin_nontemporal_load(src + min(u * kWave + lane, nvec - 1));
+        v[u] = get<V, true>(src + min(u * kWave + lane, nvec - 1));
       // The vectors come from the other end of the link, so by the time they are here every
       // store of the range before has completed, and the answers of the two counters have come:
       // nothing is waited for that is not there.
@@ -1085,10 +1106,17 @@ __device__ __forceinline__ void copy_layers(const LayersLaunch &t, const CopyKer
         if (!shares.safety_net)
           ahead = claim_ahead();
       }
+      if (nvec == kWave * kCopyUnroll) {
 #pragma unroll
-      for (int u = 0; u < kCopyUnroll; ++u)
-        if (u * kWave + lane < nvec)
-          __builtin_nontemporal_store(v[u], dst + u * kWave + lane);
+        for (int u = 0; u < kCopyUnroll; ++u)
+          put<V, true>(v[u], dst + u * kWave + lane);
+      } else {
+#pragma unroll
+        for (int u = 0; u < kCopyUnroll; ++u)
+          if (u * kWave + lane < nvec)
+            put<V, true>(v[u], dst + u * kWave + lane);
+        nothing_in_flight();
+      }
     }
     landing.copied = (int)batch;
     part = shares.safety_net ? claim_now() : ahead;

@@ -51,8 +51,8 @@ __device__ __forceinline__ void wave_copy(const uint8_t *__restrict__ src, uint8
                                           int64_t bytes, int lane) {
   int64_t done = 0;
   if (VEC16) {
-    const vec16 *s = reinterpret_cast<const vec16 *>(src);
-    vec16 *d = reinterpret_cast<vec16 *>(dst);
+    const FKV_GLOBAL vec16 *s = (const FKV_GLOBAL vec16 *)src;
+    FKV_GLOBAL vec16 *d = (FKV_GLOBAL vec16 *)dst;
     const int64_t nvec = bytes / 16;
     constexpr int U = kCopyUnroll;
     constexpr int kLane = RUNS ? U : 1, kAccess = RUNS ? 1 : 64;
@@ -63,7 +63,7 @@ __device__ __forceinline__ void wave_copy(const uint8_t *__restrict__ src, uint8
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int64_t v = v0 + u * kAccess + lane * kLane;
-        const vec16 *from = s + (v < nvec ? v : nvec - 1);
+        const FKV_GLOBAL vec16 *from = s + (v < nvec ? v : nvec - 1);
         r[u] = RUNS ? *from : __builtin_nontemporal_load(from);
       }
 #pragma unroll
@@ -258,7 +258,7 @@ int fkv_staging_transfer(const fkv_staging_transfer_desc *dp, void *stream_v) tr
   // payloads, whose last slice is short: twice the workgroups of the fixed-size
   // kernel make up for it (16-29 KiB payloads: 45 GB/s with 16 wavefronts, 55.0 with
   // 24, 55.7 with 32).
-  int grid = cta * (write_cpu ? pol.d2h_wg_per_cta : 2 * pol.h2d_wg_per_cta);
+  int grid = cta * (write_cpu ? pol.d2h_wg_per_cta * 3 / 2 : 2 * pol.h2d_wg_per_cta);
   const int threads = write_cpu ? pol.d2h_wg_threads : pol.h2d_wg_threads;
   grid = std::max(1, std::min(grid, (d.bsz + threads / 64 - 1) / (threads / 64)));
 #define FKV_LAUNCH_STAGING(...)                                                               \
