@@ -733,11 +733,11 @@ CopyKernelArgs plan_job(const KernelPlan &p, int l0, int nl) {
   a.lk = nl * p.kv_dim;
   a.vec = p.vec;
   a.nt_store = p.h2d ? 1 : 0;
-  // Packed short chunks cost a wavefront more address arithmetic per request, so
-  // such launches get half as many workgroups again.  Host->GPU, 2304-byte chunks:
-  // 16 x 64 lanes reach 45 GB/s, 24 x 64 reach 55.8, 32 x 64 reach 56.2; GPU->host:
-  // 48 x 64 lanes 50.7 GB/s, 72 x 64 52.5, 96 x 64 53.0.
-  a.packed_grid_pct = 150; // replaced by the policy's when the launch is shaped
+  // Packed chunks cost a wavefront more address arithmetic per request, so
+  // such launches get a quarter as many workgroups again.  100 / 125 / 150 % take for chunks of 18 KiB
+  // from the host 180.1 / 180.0 / 178.9 us (8 MiB) and 919 / 918 / 918 (48 MiB), to it
+  // 183.3 / 178.7 / 178.2 and 921 / 921 / 921.
+  a.packed_grid_pct = 125; // replaced by the policy's when the launch is shaped
   a.xcd_mask = 0;
   a.claim = p.claims ? p.claims + l0 : nullptr; // a launch per first layer at most
   a.host_tables = p.host_tables;
@@ -836,13 +836,16 @@ int kernel_plan_launch(const KernelPlan &p, int layer_offset, int num_layers,
   return FKV_OK;
 }
 
-bool layers_launch_fits(const KernelPlan &p) {
-  // What fkv_copy_layers_kernel is built for: 16-byte vectors, chunks of a slice at least
-  // (shorter ones need the packed form), every base address in one LDS table, single
-  // wavefronts, and a counter to claim from.
+bool layers_launch_fits(const KernelPlan &p, int layers_per_batch) {
+  // What fkv_copy_layers_kernel is built for: 16-byte vectors, of which a batch of chunks that are
+  // no whole number of slices has no more than it counts in 32 bits, every base address in one
+  // LDS table, single wavefronts, and a counter to claim from.
+  const bool whole_slices = p.chunk_size % ((int64_t)64 * kCopyUnroll * 16) == 0;
   return layers_device && p.h2d && p.host_visible && p.vec == 16 &&
-         p.chunk_size >= (int64_t)64 * kCopyUnroll * 16 && p.num_layers * p.kv_dim <= kCopyMaxLK &&
-         p.threads == 64 && p.claims && !p.no_alloc && !p.recorded;
+         (whole_slices ||
+          p.chunk_size / 16 * layers_per_batch * p.kv_dim * p.num_blocks <= kLayersMaxVectors) &&
+         p.num_layers * p.kv_dim <= kCopyMaxLK && p.threads == 64 && p.claims && !p.no_alloc &&
+         !p.recorded;
 }
 
 int kernel_plan_launch_layers(const KernelPlan &p, int layers_per_batch, LayersLaunch t,

@@ -185,7 +185,7 @@ struct CopyKernelArgs {
   int32_t unroll;   // 0: the host link bounds the launch; kCopyUnroll or kCopyUnrollDeep: HBM
                     // does, and so many vectors per lane, if launch_copy_kernel finds it fit
   int32_t per_slice; // set by launch_copy_kernel: HBM bounds it, see fkv_copy_slices_kernel
-  int32_t packed;   // set by launch_copy_kernel: chunks shorter than a slice, see the kernel
+  int32_t packed;   // set by launch_copy_kernel: chunks of no whole number of slices, see the kernel
   int32_t lane_runs; // stores into pinned host memory: a lane moves adjacent vectors (see copy_slice)
   int32_t packed_grid_pct; // workgroups to launch in packed mode, percent of the request (0 = 100)
   uint32_t xcd_mask; // bit k: workgroups that run on XCD k take part; 0 = all
@@ -243,6 +243,7 @@ int launch_copy_jobs(const CopyKernelArgs *jobs, int njobs, int num_workgroups,
 // Layers [0, a.lk / kv_dim) of a plan in batches of `pairs_per_batch` (layer, kv) pairs (the
 // last one may be shorter), copied in order by one kernel that announces each batch as it
 // lands; see fkv_copy_layers_kernel.
+constexpr int64_t kLayersMaxVectors = 1ll << 31; // of a batch, 32 GiB
 struct LayersLaunch {
   CopyKernelArgs a;
   int32_t pairs_per_batch;
@@ -391,7 +392,7 @@ int kernel_plan_launch(const KernelPlan &p, int layer_offset, int num_layers,
                        hipStream_t stream, CopyReport *report = nullptr);
 // All layers of the plan in one launch, `layers_per_batch` at a time; `t` brings the words
 // that announce the batches.  Only for plans layers_launch_fits accepts.
-bool layers_launch_fits(const KernelPlan &p);
+bool layers_launch_fits(const KernelPlan &p, int layers_per_batch);
 int kernel_plan_launch_layers(const KernelPlan &p, int layers_per_batch, LayersLaunch t,
                               hipStream_t stream);
 // The same for layer ranges of several plans of one direction in one launch (the

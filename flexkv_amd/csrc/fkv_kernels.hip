@@ -19,11 +19,11 @@
 // requests a workgroup has in flight target neighbouring addresses.  A
 // wavefront issues all kCopyUnroll loads of a slice before the first store, which
 // is what keeps enough reads outstanding to cover the host-link latency in
-// the host->GPU direction.  Chunks shorter than a slice (compressed layer
+// the host->GPU direction.  Chunks that are no whole number of slices (compressed layer
 // groups, small pages) are packed: the 16-byte vectors of all chunks form one
 // flat sequence that is cut into full slices regardless of chunk boundaries,
 // every lane resolving the chunk of each of its vectors from the LDS tables, so
-// that a wavefront keeps a full slice of requests in flight however short the
+// that a wavefront keeps a full slice of requests in flight however long the
 // chunks are.
 //
 // Launch shape.  The link is saturated by roughly 200 KB of requests in flight.
@@ -277,7 +277,7 @@ __device__ __forceinline__ void copy_share(const CopyKernelArgs &a, uint64_t num
   constexpr uint32_t kPiece = kWave * UNR; // vectors a wavefront moves per step
   const uint32_t slices = (uint32_t)a.slices_per_chunk;
   // Work units.  Normal mode: slices of a chunk, `spp` per block position.  Packed
-  // mode (chunks shorter than a slice): the vectors of all chunks form one flat
+  // mode (chunks of no whole number of slices): the vectors of all chunks form one flat
   // sequence, cut into pieces of kPiece vectors regardless of chunk boundaries.
   const uint32_t vpc = (uint32_t)(a.chunk_bytes / VEC);  // vectors per chunk
   const uint32_t spp = a.packed ? (uint32_t)a.lk * vpc : (uint32_t)a.lk * slices;
@@ -794,21 +794,22 @@ int prepare_job(CopyKernelArgs &a, int64_t *total, int *grid_pct) {
                 (long long)a.chunk_bytes, a.lk);
   a.slices_per_chunk = (int32_t)slices;
   *total = spp * a.num_blocks;
-  // Chunks shorter than one slice would leave most lanes of a wavefront idle and
-  // most of its requests unissued: pack them (the kernel indexes vectors inside an
-  // id tile with 32 bits).
+  // Chunks that are no whole number of slices would leave lanes of a wavefront idle and requests
+  // of it unissued in their last slice: they are packed (the kernel indexes vectors inside an
+  // id tile with 32 bits).  48 MiB, us, short last slices (and as many more workgroups) -> packed:
+  // host->GPU chunks of 9 KiB 951 -> 919, 18 KiB 921 -> 918; GPU->host 22 224 bytes 939 -> 930,
+  // 64 KiB less a vector 936 -> 925; 1 MiB the same or 1 us less.  Launches that HBM bounds stay
+  // with slices where a chunk has one.
   const int64_t vpp = a.chunk_bytes / a.vec * a.lk;
-  a.packed = (a.chunk_bytes < slice_bytes && vpp * kCopyIdTile <= (int64_t)UINT32_MAX) ? 1 : 0;
+  a.packed = (a.chunk_bytes % slice_bytes != 0 && !a.per_slice && vpp * kCopyIdTile <= (int64_t)UINT32_MAX) ? 1 : 0;
   if (a.packed) {
     const int64_t piece = (int64_t)kWave * a.unroll;
     *total = (vpp * a.num_blocks + piece - 1) / piece;
     if (a.packed_grid_pct > 0)
       *grid_pct = a.packed_grid_pct;
   } else {
-    // A wavefront has one slice in flight, and the last slice of a chunk is short
-    // when the chunk is no multiple of a slice (18 KiB = 8 + 8 + 2): the bytes in
-    // flight, which set the rate of a launch with few workgroups, shrink to
-    // chunk / (slices x slice).  As many workgroups more make up for it.
+    // Too large to be packed: a wavefront has one slice in flight, and the last slice of a chunk
+    // may be short.  As many workgroups more make up for it.
     *grid_pct = (int)((slices * slice_bytes * 100 + a.chunk_bytes - 1) / a.chunk_bytes);
   }
   return FKV_OK;
@@ -927,13 +928,16 @@ int launch_copy_kernel(CopyKernelArgs a, int num_workgroups, int threads_per_wor
                        hipStream_t stream) {
   int64_t total = 0;
   int grid_pct = 100;
+  const bool hbm_bound = a.unroll != 0;
   FKV_TRY(prepare_job(a, &total, &grid_pct));
   if (total == 0)
     return FKV_OK;
   int64_t grid = 1;
   int threads = kWave;
-  if (a.per_slice && threads_per_workgroup > kSliceWgThreads) {
-    // the same number of wavefronts in smaller workgroups, which find room on a CU sooner
+  if (hbm_bound && threads_per_workgroup > kSliceWgThreads) {
+    // the same number of wavefronts in smaller workgroups, which find room on a CU sooner (packed,
+    // 1024 -> 256 lanes: 146 MiB out of chunks of 2880 bytes 83 -> 76 us, 60 MiB of 2304 54 -> 51,
+    // 80 MiB of 4 KiB 57 -> 52)
     num_workgroups = (int)std::min<int64_t>(
         (int64_t)num_workgroups * threads_per_workgroup / kSliceWgThreads, INT32_MAX);
     threads_per_workgroup = kSliceWgThreads;
@@ -1027,6 +1031,12 @@ namespace {
 // to eventfds 159 -> 78, 32 x 1 MiB 773 -> 647, 61 x 7 MiB 9190 (rows gathered by host threads)
 // -> 7709, which is 56 GB/s.  Next to a fused attention of 76 us a layer: 32 x 1 MiB 2845 -> 2798,
 // 61 x 7 MiB 9193 -> 7994; next to three 2048^3 GEMMs a layer: 2691 -> 2585, 9224 -> 8076.
+// Chunks of no whole number of slices are packed, batch by batch, as in copy_share: a batch is a
+// sequence of vectors, position-major, cut into pieces of a slice.  Short chunks used to take a
+// launch a batch (us, before -> this): 55 x 122 KiB in chunks of 2304 bytes 618 -> 170, 31 x 824 KiB
+// 946 -> 521; 8 batches of 5 chunks, a stream waiting for each, 149 -> 58.  Longer ones had short last
+// slices: 41 x 4.6 MiB in chunks of 18 KiB 3567 -> 3502, 61 x 1.1 MiB 1326 -> 1324.
+template <bool PACKED>
 __device__ __forceinline__ void copy_layers(const LayersLaunch &t, const CopyKernelArgs &a) {
   using V = VecType<16>::type;
   __shared__ uint64_t s_base_src[kCopyMaxLK], s_base_dst[kCopyMaxLK];
@@ -1037,7 +1047,10 @@ __device__ __forceinline__ void copy_layers(const LayersLaunch &t, const CopyKer
     return;
   const int lane = threadIdx.x;
   constexpr int64_t kSliceBytes = (int64_t)kWave * kCopyUnroll * 16;
+  constexpr uint32_t kPiece = kWave * kCopyUnroll;
   const uint32_t slices = (uint32_t)a.slices_per_chunk;
+  const uint32_t vpc = (uint32_t)(a.chunk_bytes / 16);
+  const uint32_t q64 = kWave / vpc, r64 = kWave % vpc; // 64 vectors = q64 chunks + r64
   uint32_t tile = 0; // first of the block positions whose offsets are in LDS
   auto load_tile = [&](uint32_t at) {
     __syncthreads();
@@ -1074,26 +1087,71 @@ __device__ __forceinline__ void copy_layers(const LayersLaunch &t, const CopyKer
     const uint32_t ranges = t.ranges_of((int)batch);
     const uint32_t pair0 = batch * (uint32_t)t.pairs_per_batch;
     const uint32_t pairs = min((uint32_t)t.pairs_per_batch, (uint32_t)a.lk - pair0);
-    const uint32_t spp = pairs * slices;
-    const uint64_t units = (uint64_t)a.num_blocks * spp;
+    const uint32_t spp = pairs * (PACKED ? vpc : slices);
+    const uint32_t vectors = (uint32_t)a.num_blocks * spp; // packed: checked on the host
+    const uint64_t units = PACKED ? (vectors + kPiece - 1) / kPiece : (uint64_t)a.num_blocks * spp;
     const uint64_t s0 = units * range / ranges;
     const uint64_t s1 = units * (range + 1) / ranges;
+    const uint32_t qlk = q64 / pairs, rlk = q64 - qlk * pairs; // q64 chunks = qlk positions + rlk
     for (uint64_t s = s0; s < s1; ++s) {
-      const uint32_t p = (uint32_t)(s / spp);
-      const uint32_t r = (uint32_t)(s - (uint64_t)p * spp);
-      const uint32_t i = r / slices, sl = r - i * slices;
-      if (p - tile >= (uint32_t)kCopyIdTile) // behind the tile, or before it (wraps)
-        load_tile(p / kCopyIdTile * kCopyIdTile);
-      const int64_t off = (int64_t)sl * kSliceBytes;
-      const int64_t left = a.chunk_bytes - off;
-      const int nvec = (int)((left < kSliceBytes ? left : kSliceBytes) / 16);
-      const V *src = reinterpret_cast<const V *>(s_base_src[pair0 + i] +
-                                                 (uint64_t)s_off_src[p - tile] + off);
-      V *dst = reinterpret_cast<V *>(s_base_dst[pair0 + i] + (uint64_t)s_off_dst[p - tile] + off);
+      const V *src[kCopyUnroll];
+      V *dst[kCopyUnroll];
+      int nvec; // vectors of the piece: those of a lane are 64 apart
+      if (PACKED) {
+        const uint32_t v0 = (uint32_t)s * kPiece, last = min(v0 + kPiece, vectors) - 1;
+        const uint32_t first_p = v0 / spp, last_p = last / spp;
+        if (first_p < tile || last_p - tile >= (uint32_t)kCopyIdTile)
+          load_tile(first_p); // a piece spans 512 positions at most
+        nvec = (int)(last + 1 - v0);
+        // located by division, the further ones by adding quotients and remainders; lanes
+        // beyond the end stay on their last valid vector
+        uint32_t v = v0 + lane;
+        const uint32_t vc = min(v, last);
+        const uint32_t c = vc / vpc;
+        uint32_t w = vc - c * vpc, p = c / pairs, i = c - p * pairs;
+#pragma unroll
+        for (int u = 0; u < kCopyUnroll; ++u) {
+          if (u > 0) {
+            v += kWave;
+            uint32_t w2 = w + r64, i2 = i + rlk, p2 = p + qlk;
+            if (w2 >= vpc) {
+              w2 -= vpc;
+              i2 += 1;
+            }
+            if (i2 >= pairs) {
+              i2 -= pairs;
+              p2 += 1;
+            }
+            const bool ok = v <= last;
+            w = ok ? w2 : w;
+            i = ok ? i2 : i;
+            p = ok ? p2 : p;
+          }
+          src[u] = reinterpret_cast<const V *>(s_base_src[pair0 + i] + (uint64_t)s_off_src[p - tile]) + w;
+          dst[u] = reinterpret_cast<V *>(s_base_dst[pair0 + i] + (uint64_t)s_off_dst[p - tile]) + w;
+        }
+      } else {
+        const uint32_t p = (uint32_t)(s / spp);
+        const uint32_t r = (uint32_t)(s - (uint64_t)p * spp);
+        const uint32_t i = r / slices, sl = r - i * slices;
+        if (p - tile >= (uint32_t)kCopyIdTile) // behind the tile, or before it (wraps)
+          load_tile(p / kCopyIdTile * kCopyIdTile);
+        const int64_t off = (int64_t)sl * kSliceBytes;
+        const int64_t left = a.chunk_bytes - off;
+        nvec = (int)((left < kSliceBytes ? left : kSliceBytes) / 16);
+        const V *from = reinterpret_cast<const V *>(s_base_src[pair0 + i] +
+                                                    (uint64_t)s_off_src[p - tile] + off);
+        V *to = reinterpret_cast<V *>(s_base_dst[pair0 + i] + (uint64_t)s_off_dst[p - tile] + off);
+#pragma unroll
+        for (int u = 0; u < kCopyUnroll; ++u) {
+          src[u] = from + min(u * kWave + lane, nvec - 1);
+          dst[u] = to + u * kWave + lane;
+        }
+      }
       V v[kCopyUnroll];
 #pragma unroll
       for (int u = 0; u < kCopyUnroll; ++u)
-        v[u] = get<V, true>(src + min(u * kWave + lane, nvec - 1));
+        v[u] = get<V, true>(src[u]);
       // The vectors come from the other end of the link, so by the time they are here every
       // store of the range before has completed, and the answers of the two counters have come:
       // nothing is waited for that is not there.
@@ -1106,15 +1164,15 @@ __device__ __forceinline__ void copy_layers(const LayersLaunch &t, const CopyKer
         if (!shares.safety_net)
           ahead = claim_ahead();
       }
-      if (nvec == kWave * kCopyUnroll) {
+      if (nvec == (int)kPiece) {
 #pragma unroll
         for (int u = 0; u < kCopyUnroll; ++u)
-          put<V, true>(v[u], dst + u * kWave + lane);
+          put<V, true>(v[u], dst[u]);
       } else {
 #pragma unroll
         for (int u = 0; u < kCopyUnroll; ++u)
           if (u * kWave + lane < nvec)
-            put<V, true>(v[u], dst + u * kWave + lane);
+            put<V, true>(v[u], dst[u]);
         nothing_in_flight();
       }
     }
@@ -1127,11 +1185,14 @@ __device__ __forceinline__ void copy_layers(const LayersLaunch &t, const CopyKer
     landing.count();
   landing.announce();
 }
-__global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) { copy_layers(t, t.a); }
+template <bool PACKED> __global__ __launch_bounds__(kWave) void fkv_copy_layers_kernel(LayersLaunch t) {
+  copy_layers<PACKED>(t, t.a);
+}
+template <bool PACKED>
 __global__ __launch_bounds__(kWave) void fkv_copy_layers_args_kernel(LayersLaunch t, ArgPlan plan) {
   CopyKernelArgs a = t.a;
   tables_from_arguments(a, plan);
-  copy_layers(t, a);
+  copy_layers<PACKED>(t, a);
 }
 
 // Holds its stream until batches have landed, as an event behind them would: for as long as that
@@ -1158,7 +1219,10 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
   int64_t total = 0;
   int grid_pct = 100;
   FKV_TRY(prepare_job(t.a, &total, &grid_pct));
-  if (total == 0 || t.a.packed || t.a.vec != 16 || !t.a.claim || t.batches < 1)
+  // vectors of a batch, which the kernel counts in 32 bits
+  const int64_t vpb = t.a.chunk_bytes / 16 * t.pairs_per_batch * t.a.num_blocks;
+  if (total == 0 || t.a.vec != 16 || !t.a.claim || t.batches < 1 ||
+      (t.a.packed && vpb > kLayersMaxVectors))
     return fail(FKV_ERR_RUNTIME, "copy kernel: a restore of this shape has no single launch");
   int64_t grid = 1;
   int threads = kWave;
@@ -1170,8 +1234,15 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
                          std::max(1, __builtin_popcount(present))
                    : grid;
   const int64_t last_pairs = t.a.lk - (int64_t)(t.batches - 1) * t.pairs_per_batch;
-  const LayersCut cut = cut_layers(t.batches, t.pairs_per_batch, last_pairs,
-                                   (int64_t)t.a.num_blocks * t.a.slices_per_chunk, working);
+  constexpr int64_t kPiece = kWave * kCopyUnroll;
+  const int64_t vectors = t.a.chunk_bytes / 16 * t.a.num_blocks; // of a pair
+  LayersCut cut = cut_layers(t.batches, t.pairs_per_batch, last_pairs,
+                             t.a.packed ? std::max<int64_t>(1, vectors / kPiece)
+                                        : (int64_t)t.a.num_blocks * t.a.slices_per_chunk, working);
+  if (t.a.packed) { // none empty
+    cut.ranges = std::min(cut.ranges, (vectors * t.pairs_per_batch + kPiece - 1) / kPiece);
+    cut.last_ranges = std::min({cut.last_ranges, cut.ranges, (vectors * last_pairs + kPiece - 1) / kPiece});
+  }
   if (last_pairs < 1 || cut.claims(t.batches) > (int64_t)INT32_MAX)
     return fail(FKV_ERR_RUNTIME, "copy kernel: %d batches of %d of %d (layer, kv) pairs", t.batches,
                 t.pairs_per_batch, t.a.lk);
@@ -1182,10 +1253,11 @@ int launch_layers(LayersLaunch t, int num_workgroups, hipStream_t stream) {
   ArgPlan plan;
   int words = 0;
   if (into_arguments(with_plan.a, nullptr, 0, plan, &words)) {
-    hipLaunchKernelGGL(fkv_copy_layers_args_kernel, dim3((unsigned)grid), dim3(kWave), 0, stream,
-                       with_plan, plan);
+    hipLaunchKernelGGL(t.a.packed ? fkv_copy_layers_args_kernel<true> : fkv_copy_layers_args_kernel<false>,
+                       dim3((unsigned)grid), dim3(kWave), 0, stream, with_plan, plan);
   } else {
-    hipLaunchKernelGGL(fkv_copy_layers_kernel, dim3((unsigned)grid), dim3(kWave), 0, stream, t);
+    hipLaunchKernelGGL(t.a.packed ? fkv_copy_layers_kernel<true> : fkv_copy_layers_kernel<false>,
+                       dim3((unsigned)grid), dim3(kWave), 0, stream, t);
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess)

@@ -198,7 +198,7 @@ fkv_launch_policy defaults_for(uint32_t present) {
   p.d2h_wg_per_cta = 8;
   p.h2d_wg_per_cta = 4;
   p.d2h_wg_threads = p.h2d_wg_threads = 64;
-  p.packed_grid_pct = 150;
+  p.packed_grid_pct = 125;
   p.plan_mirror = -1;
   p.fuse_launches = 1;
   p.lane_streams = -1;

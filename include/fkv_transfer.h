@@ -707,7 +707,7 @@ typedef struct fkv_launch_policy {
   int32_t h2d_wg_per_cta;
   int32_t d2h_wg_threads;     /* lanes per workgroup */
   int32_t h2d_wg_threads;
-  int32_t packed_grid_pct;    /* packed short chunks: workgroups, percent of the normal count */
+  int32_t packed_grid_pct;    /* packed chunks: workgroups, percent of the normal count */
   int32_t plan_mirror;        /* -1 upload the plan unless one launch reads it once and it is small (it
                                  travels in the arguments, or is read in place), or the other
                                  direction is busy; 0 never, 1 always */

@@ -247,3 +247,19 @@ def test_shapes_that_go_batch_by_batch(gpu_device):
         s.oracle_transfer(ids, ids, True)
         dev.assert_matches_reference(f"chunk {chunk}")
         grp.close()
+
+
+# chunks of no whole number of slices: pieces that cross chunks, blocks, id tiles and the end of a batch
+@pytest.mark.parametrize("policy", ["default", "confined"])
+@pytest.mark.parametrize("backend,layers,kv,chunk,n,gran", [
+    (VLLM, 4, 1, 16, 1, 1),         # a vector a batch: one short piece, one range
+    (VLLM, 4, 1, 2304, 9, 1),       # the fewest batches
+    (VLLM, 9, 2, 2304, 57, 2),      # two layers a batch and a short last batch
+    (SGLANG, 5, 2, 8176, 3, 1),     # a vector less than a slice
+    (TRTLLM, 6, 1, 9936, 21, 1),    # a slice and more
+    (VLLM, 5, 1, 48, 3000, 1),      # pieces of 171 blocks: every third id tile starts inside one
+    (VLLM, 33, 1, 18432, 40, 1),
+    (VLLM, 500, 2, 256, 1, 1),      # more batches than a wavefront has lanes
+])
+def test_packed_restore_in_one_launch(gpu_device, backend, layers, kv, chunk, n, gran, policy):
+    test_restore_in_one_launch(gpu_device, backend, layers, kv, chunk, n, gran, policy)
