@@ -99,12 +99,9 @@ constexpr int kRuntimeWaits = 2;
 constexpr int64_t kLongWaitNs = 20 * 1000 * 1000;
 } // namespace
 
-hipError_t quiet_event_wait(hipEvent_t event, int device, int64_t expected_ns) {
-  const int setting = policy_peek(device).quiet_wait_us;
-  const int limit_us = setting < 0 ? -setting : setting;
-  Waiting here;
-  if (setting == 0 || (setting > 0 && here.others < kRuntimeWaits && expected_ns < kLongWaitNs))
-    return hipEventSynchronize(event);
+namespace {
+// Looks until `look` says something else than "not ready", with sleeps of up to `limit_us` between.
+template <typename Look> hipError_t quiet_poll(Look look, int limit_us, int64_t expected_ns) {
   using clock = std::chrono::steady_clock;
   const auto t0 = clock::now();
   // Where the work is expected to end: sleep up to shortly before that, look closely around
@@ -115,10 +112,9 @@ hipError_t quiet_event_wait(hipEvent_t event, int device, int64_t expected_ns) {
   const auto close_until = t0 + std::chrono::nanoseconds(std::max<int64_t>(30 * 1000, expected_ns + kCloseNs));
   int nap_us = 20;
   for (;;) {
-    const hipError_t q = hipEventQuery(event);
+    const hipError_t q = look();
     if (q != hipErrorNotReady)
       return q;
-    (void)hipGetLastError(); // "not ready" is no error of the caller's
     const auto now = clock::now();
     if (now < close_from) {
       // never long at a stretch: a core that has slept for tens of milliseconds can take
@@ -132,6 +128,23 @@ hipError_t quiet_event_wait(hipEvent_t event, int device, int64_t expected_ns) {
       nap_us = std::min(nap_us * 2, limit_us);
     }
   }
+}
+} // namespace
+
+hipError_t quiet_event_wait(hipEvent_t event, int device, int64_t expected_ns) {
+  const int setting = policy_peek(device).quiet_wait_us;
+  const int limit_us = setting < 0 ? -setting : setting;
+  Waiting here;
+  if (setting == 0 || (setting > 0 && here.others < kRuntimeWaits && expected_ns < kLongWaitNs))
+    return hipEventSynchronize(event);
+  return quiet_poll(
+      [event] {
+        const hipError_t q = hipEventQuery(event);
+        if (q == hipErrorNotReady)
+          (void)hipGetLastError(); // no error of the caller's
+        return q;
+      },
+      limit_us, expected_ns);
 }
 
 hipError_t quiet_word_wait(const uint64_t *word, uint64_t at_least, hipEvent_t behind, int device) {
@@ -167,6 +180,44 @@ hipError_t quiet_word_wait(const uint64_t *word, uint64_t at_least, hipEvent_t b
           return hipErrorUnknown;
       return hipSuccess;
     }
+  }
+}
+
+hipError_t quiet_copy_wait(const uint64_t *word, uint64_t at_least, hipStream_t stream, int device,
+                           int64_t expected_ns) {
+  const int setting = policy_peek(device).quiet_wait_us;
+  Waiting here;
+  const bool spin = setting == 0 ||
+                    (setting > 0 && here.others < kRuntimeWaits && expected_ns < kLongWaitNs);
+  // How often the stream is asked whether the kernel ended in an error: every few milliseconds of
+  // looking, every 16th time when sleeping.
+  const unsigned every = spin ? 1u << 17 : 16;
+  unsigned looks = 0;
+  auto there = [&] { return __atomic_load_n(word, __ATOMIC_ACQUIRE) >= at_least; };
+  auto look = [&]() -> hipError_t {
+    if (there())
+      return hipSuccess;
+    if (++looks % every != 0)
+      return hipErrorNotReady;
+    const hipError_t q = hipStreamQuery(stream);
+    if (q == hipErrorNotReady || capture_forbids(q)) {
+      (void)hipGetLastError();
+      return hipErrorNotReady;
+    }
+    if (q != hipSuccess)
+      return q;
+    for (const auto until = std::chrono::steady_clock::now() + kLateWord; !there();)
+      if (std::chrono::steady_clock::now() >= until)
+        return hipErrorUnknown;
+    return hipSuccess;
+  };
+  if (!spin)
+    return quiet_poll(look, setting < 0 ? -setting : setting, expected_ns);
+  for (;;) {
+    const hipError_t q = look();
+    if (q != hipErrorNotReady)
+      return q;
+    __builtin_ia32_pause();
   }
 }
 
@@ -449,6 +500,106 @@ void plan_release(PlanSlot *s, hipStream_t stream, bool drained) {
   s->busy = false;
 }
 
+// ---- words of launches somebody waits for ----------------------------------------
+bool (*copies_announce)(hipStream_t) = nullptr;
+
+namespace {
+// A word and a count per call in flight, taken from a pool per device and given back when the
+// wait is over; never freed (the link's bookkeeping looks at words of calls that are over).
+struct DonePool {
+  std::mutex mu;
+  std::map<int, std::vector<CopyDone>> idle;
+};
+DonePool &done_pool() {
+  static DonePool *p = new DonePool(); // lives until the process ends
+  return *p;
+}
+constexpr size_t kDoneChunk = 64;  // calls that share an allocation,
+constexpr size_t kDoneStride = 256; // each with lines of its own
+static_assert(sizeof(DoneCounts) <= kDoneStride, "the counts of a call fit its part");
+
+// The word of one call, for as long as somebody waits for it.
+class DoneWord {
+public:
+  DoneWord() = default;
+  DoneWord(const DoneWord &) = delete;
+  DoneWord &operator=(const DoneWord &) = delete;
+  // A word that a launch was made with and nobody waited for to the end stays out of the pool: the
+  // launch may yet count.
+  ~DoneWord() {
+    if (!used_)
+      finished();
+  }
+  // `device` is current.  Without a word (none to be had, a stream that is being captured and
+  // will not run the launch now) the call waits for an event.  The first call of 64 at a time
+  // allocates; new counts are cleared by a kernel on its own stream, which it waits for.
+  void acquire(int device, hipStream_t stream) {
+    if (!copies_announce || !copies_announce(stream))
+      return;
+    device_ = device;
+    DonePool &p = done_pool();
+    {
+      std::lock_guard<std::mutex> lk(p.mu);
+      std::vector<CopyDone> &v = p.idle[device];
+      if (!v.empty()) {
+        done_ = v.back();
+        v.pop_back();
+      }
+    }
+    if (!done_.word && !allocate(stream))
+      return;
+    ++done_.epoch;
+    done_.used = &used_;
+  }
+  // Nothing looks at it any more: the word may serve the next call.
+  void finished() {
+    if (!done_.word)
+      return;
+    done_.used = nullptr;
+    DonePool &p = done_pool();
+    std::lock_guard<std::mutex> lk(p.mu);
+    p.idle[device_].push_back(done_);
+    done_ = CopyDone{};
+  }
+  const CopyDone &get() const { return done_; }
+
+private:
+  bool allocate(hipStream_t stream) {
+    constexpr size_t kBytes = kDoneChunk * kDoneStride;
+    void *d = nullptr, *h = nullptr;
+    bool ok = hipHostMalloc(&h, kBytes, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess &&
+              hipMalloc(&d, kBytes) == hipSuccess;
+    if (ok) {
+      std::memset(h, 0, kBytes);
+      ok = launch_plan_upload(d, h, kBytes, stream) == FKV_OK;
+      ok = hipStreamSynchronize(stream) == hipSuccess && ok;
+    }
+    if (!ok) {
+      clear_error();
+      (void)hipGetLastError();
+      if (d)
+        (void)hipFree(d);
+      if (h)
+        (void)hipHostFree(h);
+      return false;
+    }
+    DonePool &p = done_pool();
+    std::lock_guard<std::mutex> lk(p.mu);
+    std::vector<CopyDone> &v = p.idle[device_];
+    for (size_t i = 0; i < kDoneChunk; ++i) {
+      done_.count = reinterpret_cast<DoneCounts *>(static_cast<uint8_t *>(d) + i * kDoneStride);
+      done_.word = reinterpret_cast<uint64_t *>(static_cast<uint8_t *>(h) + i * kDoneStride);
+      if (i + 1 < kDoneChunk)
+        v.push_back(done_);
+    }
+    return true;
+  }
+  CopyDone done_;
+  int device_ = 0;
+  bool used_ = false;
+};
+} // namespace
+
 // ---- kernel path ---------------------------------------------------------
 namespace {
 int env_int(const char *name, int fallback) {
@@ -517,6 +668,7 @@ constexpr int kActivityRing = 16;
 struct DirectionActivity {
   hipEvent_t ev[kActivityRing] = {};
   bool pending[kActivityRing] = {};
+  CopyDone done[kActivityRing] = {}; // with a word: that instead of the event
   hipStream_t stream[kActivityRing] = {};
   int64_t launched_ns[kActivityRing] = {}; // steady clock at launch
   int next = 0;
@@ -554,7 +706,10 @@ bool link_direction_busy(int device, bool h2d, hipStream_t launching_stream) {
       busy = true;
     if (!d.pending[i])
       continue;
-    if (hipEventQuery(d.ev[i]) == hipSuccess) {
+    if (d.done[i].word) {
+      d.pending[i] = __atomic_load_n(d.done[i].word, __ATOMIC_RELAXED) < d.done[i].epoch;
+      busy = busy || (d.pending[i] && d.stream[i] != launching_stream);
+    } else if (hipEventQuery(d.ev[i]) == hipSuccess) {
       d.pending[i] = false;
     } else {
       (void)hipGetLastError();
@@ -564,7 +719,8 @@ bool link_direction_busy(int device, bool h2d, hipStream_t launching_stream) {
   return busy;
 }
 
-void link_direction_mark(int device, bool h2d, hipStream_t stream, int64_t bytes) {
+void link_direction_mark(int device, bool h2d, hipStream_t stream, int64_t bytes,
+                         const CopyDone &done) {
   const fkv_launch_policy pol = policy_of(device);
   if (pol.arbiter == 0)
     return;
@@ -575,15 +731,18 @@ void link_direction_mark(int device, bool h2d, hipStream_t stream, int64_t bytes
   std::lock_guard<std::mutex> lk(a.mu);
   DirectionActivity &d = a.dir[h2d ? 1 : 0];
   const int i = d.next;
-  if (!d.ev[i] && hipEventCreateWithFlags(&d.ev[i], kBookkeepingEvent) != hipSuccess) {
-    (void)hipGetLastError();
-    d.ev[i] = nullptr;
-    return;
+  if (!done.word) {
+    if (!d.ev[i] && hipEventCreateWithFlags(&d.ev[i], kBookkeepingEvent) != hipSuccess) {
+      (void)hipGetLastError();
+      d.ev[i] = nullptr;
+      return;
+    }
+    if (hipEventRecord(d.ev[i], stream) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
   }
-  if (hipEventRecord(d.ev[i], stream) != hipSuccess) {
-    (void)hipGetLastError();
-    return;
-  }
+  d.done[i] = done;
   d.pending[i] = true;
   d.stream[i] = stream;
   d.launched_ns[i] = steady_ns();
@@ -811,7 +970,7 @@ int shape_for_now(const KernelPlan &p, int64_t bytes, hipStream_t stream, CopyKe
 } // namespace
 
 int kernel_plan_launch(const KernelPlan &p, int layer_offset, int num_layers,
-                       hipStream_t stream, CopyReport *report) {
+                       hipStream_t stream, CopyReport *report, const CopyDone &done) {
   if (!p.host_visible)
     return fail(FKV_ERR_INVALID_ARG, "kernel transfer: the host pool is not device-visible "
                 "(allocate it pinned or register it)");
@@ -822,17 +981,23 @@ int kernel_plan_launch(const KernelPlan &p, int layer_offset, int num_layers,
   const int layers_per_launch = kCopyMaxLK / p.kv_dim;
   if (layers_per_launch < 1)
     return fail(FKV_ERR_INVALID_ARG, "kv_dim %d too large", p.kv_dim);
+  CopyReport mine;
+  if (!report)
+    report = &mine;
   for (int l0 = layer_offset; l0 < layer_offset + num_layers; l0 += layers_per_launch) {
     const int nl = std::min(layers_per_launch, layer_offset + num_layers - l0);
     CopyKernelArgs a = plan_job(p, l0, nl);
     a.report = report; // tables that fit the arguments go out in one launch
+    if (nl == num_layers)
+      a.done = done;
     const int workgroups =
         shape_for_now(p, (int64_t)p.num_blocks * a.lk * p.chunk_size, stream, &a);
     FKV_TRY(launch_copy_kernel(a, workgroups, p.threads, stream));
   }
   if (!p.no_alloc) // the bookkeeping creates events on first use
     link_direction_mark(p.device, p.h2d, stream,
-                        (int64_t)p.num_blocks * num_layers * p.kv_dim * p.chunk_size);
+                        (int64_t)p.num_blocks * num_layers * p.kv_dim * p.chunk_size,
+                        report->announced ? done : CopyDone{});
   return FKV_OK;
 }
 
@@ -870,7 +1035,8 @@ int kernel_plan_launch_layers(const KernelPlan &p, int layers_per_batch, LayersL
 }
 
 int kernel_plans_launch(const KernelPlan *const *plans, const int *layer_offsets,
-                        const int *num_layers, int count, hipStream_t stream, CopyReport *report) {
+                        const int *num_layers, int count, hipStream_t stream, CopyReport *report,
+                        const CopyDone &done) {
   // One launch for all of them when they can share one: same direction, device,
   // vector width and launch shape, each range within one LDS table.
   const bool fuse = policy_of(plans[0]->device).fuse_launches != 0;
@@ -886,10 +1052,13 @@ int kernel_plans_launch(const KernelPlan *const *plans, const int *layer_offsets
                num_layers[i] * p.kv_dim <= kCopyMaxLK;
   }
   if (!together) {
-    CopyReport all{/*in_arguments=*/true, /*claims=*/false};
+    CopyReport all;
+    all.in_arguments = true;
     for (int i = 0; i < count; ++i) {
       CopyReport one;
-      FKV_TRY(kernel_plan_launch(*plans[i], layer_offsets[i], num_layers[i], stream, &one));
+      FKV_TRY(kernel_plan_launch(*plans[i], layer_offsets[i], num_layers[i], stream, &one,
+                                 count == 1 ? done : CopyDone{}));
+      all.announced = one.announced;
       all.in_arguments = all.in_arguments && one.in_arguments;
       all.claims = all.claims || one.claims;
     }
@@ -903,10 +1072,13 @@ int kernel_plans_launch(const KernelPlan *const *plans, const int *layer_offsets
     jobs[i] = plan_job(*plans[i], layer_offsets[i], num_layers[i]);
     bytes += (int64_t)plans[i]->num_blocks * jobs[i].lk * plans[i]->chunk_size;
   }
-  jobs[0].report = report;
+  CopyReport mine;
+  jobs[0].report = report ? report : &mine;
+  jobs[0].done = done;
   const int workgroups = shape_for_now(*plans[0], bytes, stream, &jobs[0]);
   FKV_TRY(launch_copy_jobs(jobs, count, workgroups, plans[0]->threads, stream));
-  link_direction_mark(plans[0]->device, plans[0]->h2d, stream, bytes);
+  link_direction_mark(plans[0]->device, plans[0]->h2d, stream, bytes,
+                      jobs[0].report->announced ? done : CopyDone{});
   return FKV_OK;
 }
 
@@ -916,15 +1088,18 @@ void kernel_plan_release(KernelPlan *p, hipStream_t stream) {
   p->slot = nullptr;
 }
 
-int run_kernel_path(const fkv_transfer_desc &d, hipStream_t stream) {
+int run_kernel_path(const fkv_transfer_desc &d, hipStream_t stream, const CopyDone &done,
+                    bool *announced) {
   set_last_path(FKV_PATH_KERNEL);
   KernelPlan plan;
   FKV_TRY(kernel_plan_build(d, stream, &plan));
   KernelPlanHold hold{&plan, stream};
   FKV_TRY(kernel_plan_publish(&plan, stream, /*one_launch=*/true));
   CopyReport report;
-  FKV_TRY(kernel_plan_launch(plan, 0, d.num_layers, stream, &report));
+  FKV_TRY(kernel_plan_launch(plan, 0, d.num_layers, stream, &report, done));
   plan.unread = report.in_arguments && !report.claims;
+  if (announced)
+    *announced = report.announced;
   return FKV_OK;
 }
 
@@ -1191,7 +1366,8 @@ int order_after(hipStream_t from, hipStream_t to, int device, int which) {
 
 // Several descriptors of one direction on the kernel path: a plan each, one launch
 // for all of them where they can share one.
-int run_kernel_path_multi(const fkv_transfer_desc *descs, int count, hipStream_t stream) {
+int run_kernel_path_multi(const fkv_transfer_desc *descs, int count, hipStream_t stream,
+                          const fkv::CopyDone &done, bool *announced) {
   fkv::set_last_path(FKV_PATH_KERNEL);
   std::vector<fkv::KernelPlan> plans(count);
   struct GiveBack { // also when a launch throws
@@ -1220,7 +1396,9 @@ int run_kernel_path_multi(const fkv_transfer_desc *descs, int count, hipStream_t
       layers[j] = descs[k + j].num_layers;
     }
     fkv::CopyReport report;
-    rc = fkv::kernel_plans_launch(group, first, layers, n, stream, &report);
+    rc = fkv::kernel_plans_launch(group, first, layers, n, stream, &report,
+                                  n == count ? done : fkv::CopyDone{});
+    *announced = n == count && report.announced;
     for (int j = 0; j < n && rc == FKV_OK; ++j)
       plans[k + j].unread = report.in_arguments && !report.claims;
   }
@@ -1272,9 +1450,13 @@ int transfer_descs(const fkv_transfer_desc *descs, int count, hipStream_t stream
     }
     all_kernel = all_kernel && engines[i] == 0;
   }
+  // A waiting call on the kernel path that is one launch learns of its end from the launch itself.
+  DoneWord word;
+  bool announced = false;
   auto run_all = [&](hipStream_t on) -> int {
     if (all_kernel)
-      return count == 1 ? run_kernel_path(d, on) : run_kernel_path_multi(descs, count, on);
+      return count == 1 ? run_kernel_path(d, on, word.get(), &announced)
+                        : run_kernel_path_multi(descs, count, on, word.get(), &announced);
     for (int i = 0; i < count; ++i)
       FKV_TRY(engines[i] ? run_ce_path(descs[i], on) : run_kernel_path(descs[i], on));
     return FKV_OK;
@@ -1285,6 +1467,8 @@ int transfer_descs(const fkv_transfer_desc *descs, int count, hipStream_t stream
                    ? lane_of(device, d.is_host_to_device != 0)
                    : nullptr;
   hipEvent_t done = nullptr;
+  if (sync && all_kernel)
+    word.acquire(device, stream);
   if (lane) {
     std::lock_guard<std::mutex> lk(lane->mu);
     // the lane starts after what the caller's stream holds; an idle stream holds nothing
@@ -1293,14 +1477,16 @@ int transfer_descs(const fkv_transfer_desc *descs, int count, hipStream_t stream
       FKV_TRY(order_after(stream, lane->stream, device, 0));
     }
     FKV_TRY(run_all(lane->stream));
-    if (sync)
+    if (announced)
+      ;
+    else if (sync)
       FKV_TRY(record_completion(lane->stream, !d.is_host_to_device, &done));
     else
       FKV_TRY(order_after(lane->stream, stream, device, 1));
     stream = lane->stream;
   } else {
     FKV_TRY(run_all(stream));
-    if (sync)
+    if (sync && !announced)
       FKV_TRY(record_completion(stream, /*host_reads_result=*/!d.is_host_to_device, &done));
   }
   (d.is_host_to_device ? stats().bytes_h2d : stats().bytes_d2h)
@@ -1312,7 +1498,9 @@ int transfer_descs(const fkv_transfer_desc *descs, int count, hipStream_t stream
     // a measurement of the device where one has been made; 3 % taken off)
     const int64_t expected_ns =
         (int64_t)((double)bytes * 1000.0 / std::max(1, policy_peek(device).model_link_mbps) * 0.97);
-    if (done)
+    if (announced)
+      FKV_HIP_TRY(quiet_copy_wait(word.get().word, word.get().epoch, stream, device, expected_ns));
+    else if (done)
       FKV_HIP_TRY(quiet_event_wait(done, device, expected_ns));
     else
       FKV_HIP_TRY(quiet_stream_wait(stream, device));
@@ -1324,6 +1512,8 @@ int transfer_descs(const fkv_transfer_desc *descs, int count, hipStream_t stream
       fprintf(stderr, "[XFER] type=%s blocks=%lld sync_ms=%.3f\n",
               d.is_host_to_device ? "H2D" : "D2H", (long long)blocks, ms);
     }
+    if (announced)
+      word.finished();
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess)

@@ -43,6 +43,10 @@ hipError_t quiet_stream_wait(hipStream_t stream, int device);
 // only a launch that has been over for kLateWord without it has ended in an error.
 constexpr std::chrono::milliseconds kLateWord{100};
 hipError_t quiet_word_wait(const uint64_t *word, uint64_t at_least, hipEvent_t behind, int device);
+// The same for the word of a launch on `stream` that has no event behind it, with `expected_ns` as
+// for events.
+hipError_t quiet_copy_wait(const uint64_t *word, uint64_t at_least, hipStream_t stream, int device,
+                           int64_t expected_ns);
 // The runtime gave no answer because some thread is capturing a stream: says nothing about the
 // work that was asked about.
 inline bool capture_forbids(hipError_t e) {
@@ -164,6 +168,21 @@ inline uint8_t *cpu_chunk_ptr(const fkv_transfer_desc &d, int64_t layer, int64_t
 #endif
 
 // ---- the gather/scatter kernel -----------------------------------------
+// How a launch tells the thread that waits for it that everything has been copied.
+struct DoneCounts { // device memory, zero between launches
+  uint64_t of_xcd[16];  // launches to the host: workgroups at work on an XCD (high half), shares they have copied
+  uint32_t reported[16]; // of those, shares in `all`
+  uint32_t all;         // shares that have been copied
+};
+struct CopyDone {
+  DoneCounts *count = nullptr;
+  uint64_t *word = nullptr;  // pinned: raised to `epoch` behind the last of them; nullptr: nobody waits
+  uint64_t epoch = 0;        // larger than that of any earlier launch with this word
+  bool *used = nullptr;      // host side: set when a launch is about to be made with them
+};
+// Whether launches on `stream` do now: not while it is being captured.  Set where the kernels are
+// part of the library (the emulated runtime's stand-ins do not announce anything).
+extern bool (*copies_announce)(hipStream_t stream);
 // One launch copies `num_blocks * lk` chunks of `chunk_bytes`:
 //   for pos, i:  src = base_src[i] + ids_src[pos]*stride_src
 //                dst = base_dst[i] + ids_dst[pos]*stride_dst
@@ -201,6 +220,7 @@ struct CopyKernelArgs {
   uint32_t epoch; // set by launch_copy_kernel: a number no other launch in flight has
   int32_t claims_per_wg; // ranges per working workgroup: confined launches (0 = 1), and
                          // launches on all XCDs that have counters (0 = fixed shares)
+  CopyDone done;         // of the launch
   int32_t host_tables;   // host side: the host reads the four arrays at these addresses too, and
                          // the launch may carry them in its arguments (fits_arguments)
   struct CopyReport *report; // host side: what became of the launch; may be null
@@ -210,6 +230,7 @@ struct CopyReport {
   bool in_arguments = false; // the tables travelled in the arguments: nothing on the device reads
                              // them where they were, whenever it runs
   bool claims = false;       // workgroups of the launch look at its claim counter, until it ends
+  bool announced = false;    // the launch raises the word of its CopyDone
 };
 // Tables in the arguments of a launch: 4 KiB in all, of which up to kCopyMaxJobs jobs take 0.8.
 constexpr int kArgPlanWords = 400;
@@ -365,7 +386,9 @@ struct PlanSlotHold {
 };
 // Link-bound launches of the last while, per device and direction (see fkv_core.cpp).
 bool link_direction_busy(int device, bool h2d, hipStream_t launching_stream);
-void link_direction_mark(int device, bool h2d, hipStream_t stream, int64_t bytes);
+// `done`: the launch is over when its word says so; else when an event behind it does.
+void link_direction_mark(int device, bool h2d, hipStream_t stream, int64_t bytes,
+                         const CopyDone &done = CopyDone{});
 // The same across processes (fkv_linkboard.cpp): post that this process keeps the
 // link busy in one direction for about `expected_ns` more, and ask whether another
 // process has posted activity that ends less than `window_ns` ago or later.
@@ -387,9 +410,11 @@ int kernel_plan_build(const fkv_transfer_desc &d, hipStream_t stream, KernelPlan
 // or carried in the arguments.  `one_launch`: the plan is read by one launch and not again.
 int kernel_plan_publish(KernelPlan *p, hipStream_t stream, bool one_launch);
 // Enqueues the copy of layers [layer_offset, layer_offset + num_layers) of the plan.
-// `report` (may be null): see CopyReport, for all launches of the call together.
+// `report` (may be null): see CopyReport, for all launches of the call together.  `done`: for a
+// caller that waits, if the call is one launch (report->announced).
 int kernel_plan_launch(const KernelPlan &p, int layer_offset, int num_layers,
-                       hipStream_t stream, CopyReport *report = nullptr);
+                       hipStream_t stream, CopyReport *report = nullptr,
+                       const CopyDone &done = CopyDone{});
 // All layers of the plan in one launch, `layers_per_batch` at a time; `t` brings the words
 // that announce the batches.  Only for plans layers_launch_fits accepts.
 bool layers_launch_fits(const KernelPlan &p, int layers_per_batch);
@@ -400,10 +425,12 @@ int kernel_plan_launch_layers(const KernelPlan &p, int layers_per_batch, LayersL
 // per plan where the plans cannot share one.
 int kernel_plans_launch(const KernelPlan *const *plans, const int *layer_offsets,
                         const int *num_layers, int count, hipStream_t stream,
-                        CopyReport *report = nullptr);
+                        CopyReport *report = nullptr, const CopyDone &done = CopyDone{});
 // The plan memory is recycled once everything enqueued on `stream` so far has run.
 void kernel_plan_release(KernelPlan *p, hipStream_t stream);
-int run_kernel_path(const fkv_transfer_desc &d, hipStream_t stream);
+// `announced` (may be null): the transfer raises the word of `done`.
+int run_kernel_path(const fkv_transfer_desc &d, hipStream_t stream, const CopyDone &done = CopyDone{},
+                    bool *announced = nullptr);
 int run_ce_path(const fkv_transfer_desc &d, hipStream_t stream);
 // Cost-model choice between the two paths for this transfer (no device call).
 int choose_engine(const fkv_transfer_desc &d, int *use_ce, double *kernel_s, double *ce_s);
