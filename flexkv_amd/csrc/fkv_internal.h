@@ -163,8 +163,12 @@ inline uint8_t *cpu_chunk_ptr(const fkv_transfer_desc &d, int64_t layer, int64_t
 // store of a slice then waits for all its loads instead of for its own.
 #if defined(__HIP__)
 #define FKV_GLOBAL __attribute__((address_space(1)))
+// Memory that nothing writes while the kernel runs: what a whole wavefront reads from one address
+// comes through the scalar cache, and is waited for apart from loads and stores of lanes.
+#define FKV_CONSTANT __attribute__((address_space(4)))
 #else // the CPU model of the device
 #define FKV_GLOBAL
+#define FKV_CONSTANT
 #endif
 
 // ---- the gather/scatter kernel -----------------------------------------

@@ -26,6 +26,8 @@
 namespace fkv {
 namespace {
 
+constexpr int64_t kShortMinBytes = 16 << 20; // calls over fewer bytes of slots are over soon
+
 struct StagingKernelArgs {
   uint8_t *staging;
   int64_t staging_stride;
@@ -37,96 +39,157 @@ struct StagingKernelArgs {
   const int64_t *cpu_ids;     // device-visible, [num_blocks]; nullptr: in the launch's arguments
   uint32_t *size_table;       // device-visible alias of the host size table
   int64_t table_block_stride, table_layer_stride; // in entries
-  int32_t start_layer, kv_dim, num_blocks, batch_start, bsz;
+  int32_t start_layer, num_blocks, batch_start, bsz;
+  uint32_t per_layer;         // chunks of a layer (no fewer than a call has, if they are more)
 };
 
 typedef unsigned int vec16 __attribute__((ext_vector_type(4)));
 
-// Copies `bytes` from src to dst with one wavefront; VEC16: both are 16-byte aligned.  RUNS: a
-// lane moves adjacent vectors, 128 bytes, so that its stores complete a line of host memory
-// (see copy_slice in fkv_kernels.hip); its loads walk through one line, without the streaming
-// hint that might let the line go in between.
+// The end of a payload, less than a slice: N accesses of a lane, 64 vectors apart, of which the last
+// reaches up to vector `nvec` (not included), and `tail` bytes behind that vector.  Lanes beyond the end
+// move the last vector (byte) once more, the same bytes to the same place, instead of sitting
+// out: every load is used, so nothing has to be waited for where this joins the path of whole slices
+// (see nothing_in_flight in fkv_kernels.hip).
+#if defined(__HIP__)
+constexpr bool kAllLanesStore = true;
+#else // work-items of the CPU model are threads, to whose sanitizer that is a race
+constexpr bool kAllLanesStore = false;
+#endif
+template <int N, bool NTS>
+__device__ __forceinline__ void copy_end(const FKV_GLOBAL vec16 *s, FKV_GLOBAL vec16 *d, int nvec, int tail,
+                                         int lane) {
+  // without a tail the last byte of the last vector
+  const int byte = nvec * 16 + (tail ? min(lane, tail - 1) : -1);
+  const uint8_t last = *((const FKV_GLOBAL uint8_t *)s + byte);
+  vec16 r[N + 1];
+  const int end = min(lane + (N - 1) * 64, nvec - 1);
+#pragma unroll
+  for (int u = 0; u < N; ++u)
+    r[u] = __builtin_nontemporal_load(s + (u + 1 < N ? lane + u * 64 : end));
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    if (!kAllLanesStore && lane + u * 64 >= nvec)
+      continue;
+    if (NTS)
+      __builtin_nontemporal_store(r[u], d + (u + 1 < N ? lane + u * 64 : end));
+    else
+      d[u + 1 < N ? lane + u * 64 : end] = r[u];
+  }
+  if (kAllLanesStore || lane < tail)
+    *((FKV_GLOBAL uint8_t *)d + byte) = last;
+  asm volatile("" ::"i"(N)); // keeps the last stores of the cases apart, which would be merged and wait
+}
+
+// Copies `bytes` from src to dst with one wavefront; VEC16: both are 16-byte aligned.  RUNS: in whole
+// slices a lane moves adjacent vectors, 128 bytes, so that its stores complete a line of host
+// memory (see copy_slice in fkv_kernels.hip); its loads walk through one line, without the
+// streaming hint that might let the line go in between.
 template <bool VEC16, bool NTS, bool RUNS>
 __device__ __forceinline__ void wave_copy(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst,
                                           int64_t bytes, int lane) {
-  int64_t done = 0;
-  if (VEC16) {
-    const FKV_GLOBAL vec16 *s = (const FKV_GLOBAL vec16 *)src;
-    FKV_GLOBAL vec16 *d = (FKV_GLOBAL vec16 *)dst;
-    const int64_t nvec = bytes / 16;
-    constexpr int U = kCopyUnroll;
-    constexpr int kLane = RUNS ? U : 1, kAccess = RUNS ? 1 : 64;
-    for (int64_t v0 = 0; v0 < nvec; v0 += 64 * U) {
-      // all loads of a slice before the first store; lanes beyond the end re-read the
-      // last vector rather than branch around the load
-      vec16 r[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t v = v0 + u * kAccess + lane * kLane;
-        const FKV_GLOBAL vec16 *from = s + (v < nvec ? v : nvec - 1);
-        r[u] = RUNS ? *from : __builtin_nontemporal_load(from);
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t v = v0 + u * kAccess + lane * kLane;
-        if (v < nvec) {
-          if (NTS)
-            __builtin_nontemporal_store(r[u], d + v);
-          else
-            d[v] = r[u];
-        }
-      }
-    }
-    done = nvec * 16;
+  if (!VEC16) {
+    for (int64_t j = lane; j < bytes; j += 64)
+      dst[j] = src[j];
+    return;
   }
-  for (int64_t j = done + lane; j < bytes; j += 64)
-    dst[j] = src[j];
+  constexpr int U = kCopyUnroll;
+  constexpr int kLane = RUNS ? U : 1, kAccess = RUNS ? 1 : 64;
+  const int64_t whole = bytes / (64 * U * 16);
+  const int rest = (int)(bytes - whole * 64 * U * 16), nvec = rest / 16, tail = rest & 15;
+  const FKV_GLOBAL vec16 *s = (const FKV_GLOBAL vec16 *)src;
+  FKV_GLOBAL vec16 *d = (FKV_GLOBAL vec16 *)dst;
+  for (int64_t k = 0; k < whole; ++k, s += 64 * U, d += 64 * U) {
+    vec16 r[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const FKV_GLOBAL vec16 *from = s + lane * kLane + u * kAccess;
+      r[u] = RUNS ? *from : __builtin_nontemporal_load(from);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      FKV_GLOBAL vec16 *to = d + lane * kLane + u * kAccess;
+      if (NTS)
+        __builtin_nontemporal_store(r[u], to);
+      else
+        *to = r[u];
+    }
+  }
+  if (rest == 0)
+    return;
+  switch ((nvec + 63) / 64) {
+  case 1: return copy_end<1, NTS>(s, d, nvec, tail, lane);
+  case 2: return copy_end<2, NTS>(s, d, nvec, tail, lane);
+  case 3: return copy_end<3, NTS>(s, d, nvec, tail, lane);
+  case 4: return copy_end<4, NTS>(s, d, nvec, tail, lane);
+  case 5: return copy_end<5, NTS>(s, d, nvec, tail, lane);
+  case 6: return copy_end<6, NTS>(s, d, nvec, tail, lane);
+  case 7: return copy_end<7, NTS>(s, d, nvec, tail, lane);
+  case 8: return copy_end<8, NTS>(s, d, nvec, tail, lane);
+  default: return copy_end<0, NTS>(s, d, nvec, tail, lane); // a few bytes
+  }
 }
 
+// Which is the same for all lanes of a wavefront, where the compiler cannot see it.
+__device__ __forceinline__ uint32_t same_for_wave(uint32_t v) {
+#if defined(__HIP__)
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+#else
+  return v;
+#endif
+}
+
+// What a payload costs its wavefront besides its bytes is what it waits for: its place and size,
+// the bytes behind its last vector, the acknowledgement of its stores.  Ids and sizes come
+// through the scalar cache, a payload ahead, which leaves the counter of loads and stores alone; the
+// bytes are asked for with the last vectors; stores of whole slices are not waited for.  With all
+// that in line (48 MiB of slots 50-90 % full, us, before -> this, wavefronts alike): written from
+// slots of 32 KiB 675 -> 656, 8 KiB 700 -> 692, 2 KiB 983 -> 849; read 650 -> 637, 683 -> 644, 1977 -> 1268.
 template <bool WRITE_CPU, bool VEC16, bool RUNS = false>
 __global__ __launch_bounds__(kCopyBlockThreads) void fkv_staging_transfer_kernel(StagingKernelArgs a,
                                                                                  ArgPlan plan) {
-  const int64_t *const cpu_ids =
-      a.cpu_ids ? a.cpu_ids : reinterpret_cast<const int64_t *>(plan.w);
+  const FKV_CONSTANT int64_t *const cpu_ids = (const FKV_CONSTANT int64_t *)(
+      a.cpu_ids ? a.cpu_ids : reinterpret_cast<const int64_t *>(plan.w));
   const int lane = threadIdx.x & 63;
-  const int64_t wave = (int64_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64;
-  const int64_t nwaves = (int64_t)gridDim.x * (blockDim.x / 64);
-  const int64_t per_layer = (int64_t)a.kv_dim * a.num_blocks;
-  // Where chunk i lives on the host side.
-  auto locate = [&](int64_t i, uint8_t **slot, uint32_t **entry) {
-    const int64_t g = (int64_t)a.batch_start + i;
-    const int64_t layer = g / per_layer;
-    const int64_t kv = (g % per_layer) / a.num_blocks;
-    const int64_t b = g % a.num_blocks;
-    const int64_t id = cpu_ids[b];
-    *slot = a.cpu + (layer + a.start_layer) * a.cpu_layer_stride + kv * a.cpu_kv_stride +
-            id * a.cpu_block_stride;
-    *entry = a.size_table + id * a.table_block_stride +
-             (a.start_layer + layer) * a.table_layer_stride + kv;
+  const uint32_t wave = blockIdx.x * (blockDim.x / 64) + same_for_wave(threadIdx.x / 64);
+  const uint32_t nwaves = gridDim.x * (blockDim.x / 64), bsz = (uint32_t)a.bsz;
+  // Where chunk i lives on the host side: (layer, kv) and the id of its block.
+  struct Place {
+    uint32_t layer, kv;
+    int64_t id;
   };
-  // The size of a chunk that is read comes out of host memory, a round trip over the
-  // link: the entry of the wavefront's next chunk is asked for before the current
-  // chunk is copied, so that it has arrived when it is needed.
-  uint8_t *slot = nullptr;
-  uint32_t *entry = nullptr;
-  int64_t sz_next = 0;
-  if (wave < a.bsz) {
-    locate(wave, &slot, &entry);
-    if (!WRITE_CPU)
-      sz_next = (int64_t)__builtin_nontemporal_load(entry);
-  }
-  for (int64_t i = wave; i < a.bsz; i += nwaves) {
-    uint8_t *cur_slot = slot;
-    uint32_t *cur_entry = entry;
-    int64_t sz = sz_next;
-    if (i + nwaves < a.bsz) {
-      locate(i + nwaves, &slot, &entry);
-      if (!WRITE_CPU)
-        sz_next = (int64_t)__builtin_nontemporal_load(entry);
-    }
+  auto place = [&](uint32_t i) {
+    const uint32_t g = (uint32_t)a.batch_start + i;
+    const uint32_t layer = g / a.per_layer, in_layer = g - layer * a.per_layer;
+    const uint32_t kv = in_layer / (uint32_t)a.num_blocks;
+    return Place{layer, kv, cpu_ids[in_layer - kv * (uint32_t)a.num_blocks]};
+  };
+  auto slot_of = [&](const Place &p) {
+    return a.cpu + ((int64_t)p.layer + a.start_layer) * a.cpu_layer_stride + p.kv * a.cpu_kv_stride +
+           p.id * a.cpu_block_stride;
+  };
+  auto entry_of = [&](const Place &p) {
+    return a.size_table + p.id * a.table_block_stride +
+           (a.start_layer + (int64_t)p.layer) * a.table_layer_stride + p.kv;
+  };
+  // out of HBM where it is written, out of host memory, a round trip over the link, where it is read
+  auto size_of = [&](uint32_t i, const Place &p) -> int64_t {
+    return WRITE_CPU ? (int64_t)((const FKV_CONSTANT uint64_t *)a.comp_sizes)[i]
+                     : (int64_t)*(const FKV_CONSTANT uint32_t *)entry_of(p);
+  };
+  if (wave >= bsz)
+    return;
+  Place here = place(wave), next = place(min(wave + nwaves, bsz - 1));
+  int64_t sz_next = size_of(wave, here);
+  for (uint32_t i = wave; i < bsz; i += nwaves) {
+    uint8_t *const cur_slot = slot_of(here);
+    uint32_t *const cur_entry = entry_of(here);
+    const int64_t sz = sz_next;
+    if (i + nwaves < bsz)
+      sz_next = size_of(i + nwaves, next);
+    here = next;
+    next = place(min(i + 2 * nwaves, bsz - 1)); // both far from 2^32
     uint8_t *payload = a.staging + i * a.staging_stride;
     if (WRITE_CPU) {
-      sz = (int64_t)a.comp_sizes[i];
       if (sz > a.chunk_capacity) { // does not fit its host slot: counted, size 0 recorded
         if (lane == 0) {
           if (a.overflow)
@@ -243,10 +306,10 @@ int fkv_staging_transfer(const fkv_staging_transfer_desc *dp, void *stream_v) tr
   a.table_block_stride = d.size_table_block_stride;
   a.table_layer_stride = d.size_table_layer_stride;
   a.start_layer = d.start_layer_id;
-  a.kv_dim = d.kv_dim;
   a.num_blocks = d.num_blocks;
   a.batch_start = d.batch_start;
   a.bsz = d.bsz;
+  a.per_layer = (uint32_t)std::min<int64_t>((int64_t)d.kv_dim * d.num_blocks, UINT32_MAX);
   const uint64_t align = (uint64_t)(uintptr_t)a.staging | (uint64_t)a.staging_stride |
                          (uint64_t)(uintptr_t)a.cpu | (uint64_t)a.cpu_kv_stride |
                          (uint64_t)a.cpu_layer_stride | (uint64_t)a.cpu_block_stride;
@@ -254,11 +317,17 @@ int fkv_staging_transfer(const fkv_staging_transfer_desc *dp, void *stream_v) tr
   const bool write_cpu = d.is_write_cpu != 0;
   const fkv_launch_policy pol = policy_of(device);
   const int cta = d.transfer_num_cta > 0 ? d.transfer_num_cta : default_num_cta(!write_cpu);
-  // Reading from the host, a wavefront has one payload in flight and drains between
-  // payloads, whose last slice is short: twice the workgroups of the fixed-size
-  // kernel make up for it (16-29 KiB payloads: 45 GB/s with 16 wavefronts, 55.0 with
-  // 24, 55.7 with 32).
-  int grid = cta * (write_cpu ? pol.d2h_wg_per_cta * 3 / 2 : 2 * pol.h2d_wg_per_cta);
+  // The wavefronts of a plain copy to the host, half as many again for a call that is over soon;
+  // from the host also, because a wavefront has one payload in flight, whose last slice is short.
+  // 48 MiB of slots of 32 KiB, us, and what a 2048^3 GEMM next to it takes longer: written with 30 / 40
+  // / 50 wavefronts 667 (3.9x) / 657 (7.1x) / 655 (7.0x), read with 16 / 24 / 32 653 / 643 / 637 (3.6x).
+  // Slots shorter than a slice hold less, and as many more wavefronts have the same bytes
+  // under way: 48 MiB of slots of 2 KiB written 931 -> 715, read 1268 -> 677.
+  const int64_t slots = (int64_t)d.bsz * d.staging_stride;
+  const int64_t shorter = std::max<int64_t>(1, std::min<int64_t>(4, 64 * kCopyUnroll * 16 / d.staging_stride));
+  int grid = cta * (write_cpu ? pol.d2h_wg_per_cta : pol.h2d_wg_per_cta) * (int)shorter;
+  if (!write_cpu || slots < kShortMinBytes)
+    grid = grid * 3 / 2;
   const int threads = write_cpu ? pol.d2h_wg_threads : pol.h2d_wg_threads;
   grid = std::max(1, std::min(grid, (d.bsz + threads / 64 - 1) / (threads / 64)));
 #define FKV_LAUNCH_STAGING(...)                                                               \
@@ -267,13 +336,10 @@ int fkv_staging_transfer(const fkv_staging_transfer_desc *dp, void *stream_v) tr
   // Adjacent vectors per lane on the same terms as the fixed-size kernel: not next to a
   // transfer from the host, where the plain order moves 2 % more in sum.  And only for calls
   // that fill the link for a while: the loads of a slice take longer in this order, which a
-  // shorter call waits for.  The line lies at the same bytes for all sizes (us, plain / adjacent,
-  // by MiB of slots 50-90 % full): slots of 2 KiB 8: 219 / 241, 16: 415 / 403, 24: 603 / 553;
-  // 4 KiB 8: 173 / 188, 16: 320 / 308, 24: 455 / 425; 8 KiB 8: 153 / 163, 12: 216 / 222,
-  // 16: 283 / 274; 32 KiB 8: 143 / 150, 12: 201 / 201, 16: 260 / 254, 48: 687 / 679.
-  constexpr int64_t kRunsMinBytes = 16 << 20; // of slots
+  // shorter call waits for.  Slots of 32 KiB, us, plain / adjacent: 8 MiB 128 / 133, 16 MiB 237 / 238,
+  // 48 MiB 667 / 656; of 8 and 2 KiB the same either way.
   const bool runs = pol.d2h_lane_runs == 2 ||
-                    (pol.d2h_lane_runs == 1 && d.bsz * d.staging_stride >= kRunsMinBytes &&
+                    (pol.d2h_lane_runs == 1 && slots >= kShortMinBytes &&
                      !(pol.arbiter != 0 && link_direction_busy(device, /*h2d=*/true, stream)));
   if (write_cpu && vec16 && runs)
     FKV_LAUNCH_STAGING(true, true, true);
