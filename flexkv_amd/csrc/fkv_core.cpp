@@ -915,9 +915,7 @@ CopyKernelArgs plan_job(const KernelPlan &p, int l0, int nl) {
 // next to it grows with their number (a 2048^3 GEMM takes 47 us next to 16 host->GPU
 // workgroups, confined or not, and 67 us next to 24), and 16 on four XCDs already
 // reach the link rate.
-// Ranges per workgroup: next to a transfer in the other direction one each is best
-// (finer ranges shift the balance towards GPU->host and lower the sum: two threads
-// with 25 MB requests 88.9 against 87.5 GB/s).  On an idle link the neighbours are
+// Ranges per workgroup: see defaults_for in fkv_policy.cpp.  On an idle link the neighbours are
 // the engine's compute kernels, which slow down single workgroups of a copy, and
 // with one range each the slowest one holds up the launch: a restore next to
 // fused-attention calls moves 37 GB/s with one range per workgroup and 54 GB/s with
@@ -960,8 +958,9 @@ int shape_for_now(const KernelPlan &p, int64_t bytes, hipStream_t stream, CopyKe
   // A short copy to the host spends its time getting under way, which more wavefronts do sooner,
   // and its neighbours are free again in no time: 48 instead of 32 take 61.8 instead of 63.2 us
   // for 2 MiB, 216.0 instead of 218.6 for 10 MiB, and no less for 64 MiB.
+  // (Next to a transfer the other way the same: see defaults_for in fkv_policy.cpp.)
   constexpr int64_t kShortCopyBytes = 16 << 20;
-  if (!p.h2d && !next_to_other && bytes < kShortCopyBytes)
+  if (!p.h2d && bytes < kShortCopyBytes)
     workgroups = workgroups * 3 / 2;
   if (beside)
     *beside = next_to_other;

@@ -183,14 +183,17 @@ fkv_launch_policy defaults_for(uint32_t present) {
   p.arbiter = p.xcd_count >= 4 ? 1 : 0;
   p.busy_window_ms = 20;
   p.home_min_kb = 8192;
-  p.d2h_busy_pct = 150;
-  // A wavefront more or less shifts the balance: reads keep writes from the link, not the other
-  // way round.  Six puts and six gets of 64 MiB on the mean, on two threads (three sets of sizes;
+  // A host->GPU wavefront more or less shifts the balance: reads keep writes from the link, not the
+  // other way round.  Six puts and six gets of 64 MiB on the mean, on two threads (three sets of sizes;
   // GPU->host / host->GPU done after, ms), with 16 host->GPU wavefronts 7.4 / 10.3, 21 8.0 / 8.9,
-  // 23 8.5 / 8.5, 24 8.8 / 8.4, 36 11.7 / 8.1.  Of GPU->host wavefronts, 24 take 2 % longer in sum
-  // than 48.
-  p.h2d_busy_pct = 144; // 23
-  p.busy_claims_per_wg = 1;
+  // 23 8.5 / 8.5, 24 8.8 / 8.4, 36 11.7 / 8.1.  15 mixes of 4 to 12 requests of 4 to 45 MiB take 4.5 %
+  // less time with 22 than before these figures, 3.7 % with 23, and none takes more.  Two ranges a
+  // wavefront: with one 9.57 ms for eight other sets of the large requests, with two 9.41, with four 9.56.
+  // GPU->host wavefronts of large requests, 32 / 48 / 80: as much within 1 %, but a 2048^3 GEMM next to
+  // both takes 160 / 192 / 252 us, a fused attention 378 / 454 / 680.
+  p.d2h_busy_pct = 100;
+  p.h2d_busy_pct = 138; // 22
+  p.busy_claims_per_wg = 2;
   p.home_claims_per_wg = 2;
   p.all_claims_per_wg = 0;
   p.safety_net_wait_us = 50;
