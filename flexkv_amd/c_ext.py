@@ -36,7 +36,7 @@ __all__ = ["transfer_kv_blocks", "transfer_kv_blocks_multi", "transfer_kv_blocks
 def _ids(t: torch.Tensor, name: str) -> torch.Tensor:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
-    if t.device.type != "cpu":
+    if not t.is_cpu:  # (t.device.type makes two objects)
         raise ValueError(f"{name} must live in host memory")
     if t.dtype != torch.int64:
         raise TypeError(f"{name} must be int64, got {t.dtype}")
@@ -71,16 +71,8 @@ def _engine_code(use_ce_transfer) -> int:
 
 def _ce_config(segment_threshold, path_opt, force_path, enable_memcpy2d, is_blockfirst,
                num_kv_heads, gather_threads, gather_nt) -> CEConfig:
-    cfg = CEConfig()
-    cfg.segment_threshold = int(segment_threshold)
-    cfg.path_opt_enabled = int(bool(path_opt))
-    cfg.force_path = int(force_path)
-    cfg.enable_memcpy2d = int(bool(enable_memcpy2d))
-    cfg.is_blockfirst = int(bool(is_blockfirst))
-    cfg.num_kv_heads = int(num_kv_heads)
-    cfg.gather_threads = int(gather_threads)
-    cfg.gather_nt = int(bool(gather_nt))
-    return cfg
+    return CEConfig(int(segment_threshold), bool(path_opt), int(force_path), bool(enable_memcpy2d),
+                    bool(is_blockfirst), int(num_kv_heads), int(gather_threads), bool(gather_nt))
 
 
 def _transfer_desc(
@@ -104,42 +96,28 @@ def _transfer_desc(
     if gpu_ids.numel() != cpu_ids.numel():
         raise ValueError("gpu_block_id_tensor and cpu_block_id_tensor differ in length")
     ptrs = _ids(gpu_tensor_ptrs_tensor, "gpu_tensor_ptrs_tensor")
-    if cpu_tensor.device.type != "cpu":
+    if not cpu_tensor.is_cpu:
         raise ValueError("cpu_tensor must live in host memory")
 
-    d = TransferDesc()
-    d.backend = int(gpu_block_type)
+    backend, num_layers, pointers = int(gpu_block_type), int(num_layers), ptrs.numel()
     # The reference builds its GTensorHandler with the num_layers of the call
     # (csrc/bindings.cpp:108-111), which indexes SGLang's K-then-V pointer table
     # correctly only for whole-model calls; take the true layer count from the
     # table itself so partial-layer calls address V tensors correctly too.
-    d.num_layers_total = ptrs.numel() // 2 if int(gpu_block_type) == 2 else int(num_layers)
-    d.gpu_tensor_ptrs = ptrs.data_ptr()
-    d.num_gpu_tensor_ptrs = ptrs.numel()
-    d.device = -1
-    d.gpu_kv_stride = int(gpu_kv_stride_in_bytes)
-    d.gpu_block_stride = int(gpu_block_stride_in_bytes)
-    d.gpu_layer_stride = int(gpu_layer_stride_in_bytes)
-    d.gpu_startoff_inside_chunks = 0
-    d.cpu_ptr = cpu_tensor.data_ptr()
-    d.cpu_kv_stride = int(cpu_kv_stride_in_bytes)
-    d.cpu_layer_stride = int(cpu_layer_stride_in_bytes)
-    d.cpu_block_stride = int(cpu_block_stride_in_bytes)
-    d.cpu_startoff_inside_chunks = 0
-    d.chunk_size = int(chunk_size_in_bytes)
-    d.start_layer_id = int(start_layer_id)
-    d.num_layers = int(num_layers)
-    d.kv_dim = int(kv_dim)
-    d.num_blocks = gpu_ids.numel()
-    d.gpu_block_ids = gpu_ids.data_ptr()
-    d.cpu_block_ids = cpu_ids.data_ptr()
-    d.is_host_to_device = int(bool(is_host_to_device))
-    d.use_ce_transfer = _engine_code(use_ce_transfer)
-    d.transfer_num_cta = int(transfer_num_cta)
-    d.sync = int(bool(sync))
-    d.enable_trace = int(bool(enable_transfer_trace))
-    d.ce = _ce_config(ce_segment_threshold, ce_path_opt, ce_force_path, ce_enable_memcpy2d,
-                      is_blockfirst, num_kv_heads, ce_gather_threads, ce_gather_nt)
+    num_layers_total = pointers // 2 if backend == 2 else num_layers
+    # All fields at once, in their order: a call per field costs a small transfer 4 us.
+    d = TransferDesc(
+        backend, num_layers_total, ptrs.data_ptr(), pointers, -1,
+        int(gpu_kv_stride_in_bytes), int(gpu_block_stride_in_bytes),
+        int(gpu_layer_stride_in_bytes), 0, cpu_tensor.data_ptr(),
+        int(cpu_kv_stride_in_bytes), int(cpu_layer_stride_in_bytes),
+        int(cpu_block_stride_in_bytes), 0, int(chunk_size_in_bytes),
+        int(start_layer_id), num_layers, int(kv_dim), gpu_ids.numel(),
+        gpu_ids.data_ptr(), cpu_ids.data_ptr(), bool(is_host_to_device),
+        _engine_code(use_ce_transfer), int(transfer_num_cta), bool(sync),
+        bool(enable_transfer_trace), 0,
+        _ce_config(ce_segment_threshold, ce_path_opt, ce_force_path, ce_enable_memcpy2d,
+                   is_blockfirst, num_kv_heads, ce_gather_threads, ce_gather_nt))
     return d, (gpu_ids, cpu_ids, ptrs, cpu_tensor)
 
 
@@ -210,31 +188,19 @@ def layout_transform(
     """
     ids = _ids(gpu_block_id_tensor, "gpu_block_id_tensor")
     ptrs = _ids(gpu_tensor_ptrs_tensor, "gpu_tensor_ptrs_tensor")
-    if buffer.device.type != "cuda":
+    if not buffer.is_cuda:
         raise ValueError("buffer must live in device memory")
-    d = _lib.LayoutTransformDesc()
-    d.backend = int(gpu_block_type)
-    d.num_layers_total = ptrs.numel() // 2 if int(gpu_block_type) == 2 else int(num_layers)
-    d.gpu_tensor_ptrs = ptrs.data_ptr()
-    d.num_gpu_tensor_ptrs = ptrs.numel()
-    d.device = buffer.device.index if buffer.device.index is not None else -1
-    d.gpu_kv_stride = int(gpu_kv_stride_in_bytes)
-    d.gpu_block_stride = int(gpu_block_stride_in_bytes)
-    d.gpu_layer_stride = int(gpu_layer_stride_in_bytes)
-    d.buffer_ptr = buffer.data_ptr()
-    d.buffer_layer_stride = int(buffer_layer_stride_in_bytes)
-    d.buffer_kv_stride = int(buffer_kv_stride_in_bytes)
-    d.buffer_block_stride = int(buffer_block_stride_in_bytes)
-    d.chunk_size = int(chunk_size_in_bytes)
-    d.start_layer_id = int(start_layer_id)
-    d.num_layers = int(num_layers)
-    d.kv_dim = int(kv_dim)
-    d.num_blocks = ids.numel()
-    d.gpu_block_ids = ids.data_ptr()
-    d.buffer_to_target = int(bool(buffer_to_target))
-    d.sync = int(bool(sync))
-    need = ((d.num_blocks - 1) * d.buffer_block_stride + (d.num_layers - 1) * d.buffer_layer_stride
-            + (d.kv_dim - 1) * d.buffer_kv_stride + d.chunk_size) if d.num_blocks and d.num_layers else 0
+    backend, layers, kv, blocks = int(gpu_block_type), int(num_layers), int(kv_dim), ids.numel()
+    layer_stride, kv_stride = int(buffer_layer_stride_in_bytes), int(buffer_kv_stride_in_bytes)
+    block_stride, chunk, pointers = int(buffer_block_stride_in_bytes), int(chunk_size_in_bytes), ptrs.numel()
+    d = _lib.LayoutTransformDesc(  # in the order of the fields
+        backend, pointers // 2 if backend == 2 else layers, ptrs.data_ptr(), pointers,
+        buffer.get_device(), int(gpu_kv_stride_in_bytes), int(gpu_block_stride_in_bytes),
+        int(gpu_layer_stride_in_bytes), buffer.data_ptr(), layer_stride, kv_stride, block_stride,
+        chunk, int(start_layer_id), layers, kv, blocks, ids.data_ptr(), bool(buffer_to_target),
+        bool(sync))
+    need = ((blocks - 1) * block_stride + (layers - 1) * layer_stride + (kv - 1) * kv_stride
+            + chunk) if blocks and layers else 0
     if need > buffer.numel() * buffer.element_size():
         raise ValueError(f"buffer of {buffer.numel() * buffer.element_size()} bytes is shorter than "
                          f"the {need} bytes the strides address")
@@ -259,7 +225,7 @@ def staging_transfer(
     counter of payloads that did not fit (may be None when reading).  ``cpu_tensor``
     and ``cpu_size_table`` are pinned host tensors, the block ids a host tensor."""
     ids = _ids(cpu_block_id_tensor, "cpu_block_id_tensor")
-    if comp_staging.device.type != "cuda" or comp_sizes.device.type != "cuda":
+    if not comp_staging.is_cuda or not comp_sizes.is_cuda:
         raise ValueError("comp_staging and comp_sizes must live in device memory")
     if comp_sizes.dtype not in (torch.int64, torch.uint64) or comp_sizes.numel() < bsz:
         raise ValueError("comp_sizes must hold bsz 64-bit sizes")
@@ -267,28 +233,17 @@ def staging_transfer(
         raise ValueError("cpu_size_table must hold 32-bit entries")
     if comp_staging.numel() * comp_staging.element_size() < int(bsz) * int(staging_stride_in_bytes):
         raise ValueError("comp_staging is shorter than bsz slots of staging_stride bytes")
-    if overflow is not None and (overflow.device.type != "cuda" or overflow.dtype != torch.int32):
+    if overflow is not None and (not overflow.is_cuda or overflow.dtype != torch.int32):
         raise ValueError("overflow must be a device int32 tensor")
-    d = _lib.StagingTransferDesc()
-    d.staging = comp_staging.data_ptr()
-    d.staging_stride = int(staging_stride_in_bytes)
-    d.comp_sizes = comp_sizes.data_ptr()
-    d.cpu_ptr = cpu_tensor.data_ptr()
-    d.chunk_capacity = int(chunk_capacity_in_bytes)
-    d.overflow = overflow.data_ptr() if overflow is not None else None
-    d.cpu_kv_stride = int(cpu_kv_stride_in_bytes)
-    d.cpu_layer_stride = int(cpu_layer_stride_in_bytes)
-    d.cpu_block_stride = int(cpu_block_stride_in_bytes)
-    d.cpu_block_ids = ids.data_ptr()
-    d.size_table = cpu_size_table.data_ptr()
-    d.size_table_block_stride = int(cpu_size_table_block_stride)
-    d.size_table_layer_stride = int(cpu_size_table_layer_stride)
-    d.start_layer_id, d.kv_dim, d.num_blocks = int(start_layer_id), int(kv_dim), ids.numel()
-    d.batch_start, d.bsz = int(batch_start), int(bsz)
-    d.is_write_cpu = int(bool(is_write_cpu))
-    d.transfer_num_cta = int(transfer_num_cta)
-    d.device = comp_staging.device.index if comp_staging.device.index is not None else -1
-    d.sync = int(bool(sync))
+    d = _lib.StagingTransferDesc(  # in the order of the fields
+        comp_staging.data_ptr(), int(staging_stride_in_bytes), comp_sizes.data_ptr(),
+        cpu_tensor.data_ptr(), int(chunk_capacity_in_bytes),
+        overflow.data_ptr() if overflow is not None else None, int(cpu_kv_stride_in_bytes),
+        int(cpu_layer_stride_in_bytes), int(cpu_block_stride_in_bytes), ids.data_ptr(),
+        cpu_size_table.data_ptr(), int(cpu_size_table_block_stride),
+        int(cpu_size_table_layer_stride), int(start_layer_id), int(kv_dim), ids.numel(),
+        int(batch_start), int(bsz), bool(is_write_cpu), int(transfer_num_cta),
+        comp_staging.get_device(), bool(sync))
     check(_L.fkv_staging_transfer(ctypes.byref(d), _current_stream_handle()))
 
 
@@ -1054,7 +1009,8 @@ class LayerwiseTransferGroup:
                    gpu_index: int = 0) -> None:
         """Make ``stream`` (default: torch's current stream) wait until ``layer``
         of the last ``layerwise_transfer`` has landed."""
-        handle = int((stream or torch.cuda.current_stream()).cuda_stream)
+        # (torch's stream object alone costs as much as the rest of a call per layer)
+        handle = int(stream.cuda_stream) if stream else _current_stream_handle()
         check(_L.fkv_layerwise_wait_layer(self._h, int(gpu_index), int(layer), handle))
 
     def set_compute_stream(self, stream: Optional["torch.cuda.Stream"] = None,
