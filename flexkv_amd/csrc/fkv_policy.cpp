@@ -192,7 +192,7 @@ fkv_launch_policy defaults_for(uint32_t present) {
   // GPU->host wavefronts of large requests, 32 / 48 / 80: as much within 1 %, but a 2048^3 GEMM next to
   // both takes 160 / 192 / 252 us, a fused attention 378 / 454 / 680.
   p.d2h_busy_pct = 100;
-  p.h2d_busy_pct = 138; // 22
+  p.h2d_busy_pct = 138; // 22, which makes 44 ranges; on four XCDs 24 wavefronts share them
   p.busy_claims_per_wg = 2;
   p.home_claims_per_wg = 2;
   p.all_claims_per_wg = 0;
