@@ -912,8 +912,8 @@ CopyKernelArgs plan_job(const KernelPlan &p, int l0, int nl) {
 // launches keep to their direction's home XCDs, so that a transfer of the other
 // direction that starts while they run finds its own XCDs free.  On the home XCDs
 // a launch gets no more workgroups than on all XCDs: what a copy costs the kernels
-// next to it grows with their number (a 2048^3 GEMM takes 47 us next to 16 host->GPU
-// workgroups, confined or not, and 67 us next to 24), and 16 on four XCDs already
+// next to it grows with their number (a 2048^3 GEMM takes 49 us next to 16 host->GPU
+// workgroups and 74 next to 24, confined or not), and 16 on four XCDs already
 // reach the link rate.
 // Ranges per workgroup: see defaults_for in fkv_policy.cpp.  On an idle link the neighbours are
 // the engine's compute kernels, which slow down single workgroups of a copy, and
@@ -1020,14 +1020,15 @@ int kernel_plan_launch_layers(const KernelPlan &p, int layers_per_batch, LayersL
   t.batches = (p.num_layers + layers_per_batch - 1) / layers_per_batch;
   bool beside = false;
   const int workgroups = shape_for_now(p, bytes, stream, &t.a, &beside);
-  // Half as many workgroups again as for a plain copy: the fence behind every range takes a
-  // wavefront out for a few microseconds.  (16 / 20 / 24 wavefronts: 32 layers of 1 MiB 874 / 765 /
-  // 732 us, 61 of 7 MiB 9.52 / 8.23 / 7.84 ms; next to the latter three 2048^3 GEMMs take 118 /
-  // 121 / 126 us, 80 alone, a fused attention 112 / 113 / 115, 82 alone.)  Next to a transfer the
-  // other way there are half as many again already, and more would slow that one down: a put of
-  // 512 MiB takes 10.97 instead of 12.56 ms with 24 instead of 36 wavefronts beside it, the restore
+  // A quarter more workgroups than for a plain copy: the fence behind every range takes a
+  // wavefront out for a few microseconds.  (19 / 24 wavefronts: 32 layers of 1 MiB 695 / 693 us,
+  // 61 of 7 MiB 7.73 / 7.71 ms; with three 2048^3 GEMMs a layer that wait for it 8.04 / 8.35 ms, with a
+  // fused attention 7.86 / 8.06; those kernels on another stream 135 / 144 us, 79 alone, and 122 / 124,
+  // 75 alone.)  Next to a transfer the
+  // other way there are more already, and still more would slow that one down: a put of
+  // 512 MiB took 10.97 instead of 12.56 ms with 24 instead of 36 wavefronts beside it, the restore
   // 10.35 instead of 8.49, both together 11.16 instead of 12.71 ms.
-  t.grid_pct = beside ? 100 : 150;
+  t.grid_pct = beside ? 100 : 125;
   FKV_TRY(layers_device->launch(t, workgroups, stream));
   link_direction_mark(p.device, p.h2d, stream, bytes);
   return FKV_OK;

@@ -1123,10 +1123,10 @@ namespace {
 // writes its epoch to a word in device memory, which streams wait for, and one in pinned
 // memory, which the host looks at (see Landing).
 //
-// Whole restores, the forward stream waiting for every layer (us, before -> this): 8 x 256 KiB
-// to eventfds 159 -> 78, 32 x 1 MiB 773 -> 647, 61 x 7 MiB 9190 (rows gathered by host threads)
-// -> 7709, which is 56 GB/s.  Next to a fused attention of 76 us a layer: 32 x 1 MiB 2845 -> 2798,
-// 61 x 7 MiB 9193 -> 7994; next to three 2048^3 GEMMs a layer: 2691 -> 2585, 9224 -> 8076.
+// Whole restores, the forward stream waiting for every layer (us, a launch a batch -> this):
+// 8 x 256 KiB to eventfds 159 -> 72, 32 x 1 MiB 773 -> 627, 61 x 7 MiB 9190 (rows gathered by host threads)
+// -> 7631, which is 56.6 GB/s.  Next to a fused attention of 76 us a layer: 32 x 1 MiB 2845 -> 2807,
+// 61 x 7 MiB 9193 -> 7855; next to three 2048^3 GEMMs a layer: 2691 -> 2561, 9224 -> 8044.
 // Chunks of no whole number of slices are packed, batch by batch, as in copy_share: a batch is a
 // sequence of vectors, position-major, cut into pieces of a slice.  Short chunks used to take a
 // launch a batch (us, before -> this): 55 x 122 KiB in chunks of 2304 bytes 618 -> 170, 31 x 824 KiB
