@@ -515,7 +515,7 @@ DonePool &done_pool() {
   return *p;
 }
 constexpr size_t kDoneChunk = 64;  // calls that share an allocation,
-constexpr size_t kDoneStride = 256; // each with lines of its own
+constexpr size_t kDoneStride = 512; // each with lines of its own
 static_assert(sizeof(DoneCounts) <= kDoneStride, "the counts of a call fit its part");
 
 // The word of one call, for as long as somebody waits for it.

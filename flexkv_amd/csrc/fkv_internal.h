@@ -173,11 +173,13 @@ inline uint8_t *cpu_chunk_ptr(const fkv_transfer_desc &d, int64_t layer, int64_t
 
 // ---- the gather/scatter kernel -----------------------------------------
 // How a launch tells the thread that waits for it that everything has been copied.
-struct DoneCounts { // device memory, zero between launches
-  uint64_t of_xcd[16];  // launches to the host: workgroups at work on an XCD (high half), shares they have copied
-  uint32_t reported[16]; // of those, shares in `all`
-  uint32_t all;         // shares that have been copied
+struct DoneCounts { // device memory, one launch at a time
+  // Launches to the host, by XCD: workgroups at work there (fewer than kDoneShare), plus kDoneShare times
+  // the shares copied there since the counts were made; and those of them that have been reported.
+  uint64_t of_xcd[16], reported[16];
+  uint32_t all; // shares of the launch that have been reported, zero between launches
 };
+constexpr uint64_t kDoneShare = 1 << 16;
 struct CopyDone {
   DoneCounts *count = nullptr;
   uint64_t *word = nullptr;  // pinned: raised to `epoch` behind the last of them; nullptr: nobody waits

@@ -49,6 +49,7 @@
 // memory are plain, which measured about 1 GB/s faster over the link.
 #include "fkv_internal.h"
 #include "fkv_landing.h"
+#include "fkv_done.h"
 
 #include <algorithm>
 #include <chrono>
@@ -293,18 +294,19 @@ __device__ __forceinline__ void drain_wave() {
 // its shares.  To the host that would be a release to the system, which waits for whatever its XCD has
 // under way: with one for each of 16 workgroups of an XCD a copy of 10 MiB took 9 us longer, one of
 // 512 MiB, whose workgroups end milliseconds apart, 40.  So there the workgroups of an XCD, which
-// share an L2, count among themselves, and the last one at work on it releases for all: their
-// stores have been acknowledged by that L2 before they count.
+// share an L2, count among themselves, and the last one at work on it releases for all (fkv_done.h).
+// The L2 knows no owners: that one's release writes back every line which is dirty there, and
+// waits for every line on its way out of it, evicted ones too, as it must for its own stores, of
+// which some may have been evicted.  The others' stores have been acknowledged by that L2 before they
+// leave, so they are among those lines.
 template <bool TO_HOST> __device__ __forceinline__ void count_started(const CopyDone &done) {
   if (TO_HOST && done.word && threadIdx.x == 0)
-    (void)atomicAdd(reinterpret_cast<unsigned long long *>(&done.count->of_xcd[xcd_of_this_wave()]),
-                    1ull << 32);
+    begin_on_xcd(done, xcd_of_this_wave());
 }
 template <bool TO_HOST>
 __device__ __forceinline__ void count_copied(const CopyDone &done, uint32_t mine, uint32_t all) {
   if (!done.word || mine == 0) // the same for the whole workgroup
     return;
-  DoneCounts &c = *done.count;
   if (TO_HOST)
     drain_wave();
   else
@@ -313,42 +315,14 @@ __device__ __forceinline__ void count_copied(const CopyDone &done, uint32_t mine
   if (threadIdx.x != 0)
     return;
   if (TO_HOST) {
-#if defined(__HIP__)
-    constexpr int kOrder = __ATOMIC_RELAXED; // through the one L2
-#else // threads of the CPU model have none
-    constexpr int kOrder = __ATOMIC_ACQ_REL;
-#endif
     const uint32_t xcd = xcd_of_this_wave();
-    const uint64_t change = (uint64_t)mine - (1ull << 32);
-    const uint64_t now =
-        __hip_atomic_fetch_add(&c.of_xcd[xcd], change, kOrder, __HIP_MEMORY_SCOPE_AGENT) + change;
-    if (now >> 32) // others are at work: the last of them releases
+    const uint64_t far = leave_xcd(done, xcd, mine);
+    if (far == 0)
       return;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-    // Another workgroup may start here later and be the last one again; each reports what the
-    // one before did not.
-    mine = 0;
-    for (uint32_t before = __hip_atomic_load(&c.reported[xcd], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-         mine == 0 && before < (uint32_t)now;) {
-      const uint32_t seen = atomicCAS(&c.reported[xcd], before, (uint32_t)now);
-      if (seen == before)
-        mine = (uint32_t)now - before;
-      before = seen;
-    }
-    if (mine == 0)
-      return;
+    mine = newly_released(done, xcd, far);
   }
-  if (__hip_atomic_fetch_add(&c.all, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + mine == all) {
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    // for the next launch: nobody of this one counts any more
-    if (TO_HOST)
-      for (int i = 0; i < 16; ++i) {
-        __hip_atomic_store(&c.of_xcd[i], (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&c.reported[i], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-    __hip_atomic_store(&c.all, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(done.word, done.epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-  }
+  report_copied(done, mine, all);
 }
 
 // Copies the work units of `a` that fall into [num0/den, num1/den) of the job.

@@ -4,7 +4,8 @@
 // the deep unroll; one to 1024 (layer, kv) pairs; more block positions than one id tile
 // holds; id lists or none; plain and nontemporal stores; lanes that move adjacent vectors;
 // fixed shares, claimed ranges, launches confined to some XCDs with a dirty claim counter;
-// one to four jobs in one launch), every byte of every destination against a plain model.
+// one to four jobs in one launch; waited for, on one set of counts, or not; tables in the
+// arguments or in memory), every byte of every destination against a plain model.
 //
 // Every table, id list and chunk region is an allocation of exactly the size the kernel may
 // touch, the last chunk of a region ending where the allocation ends: an address one vector
@@ -159,6 +160,41 @@ uint64_t *share_out(std::mt19937_64 &rng, fkv::CopyKernelArgs &a) {
   return claim;
 }
 
+// One set of counts and one word for all launches that are waited for, as in the library's pool.
+struct Waiting {
+  fkv::DoneCounts counts{};
+  uint64_t word = 0, epoch = 0;
+};
+Waiting waiting;
+
+// Some launches are waited for, and some may carry their tables in their arguments, whether they fit or not
+// (numbers of their own, so that the shapes stay as they are without).
+void wait_and_carry(unsigned long long seed, std::vector<fkv::CopyKernelArgs *> jobs, fkv::CopyReport *report) {
+  std::mt19937_64 rng(seed * 2654435761ull + 1);
+  jobs[0]->report = report;
+  if (rng() % 4) {
+    jobs[0]->done.count = &waiting.counts, jobs[0]->done.word = &waiting.word;
+    jobs[0]->done.epoch = ++waiting.epoch;
+  }
+  const bool carry = rng() & 1;
+  for (fkv::CopyKernelArgs *a : jobs)
+    a->host_tables = carry;
+}
+
+// Behind a launch that has ended: its word is up, nobody is at work, everything has been reported.
+void check_waiting(unsigned long long seed, const fkv::CopyKernelArgs &a, const fkv::CopyReport &report) {
+  const bool slices = a.done.word && !report.announced; // those of HBM-bound launches announce nothing
+  REQUIRE(!slices || a.unroll != 0, "seed %llu: a launch that nobody is told about", seed);
+  if (slices)
+    --waiting.epoch;
+  REQUIRE(waiting.word == waiting.epoch, "seed %llu: word %llu of %llu", seed,
+          (unsigned long long)waiting.word, (unsigned long long)waiting.epoch);
+  bool rest = waiting.counts.all == 0;
+  for (int x = 0; x < 16; ++x)
+    rest = rest && waiting.counts.of_xcd[x] == waiting.counts.reported[x] * fkv::kDoneShare;
+  REQUIRE(rest, "seed %llu: counts behind the launch", seed);
+}
+
 void single(unsigned long long seed, hipStream_t stream) {
   std::mt19937_64 rng(seed);
   const int vec = 1 << pick(rng, 0, 4);
@@ -166,9 +202,12 @@ void single(unsigned long long seed, hipStream_t stream) {
   make_job(rng, vec, rng() & 1, false, j);
   uint64_t *claim = share_out(rng, j.a);
   const int threads = std::vector<int>{1, 64, 128, 256, 1024, 4096}[pick(rng, 0, 5)];
+  fkv::CopyReport report;
+  wait_and_carry(seed, {&j.a}, &report);
   REQUIRE(fkv::launch_copy_kernel(j.a, pick(rng, 1, 40), threads, stream) == FKV_OK, "seed %llu: %s",
           seed, fkv_last_error());
   REQUIRE(hipStreamSynchronize(stream) == hipSuccess, "synchronize");
+  check_waiting(seed, j.a, report);
   check_and_release(j, seed, 0);
   if (claim)
     REQUIRE(hipFree(claim) == hipSuccess, "free counter");
@@ -185,10 +224,16 @@ void several(unsigned long long seed, hipStream_t stream) {
     args.push_back(j.a);
   }
   uint64_t *claim = share_out(rng, args[0]);
+  fkv::CopyReport report;
+  std::vector<fkv::CopyKernelArgs *> each;
+  for (fkv::CopyKernelArgs &a : args)
+    each.push_back(&a);
+  wait_and_carry(seed, each, &report);
   REQUIRE(fkv::launch_copy_jobs(args.data(), njobs, pick(rng, 1, 24),
                                 std::vector<int>{64, 256, 1024}[pick(rng, 0, 2)], stream) == FKV_OK,
           "seed %llu: %s", seed, fkv_last_error());
   REQUIRE(hipStreamSynchronize(stream) == hipSuccess, "synchronize");
+  check_waiting(seed, args[0], report);
   for (int k = 0; k < njobs; ++k)
     check_and_release(jobs[k], seed, k);
   if (claim)

@@ -48,6 +48,12 @@ inline void fence(int order) {
   if (order == __ATOMIC_ACQUIRE || order == __ATOMIC_ACQ_REL)
     (void)fence_word.load(std::memory_order_acquire);
 }
+template <typename T> inline T fetch_max(T *p, T v, int order) {
+  T seen = __atomic_load_n(p, __ATOMIC_RELAXED);
+  while (seen < v && !__atomic_compare_exchange_n(p, &seen, v, false, order, __ATOMIC_RELAXED))
+    ;
+  return seen;
+}
 // The launch's dynamically sized LDS, one array per workgroup, zeroed never (as on the device).
 void *dynamic_lds();
 // XCDs take the workgroups of a launch in turn; which one takes workgroup 0 changes
@@ -92,6 +98,7 @@ void launch(hipStream_t stream, dim3 grid, dim3 block, size_t lds_bytes, std::fu
 #define __hip_atomic_load(pointer, order, scope) __atomic_load_n(pointer, order)
 #define __hip_atomic_store(pointer, value, order, scope) __atomic_store_n(pointer, value, order)
 #define __hip_atomic_fetch_add(pointer, value, order, scope) __atomic_fetch_add(pointer, value, order)
+#define __hip_atomic_fetch_max(pointer, value, order, scope) cpu_device_model::fetch_max(pointer, value, order)
 #define __builtin_amdgcn_fence(order, scope) cpu_device_model::fence(order)
 #undef hipLaunchKernelGGL
 #define hipLaunchKernelGGL(kernel, grid, block, lds_bytes, stream, ...)                             \

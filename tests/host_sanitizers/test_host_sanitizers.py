@@ -290,3 +290,13 @@ def test_landing_of_batches_and_waits_for_them(tmp_path, sanitizer):
     r = subprocess.run([exe, "300"], capture_output=True, text=True, env=env, timeout=300)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-6000:]
     assert "ok: 300 landings by turns and by threads" in r.stdout
+
+
+@pytest.mark.parametrize("sanitizer", SANITIZERS)
+def test_launches_that_tell_when_everything_has_been_copied(tmp_path, sanitizer):
+    """The counts behind the word that a waiting call looks at (fkv_done.h): workgroups take turns in
+    seeded orders, some dispatched late, some long in their release, launch after launch on one set
+    of counts; the word is raised when every share has been copied and released, and what the counts
+    hold then is no part of the next launch."""
+    out = build_and_run(tmp_path, "done_driver.cpp", sanitizer, extra=("-I" + HERE,))
+    assert "ok: 1000 sets of counted launches" in out
