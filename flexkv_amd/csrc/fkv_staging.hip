@@ -172,25 +172,26 @@ __global__ __launch_bounds__(kCopyBlockThreads) void fkv_staging_transfer_kernel
            (a.start_layer + (int64_t)p.layer) * a.table_layer_stride + p.kv;
   };
   // out of HBM where it is written, out of host memory, a round trip over the link, where it is read
-  auto size_of = [&](uint32_t i, const Place &p) -> int64_t {
-    return WRITE_CPU ? (int64_t)((const FKV_CONSTANT uint64_t *)a.comp_sizes)[i]
-                     : (int64_t)*(const FKV_CONSTANT uint32_t *)entry_of(p);
+  // (64 bits without a sign: a compressor's "failed" may be the largest of them)
+  auto size_of = [&](uint32_t i, const Place &p) -> uint64_t {
+    return WRITE_CPU ? ((const FKV_CONSTANT uint64_t *)a.comp_sizes)[i]
+                     : (uint64_t)*(const FKV_CONSTANT uint32_t *)entry_of(p);
   };
   if (wave >= bsz)
     return;
   Place here = place(wave), next = place(min(wave + nwaves, bsz - 1));
-  int64_t sz_next = size_of(wave, here);
+  uint64_t sz_next = size_of(wave, here);
   for (uint32_t i = wave; i < bsz; i += nwaves) {
     uint8_t *const cur_slot = slot_of(here);
     uint32_t *const cur_entry = entry_of(here);
-    const int64_t sz = sz_next;
+    const uint64_t sz = sz_next;
     if (i + nwaves < bsz)
       sz_next = size_of(i + nwaves, next);
     here = next;
     next = place(min(i + 2 * nwaves, bsz - 1)); // both far from 2^32
     uint8_t *payload = a.staging + i * a.staging_stride;
     if (WRITE_CPU) {
-      if (sz > a.chunk_capacity) { // does not fit its host slot: counted, size 0 recorded
+      if (sz > (uint64_t)a.chunk_capacity) { // does not fit its host slot: counted, size 0 recorded
         if (lane == 0) {
           if (a.overflow)
             atomicAdd(a.overflow, 1);
@@ -200,9 +201,9 @@ __global__ __launch_bounds__(kCopyBlockThreads) void fkv_staging_transfer_kernel
       }
       if (lane == 0)
         *cur_entry = (uint32_t)sz;
-      wave_copy<VEC16, false, RUNS>(payload, cur_slot, sz, lane);
+      wave_copy<VEC16, false, RUNS>(payload, cur_slot, (int64_t)sz, lane);
     } else {
-      if (sz > a.staging_stride) { // a stale or corrupt entry must not overrun the staging slot
+      if (sz > (uint64_t)a.staging_stride) { // a stale or corrupt entry must not overrun the staging slot
         if (lane == 0) {
           if (a.overflow)
             atomicAdd(a.overflow, 1);
@@ -211,8 +212,8 @@ __global__ __launch_bounds__(kCopyBlockThreads) void fkv_staging_transfer_kernel
         continue;
       }
       if (lane == 0)
-        a.comp_sizes[i] = (uint64_t)sz;
-      wave_copy<VEC16, true, false>(cur_slot, payload, sz, lane);
+        a.comp_sizes[i] = sz;
+      wave_copy<VEC16, true, false>(cur_slot, payload, (int64_t)sz, lane);
     }
   }
 }

@@ -300,3 +300,18 @@ def test_launches_that_tell_when_everything_has_been_copied(tmp_path, sanitizer)
     hold then is no part of the next launch."""
     out = build_and_run(tmp_path, "done_driver.cpp", sanitizer, extra=("-I" + HERE,))
     assert "ok: 1000 sets of counted launches" in out
+
+
+@pytest.mark.parametrize("sanitizer,calls", [(SANITIZERS[0].values[0], 60),
+                                             (SANITIZERS[1].values[0], 30)],
+                         ids=["asan-ubsan", "tsan"])
+def test_payload_transfers_on_a_cpu_device_model(tmp_path, sanitizer, calls):
+    """Payloads of every kind of length out and back, sizes that do not fit their slots among them (up
+    to 2^64 - 1, which a compressor may give for "failed"), against the oracle."""
+    exe = build_over_emulated_runtime(tmp_path, "staging_model_driver.cpp", sanitizer,
+                                      kernels_from_source=True)
+    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:verify_asan_link_order=0",
+               TSAN_OPTIONS="halt_on_error=1", TMPDIR=str(tmp_path))
+    r = subprocess.run([exe, str(calls)], capture_output=True, text=True, env=env, timeout=600)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-6000:]
+    assert "ok: %d payload transfers" % calls in r.stdout

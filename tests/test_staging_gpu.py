@@ -177,3 +177,16 @@ def test_chunk_ptrs_match_the_oracle_and_address_the_chunks(gpu_device, backend,
         dev_bytes = off[0][off[1]:off[1] + 16].cpu().numpy()
         ref_bytes = np.frombuffer((ctypes.c_uint8 * 16).from_address(int(ref[i])), dtype=np.uint8)
         np.testing.assert_array_equal(dev_bytes, ref_bytes)
+
+
+@pytest.mark.parametrize("cap", [4608, 1001])
+def test_sizes_of_64_bits_do_not_fit(gpu_device, cap):
+    """A compressor's "failed" (2^64 - 1, or any size with its upper half set) is a payload that does not
+    fit: counted, 0 in the size table, nothing copied."""
+    rng = np.random.default_rng(cap)
+    c = Case(gpu_device, rng, 3, 2, 9, 12, cap, cap, "BLOCKFIRST", (0, cap), 54)
+    large = [2**64 - 1, 2**64 - 17, 2**64 - 8191, 2**63, 2**63 + 100, 2**32, 2**32 + 16]
+    c.sizes_ref[5:5 + len(large)] = np.array(large, dtype=np.uint64)
+    c.sizes.copy_(torch.from_numpy(c.sizes_ref.view(np.int64)))
+    assert c.run(0, 0, 54, True) == len(large) == int(c.overflow.item())
+    c.check("after the write")
