@@ -509,6 +509,7 @@ namespace {
 struct DonePool {
   std::mutex mu;
   std::map<int, std::vector<CopyDone>> idle;
+  std::mutex growing; // held by the call that allocates
 };
 DonePool &done_pool() {
   static DonePool *p = new DonePool(); // lives until the process ends
@@ -532,7 +533,9 @@ public:
   }
   // `device` is current.  Without a word (none to be had, a stream that is being captured and
   // will not run the launch now) the call waits for an event.  The first call of 64 at a time
-  // allocates; new counts are cleared by a kernel on its own stream, which it waits for.
+  // allocates; new counts are cleared by a kernel on its own stream, which it waits for.  Calls that
+  // find the pool empty meanwhile wait for events, so that threads which start together do not allocate a
+  // set each next to the others' transfers, nor wait for that stream.
   void acquire(int device, hipStream_t stream) {
     if (!copies_announce || !copies_announce(stream))
       return;
@@ -565,6 +568,10 @@ public:
 
 private:
   bool allocate(hipStream_t stream) {
+    DonePool &p = done_pool();
+    std::unique_lock<std::mutex> only(p.growing, std::try_to_lock);
+    if (!only)
+      return false;
     constexpr size_t kBytes = kDoneChunk * kDoneStride;
     void *d = nullptr, *h = nullptr;
     bool ok = hipHostMalloc(&h, kBytes, hipHostMallocPortable | hipHostMallocMapped) == hipSuccess &&
@@ -583,7 +590,6 @@ private:
         (void)hipHostFree(h);
       return false;
     }
-    DonePool &p = done_pool();
     std::lock_guard<std::mutex> lk(p.mu);
     std::vector<CopyDone> &v = p.idle[device_];
     for (size_t i = 0; i < kDoneChunk; ++i) {

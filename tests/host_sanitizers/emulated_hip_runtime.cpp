@@ -126,6 +126,7 @@ std::atomic<long> g_fail_after[kCategories];
 std::atomic<long> g_fail_count[kCategories];
 std::atomic<long> g_failed_calls{0};
 std::atomic<long> g_host_waited_copies{0}; // hipMemcpy calls: the host waits for each
+std::atomic<long> g_small_pinned_allocations{0}; // of less than 64 KiB, which plan memory never is
 bool refused(Category c) {
   if (g_fail_count[c].load(std::memory_order_relaxed) <= 0)
     return false;
@@ -423,6 +424,8 @@ hipError_t hipMalloc(void **p, size_t size) {
 }
 hipError_t hipFree(void *p) { return release(p, false); }
 hipError_t hipHostMalloc(void **p, size_t size, unsigned int) {
+  if (size < 64 * 1024)
+    g_small_pinned_allocations.fetch_add(1);
   *p = refused(kPinnedAlloc) ? nullptr : allocate(size, true);
   return *p ? hipSuccess : remember(hipErrorOutOfMemory);
 }
@@ -847,6 +850,7 @@ extern "C" unsigned long long fkv_emulated_workgroups_run() { return 0; }
 
 // Copies the host has waited for since the process started (hipMemcpy): a library that
 // makes one per request under load holds every thread up for as long as the device is busy.
+extern "C" long fkv_emulated_small_pinned_allocations() { return g_small_pinned_allocations.load(); }
 extern "C" long fkv_emulated_host_waited_copies() { return g_host_waited_copies.load(); }
 
 // Test hook: the next `count` calls of `category` (0 device allocation, 1 pinned allocation,

@@ -315,3 +315,16 @@ def test_payload_transfers_on_a_cpu_device_model(tmp_path, sanitizer, calls):
     r = subprocess.run([exe, str(calls)], capture_output=True, text=True, env=env, timeout=600)
     assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-6000:]
     assert "ok: %d payload transfers" % calls in r.stdout
+
+
+@pytest.mark.parametrize("sanitizer", SANITIZERS)
+def test_words_for_threads_that_start_together_are_allocated_once(tmp_path, sanitizer):
+    """A dozen threads whose first waiting transfers start together, on a busy device: one allocation
+    of words, none later, every call returns when its own copy has been made."""
+    exe = build_over_emulated_runtime(tmp_path, "copy_wait_emulated_driver.cpp", sanitizer,
+                                      kernels_from_source=True)
+    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:verify_asan_link_order=0",
+               TSAN_OPTIONS="halt_on_error=1", TMPDIR=str(tmp_path))
+    r = subprocess.run([exe], capture_output=True, text=True, env=env, timeout=60)
+    assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-6000:]
+    assert "ok: 12 threads waiting at once" in r.stdout
