@@ -241,3 +241,78 @@ def test_link_activity_board_is_shared_between_processes():
         path = f"/dev/shm/fkv_link_{os.getuid()}_{key}_{dev}"
         if os.path.exists(path):
             os.unlink(path)
+
+
+class _OnDevice:
+    """What the operators ask of a device tensor."""
+    is_cuda, is_cpu = True, False
+
+    def __init__(self, address, numel, dtype):
+        self._address, self._numel, self.dtype = address, numel, dtype
+
+    def data_ptr(self):
+        return self._address
+
+    def numel(self):
+        return self._numel
+
+    def element_size(self):
+        return self.dtype.itemsize
+
+    def get_device(self):
+        return 3
+
+
+def _fields(desc):
+    return {name: getattr(desc, name) for name, _ in desc._fields_}
+
+
+def test_operators_fill_descriptors_field_by_field(monkeypatch):
+    """The operators pass all fields of a descriptor at once, in order: each argument in its own field."""
+    from flexkv_amd import c_ext
+    gids, cids, ptrs = (torch.arange(n, dtype=torch.int64) for n in (2, 2, 6))
+    host = torch.empty(64, dtype=torch.uint8)
+    d, _ = c_ext._transfer_desc(
+        gids, ptrs, 11, 12, 13, cids, host, 14, 15, 16, 17, 1, 2, transfer_num_cta=18,
+        is_host_to_device=False, use_ce_transfer=True, kv_dim=1, num_kv_heads=19, gpu_block_type=2, sync=False,
+        ce_path_opt=True, ce_segment_threshold=20, ce_force_path=4, ce_enable_memcpy2d=False,
+        is_blockfirst=True, ce_gather_threads=21, ce_gather_nt=False, enable_transfer_trace=True)
+    got = _fields(d)
+    assert _fields(got.pop("ce")) == dict(_fields(_lib.CEConfig()), segment_threshold=20, path_opt_enabled=1,
+                                          force_path=4, enable_memcpy2d=0, is_blockfirst=1, num_kv_heads=19,
+                                          gather_threads=21, gather_nt=0)
+    assert got == dict(
+        backend=2, num_layers_total=3, gpu_tensor_ptrs=ptrs.data_ptr(), num_gpu_tensor_ptrs=6, device=-1,
+        gpu_kv_stride=11, gpu_block_stride=12, gpu_layer_stride=13, gpu_startoff_inside_chunks=0,
+        cpu_ptr=host.data_ptr(), cpu_kv_stride=14, cpu_layer_stride=15, cpu_block_stride=16,
+        cpu_startoff_inside_chunks=0, chunk_size=17, start_layer_id=1, num_layers=2, kv_dim=1, num_blocks=2,
+        gpu_block_ids=gids.data_ptr(), cpu_block_ids=cids.data_ptr(), is_host_to_device=0, use_ce_transfer=1,
+        transfer_num_cta=18, sync=0, enable_trace=1, reserved=0)
+
+    seen = {}
+
+    class Library:
+        def __getattr__(self, name):
+            def entry(desc, stream):
+                seen[name] = _fields(desc._obj)
+                return 0
+            return entry
+
+    monkeypatch.setattr(c_ext, "_L", Library())
+    c_ext.layout_transform(_OnDevice(4096, 10 ** 6, torch.uint8), 21, 22, 23, 24, ptrs, 25, 26, 27, gids, 2, 1,
+                           True, gpu_block_type=2, start_layer_id=1, sync=False)
+    assert seen["fkv_layout_transform"] == dict(
+        backend=2, num_layers_total=3, gpu_tensor_ptrs=ptrs.data_ptr(), num_gpu_tensor_ptrs=6, device=3,
+        gpu_kv_stride=25, gpu_block_stride=26, gpu_layer_stride=27, buffer_ptr=4096, buffer_layer_stride=21,
+        buffer_kv_stride=22, buffer_block_stride=23, chunk_size=24, start_layer_id=1, num_layers=2, kv_dim=1,
+        num_blocks=2, gpu_block_ids=gids.data_ptr(), buffer_to_target=1, sync=0)
+    table = torch.zeros(8, dtype=torch.int32)
+    c_ext.staging_transfer(_OnDevice(8192, 10 ** 6, torch.uint8), 31, _OnDevice(12288, 99, torch.int64), host, 32,
+                           _OnDevice(16384, 1, torch.int32), 33, 34, 35, cids, table, 36, 37, 38, 2, 39, 40, True,
+                           transfer_num_cta=41, sync=False)
+    assert seen["fkv_staging_transfer"] == dict(
+        staging=8192, staging_stride=31, comp_sizes=12288, cpu_ptr=host.data_ptr(), chunk_capacity=32,
+        overflow=16384, cpu_kv_stride=33, cpu_layer_stride=34, cpu_block_stride=35,
+        cpu_block_ids=cids.data_ptr(), size_table=table.data_ptr(), size_table_block_stride=36,
+        size_table_layer_stride=37, start_layer_id=38, kv_dim=2, num_blocks=2, batch_start=39, bsz=40,
+        is_write_cpu=1, transfer_num_cta=41, device=3, sync=0)
