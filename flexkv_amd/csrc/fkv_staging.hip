@@ -50,11 +50,11 @@ typedef unsigned int vec16 __attribute__((ext_vector_type(4)));
 // move the last vector (byte) once more, the same bytes to the same place, instead of sitting
 // out: every load is used, so nothing has to be waited for where this joins the path of whole slices
 // (see nothing_in_flight in fkv_kernels.hip).
-#if defined(__HIP__)
-constexpr bool kAllLanesStore = true;
-#else // work-items of the CPU model are threads, to whose sanitizer that is a race
-constexpr bool kAllLanesStore = false;
+// (To ThreadSanitizer, under which work-items are threads, that is a race.)
+#ifndef __has_feature
+#define __has_feature(name) 0
 #endif
+constexpr bool kAllLanesStore = !__has_feature(thread_sanitizer);
 template <int N, bool NTS>
 __device__ __forceinline__ void copy_end(const FKV_GLOBAL vec16 *s, FKV_GLOBAL vec16 *d, int nvec, int tail,
                                          int lane) {
