@@ -28,8 +28,9 @@ hipError_t pooled_stream_acquire(int device, bool non_blocking, hipStream_t *out
 void pooled_stream_release(int device, bool non_blocking, hipStream_t stream);
 // Waits of the host for device work.  The runtime's own (hipEventSynchronize,
 // hipStreamSynchronize, also on events made for blocking waits) keep a core busy for as long
-// as they last; these poll instead when quiet_wait_us of the device's launch policy says so
-// and two threads of the process are already waiting the runtime's way:
+// as they last, and so does looking at a word without a pause; these sleep instead when
+// quiet_wait_us of the device's launch policy says so
+// and two threads of the process are already waiting the busy way:
 // a spin of 30 us for work that is nearly done, then sleeps that double from 20 us up to
 // that limit; with `expected_ns` (how long the work takes when nothing else holds it up, 0 =
 // unknown) the thread sleeps towards that moment first, a millisecond at a time at most, and

@@ -105,10 +105,14 @@ typedef struct fkv_transfer_desc {
   int32_t is_host_to_device;
   int32_t use_ce_transfer;  /* 0 kernel, 1 copy engine, 2 pick per transfer (fkv_choose_engine) */
   int32_t transfer_num_cta; /* CTAs as the reference counts them; each becomes 4 (host->GPU)
-                               or 12 (GPU->host) single-wavefront workgroups;
-                               <= 0 = library default (4) */
+                               or 8 (GPU->host; 12 for transfers below 16 MiB) single-wavefront
+                               workgroups; <= 0 = library default (4) */
   int32_t sync;             /* 1: return when the transfer (and what `stream` held before it)
-                               has finished; where the reference calls cudaStreamSynchronize */
+                               has finished; where the reference calls cudaStreamSynchronize.  The
+                               bytes are in place for the host, for copies and for kernels on any
+                               stream.  The stream itself may be busy for some microseconds more,
+                               with the end of a kernel that has told the host so: hipStreamQuery
+                               right behind the call can say hipErrorNotReady */
   int32_t enable_trace;     /* 1: print an "[XFER]" line per call to stderr */
   int32_t reserved;
   fkv_ce_config ce;
@@ -805,13 +809,16 @@ typedef struct fkv_launch_policy {
                                  announces its batches itself where its shape allows that, and as
                                  with 4096 otherwise */
   int32_t quiet_wait_us;        /* how a call waits for its transfer (sync = 1, the thread group, the
-                                 layerwise restore in HOSTFUNC mode, fkv_layerwise_synchronize): the
-                                 runtime's own waits keep a core busy for as long as they last (a
+                                 layerwise restore in HOSTFUNC mode, fkv_layerwise_synchronize).  The
+                                 soonest way back keeps a core busy for as long as the wait lasts: a
+                                 synchronous transfer that is one launch of the copy kernel looks at
+                                 a word in pinned memory without a pause, anything else uses the
+                                 runtime's own wait (a
                                  synchronous 9 ms transfer costs 9 ms of CPU time, 64 waiting
                                  requests 13 of 16 cores, and the threads that still have to submit
                                  theirs wait for a core).  > 0 (default 100): while two threads of the
-                                 process are already waiting the runtime's way, further ones poll
-                                 their event instead: they sleep towards the moment the transfer
+                                 process are already waiting that way, further ones look at
+                                 their word or event now and then: they sleep towards the moment the transfer
                                  would end alone on the link, spin for the 80 us around it, and
                                  after that sleep for spells that double from 20 us up to this many
                                  microseconds (2 % of a core each; such a wait ends up to that much
@@ -821,7 +828,8 @@ typedef struct fkv_launch_policy {
                                  thousand.  < 0: every waiting thread polls, with -value as the
                                  limit (a worker then costs 2 % of a core while it waits instead of a
                                  whole one, and its 9.4 ms op ends up to 0.1 ms later).  0 = always
-                                 the runtime's wait */
+                                 the busy way, for as long as the stream takes, what it held before
+                                 the transfer included */
 } fkv_launch_policy;
 /* The table of `device` (-1 = current).  The first call for a device runs the probe kernel. */
 int fkv_launch_policy_get(int32_t device, fkv_launch_policy *out);
