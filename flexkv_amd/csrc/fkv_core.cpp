@@ -861,7 +861,8 @@ int kernel_plan_publish(KernelPlan *p, hipStream_t stream, bool one_launch) {
   // stays where it is, as long as a workgroup's part of it is one round trip: the ids of its
   // blocks one a lane, and two tables of two entries a lane (1024
   // blocks of 2304 bytes 72.6 -> 70.1 us; with 160 (layer, kv) pairs 37.5 -> 37.7, with 256
-  // 73.0 -> 73.9).  A restore that reads its plan a launch a batch is 1.5 % slower
+  // 73.0 -> 73.9; plans that fit the arguments one by one but not together with the others of
+  // their launch are read in place too, of 200 pairs at most).  A restore that reads its plan a launch a batch is 1.5 % slower
   // in place; but next to a transfer in the other direction every command on a stream costs
   // idle time, and nothing is uploaded then: two threads that put and get 25 MB (100 MB)
   // requests move 88.8 (95.4) instead of 87.0 (94.1) GB/s.  plan_mirror of the launch

@@ -284,11 +284,10 @@ __device__ __forceinline__ void drain_wave() {
 //
 // A waiting thread learns it 5 us sooner than from an event behind the launch (an event is a
 // command of its own, which the stream takes up when the kernel has been retired), and 10 us
-// sooner than with the two more events that plan memory and the link's bookkeeping used to need;
-// next to traffic the other way, where every command costs a stream idle time, by more.  Whole
+// sooner than with the two more events that plan memory and the link's bookkeeping used to need.  Whole
 // calls, event -> word (us): 53 KiB from the host 28.2 -> 17.2, 2 MiB 58.4 -> 52.7, 72 MiB
 // 1340 -> 1332; 130 KiB to it 32.3 -> 21.3, 10 MiB 216.4 -> 207.2, 512 MiB 9450 -> 9444; three layer
-// groups 808 -> 793; six puts and six gets of 64 MiB at the same time 9336 -> 9191.
+// groups 808 -> 793; six puts and six gets of 64 MiB at the same time the same.
 //
 // Into HBM every workgroup releases what it wrote to whatever runs on the device next, and counts
 // its shares.  To the host that would be a release to the system, which waits for whatever its XCD has

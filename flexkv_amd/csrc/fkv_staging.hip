@@ -320,8 +320,11 @@ int fkv_staging_transfer(const fkv_staging_transfer_desc *dp, void *stream_v) tr
   const int cta = d.transfer_num_cta > 0 ? d.transfer_num_cta : default_num_cta(!write_cpu);
   // The wavefronts of a plain copy to the host, half as many again for a call that is over soon;
   // from the host also, because a wavefront has one payload in flight, whose last slice is short.
-  // 48 MiB of slots of 32 KiB, us, and what a 2048^3 GEMM next to it takes longer: written with 30 / 40
-  // / 50 wavefronts 667 (3.9x) / 657 (7.1x) / 655 (7.0x), read with 16 / 24 / 32 653 / 643 / 637 (3.6x).
+  // 48 MiB of slots of 32 KiB, us, and what a 2048^3 GEMM (alone 27) / a streaming kernel (37) next to it
+  // takes: written with 16 / 24 / 32 wavefronts 683 (59 / 43) / 663 (105 / 51) / 654 (160 / 72), read with
+  // 12 / 18 / 24 715 (44 / 40) / 643 (54 / 41) / 629 (67 / 43).  The wavefronts that waited for their stores, 48
+  // and 32 of them, took 662 (67 / 58) and 637 (50 / 41), of slots of 8 KiB 688 (43 / 42) and 657 (40 / 39)
+  // against 695 (73 / 63) and 632 (51 / 41) now: a caller whose own kernels matter more takes 3 CTAs, not 4.
   // Slots shorter than a slice hold less, and as many more wavefronts have the same bytes
   // under way: 48 MiB of slots of 2 KiB written 931 -> 715, read 1268 -> 677.
   const int64_t slots = (int64_t)d.bsz * d.staging_stride;

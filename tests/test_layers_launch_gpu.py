@@ -224,7 +224,7 @@ def test_wait_layer_while_the_stream_is_captured(gpu_device):
 
 
 def test_shapes_that_go_batch_by_batch(gpu_device):
-    """Packed chunks and odd vector widths keep a launch a batch."""
+    """Few batches of short chunks, and odd vector widths, keep a launch a batch."""
     from flexkv_amd.c_ext import get_stats, launch_policy, reset_stats
     from flexkv_amd.c_ext import LayerwiseTransferGroup
     i64 = lambda v: torch.tensor([v], dtype=torch.int64)  # noqa: E731
