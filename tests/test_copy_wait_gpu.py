@@ -78,7 +78,7 @@ def test_threads_that_wait_at_once(gpu_device):
 @pytest.mark.parametrize("policy", ["default", "everywhere", "claimed"])
 def test_a_put_larger_than_the_caches_is_all_there(gpu_device, policy):
     """192 MiB, many times what the L2s hold: most lines leave them before the release that the
-    word stands behind.  (On four XCDs, on all, and in many small ranges, several launches on one word.)"""
+    word stands behind.  (On three XCDs, on all, and in many small ranges, several launches on one word.)"""
     from flexkv_amd.c_ext import launch_policy
     s = KVSetup(VLLM, 8, 2, 100, 96, 131072, "BLOCKFIRST", seed=96)
     dev = s.to_device(gpu_device)
@@ -91,3 +91,31 @@ def test_a_put_larger_than_the_caches_is_all_there(gpu_device, policy):
             put = dev.host_bytes().copy()  # straight away
             s.oracle_transfer(gids, cids, is_h2d=False)
             assert np.array_equal(put, s.host_ref)
+
+
+@pytest.mark.parametrize("policy", ["default", "everywhere", "claimed", "confined", "fat"])
+def test_puts_next_to_compute_that_holds_the_compute_units(gpu_device, policy):
+    """Workgroups that find no room until others of their launch have ended: each put is all there when
+    its call returns, many of them on one word."""
+    from flexkv_amd.c_ext import launch_policy
+    s = KVSetup(VLLM, 8, 2, 24, 20, 24592, "BLOCKFIRST", seed=24)
+    dev = s.to_device(gpu_device)
+    rng = np.random.default_rng(24)
+    a = torch.randn(4096, 4096, device=gpu_device, dtype=torch.bfloat16)
+    out, beside, own = torch.empty_like(a), torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with launch_policy(**POLICIES[policy]):
+        for rep in range(12):
+            with torch.cuda.stream(beside):
+                for _ in range(6):
+                    torch.mm(a, a, out=out)
+            n = int(rng.integers(1, 20))
+            gids, cids = block_ids(rng, 24, n), block_ids(rng, 20, n)
+            dev.host.fill_(rep)
+            s.host_ref[:] = rep
+            with torch.cuda.stream(own):
+                dev.transfer(gids, cids, is_h2d=False)
+            put = dev.host_bytes().copy()  # straight away
+            s.oracle_transfer(gids, cids, is_h2d=False)
+            assert np.array_equal(put, s.host_ref), (rep, n)
+    torch.cuda.synchronize()
