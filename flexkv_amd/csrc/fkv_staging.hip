@@ -27,6 +27,8 @@ namespace fkv {
 namespace {
 
 constexpr int64_t kShortMinBytes = 16 << 20; // calls over fewer bytes of slots are over soon
+constexpr int64_t kSliceBytes = 64 * kCopyUnroll * 16;
+constexpr int64_t kFewWholeSlices = kSliceBytes * 3 / 2; // most payloads in smaller slots have none
 
 struct StagingKernelArgs {
   uint8_t *staging;
@@ -80,8 +82,36 @@ __device__ __forceinline__ void copy_end(const FKV_GLOBAL vec16 *s, FKV_GLOBAL v
   asm volatile("" ::"i"(N)); // keeps the last stores of the cases apart, which would be merged and wait
 }
 
+// The same for a payload without a whole slice but with more than half of one, in the order of adjacent
+// vectors.  Slots of 8 KiB, 50-90 % full, hold little else.  Us, and what a 2048^3 GEMM (27) / a streaming kernel (37)
+// beside it takes, vectors 64 apart with 32 wavefronts -> this with 24: 24 MiB 373 (69 / 58) -> 355 (52 / 41),
+// 48 MiB 697 (72 / 62) -> 672 (55 / 42).
+template <bool NTS>
+__device__ __forceinline__ void copy_end_runs(const FKV_GLOBAL vec16 *s, FKV_GLOBAL vec16 *d, int nvec, int tail,
+                                              int lane) {
+  const int byte = nvec * 16 + (tail ? min(lane, tail - 1) : -1);
+  const uint8_t last = *((const FKV_GLOBAL uint8_t *)s + byte);
+  vec16 r[kCopyUnroll];
+#pragma unroll
+  for (int u = 0; u < kCopyUnroll; ++u)
+    r[u] = s[min(lane * kCopyUnroll + u, nvec - 1)];
+#pragma unroll
+  for (int u = 0; u < kCopyUnroll; ++u) {
+    if (!kAllLanesStore && lane * kCopyUnroll + u >= nvec)
+      continue;
+    FKV_GLOBAL vec16 *to = d + min(lane * kCopyUnroll + u, nvec - 1);
+    if (NTS)
+      __builtin_nontemporal_store(r[u], to);
+    else
+      *to = r[u];
+  }
+  if (kAllLanesStore || lane < tail)
+    *((FKV_GLOBAL uint8_t *)d + byte) = last;
+  asm volatile("" ::"i"(16)); // as above
+}
+
 // Copies `bytes` from src to dst with one wavefront; VEC16: both are 16-byte aligned.  RUNS: in whole
-// slices a lane moves adjacent vectors, 128 bytes, so that its stores complete a line of host
+// slices, and in payloads that come near one, a lane moves adjacent vectors, 128 bytes, so that its stores complete a line of host
 // memory (see copy_slice in fkv_kernels.hip); its loads walk through one line, without the
 // streaming hint that might let the line go in between.
 template <bool VEC16, bool NTS, bool RUNS>
@@ -116,6 +146,8 @@ __device__ __forceinline__ void wave_copy(const uint8_t *__restrict__ src, uint8
   }
   if (rest == 0)
     return;
+  if (RUNS && whole == 0 && nvec > 64 * U / 2)
+    return copy_end_runs<NTS>(s, d, nvec, tail, lane);
   switch ((nvec + 63) / 64) {
   case 1: return copy_end<1, NTS>(s, d, nvec, tail, lane);
   case 2: return copy_end<2, NTS>(s, d, nvec, tail, lane);
@@ -324,27 +356,32 @@ int fkv_staging_transfer(const fkv_staging_transfer_desc *dp, void *stream_v) tr
   // takes: written with 16 / 24 / 32 wavefronts 683 (59 / 43) / 663 (105 / 51) / 654 (160 / 72), read with
   // 12 / 18 / 24 715 (44 / 40) / 643 (54 / 41) / 629 (67 / 43).  The wavefronts that waited for their stores, 48
   // and 32 of them, took 662 (67 / 58) and 637 (50 / 41), of slots of 8 KiB 688 (43 / 42) and 657 (40 / 39)
-  // against 695 (73 / 63) and 632 (51 / 41) now: a caller whose own kernels matter more takes 3 CTAs, not 4.
+  // against 672 (55 / 42) and 632 (51 / 41) now: a caller whose own kernels matter more takes 3 CTAs, not 4.
   // Slots shorter than a slice hold less, and as many more wavefronts have the same bytes
   // under way: 48 MiB of slots of 2 KiB written 931 -> 715, read 1268 -> 677.
   const int64_t slots = (int64_t)d.bsz * d.staging_stride;
-  const int64_t shorter = std::max<int64_t>(1, std::min<int64_t>(4, 64 * kCopyUnroll * 16 / d.staging_stride));
+  const int64_t shorter = std::max<int64_t>(1, std::min<int64_t>(4, kSliceBytes / d.staging_stride));
   int grid = cta * (write_cpu ? pol.d2h_wg_per_cta : pol.h2d_wg_per_cta) * (int)shorter;
   if (!write_cpu || slots < kShortMinBytes)
     grid = grid * 3 / 2;
+  // Adjacent vectors per lane on the same terms as the fixed-size kernel: not next to a
+  // transfer from the host, where the plain order moves 2 % more in sum.  And only for calls
+  // that fill the link for a while: the loads of a slice take longer in this order, which a
+  // shorter call waits for.  Slots of 32 KiB, us, plain / adjacent: 8 MiB 128 / 133, 16 MiB 237 / 238,
+  // 48 MiB 667 / 656; of 2 KiB the same either way.  Such calls reach the link's rate with fewer wavefronts
+  // where most payloads have no whole slice and come near one: 24 and 32 take, 48 MiB of slots of 8 KiB, 672 (55 / 42) and
+  // 658 (125 / 65), of 10 KiB 674 (57 / 43) and 661 (115 / 63); of 12 KiB 32 are kept, 665 (71 / 49), with
+  // 24 675 (59 / 44).
+  const bool runs = pol.d2h_lane_runs == 2 ||
+                    (pol.d2h_lane_runs == 1 && slots >= kShortMinBytes &&
+                     !(pol.arbiter != 0 && link_direction_busy(device, /*h2d=*/true, stream)));
+  if (write_cpu && vec16 && runs && d.staging_stride >= kSliceBytes && d.staging_stride < kFewWholeSlices)
+    grid = grid * 3 / 4;
   const int threads = write_cpu ? pol.d2h_wg_threads : pol.h2d_wg_threads;
   grid = std::max(1, std::min(grid, (d.bsz + threads / 64 - 1) / (threads / 64)));
 #define FKV_LAUNCH_STAGING(...)                                                               \
   hipLaunchKernelGGL((fkv_staging_transfer_kernel<__VA_ARGS__>), dim3(grid), dim3(threads), 0,  \
                      stream, a, plan)
-  // Adjacent vectors per lane on the same terms as the fixed-size kernel: not next to a
-  // transfer from the host, where the plain order moves 2 % more in sum.  And only for calls
-  // that fill the link for a while: the loads of a slice take longer in this order, which a
-  // shorter call waits for.  Slots of 32 KiB, us, plain / adjacent: 8 MiB 128 / 133, 16 MiB 237 / 238,
-  // 48 MiB 667 / 656; of 8 and 2 KiB the same either way.
-  const bool runs = pol.d2h_lane_runs == 2 ||
-                    (pol.d2h_lane_runs == 1 && slots >= kShortMinBytes &&
-                     !(pol.arbiter != 0 && link_direction_busy(device, /*h2d=*/true, stream)));
   if (write_cpu && vec16 && runs)
     FKV_LAUNCH_STAGING(true, true, true);
   else if (write_cpu && vec16)

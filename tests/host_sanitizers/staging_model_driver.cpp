@@ -1,7 +1,7 @@
 // Payload transfers (fkv_staging_transfer) with the kernel on the CPU device model, for sanitizer
 // builds: seeded calls over slots that are and are not multiples of a vector, payloads from nothing
 // to the whole slot (ends of every number of vectors and bytes), sizes that do not fit, up to the
-// largest 64 bits hold, split batches, both directions, against the oracle byte for byte.  Staging
+// largest 64 bits hold, split batches, both directions, both orders of vectors, against the oracle byte for byte.  Staging
 // buffer, host cache, sizes and size table are allocations of exactly the size the call may touch.
 #include <hip/hip_runtime.h>
 
@@ -112,6 +112,10 @@ void call(unsigned long long seed, hipStream_t stream) {
   d.size_table_block_stride = all_layers * kv, d.size_table_layer_stride = kv;
   d.start_layer_id = start_layer, d.kv_dim = kv, d.num_blocks = blocks, d.batch_start = batch_start, d.bsz = bsz;
   d.is_write_cpu = write, d.transfer_num_cta = pick(rng, 0, 2), d.device = -1, d.sync = 1;
+  fkv_launch_policy policy{}; // the order of vectors towards the host: not a number of `rng`, whose shapes stay
+  REQUIRE(fkv_launch_policy_get(-1, &policy) == FKV_OK, "policy");
+  policy.d2h_lane_runs = seed % 3 ? 2 : 0;
+  REQUIRE(fkv_launch_policy_set(-1, &policy) == FKV_OK, "policy");
   REQUIRE(fkv_staging_transfer(&d, stream) == FKV_OK, "seed %llu: %s", seed, fkv_last_error());
   fkv_oracle_staging_transfer(staging.data(), stride, sizes.data(), host.data(), capacity,
                               counted ? overflow.data() : nullptr, kv_stride, layer_stride, block_stride,

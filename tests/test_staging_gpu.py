@@ -104,6 +104,21 @@ def test_many_payloads_in_either_order_of_vectors(gpu_device, lane_runs, size_ra
     c.check("after the writes")
 
 
+@pytest.mark.parametrize("slot", [8192, 8208, 12272, 12288])
+@pytest.mark.parametrize("size_range", [(4080, 4128), (4096, 8191), (8176, 8208)])
+def test_payloads_without_a_whole_slice_in_the_order_of_adjacent_vectors(gpu_device, slot, size_range):
+    """More than half a slice and less than one: the lane in which the payload ends, the lanes beyond
+    it, the bytes behind the last vector."""
+    from flexkv_amd.c_ext import launch_policy
+    rng = np.random.default_rng(slot + size_range[0])
+    L, NB = 3, 70
+    c = Case(gpu_device, rng, L, 1, NB, NB + 3, slot, slot, "BLOCKFIRST", size_range, L * NB)
+    with launch_policy(d2h_lane_runs=2):
+        over = c.run(0, 0, L * NB, True)
+    c.check("after the writes")
+    assert int(c.overflow.item()) == over
+
+
 def test_unaligned_addresses_take_the_byte_path(gpu_device):
     """A staging stride and a host slot that are no multiples of 16."""
     rng = np.random.default_rng(4)
